@@ -7,8 +7,10 @@
 
 #include <algorithm>
 #include <cstring>
+#include <functional>
 #include <new>
 #include <unordered_map>
+#include <utility>
 #include <vector>
 
 struct spinf_tileplan {
@@ -27,10 +29,12 @@ namespace {
 struct Blk {            // aggregates of one 32-token block
     int32_t lo, hi;     // token range [lo, hi)
     bool all_real;      // every token is a real token
-    int32_t job;        // the single job of its tokens, -2 if mixed / pads present
-    int32_t min_end, max_end;   // over all tokens (pads count as -1)
-    int64_t min_pos, max_pos;   // over real tokens
     bool any_real;
+    int32_t job;        // the single job of its tokens, -2 if mixed / pads present
+    int32_t lead;       // job of the first real token, -1 if there is none
+    int32_t first;      // lowest key any of its rows may see: where the earliest job of its rows begins
+    int32_t min_end, max_end;   // over all tokens (pads count as -1)
+    int32_t min_pos, max_pos;   // over real tokens
 };
 
 // grp_mode 1: the group term holds past the window; 2: it is windowed like the rest (scorer.py:186-198)
@@ -51,6 +55,39 @@ inline bool share(const std::vector<int32_t>& a, const std::vector<int32_t>& b) 
         if (a[i] < b[j]) i++; else j++;
     }
     return false;
+}
+
+// Does some row of R see some key of K, and does every row see every key?  The plain rule (no image groups), one key at a time: the
+// rows that see a key are a 32-bit set: its subtree's interval, the rows of its job, and on a sliding layer the rows within the window.
+// (A block pair that is partly visible, the common case here, is settled by its first two or three keys; evaluating the rule for
+// all 1,024 pairs was nine tenths of a build; 64,896 tokens, 64-key entries: 10.7 -> 1.2 ms of one host core.)
+inline void rows_of_keys(const int32_t* art, const int32_t* end, const int32_t* pos, int32_t window, const Blk& R, const Blk& K, bool* any, bool* all) {
+    const int rows = R.hi - R.lo;
+    const uint32_t full = rows == 32 ? ~0u : (1u << rows) - 1;
+    *any = false;
+    *all = rows == SPINF_SUB && K.hi - K.lo == SPINF_SUB;
+    uint32_t mates = 0;      // rows of job `job`
+    int32_t job = -1;
+    for (int32_t k = K.lo; k < K.hi && (!*any || *all); k++) {
+        uint32_t see = 0;
+        const int32_t from = std::max(k, R.lo), to = std::min(end[k], R.hi);
+        if (art[k] >= 0 && from < to) {
+            if (art[k] != job) {
+                job = art[k];
+                mates = 0;
+                if (R.job == job) mates = full;
+                else
+                    for (int i = 0; i < rows; i++) mates |= (uint32_t)(art[R.lo + i] == job) << i;
+            }
+            see = mates & (~0u << (from - R.lo)) & (~0u >> (32 - (to - R.lo)));
+            if (window > 0 && see && R.max_pos - (int64_t)pos[k] >= window)
+                for (int i = from - R.lo; i < to - R.lo; i++)
+                    if (pos[R.lo + i] - (int64_t)pos[k] >= window) see &= ~(1u << i);
+        }
+        if (k >= R.lo && k < R.hi) see |= 1u << (k - R.lo);
+        *any |= see != 0;
+        *all &= see == full;
+    }
 }
 
 }  // namespace
@@ -83,25 +120,33 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
         const int64_t nqt = (n + SPINF_QTILE - 1) / SPINF_QTILE;
         const int64_t nb = (n + SPINF_SUB - 1) / SPINF_SUB;
         std::vector<Blk> blk(nb);
+        std::unordered_map<int32_t, int32_t> first;   // first stream position of every job
+        int32_t run_job = -1, run_first = 0;
         for (int64_t b = 0; b < nb; b++) {
             Blk& B = blk[b];
             B.lo = (int32_t)(b * SPINF_SUB);
             B.hi = (int32_t)std::min<int64_t>(n, (b + 1) * SPINF_SUB);
-            B.all_real = true; B.any_real = false; B.job = -3;
-            B.min_end = INT32_MAX; B.max_end = INT32_MIN; B.min_pos = INT64_MAX; B.max_pos = INT64_MIN;
+            B.all_real = true; B.any_real = false; B.job = -3; B.lead = -1; B.first = INT32_MAX;
+            B.min_end = INT32_MAX; B.max_end = INT32_MIN; B.min_pos = INT32_MAX; B.max_pos = INT32_MIN;
             for (int32_t i = B.lo; i < B.hi; i++) {
-                const bool real = art[i] >= 0;
-                B.all_real &= real;
+                const int32_t a = art[i];
                 B.min_end = std::min(B.min_end, end[i]);
                 B.max_end = std::max(B.max_end, end[i]);
-                if (real) {
-                    B.any_real = true;
-                    B.min_pos = std::min<int64_t>(B.min_pos, pos[i]);
-                    B.max_pos = std::max<int64_t>(B.max_pos, pos[i]);
-                    if (B.job == -3) B.job = art[i]; else if (B.job != art[i]) B.job = -2;
-                } else {
+                if (a < 0) {
+                    B.all_real = false;
                     B.job = -2;
+                    continue;
                 }
+                B.min_pos = std::min(B.min_pos, pos[i]);
+                B.max_pos = std::max(B.max_pos, pos[i]);
+                if (!B.any_real) B.lead = a;
+                B.any_real = true;
+                if (B.job == -3) B.job = a; else if (B.job != a) B.job = -2;
+                if (a != run_job) {   // a job's tokens lie together: one look-up per run
+                    run_job = a;
+                    run_first = first.emplace(a, i).first->second;
+                }
+                B.first = std::min(B.first, run_first);
             }
             if (B.job == -3) B.job = -2;
         }
@@ -117,15 +162,6 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
             }
             for (auto& g : bgrp) std::sort(g.begin(), g.end());
         }
-        // first stream position of every job: the lowest key any of its rows may see
-        std::unordered_map<int32_t, int64_t> first;
-        std::vector<int64_t> jfirst(n);
-        for (int64_t i = 0; i < n; i++) {
-            if (art[i] < 0) { jfirst[i] = i; continue; }
-            auto it = first.find(art[i]);
-            if (it == first.end()) it = first.emplace(art[i], i).first;
-            jfirst[i] = it->second;
-        }
         p->qt_ptr.assign(nqt + 1, 0);
         std::vector<int64_t>& weight = p->weight;
         std::vector<int32_t>& group = p->group;
@@ -134,11 +170,12 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
         for (int64_t t = 0; t < nqt; t++) {
             const int64_t q0 = t * SPINF_QTILE, q1 = std::min<int64_t>(n, q0 + SPINF_QTILE);
             int64_t lo_key = q0, hi_key = q1;   // keys [lo_key, hi_key) can matter: the rows' jobs so far, and their groups to the end
-            for (int64_t q = q0; q < q1; q++) {
-                lo_key = std::min(lo_key, jfirst[q]);
-                if (group[t] < 0 && art[q] >= 0) group[t] = art[q];
-                if (grp && grp[q] >= 0) hi_key = std::max(hi_key, glast[grp[q]] + 1);
+            for (int64_t rb = q0 / SPINF_SUB; rb < nb && blk[rb].lo < q1; rb++) {
+                lo_key = std::min<int64_t>(lo_key, blk[rb].first);
+                if (group[t] < 0) group[t] = blk[rb].lead;
             }
+            for (int64_t q = q0; grp && q < q1; q++)
+                if (grp[q] >= 0) hi_key = std::max(hi_key, glast[grp[q]] + 1);
             for (int64_t j = lo_key / ktile; j * ktile < hi_key; j++) {
                 uint32_t bits = 0;
                 for (int w = 0; w < SPINF_QTILE / SPINF_SUB; w++) {
@@ -161,17 +198,12 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
                                     any |= v; all &= v;
                                 }
                         } else if (below && K.max_end <= R.lo) { any = false; all = false; }
-                        else if (below && W > 0 && R.any_real && K.any_real && R.min_pos - K.max_pos >= W) { any = false; all = false; }
+                        else if (below && W > 0 && R.any_real && K.any_real && (int64_t)R.min_pos - K.max_pos >= W) { any = false; all = false; }
                         else if (K.hi - 1 <= R.lo && R.all_real && K.all_real && R.job >= 0 && R.job == K.job && K.min_end >= R.hi &&
-                                 (W == 0 || R.max_pos - K.min_pos < W) && (R.hi - R.lo) == SPINF_SUB && (K.hi - K.lo) == SPINF_SUB) {
+                                 (W == 0 || (int64_t)R.max_pos - K.min_pos < W) && (R.hi - R.lo) == SPINF_SUB && (K.hi - K.lo) == SPINF_SUB) {
                             any = true; all = true;
                         } else {
-                            any = false; all = (R.hi - R.lo) == SPINF_SUB && (K.hi - K.lo) == SPINF_SUB;
-                            for (int64_t q = R.lo; q < R.hi; q++)
-                                for (int64_t k = K.lo; k < K.hi; k++) {
-                                    const bool v = visible(art, end, pos, nullptr, 0, W, q, k);
-                                    any |= v; all &= v;
-                                }
+                            rows_of_keys(art, end, pos, W, R, K, &any, &all);
                         }
                         if (any) {
                             bits |= 1u << (2 * w + s);
@@ -285,10 +317,12 @@ extern "C" int spinf_tileplan_schedule(const spinf_tileplan* p, int32_t head_gro
             auto cost = [&](int64_t i) { return cum[i + 1] - cum[i]; };
             idx.resize(hi - lo);
             for (int64_t i = lo; i < hi; i++) idx[i - lo] = (int32_t)i;
-            std::stable_sort(idx.begin(), idx.end(), [&](int32_t x, int32_t y) { return cost(x) < cost(y); });
+            // (the TAIL_ITEMS lightest in order are all that can move)
+            const size_t lightest = std::min<size_t>(idx.size(), (size_t)TAIL_ITEMS);
+            std::partial_sort(idx.begin(), idx.begin() + lightest, idx.end(), [&](int32_t x, int32_t y) { return cost(x) != cost(y) ? cost(x) < cost(y) : x < y; });
             const int64_t budget = (int64_t)(TAIL_SHARE * (double)(cum[hi] - cum[lo]));
             int64_t taken = 0, n_tail = 0;
-            while (n_tail < (int64_t)idx.size() && n_tail < TAIL_ITEMS && taken + cost(idx[n_tail]) <= budget) taken += cost(idx[n_tail++]);
+            while (n_tail < (int64_t)lightest && taken + cost(idx[n_tail]) <= budget) taken += cost(idx[n_tail++]);
             if (n_tail == 0) continue;
             moved.assign((size_t)(hi - lo), 0);
             for (int64_t j = 0; j < n_tail; j++) moved[idx[j] - lo] = 1;
@@ -319,35 +353,36 @@ extern "C" int spinf_tileplan_schedule_static(const spinf_tileplan* p, int32_t h
         std::vector<int32_t> base((size_t)std::max<int64_t>(1, nqt * head_groups) * 4);
         int32_t lp[9];
         if (int rc = spinf_tileplan_schedule(p, head_groups, base.data(), lp)) return rc;
-        const int nsub = p->ktile / SPINF_SUB;
+        // per 32-key block of an entry: does any row group see it, and how many blocks of each SIMD pair need the mask
         std::vector<float> cost(nqt, 0.f);
         for (int64_t t = 0; t < nqt; t++) {
-            float tiles = 0.f, ma = 0.f, mb = 0.f;
-            for (int32_t e = p->qt_ptr[t]; e < p->qt_ptr[t + 1]; e++) {
-                const uint32_t bits = p->kv_bits[e];
-                for (int sb = 0; sb < nsub; sb++) {
-                    bool any = false;
-                    for (int w = 0; w < 4; w++) {
-                        if (!((bits >> (2 * w + sb)) & 1u)) continue;
-                        any = true;
-                        if ((bits >> (8 + 2 * w + sb)) & 1u) (w == 0 || w == 3 ? ma : mb) += 1.f;
-                    }
-                    if (any) tiles += 1.f;
-                }
+            if (p->ktile != SPINF_SUB) {   // 64-key entries: the lockstep kernels, whose items cost what spinf_tileplan_schedule weighs them with
+                cost[t] = (float)(p->weight[t] + 15);
+                continue;
             }
-            // 64-key entries: the lockstep kernels, whose items cost what spinf_tileplan_schedule weighs them with
-            cost[t] = p->ktile == SPINF_SUB ? 3.2f + tiles + 0.3f * std::max(ma, mb) : (float)(p->weight[t] + 15);
+            int tiles = 0, ma = 0, mb = 0;
+            for (int32_t e = p->qt_ptr[t]; e < p->qt_ptr[t + 1]; e++) {
+                const uint32_t bits = p->kv_bits[e], masked = bits & (bits >> 8);
+                tiles += (bits & 0x55u) != 0;
+                ma += __builtin_popcount(masked & 0x41u);   // row groups 0 and 3
+                mb += __builtin_popcount(masked & 0x14u);   // row groups 1 and 2
+            }
+            cost[t] = 3.2f + (float)tiles + 0.3f * (float)std::max(ma, mb);
         }
+        // the workgroup of a list that is free first (the lowest numbered of equals) takes its next item: a heap per list
         const int nl = std::min<int32_t>(8, n_lists);
         std::vector<std::vector<int32_t>> mine((size_t)n_lists);
-        std::vector<float> load((size_t)n_lists, 0.f);
+        std::vector<std::vector<std::pair<float, int>>> free_at((size_t)nl);
+        for (int w = 0; w < n_lists; w++) free_at[w % nl].emplace_back(0.f, w);
+        const auto later = std::greater<std::pair<float, int>>();
+        for (auto& f : free_at) std::make_heap(f.begin(), f.end(), later);
         for (int l = 0; l < 8; l++)
             for (int64_t i = lp[l]; i < lp[l + 1]; i++) {
-                int best = -1;
-                for (int w = l % nl; w < n_lists; w += nl)
-                    if (best < 0 || load[w] < load[best]) best = w;
-                mine[best].push_back((int32_t)i);
-                load[best] += cost[base[4 * i]];
+                auto& f = free_at[l % nl];
+                std::pop_heap(f.begin(), f.end(), later);
+                mine[f.back().second].push_back((int32_t)i);
+                f.back().first += cost[base[4 * i]];
+                std::push_heap(f.begin(), f.end(), later);
             }
         int64_t k = 0;
         for (int w = 0; w < n_lists; w++) {
