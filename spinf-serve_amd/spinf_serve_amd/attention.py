@@ -62,7 +62,7 @@ def _check_tensors(q, k, v, n_mask, compact, others=()):
             raise ValueError(f"all tensors of the call must be on {q.device}, one is on {t.device}")
 
 
-def _ring_lists(q, hq, hkv, d, variant, sidx, mask):
+def _ring_lists(device, hq, hkv, d, variant, compact, mask):
     """-> (workgroups of the static schedule or 0, whether the call goes to the kernel with decoupled waves).
 
     Measured on MI355X: the decoupled kernel wins where a workgroup gets only a handful of items (C2: 6.75 per workgroup), since
@@ -75,10 +75,10 @@ def _ring_lists(q, hq, hkv, d, variant, sidx, mask):
     SPINF_ATTN_RING=1 select it)."""
     from .masks import _static_lists
 
-    n_wg = _static_lists(q.device)
-    ring = (d == 512 or (variant == 0 and d in (128, 256) and (hq // hkv) % 2 == 0)) and sidx is None and mask.grp is None
+    n_wg = _static_lists(device)
+    ring = (d == 512 or (variant == 0 and d in (128, 256) and (hq // hkv) % 2 == 0)) and not compact and mask.grp is None
     if ring and RING < 0:
-        ring = d == 512 or (d == 256 and mask.plan.n_qtiles * (hq // 2) <= RING_MAX_ITEMS_PER_WG * n_wg) or (d == 128 and RING_128)
+        ring = d == 512 or (d == 256 and mask.n_qtiles * (hq // 2) <= RING_MAX_ITEMS_PER_WG * n_wg) or (d == 128 and RING_128)
     elif not RING:
         ring = False
     static = d != 512 and STATIC > 0
@@ -139,10 +139,7 @@ def _tree_attn_op(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, art: torch.
     else:
         out = torch.empty((rows, hq, d), dtype=torch.bfloat16, device=q.device)
     a = _attn_args(q, k, v, out, n, art, end, pos, kv_idx, kv_bits, items, list_ptr, n_items, scale, window, variant, row_of, kv_row0, grp, grp_mode, ktile, n_lists)
-    lib = _lib.load_library()
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        _lib.check(lib.spinf_tree_attn_fwd(C.byref(a), C.c_void_p(stream)), "spinf_tree_attn_fwd")
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, q.device, "spinf_tree_attn_fwd")
     return out
 
 
@@ -151,13 +148,57 @@ def _(q, k, v, art, end, pos, kv_idx, kv_bits, items, list_ptr, n_items, scale, 
     return torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
 
 
+class _Layer:
+    """what the calls of one mask at one head geometry share: the schedule on the device and the argument block with everything in it
+    that does not belong to one layer's tensors (the mask owns the memory it points to)"""
+
+    def __init__(self, mask, hq, hkv, d, variant, compact, device):
+        n_lists, ring = _ring_lists(device, hq, hkv, d, variant, compact, mask)
+        if ring and d == 128:
+            variant = 3   # (64-key plan entries, as the lockstep kernels take)
+        self.ring = ring and d != 128
+        m = mask.for_head_dim(d, ring=self.ring)
+        per_item = _lib.load_library().spinf_attn_heads_per_item(hq, hkv, d, variant)
+        if per_item <= 0:
+            raise ValueError(f"{hq} query heads do not group over {hkv} key / value heads")
+        self.items, self.list_ptr, self.n_items = m.schedule(hq // per_item, n_lists)
+        self.variant, self.n_lists = variant, n_lists
+        a = self.args = _lib.AttnArgs()
+        a.n, a.hq, a.hkv, a.d, a.window = m.n, hq, hkv, d, m.window
+        a.art, a.end, a.pos = m.art.data_ptr(), m.end.data_ptr(), m.pos.data_ptr()
+        a.kv_idx, a.kv_bits, a.items, a.list_ptr = m.kv_idx.data_ptr(), m.kv_bits.data_ptr(), self.items.data_ptr(), self.list_ptr.data_ptr()
+        a.n_items, a.variant, a.ktile, a.n_lists = self.n_items, variant, m._ktile, n_lists
+        if m.grp is not None:
+            a.grp, a.grp_mode = m.grp.data_ptr(), m.grp_mode
+
+    @classmethod
+    def of(cls, mask, q, k, variant, compact):
+        hq, hkv, d = q.shape[1], k.shape[1], q.shape[2]
+        key = (hq, hkv, d, variant, compact, RING, STATIC, RING_128)
+        got = mask._layers.get(key)
+        if got is None:
+            got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, q.device)
+        return got
+
+    def bound(self, q, k, v, out, scale):
+        """the argument block of one call (a block of its own: calls may come from several threads)"""
+        a = _lib.AttnArgs.from_buffer_copy(self.args)
+        a.q, a.k, a.v, a.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
+        a.q_tok, a.q_head, _ = q.stride()
+        a.k_tok, a.k_head, _ = k.stride()
+        a.v_tok, a.v_head, _ = v.stride()
+        a.o_tok, a.o_head, _ = out.stride()
+        a.scale, a.debug_expire = scale, DEBUG_EXPIRE
+        return a
+
+
 def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
     """q [n, hq, d], k / v [n, hkv, d] bf16 -> [n, hq, d]: softmax(scale q k^T under the tree mask) v.
     sidx [R] (compact rows): q, k, v hold real tokens only, row r is stream position sidx[r]; the kernel reads and writes them
     in place of the scatter into stream layout and the gather back (rows >= R come back zero)."""
     if not isinstance(mask, TreeMask):
         raise TypeError("attention_mask must be a TreeMask (masks.block_masks)")
-    _check_tensors(q, k, v, mask.n, sidx is not None, (mask.art, mask.end, mask.pos, mask.kv_idx, mask.kv_bits, mask.grp, sidx))
+    _check_tensors(q, k, v, mask.n, sidx is not None, (mask.art, sidx))
     if sidx is not None and sidx.shape[0] > q.shape[0]:
         raise ValueError(f"sidx names {sidx.shape[0]} rows, q has {q.shape[0]}")
     scale = float(q.shape[-1] ** -0.5 if scale is None else scale)
@@ -166,19 +207,21 @@ def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
         variant = 0   # the two-heads-per-wave kernels take neither compact rows nor image groups
     if sidx is not None and mask.grp is not None:
         raise ValueError("image groups go with the stream layout (no sidx)")
-    hq, hkv, d = q.shape[1], k.shape[1], q.shape[2]
-    n_lists, ring = _ring_lists(q, hq, hkv, d, variant, sidx, mask)
-    if ring and d == 128:
-        variant = 3   # (64-key plan entries, as the lockstep kernels take)
-    mask = mask.for_head_dim(d, ring=ring and d != 128)
-    per_item = _lib.load_library().spinf_attn_heads_per_item(hq, hkv, d, variant)
-    if per_item <= 0:
-        raise ValueError(f"{hq} query heads do not group over {hkv} key / value heads")
-    items, list_ptr, n_items = mask.schedule(hq // per_item, n_lists)
-    row_of, kv_row0 = mask.rows(sidx) if sidx is not None else (None, None)
-    return _tree_attn_op(q, k, v, mask.art, mask.end, mask.pos, mask.kv_idx, mask.kv_bits, items, list_ptr, n_items,
-                         scale, int(mask.window), variant, row_of, kv_row0, 0 if sidx is None else int(sidx.shape[0]),
-                         mask.grp, int(mask.grp_mode), int(mask.plan.ktile), n_lists)
+    layer = _Layer.of(mask, q, k, variant, sidx is not None)
+    m = mask.for_head_dim(q.shape[2], ring=layer.ring)   # the plan of the kernel's key-tile size
+    row_of, kv_row0 = m.rows(sidx) if sidx is not None else (None, None)
+    if not _lib.eager(q, k, v, sidx):
+        return _tree_attn_op(q, k, v, m.art, m.end, m.pos, m.kv_idx, m.kv_bits, layer.items, layer.list_ptr, layer.n_items,
+                             scale, int(m.window), layer.variant, row_of, kv_row0, 0 if sidx is None else int(sidx.shape[0]),
+                             m.grp, int(m.grp_mode), int(m._ktile), layer.n_lists)
+    out = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
+    a = layer.bound(q, k, v, out, scale)
+    if sidx is not None:
+        if sidx.shape[0] < q.shape[0]:
+            out[sidx.shape[0] :].zero_()
+        a.row_of, a.kv_row0 = row_of.data_ptr(), kv_row0.data_ptr()
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, q.device, "spinf_tree_attn_fwd")
+    return out
 
 
 def tree_attn_noalloc(q, k, v, mask: TreeMask, out, scale=None):
@@ -190,23 +233,9 @@ def tree_attn_noalloc(q, k, v, mask: TreeMask, out, scale=None):
         raise TypeError("attention_mask must be a TreeMask (masks.block_masks)")
     if out.shape != q.shape or out.dtype != torch.bfloat16 or not out.is_contiguous():
         raise ValueError("out must be a contiguous bf16 tensor of q's shape")
-    _check_tensors(q, k, v, mask.n, False, (out, mask.art, mask.end, mask.pos, mask.kv_idx, mask.kv_bits, mask.grp))
-    n, hq, d = q.shape
-    hkv = k.shape[1]
-    n_lists, ring = _ring_lists(q, hq, hkv, d, 0, None, mask)
-    variant = 3 if ring and d == 128 else 0
-    mask = mask.for_head_dim(d, ring=ring and d != 128)
-    per_item = _lib.load_library().spinf_attn_heads_per_item(hq, hkv, d, variant)
-    if per_item <= 0:
-        raise ValueError(f"{hq} query heads do not group over {hkv} key / value heads")
-    items, list_ptr, n_items = mask.schedule(hq // per_item, n_lists)
-    scale = float(d ** -0.5 if scale is None else scale)
-    a = _attn_args(q, k, v, out, n, mask.art, mask.end, mask.pos, mask.kv_idx, mask.kv_bits, items, list_ptr, n_items, scale, int(mask.window), variant,
-                   None, None, mask.grp, int(mask.grp_mode), int(mask.plan.ktile), n_lists)
-    lib = _lib.load_library()
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        _lib.check(lib.spinf_tree_attn_fwd_noalloc(C.byref(a), C.c_void_p(stream)), "spinf_tree_attn_fwd_noalloc")
+    _check_tensors(q, k, v, mask.n, False, (out, mask.art))
+    a = _Layer.of(mask, q, k, 0, False).bound(q, k, v, out, float(q.shape[-1] ** -0.5 if scale is None else scale))
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd_noalloc, a, q.device, "spinf_tree_attn_fwd_noalloc")
     return out
 
 

@@ -3,27 +3,30 @@
 
 A TreeMask holds the stream's art / end / pos on the device and, instead of FlexAttention's nb x nb block tables
 (spinf_serve/packer.py:426-491), a compact per-query-tile list of visible key tiles compiled on the host by the
-library's tile-plan compiler.  No dense mask is built anywhere.
+library's tile-plan compiler: for the window and the key-tile size the layers ask for, at the first layer that asks (a pass
+whose global layers have 512-dim heads never compiles the 64-key plan of its global mask).  No dense mask is built anywhere.
 """
 
 from __future__ import annotations
 
 import ctypes as C
+import weakref
+
 import numpy as np
 
 from . import _lib
 
 
 class TilePlan:
-    """host arrays of a compiled plan (see include/spinf_tree.h) and the native handle that makes its work lists"""
+    """a compiled plan (see include/spinf_tree.h): the native handle, and on first use its host arrays qt_ptr, kv_idx, kv_bits, order"""
 
-    def __init__(self, handle, qt_ptr, kv_idx, kv_bits, order, n, window, active_blocks, masked_blocks, grp_mode=0, ktile=64):
+    def __init__(self, handle, counts, n, window, grp_mode=0, ktile=64):
         self._handle = handle
         self.ktile = ktile
-        self.qt_ptr, self.kv_idx, self.kv_bits, self.order = qt_ptr, kv_idx, kv_bits, order
+        self.n_qtiles, self.n_entries, self.active_blocks, self.masked_blocks = (int(c) for c in counts[:4])
         self.n, self.window, self.grp_mode = n, window, grp_mode
-        self.active_blocks, self.masked_blocks = active_blocks, masked_blocks
         self._schedules = {}
+        self._arrays = None
 
     def __del__(self):
         h, self._handle = getattr(self, "_handle", None), None
@@ -38,116 +41,151 @@ class TilePlan:
         """grp (image groups, spinf_serve/scorer.py:184-198): [n] int32, -1 none; the tokens of a group also see each other both
         ways, past the window unless grp_windowed.  ktile: keys per entry, 64, or 32 for the head dim 512 kernel."""
         lib = _lib.load_library()
-        art = np.ascontiguousarray(art, np.int32)
-        end = np.ascontiguousarray(end, np.int32)
-        pos = np.ascontiguousarray(pos, np.int32)
+        art, end, pos, grp = _host_arrays(art, end, pos, grp)
         n = len(art)
-        if len(end) != n or len(pos) != n:
-            raise ValueError("art, end and pos differ in length")
         w = int(window) if window else 0
         h = C.c_void_p()
-        mode = 0
-        gptr = None
-        if grp is not None:
-            grp = np.ascontiguousarray(grp, np.int32)
-            if len(grp) != n:
-                raise ValueError("grp differs in length from art")
-            mode = 2 if grp_windowed else 1
-            gptr = grp.ctypes.data
-        _lib.check(lib.spinf_tileplan_build_ktile(art.ctypes.data, end.ctypes.data, pos.ctypes.data, gptr, mode, n, w, int(ktile), C.byref(h)),
-                   "tileplan_build")
-        try:
-            counts = (C.c_int64 * 5)()
-            _lib.check(lib.spinf_tileplan_counts(h, counts), "tileplan_counts")
-            nqt, nent = int(counts[0]), int(counts[1])
-            qt_ptr = np.zeros(nqt + 1, np.int32)
-            kv_idx = np.zeros(max(nent, 1), np.int32)
-            kv_bits = np.zeros(max(nent, 1), np.uint32)
-            order = np.zeros(max(nqt, 1), np.int32)
-            _lib.check(lib.spinf_tileplan_export(h, qt_ptr.ctypes.data, kv_idx.ctypes.data, kv_bits.ctypes.data, order.ctypes.data), "tileplan_export")
-        except Exception:
-            lib.spinf_tileplan_free(h)
-            raise
-        return cls(h, qt_ptr, kv_idx[:nent], kv_bits[:nent], order[:nqt], n, w, int(counts[2]), int(counts[3]), mode, int(ktile))
+        mode = 0 if grp is None else 2 if grp_windowed else 1
+        _lib.check(lib.spinf_tileplan_build_ktile(art.ctypes.data, end.ctypes.data, pos.ctypes.data, None if grp is None else grp.ctypes.data, mode, n, w,
+                                                  int(ktile), C.byref(h)), "tileplan_build")
+        counts = (C.c_int64 * 5)()
+        _lib.check(lib.spinf_tileplan_counts(h, counts), "tileplan_counts")
+        return cls(h, counts, n, w, mode, int(ktile))
 
-    @property
-    def n_qtiles(self) -> int:
-        return len(self.order)
+    def export(self, qt_ptr, kv_idx, kv_bits, order) -> None:
+        """the plan's arrays into host memory at these addresses (qt_ptr [n_qtiles + 1], kv_idx / kv_bits [entries], order [n_qtiles])"""
+        _lib.check(_lib.load_library().spinf_tileplan_export(self._handle, qt_ptr, kv_idx, kv_bits, order), "tileplan_export")
+
+    def _array(self, i):
+        if self._arrays is None:
+            out = [np.zeros(max(k, 1), t) for k, t in ((self.n_qtiles + 1, np.int32), (self.n_entries, np.int32), (self.n_entries, np.uint32), (self.n_qtiles, np.int32))]
+            self.export(*(x.ctypes.data for x in out))
+            self._arrays = [out[0], out[1][: self.n_entries], out[2][: self.n_entries], out[3][: self.n_qtiles]]
+        return self._arrays[i]
+
+    qt_ptr = property(lambda self: self._array(0))
+    kv_idx = property(lambda self: self._array(1))
+    kv_bits = property(lambda self: self._array(2))
+    order = property(lambda self: self._array(3))
+
+    def schedule_into(self, head_groups: int, n_lists: int, items, list_ptr) -> None:
+        """the work lists into host memory at these addresses: items [4 n_qtiles head_groups], list_ptr [9] or, for a static schedule
+        (n_lists > 0), [n_lists + 1]"""
+        lib = _lib.load_library()
+        if n_lists:
+            _lib.check(lib.spinf_tileplan_schedule_static(self._handle, head_groups, n_lists, items, list_ptr), "tileplan_schedule_static")
+        else:
+            _lib.check(lib.spinf_tileplan_schedule(self._handle, head_groups, items, list_ptr), "tileplan_schedule")
+
+    def _schedule(self, head_groups: int, n_lists: int):
+        got = self._schedules.get((head_groups, n_lists))
+        if got is None:
+            items = np.zeros((max(self.n_qtiles * head_groups, 1), 4), np.int32)
+            list_ptr = np.zeros((n_lists or 8) + 1, np.int32)
+            self.schedule_into(head_groups, n_lists, items.ctypes.data, list_ptr.ctypes.data)
+            got = self._schedules[(head_groups, n_lists)] = (items[: self.n_qtiles * head_groups], list_ptr)
+        return got
 
     def schedule(self, head_groups: int):
         """-> (items [n_qtiles * head_groups, 4] int32, list_ptr [9] int32): the kernel's work lists"""
-        got = self._schedules.get(head_groups)
-        if got is None:
-            items = np.zeros((max(self.n_qtiles * head_groups, 1), 4), np.int32)
-            list_ptr = np.zeros(9, np.int32)
-            _lib.check(_lib.load_library().spinf_tileplan_schedule(self._handle, head_groups, items.ctypes.data, list_ptr.ctypes.data), "tileplan_schedule")
-            got = self._schedules[head_groups] = (items[: self.n_qtiles * head_groups], list_ptr)
-        return got
+        return self._schedule(head_groups, 0)
 
     def schedule_static(self, head_groups: int, n_lists: int):
         """-> (items [n_qtiles * head_groups, 4] int32, list_ptr [n_lists + 1] int32): the items dealt out to n_lists workgroups
         ahead of the launch (the kernel with decoupled waves)"""
-        got = self._schedules.get((head_groups, n_lists))
-        if got is None:
-            items = np.zeros((max(self.n_qtiles * head_groups, 1), 4), np.int32)
-            list_ptr = np.zeros(n_lists + 1, np.int32)
-            _lib.check(_lib.load_library().spinf_tileplan_schedule_static(self._handle, head_groups, n_lists, items.ctypes.data, list_ptr.ctypes.data),
-                       "tileplan_schedule_static")
-            got = self._schedules[(head_groups, n_lists)] = (items[: self.n_qtiles * head_groups], list_ptr)
-        return got
+        return self._schedule(head_groups, n_lists)
+
+
+def _host_arrays(art, end, pos, grp=None):
+    art, end, pos = (np.ascontiguousarray(a, np.int32) for a in (art, end, pos))
+    if len(end) != len(art) or len(pos) != len(art):
+        raise ValueError("art, end and pos differ in length")
+    if grp is not None:
+        grp = np.ascontiguousarray(grp, np.int32)
+        if len(grp) != len(art):
+            raise ValueError("grp differs in length from art")
+    return art, end, pos, grp
+
+
+_CUS: dict = {}   # compute units by device index
 
 
 def _static_lists(device) -> int:
     """workgroups of a static schedule on this device: one per compute unit"""
     import torch
 
-    return int(torch.cuda.get_device_properties(device).multi_processor_count)
+    got = _CUS.get(device.index)
+    if got is None:
+        got = _CUS[device.index] = int(torch.cuda.get_device_properties(device).multi_processor_count)
+    return got
 
 
-def _upload(a, dtype, device):
+def _staging(n: int, device):
+    """-> host tensor of n int32, in pinned memory where it is to be copied to a GPU"""
     import torch
 
-    t = torch.from_numpy(np.ascontiguousarray(a, dtype))
-    if device.type == "cuda":
-        t = t.pin_memory().to(device, non_blocking=True)
-    return t
+    return torch.empty(n, dtype=torch.int32, pin_memory=device.type == "cuda")
 
 
 class TreeMask:
-    """Device-side handle: the stream's metadata + one compiled plan.  ``seq_lengths`` mirrors BlockMask.seq_lengths
-    (spinf_serve/models/qwen35/qwen.py:615 reads it)."""
+    """Device-side handle: the stream's metadata, and per key-tile size a plan compiled when the first call that takes it comes (a
+    forward's layers share it).  ``seq_lengths`` mirrors BlockMask.seq_lengths (spinf_serve/models/qwen35/qwen.py:615 reads it)."""
 
-    def __init__(self, plan: TilePlan, meta, device, grp=None, host=None):
-        self.plan = plan
-        self._host = host                   # (art, end, pos, grp, grp_windowed) on the host, for a plan of another key-tile size
-        self._other = None
-        self.grp = grp                      # device copy of the image groups the plan was built with, or None
-        self.grp_mode = plan.grp_mode if grp is not None else 0
-        self.n = plan.n
-        self.window = plan.window
-        self.seq_lengths = (plan.n, plan.n)
+    def __init__(self, plan, meta, device, grp=None, host=None, window=None, ktile=64):
+        """plan: a compiled plan, or None: compiled from host = (art, end, pos, grp or None, grp_windowed) for this window and ktile"""
+        self._host = host
+        self._plan = plan
+        self._ktile = plan.ktile if plan is not None else ktile
+        self._other = None                  # the same mask with the other key-tile size
+        self.grp = grp                      # device copy of the image groups, or None
+        self.grp_mode = 0 if grp is None else plan.grp_mode if plan is not None else 2 if host[4] else 1
+        self.n = plan.n if plan is not None else len(host[0])
+        self.window = plan.window if plan is not None else int(window) if window else 0
+        self.seq_lengths = (self.n, self.n)
         self.device = device
         self.art, self.end, self.pos = meta
-        one = np.zeros(1, np.int32)
-        self.kv_idx = _upload(plan.kv_idx if len(plan.kv_idx) else one, np.int32, device)
-        self.kv_bits = _upload((plan.kv_bits if len(plan.kv_bits) else one.view(np.uint32)).view(np.int32), np.int32, device)
+        self._kv = None                     # device copies of the plan's kv_idx, kv_bits
         self._sched = {}
+        self._layers = {}                   # prepared calls by head geometry (attention.py)
         self._rows = None
+
+    @property
+    def plan(self) -> TilePlan:
+        if self._plan is None:
+            art, end, pos, grp, grp_windowed = self._host
+            self._plan = TilePlan.build(art, end, pos, self.window, grp, grp_windowed, self._ktile)
+        return self._plan
+
+    @property
+    def n_qtiles(self) -> int:
+        return -(-self.n // 128)
+
+    @property
+    def kv_idx(self):
+        return self._entries()[0]
+
+    @property
+    def kv_bits(self):
+        return self._entries()[1]
+
+    def _entries(self):
+        if self._kv is None:
+            self._upload(1, 0)
+        return self._kv
 
     def for_head_dim(self, d: int, ring: bool = False) -> "TreeMask":
         """the mask with the plan granularity the kernel takes: 32-key entries at head dim 512 and for the kernel with decoupled
-        waves (ring), 64-key ones otherwise (the second plan is compiled on first use and shares the device metadata)"""
+        waves (ring), 64-key ones otherwise (each plan is compiled on first use; both share the device metadata)"""
         ktile = 32 if d == 512 or ring else 64
-        if ktile == self.plan.ktile:
+        if ktile == self._ktile:
             return self
-        if self._other is None:
+        other = self._other() if isinstance(self._other, weakref.ref) else self._other
+        if other is None:
             if self._host is None:
-                raise ValueError(f"this mask was built for key tiles of {self.plan.ktile}; head dim {d} takes {ktile}")
-            art, end, pos, grp, grp_windowed = self._host
-            plan = TilePlan.build(art, end, pos, self.window, grp, grp_windowed, ktile)
-            self._other = TreeMask(plan, (self.art, self.end, self.pos), self.device, self.grp)
-            self._other._other = self
-        return self._other
+                raise ValueError(f"this mask was built for key tiles of {self._ktile}; head dim {d} takes {ktile}")
+            other = self._other = TreeMask(None, (self.art, self.end, self.pos), self.device, self.grp, self._host, self.window, ktile)
+            other._other = weakref.ref(self)   # (no cycle: a pass's masks go, and give their device memory back, with the last reference)
+        return other
 
     def rows(self, sidx):
         """compact rows (spinf_serve/models/qwen35/qwen.py:613-622): sidx [R] = stream position of each real row (a device
@@ -161,7 +199,7 @@ class TreeMask:
         n = self.n
         row_of = torch.full((n + 63,), -1, dtype=torch.int32, device=self.device)   # padded: every key tile is 64 long
         row_of[sidx.to(self.device, torch.long)] = torch.arange(sidx.shape[0], dtype=torch.int32, device=self.device)
-        kt = self.plan.ktile
+        kt = self._ktile
         tiles = row_of[: (n + kt - 1) // kt * kt].view(-1, kt)
         run = (tiles - tiles[:, :1]) == torch.arange(kt, dtype=torch.int32, device=self.device)
         tile_row0 = torch.where((tiles[:, 0] >= 0) & run.all(1), tiles[:, 0], torch.full_like(tiles[:, 0], -1))
@@ -169,30 +207,51 @@ class TreeMask:
         self._rows = (sidx, row_of[:n].contiguous(), kv_row0)
         return self._rows[1], self._rows[2]
 
+    def _upload(self, head_groups: int, n_lists: int):
+        """one staging buffer, one copy: items | list_ptr and, with the plan's first schedule, kv_idx | kv_bits.  (A copy per array, each
+        from pinned memory of its own, was 11 copies and 150 us of a new stream's two masks.)"""
+        plan, first = self.plan, self._kv is None
+        ni, nl, ne, nq = 4 * max(plan.n_qtiles * head_groups, 1), (n_lists or 8) + 1, max(plan.n_entries, 1), plan.n_qtiles
+        at = [0, ni, ni + nl, ni + nl + ne, ni + nl + 2 * ne]   # items (16-byte aligned), list_ptr, kv_idx, kv_bits, host only: qt_ptr, order
+        used = at[4] if first else at[2]
+        buf = _staging(at[4] + 2 * nq + 1 if first else at[2], self.device)
+        p = buf.data_ptr()
+        plan.schedule_into(head_groups, n_lists, p, p + 4 * at[1])
+        if first:
+            plan.export(p + 4 * at[4], p + 4 * at[2], p + 4 * at[3], p + 4 * (at[4] + nq + 1))
+        dev = buf[:used].to(self.device, non_blocking=True)
+        if first:
+            self._kv = dev[at[2] : at[3]], dev[at[3] : at[4]]
+        got = self._sched[(head_groups, n_lists)] = (dev[:ni].view(-1, 4), dev[ni : at[2]], plan.n_qtiles * head_groups)
+        return got
+
     def schedule(self, head_groups: int, n_lists: int = 0):
         """device copy of the work lists for this many head groups (built on first use, then kept); n_lists > 0: the static
         schedule for that many workgroups"""
-        got = self._sched.get((head_groups, n_lists))
-        if got is None:
-            items, list_ptr = self.plan.schedule_static(head_groups, n_lists) if n_lists else self.plan.schedule(head_groups)
-            if not len(items):
-                items = np.zeros((1, 4), np.int32)
-            got = self._sched[(head_groups, n_lists)] = (_upload(items, np.int32, self.device), _upload(list_ptr, np.int32, self.device), self.plan.n_qtiles * head_groups)
-        return got
+        return self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
 
     @classmethod
     def build(cls, art, end, pos, window=None, device="cuda", meta=None, grp=None, grp_windowed=False, grp_dev=None):
-        """compile the plan on the host and upload it; ``meta``: device art / end / pos tensors to share with another mask;
-        grp: image groups (see TilePlan.build), grp_dev: their device copy to share"""
+        """the handle of a stream: its metadata is copied to the device; ``meta``: device art / end / pos tensors to share with another
+        mask; grp: image groups (see TilePlan.build), grp_dev: their device copy to share"""
         import torch
 
         device = torch.device(device)
-        if meta is None:
-            meta = tuple(_upload(a, np.int32, device) for a in (art, end, pos))
-        if grp is not None and grp_dev is None:
-            grp_dev = _upload(grp, np.int32, device)
-        return cls(TilePlan.build(art, end, pos, window, grp, grp_windowed), meta, device, grp_dev if grp is not None else None,
-                   host=(art, end, pos, grp, grp_windowed))
+        host = _host_arrays(art, end, pos, grp)
+        n = len(host[0])
+        given = [i for i in range(4) if host[i] is not None and not (grp_dev is not None if i == 3 else meta is not None)]
+        if given:
+            buf = _staging(len(given) * n, device).view(len(given), n)
+            rows = buf.numpy()
+            for r, i in enumerate(given):
+                rows[r] = host[i]
+            host = tuple(rows[given.index(i)] if i in given else h for i, h in enumerate(host))   # (the caller may reuse its arrays)
+            dev = buf.to(device, non_blocking=True)
+            if meta is None:
+                meta = tuple(dev[:3])
+            if 3 in given:
+                grp_dev = dev[-1]
+        return cls(None, meta, device, grp_dev if grp is not None else None, (*host, grp_windowed), window)
 
 
 def block_masks(batch, sliding_window=None, device="cuda", grp=None, bidir_all=True):
@@ -205,7 +264,9 @@ def block_masks(batch, sliding_window=None, device="cuda", grp=None, bidir_all=T
     full = TreeMask.build(batch.art, batch.end, batch.pos, None, device, grp=grp if bidir_all else None)
     if not sliding_window:
         return {"full_attention": full, "sliding_attention": full}
-    grp_dev = full.grp if grp is not None else None
-    slid = TreeMask.build(batch.art, batch.end, batch.pos, sliding_window, device, meta=(full.art, full.end, full.pos), grp=grp,
-                          grp_windowed=not bidir_all, grp_dev=grp_dev)
+    meta = (full.art, full.end, full.pos)
+    if grp is None or bidir_all:
+        slid = TreeMask(None, meta, full.device, full.grp, full._host, sliding_window)
+    else:
+        slid = TreeMask.build(*full._host[:3], sliding_window, device, meta=meta, grp=grp, grp_windowed=True)
     return {"full_attention": full, "sliding_attention": slid}
