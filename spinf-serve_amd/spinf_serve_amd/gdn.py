@@ -9,7 +9,6 @@ q and k arrive l2-normalised; g is the log decay (fp32), beta the write strength
 
 from __future__ import annotations
 
-import ctypes as C
 from typing import Optional
 
 import torch
@@ -33,7 +32,8 @@ def _run(mode, q, k, v, g, beta, scale, cu, n, h0, h0_idx, ht, ht_idx, idx, o, m
     beta = beta if beta.dtype == torch.bfloat16 else beta.to(torch.bfloat16)
     if o is None:
         o = torch.zeros_like(v) if idx is not None else torch.empty_like(v)
-    _gdn_scan_op(mode, q, k, v, g, beta, float(scale), cu, int(n), h0, h0_idx, ht, ht_idx, idx, o, int(max_len))
+    run = _launch if _lib.eager(q, k, v, g, beta, h0, ht, o) else _gdn_scan_op
+    run(mode, q, k, v, g, beta, float(scale), cu, int(n), h0, h0_idx, ht, ht_idx, idx, o, int(max_len))
     return o
 
 
@@ -68,10 +68,7 @@ def _launch(mode, q, k, v, g, beta, scale, cu, n, h0, h0_idx, ht, ht_idx, idx, o
     a.ht = ht.data_ptr() if (ht is not None and ht_idx is not None) else None
     a.ht_idx = ht_idx.data_ptr() if (ht is not None and ht_idx is not None) else None
     a.mode = mode
-    lib = _lib.load_library()
-    with torch.cuda.device(q.device):
-        stream = torch.cuda.current_stream(q.device).cuda_stream
-        _lib.check(lib.spinf_gdn_fwd(C.byref(a), C.c_void_p(stream)), "spinf_gdn_fwd")
+    _lib.launch(_lib.load_library().spinf_gdn_fwd, a, q.device, "spinf_gdn_fwd")
     return o
 
 

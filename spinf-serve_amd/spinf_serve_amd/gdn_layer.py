@@ -10,15 +10,12 @@ y is the input projection's output [T, conv_dim + hv dv + 2 hv] (q k v | z | b |
 
 from __future__ import annotations
 
-import ctypes as C
-
 import torch
 
 from . import _lib
 
 
-@torch.library.custom_op("spinf::gdn_prologue", mutates_args=())
-def _prologue_op(y: torch.Tensor, conv: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
+def _prologue(y: torch.Tensor, conv: torch.Tensor, conv_w: torch.Tensor, a_log: torch.Tensor, dt_bias: torch.Tensor,
                  h: int, hv: int, dk: int, dv: int, normalize: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     if not y.is_cuda:
         raise RuntimeError("spinf::gdn_prologue runs on ROCm device tensors only (no CPU path)")
@@ -47,10 +44,11 @@ def _prologue_op(y: torch.Tensor, conv: torch.Tensor, conv_w: torch.Tensor, a_lo
     a.conv, a.conv_w, a.a_log, a.dt_bias = conv.data_ptr(), conv_w.data_ptr(), a_log.data_ptr(), dt_bias.data_ptr()
     a.q, a.k, a.v, a.g, a.beta = q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr()
     a.T, a.h, a.hv, a.dk, a.dv, a.normalize = T, h, hv, dk, dv, int(normalize)
-    lib = _lib.load_library()
-    with torch.cuda.device(dev):
-        _lib.check(lib.spinf_gdn_prologue(C.byref(a), C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)), "spinf_gdn_prologue")
+    _lib.launch(_lib.load_library().spinf_gdn_prologue, a, dev, "spinf_gdn_prologue")
     return q, k, v, g, beta
+
+
+_prologue_op = torch.library.custom_op("spinf::gdn_prologue", _prologue, mutates_args=())
 
 
 @_prologue_op.register_fake
@@ -63,11 +61,11 @@ def _(y, conv, conv_w, a_log, dt_bias, h, hv, dk, dv, normalize):
 
 def gdn_prologue(y, conv, conv_w, a_log, dt_bias, h, hv, dk, dv, normalize=True):
     """-> q, k [T, h, dk], v [T, hv, dv] bf16, g [T, hv] fp32, beta [T, hv] bf16   (qwen.py:657-668 in one pass over y)"""
-    return _prologue_op(y, conv, conv_w, a_log, dt_bias, int(h), int(hv), int(dk), int(dv), bool(normalize))
+    run = _prologue if _lib.eager(y, conv_w, a_log, dt_bias) else _prologue_op
+    return run(y, conv, conv_w, a_log, dt_bias, int(h), int(hv), int(dk), int(dv), bool(normalize))
 
 
-@torch.library.custom_op("spinf::gdn_gate", mutates_args=())
-def _gate_op(o: torch.Tensor, z: torch.Tensor, norm_w: torch.Tensor, eps: float) -> torch.Tensor:
+def _gate(o: torch.Tensor, z: torch.Tensor, norm_w: torch.Tensor, eps: float) -> torch.Tensor:
     if not o.is_cuda:
         raise RuntimeError("spinf::gdn_gate runs on ROCm device tensors only (no CPU path)")
     if o.dtype != torch.bfloat16 or z.dtype != torch.bfloat16 or o.dim() != 3:
@@ -80,10 +78,11 @@ def _gate_op(o: torch.Tensor, z: torch.Tensor, norm_w: torch.Tensor, eps: float)
     a = _lib.GdnGateArgs()
     a.o, a.o_tok, a.z, a.z_tok, a.norm_w, a.eps = o.data_ptr(), o.stride(0), z.data_ptr(), z.stride(0), norm_w.data_ptr(), eps
     a.out, a.T, a.hv, a.dv = out.data_ptr(), T, hv, dv
-    lib = _lib.load_library()
-    with torch.cuda.device(o.device):
-        _lib.check(lib.spinf_gdn_gate(C.byref(a), C.c_void_p(torch.cuda.current_stream(o.device).cuda_stream)), "spinf_gdn_gate")
+    _lib.launch(_lib.load_library().spinf_gdn_gate, a, o.device, "spinf_gdn_gate")
     return out
+
+
+_gate_op = torch.library.custom_op("spinf::gdn_gate", _gate, mutates_args=())
 
 
 @_gate_op.register_fake
@@ -93,4 +92,4 @@ def _(o, z, norm_w, eps):
 
 def gdn_gate(o, z, norm_w, eps):
     """o [T, hv, dv], z [T, hv dv] (a column range of y is fine) -> [T, hv dv]: norm_w * rms_norm(o) * silu(z)   (qwen.py:670-672)"""
-    return _gate_op(o, z, norm_w, float(eps))
+    return (_gate if _lib.eager(o, z, norm_w) else _gate_op)(o, z, norm_w, float(eps))

@@ -43,6 +43,7 @@ class TreePlan:
     seg_slot: object | None = None
     cap: dict | None = None
     pad_rows: object | None = None   # [pads] int64 (device): rows of the tensors no segment covers; their outputs are zero
+    launches: list | None = None     # indexed path: per level the kernel launches (tuples for gdn.launch), neighbouring calls of one kind as one
 
 
 _PATHS = {"indexed": 0, "levels": 1}
@@ -87,28 +88,59 @@ def tree_plan(prev, real, device, max_init: int = 96, path: str = "indexed", sho
     a = _compile(prev, real, path, short, call_tokens, max_init, rows, keep)
     dev = torch.device(device)
 
-    def up(x):
-        return torch.from_numpy(np.ascontiguousarray(x)).to(dev, non_blocking=True)
-
     indexed = path == "indexed"
-    levels = []
-    for d in range(len(a["level_ptr"]) - 1):
+    seg_len, call_kind, call_keep = a["seg_len"], a["call_kind"], a["call_keep"]
+    seg_ptr, row_ptr, level_ptr = a["call_seg_ptr"].tolist(), a["call_row_ptr"].tolist(), a["level_ptr"].tolist()
+    # A call's cumulative lengths, and those of the run of neighbouring calls of one kind and level that it belongs to: the indexed
+    # path cuts a level's long segments into calls of call_tokens tokens (which bounded the reference's per-chunk snapshots), but the
+    # kernel keeps none and wants all the segments of a level at once: 8 calls of 4 segments x 32 heads fill half the GPU eight times.
+    runs = []   # per level: (first call, one past the last)
+    for d in range(len(level_ptr) - 1):
+        cuts = [c for c in range(level_ptr[d], level_ptr[d + 1]) if c == level_ptr[d] or call_kind[c] != call_kind[c - 1]] + [level_ptr[d + 1]]
+        runs.append(list(zip(cuts[:-1], cuts[1:])))
+    total = np.concatenate([[0], np.cumsum(seg_len)]).astype(np.int64)
+    spans = [(c, c + 1) for c in range(len(call_kind))] + [r for lv in runs for r in lv if indexed and r[1] - r[0] > 1]
+    cu_host = torch.from_numpy(np.concatenate([total[seg_ptr[i] : seg_ptr[j] + 1] - total[seg_ptr[i]] for i, j in spans]) if spans else np.zeros(0, np.int64))
+    cu_at = np.concatenate([[0], np.cumsum([seg_ptr[j] - seg_ptr[i] + 1 for i, j in spans])]).astype(np.int64).tolist()
+    # everything the kernels read, in one copy
+    sidx_host = np.flatnonzero(real) if rows is not None else np.zeros(0, np.int64)
+    parts = [a["conv"], a["idx"], a["h0_idx"], a["ht_idx"], cu_host.numpy(), sidx_host, np.flatnonzero(a["seg_of_row"] < 0)]
+    at = np.concatenate([[0], np.cumsum([-(-len(x) // 2) * 2 for x in parts])]).tolist()   # (each part 16-byte aligned)
+    stage = torch.empty(at[-1], dtype=torch.int64, pin_memory=dev.type == "cuda")
+    host = stage.numpy()
+    for x, o in zip(parts, at):
+        host[o : o + len(x)] = x
+    on_dev = stage.to(dev, non_blocking=True)
+    conv, idx_all, h0_all, ht_all, cu_all, sidx, pad_rows = (on_dev[o : o + len(x)] for x, o in zip(parts, at))
+    cu_of = {span: k for k, span in enumerate(spans)}
+
+    def cut(i, j):
+        """calls i .. j - 1 as one: rows, cumulative lengths (device, host), start and end slots"""
+        k = cu_of[(i, j)]
+        seg, row = slice(seg_ptr[i], seg_ptr[j]), slice(row_ptr[i], row_ptr[j])
+        return idx_all[row], cu_all[cu_at[k] : cu_at[k + 1]], cu_host[cu_at[k] : cu_at[k + 1]], h0_all[seg], ht_all[seg]
+
+    levels, launches = [], []
+    for d, lv in enumerate(runs):
         calls = []
-        for c in range(a["level_ptr"][d], a["level_ptr"][d + 1]):
-            s0, s1 = a["call_seg_ptr"][c], a["call_seg_ptr"][c + 1]
-            cu = torch.from_numpy(np.concatenate([[0], np.cumsum(a["seg_len"][s0:s1])]).astype(np.int64))
-            idx = up(a["idx"][a["call_row_ptr"][c] : a["call_row_ptr"][c + 1]])
-            starts = None if d == 0 else up(a["h0_idx"][s0:s1])
+        for c in range(level_ptr[d], level_ptr[d + 1]):
+            idx, cu, cu_cpu, starts, ends = cut(c, c + 1)
+            starts = None if d == 0 else starts
             if indexed:
-                ends = up(a["ht_idx"][s0:s1]) if a["call_keep"][c] else None
-                calls.append(Call(idx, cu.to(dev, non_blocking=True), cu, None, False, "chunked" if a["call_kind"][c] else "recurrent", starts, ends))
+                calls.append(Call(idx, cu, cu_cpu, None, False, "chunked" if call_kind[c] else "recurrent", starts, ends if call_keep[c] else None))
             else:
-                calls.append(Call(idx, cu.to(dev, non_blocking=True), cu, starts, bool(a["call_keep"][c])))
+                calls.append(Call(idx, cu, cu_cpu, starts, bool(call_keep[c])))
         levels.append(calls)
+        merged = []
+        for i, j in lv:
+            idx, cu, _, starts, ends = cut(i, j) if indexed else (None,) * 5
+            if indexed:
+                lens = seg_len[seg_ptr[i] : seg_ptr[j]]
+                merged.append((int(call_kind[i]), cu, len(lens), starts if d else None, ends if call_keep[i:j].any() else None, idx, int(lens.max()) if call_kind[i] else 0))
+        launches.append(merged)
     seg_of_row = a["seg_of_row"]
-    sidx = up(np.flatnonzero(real)) if rows is not None else None
-    return TreePlan(up(a["conv"].reshape(-1, 4)), levels, a["n_segments"], path, a["n_keep"].tolist() if indexed else None, rows, sidx, seg_of_row,
-                    a["seg_level"], a["seg_slot"], pad_rows=up(np.flatnonzero(seg_of_row < 0)))
+    return TreePlan(conv.view(-1, 4), levels, a["n_segments"], path, a["n_keep"].tolist() if indexed else None, rows, sidx if rows is not None else None, seg_of_row,
+                    a["seg_level"], a["seg_slot"], pad_rows=pad_rows, launches=launches if indexed else None)
 
 
 def _kept_state_requests(plan: TreePlan, cap):
@@ -150,11 +182,16 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
     g32 = g if g.dtype == torch.float32 else g.float()
     b16 = beta if beta.dtype == torch.bfloat16 else beta.to(torch.bfloat16)
     indexed = plan.path == "indexed"
+    direct = indexed and plan.launches is not None and _lib.eager(q, k, v, g, beta)
     above = None   # the states the level above left
     for d, calls in enumerate(plan.levels):
         n_slots = plan.n_keep[d] if indexed else sum(len(c.cu_cpu) - 1 for c in calls if c.keep)
         states = q.new_empty((n_slots, v.shape[1], q.shape[-1], v.shape[-1]), dtype=torch.float32) if n_slots else None
         next_slot = 0
+        if direct:
+            for mode, cu, n_seg, h0_idx, ht_idx, idx, longest in plan.launches[d]:
+                gdn._launch(mode, q[None], k[None], v[None], g32[None], b16[None], scale, cu, n_seg, above, h0_idx, states, ht_idx, idx, o[None], longest)
+            calls = ()
         for c in calls:
             n_seg = len(c.cu_cpu) - 1
             if indexed:
