@@ -241,6 +241,7 @@ typedef struct spinf_lm_args {
     int64_t rows, vocab; float softcap;
     const int64_t* cols; int64_t n_cols;
     float* out; int64_t out_ld;
+    int32_t cols_wrap;                       /* nonzero: a column in -vocab .. -1 counts from the end, as in tensor indexing */
 } spinf_lm_args;
 int spinf_lm_logprobs(const spinf_lm_args* args, void* stream);
 
@@ -268,6 +269,7 @@ typedef struct spinf_lm_head_args {
     float* out; int64_t out_ld;
     void* workspace; int64_t workspace_bytes;
     int64_t h_rows;                          /* rows of h (> 0): what sel is checked against */
+    int32_t cols_wrap;                       /* nonzero: a column in -vocab .. -1 counts from the end, as in tensor indexing */
 } spinf_lm_head_args;
 int spinf_lm_head_workspace(const spinf_lm_head_args* args, int64_t* bytes);
 int spinf_lm_head_fwd(const spinf_lm_head_args* args, void* stream);
@@ -310,6 +312,11 @@ int spinf_xdecode_plan(const spinf_xdec_args* args, int32_t* nsplit, int64_t* wo
 /* tiles of the longest list of these sizes (a group whose prefix and template ranges are full) */
 int spinf_xdecode_tiles(const spinf_xdec_args* args, int32_t* tiles);
 int spinf_xdecode_attn_fwd(const spinf_xdec_args* args, void* stream);
+/* Replaces the two index_copy_ of GroupKV.update (spinf_serve/decode.py:51-68): the new tokens' keys and values [G, h, Q, d] (bf16,
+ * head dim contiguous, element strides *_g, *_h, *_q, multiples of 8) become entry *step (device scalar) of gk / gv [G, h, Q, S, d].
+ * A step outside 0 .. S - 1 writes nothing.  d a multiple of 8, everything 16-byte aligned. */
+int spinf_xdecode_put(const void* k, int64_t k_g, int64_t k_h, int64_t k_q, const void* v, int64_t v_g, int64_t v_h, int64_t v_q,
+                      void* gk, void* gv, const int64_t* step, int32_t G, int32_t h, int32_t Q, int32_t S, int32_t d, void* stream);
 
 /* ------------------------------------------------------------------------------------------------ yardstick
  * No counterpart in the reference: one launch of a pure v_mfma_f32_32x32x16_bf16 loop on every compute unit (one workgroup of eight

@@ -296,3 +296,23 @@ def test_seeded_random_shapes(dev):
         out = sa.xdecode_attn(q, c, 0, scale, window, softcap, nsplit=nsplit)
         err = np.abs(_np(out) - _oracle(q, c, scale, window, softcap)).max()
         assert err <= TOL, (case, err)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("G,h,Q,S,d", [(1, 1, 1, 1, 64), (3, 4, 7, 5, 128), (2, 1, 13, 33, 512), (5, 8, 48, 17, 256)])
+def test_cache_update_equals_index_copy(dev, G, h, Q, S, d):
+    """GroupKV.update in one launch: entry `step` of both caches and nothing else, from strided views as the model hands them over;
+    tensors the kernel does not take still go through index_copy_"""
+    gen = torch.Generator().manual_seed(G + Q)
+    rnd = lambda *s: torch.randn(*s, generator=gen).to(torch.bfloat16).to(dev)  # noqa: E731
+    c = decode.XCaches()
+    c.gk[0], c.gv[0] = rnd(G, h, Q, S, d), rnd(G, h, Q, S, d)
+    k, v = rnd(G, Q, h, d).transpose(1, 2), rnd(G, h, Q, d)
+    for step in (0, S // 2, S - 1):
+        c.step_t = torch.full((1,), step, dtype=torch.int64, device=dev)
+        want = [t.clone().index_copy_(3, c.step_t, n.unsqueeze(3)) for t, n in ((c.gk[0], k), (c.gv[0], v))]
+        assert decode.GroupKV(c).update(k, v, 0) == (("x", 0), ("x", 0))
+        assert torch.equal(c.gk[0], want[0]) and torch.equal(c.gv[0], want[1])
+    c.gk[0], c.gv[0] = c.gk[0].float(), c.gv[0].float()
+    decode.GroupKV(c).update(v.float(), k.float(), 0)
+    assert torch.equal(c.gk[0][:, :, :, S - 1], v.float()) and torch.equal(c.gv[0][:, :, :, S - 1], k.float())
