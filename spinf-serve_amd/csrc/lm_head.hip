@@ -18,11 +18,12 @@
 // pads its last chunk to 1,024 rows for (lm_fixed_rows, spinf_serve/config.py:56-57).
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "spinf_tree.h"
 #include "common.h"
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
+#include "attn_tiles.h"
 
 namespace {
 
@@ -30,6 +31,7 @@ constexpr int TV = 256, TR = 256, BK = 64;      // tile: vocabulary rows, read r
 constexpr int WT = 128;                         // a wave's quarter: 128 vocabulary rows x 128 read rows
 constexpr int PITCH = BK * 2 + 16;              // bytes of a staged row (padded: the fragment reads of 32 rows spread over the banks)
 constexpr int STAGE = (TV + TR) * PITCH;        // one buffer: W rows then h rows
+constexpr int ROWS_MAX = 96;                    // read rows up to which lm_head_rows_kernel takes the call
 constexpr int BP = 33;                          // floats of a row of a wave's 32 x 32 output block in LDS ([vocabulary][read row])
 constexpr float LOG2E = 1.4426950408889634f;
 
@@ -39,11 +41,24 @@ struct HeadParams {
     const __bf16* w; long w_ld;
     int vocab, hidden;
     float cap, inv_cap;
-    const long* cols; int n_cols;
+    const long* cols; int n_cols; bool cols_wrap;
     float* out; long out_ld;
     float2* part; int n_part;   // [rows, n_part] pairs; n_part = 2 * vocabulary tiles
     int row_tiles;
 };
+
+// row of h that entry r of the row list names: a negative one counts from the end, as tensor indexing does; one that names no row of h
+// reads row 0 (the finishing kernel turns its output row into NaN)
+__device__ __forceinline__ long row_of_h(const HeadParams& p, const int r) {
+    long hr = p.sel ? p.sel[r] : r;
+    hr = hr < 0 ? hr + p.h_rows : hr;
+    return hr >= 0 && hr < p.h_rows ? hr : 0;
+}
+
+__device__ __forceinline__ long column(const HeadParams& p, const int c) {
+    const long col = p.cols[c];
+    return p.cols_wrap && col < 0 ? col + p.vocab : col;
+}
 
 __device__ __forceinline__ float to_bf16(float x) { return (float)(__bf16)x; }
 
@@ -59,6 +74,179 @@ __device__ __forceinline__ float softcap(float x, float cap, float inv_cap) {
     }
     const float e = __builtin_amdgcn_exp2f(2.0f * LOG2E * x * inv_cap);
     return cap * (1.0f - 2.0f * __builtin_amdgcn_rcpf(e + 1.0f));
+}
+
+// What leaves a wave's 128 vocabulary rows x 32 NB read rows: the capped logits replace the accumulators (register i of block (a, b)
+// holds vocabulary row vw0 + 32 a + 8 (i / 4) + 4 g + i % 4 for read row rw0 + 32 b + m), each read row's (reference, sum of
+// exponentials) pair over the 128 vocabulary rows goes to p.part[.][pair], and blocks with a selected column (or all of them) pass
+// through `blk`, a 32 x 32 tile of the wave's own in LDS, to the output.
+template <int NB, bool CAPPED, bool BF16>
+__device__ __forceinline__ void leave_tile(const HeadParams& p, f32x16 (&acc)[4][NB], const int vw0, const int rw0, const int pair, float* blk, const int lane) {
+    const int m = lane & 31, g = lane >> 5;
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                float x = acc[a][b][i];
+                if (BF16) x = to_bf16(x);
+                if (CAPPED) x = softcap<BF16>(x, p.cap, p.inv_cap);
+                acc[a][b][i] = x;
+            }
+    // per read row one pair: 64 values in this lane, 64 in lane ^ 32
+    const bool tail = vw0 + WT > p.vocab;   // wave-uniform: some of the wave's vocabulary rows do not exist
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        float ref = CAPPED ? p.cap : -INFINITY;
+        if (!CAPPED) {
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (!tail || vw0 + 32 * a + 8 * (i >> 2) + 4 * g + (i & 3) < p.vocab) ref = fmaxf(ref, acc[a][b][i]);
+            ref = fmaxf(ref, __shfl_xor(ref, 32));
+        }
+        float sum = 0.f;
+        if (ref != -INFINITY) {
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (!tail || vw0 + 32 * a + 8 * (i >> 2) + 4 * g + (i & 3) < p.vocab) sum += __builtin_amdgcn_exp2f((acc[a][b][i] - ref) * LOG2E);
+        }
+        const float other = __shfl_xor(sum, 32);
+        sum = g == 0 ? sum + other : other + sum;   // both halves add in the same order
+        const int row = rw0 + 32 * b + m;
+        if (g == 0 && row < p.rows) p.part[(long)row * p.n_part + pair] = make_float2(ref, sum);
+    }
+    auto put = [&](const f32x16& x) __attribute__((always_inline)) {   // a 32 x 32 block, vocabulary-major
+#pragma unroll
+        for (int i = 0; i < 16; i++) blk[(8 * (i >> 2) + 4 * g + (i & 3)) * BP + m] = x[i];
+    };
+    if (p.cols) {   // the selected columns: rarely one of them lies in this wave's 128 vocabulary rows (64 of them looked at at a time)
+        for (int c0 = 0; c0 < p.n_cols; c0 += 64) {
+            long mine = c0 + lane < p.n_cols ? column(p, c0 + lane) : -1;
+            unsigned long long hits = __builtin_amdgcn_ballot_w64(mine >= vw0 && mine < vw0 + WT);
+            for (; hits; hits &= hits - 1) {
+                const int c = c0 + __builtin_ctzll(hits);
+                const int at = __builtin_amdgcn_readlane((int)(mine - vw0), c - c0);
+                const int ca = at >> 5, cv = at & 31;
+#pragma unroll
+                for (int a = 0; a < 4; a++) {
+                    if (a != ca) continue;
+#pragma unroll
+                    for (int b = 0; b < NB; b++) {
+                        put(acc[a][b]);
+                        const int row = rw0 + 32 * b + m;
+                        if (g == 0 && row < p.rows) p.out[(long)row * p.out_ld + c] = blk[cv * BP + m];
+                    }
+                }
+            }
+        }
+    } else {        // the extraction rows: every block, a read row's 32 values of the block as one 128-byte run
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int b = 0; b < NB; b++) {
+                put(acc[a][b]);
+                const int vb = vw0 + 32 * a + m;
+                for (int r = g; r < 32; r += 2) {
+                    const int row = rw0 + 32 * b + r;
+                    if (row < p.rows && vb < p.vocab) p.out[(long)row * p.out_ld + vb] = blk[m * BP + r];
+                }
+            }
+    }
+}
+
+// Few read rows (at most ROWS_MAX): bound by reading W once.  One wave owns 128 vocabulary rows and all the read rows, 32 NB of them,
+// so W goes straight from HBM into that wave's own LDS (global -> LDS requests, no barrier anywhere, two buffers of 64 hidden dims:
+// 16 KB in flight per wave, five waves per CU) and each fragment of h, which lies in L2, into registers.  The 16-byte pieces of a row
+// are swapped inside its 128 bytes (piece ^ row % 8, on the request's source side), so that the fragment reads of eight
+// neighbouring rows cover all banks.  Same products in the same order as the tile kernel: a row's bits do not depend on which of
+// the two computed it.  24 rows x 262,144 x 2,560, 1.34 GB
+// of W: 0.238 ms = 5.65 TB/s (the 256-row tile kernel 0.362); 64 rows 0.262 (0.356), 96 rows 0.290 (0.366).  Beyond that the accumulators leave
+// room for one wave per SIMD and each wave's own copy of h through L1 costs as much as the tile kernel's padding: 128 rows 0.327 (0.367) at
+// hidden 2,560 but 0.371 (0.350) at 3,840 x 151,936, so ROWS_MAX is 96.
+template <int NB, bool CAPPED, bool BF16>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(NB <= 2 ? 2 : 1))) void lm_head_rows_kernel(const HeadParams p) {
+    constexpr int STEP = WT * BK * 2;
+    __shared__ __attribute__((aligned(16))) char lds[2 * STEP];
+    const int lane = threadIdx.x, m = lane & 31, g = lane >> 5;
+    const int vw0 = blockIdx.x * WT, rw0 = blockIdx.y * 32 * NB;
+    if (vw0 >= p.vocab) {   // the last pair of a vocabulary whose last tile is half empty
+        for (int row = rw0 + lane; row < p.rows && row < rw0 + 32 * NB; row += 64) p.part[(long)row * p.n_part + blockIdx.x] = make_float2(0.f, 0.f);
+        return;
+    }
+    const __bf16* hp[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++) {
+        const int rr = rw0 + 32 * b + m < p.rows ? rw0 + 32 * b + m : p.rows - 1;
+        hp[b] = p.h + row_of_h(p, rr) * p.h_ld + 8 * g;
+    }
+    // request i of a step: rows 8 i .. 8 i + 7, lane -> row lane / 8, piece (lane % 8) ^ (row % 8)
+    const bool whole = vw0 + WT <= p.vocab;
+    const unsigned lane_off = (unsigned)((lane >> 3) * p.w_ld * 2 + (((lane & 7) ^ (lane >> 3)) << 4));
+    const char* const wbase = (const char*)(p.w + (long)vw0 * p.w_ld);
+    auto request = [&](const int k0, const unsigned to) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < WT / 8; i++) {
+            if (whole) dma16_uniform(wbase + (long)8 * i * p.w_ld * 2 + k0 * 2, lane_off, to + 1024 * i);
+            else {   // rows past the vocabulary: its last row (their logits are left out of the sums and never stored)
+                const int row = vw0 + 8 * i + (lane >> 3);
+                dma16_lane((const char*)(p.w + (long)(row < p.vocab ? row : p.vocab - 1) * p.w_ld + k0) + (((lane & 7) ^ (lane >> 3)) << 4), to + 1024 * i);
+            }
+        }
+    };
+    bf16x8 h[2][NB][4];
+    auto request_h = [&](const int set, const int k0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int ks = 0; ks < 4; ks++) h[set][b][ks] = *(const bf16x8*)(hp[b] + k0 + 16 * ks);
+    };
+    int piece[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ks++) piece[ks] = m * (BK * 2) + (((2 * ks + g) ^ (m & 7)) << 4);
+    f32x16 acc[4][NB];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < 16; i++) acc[a][b][i] = 0.f;
+    const int nk = p.hidden / BK;
+    const unsigned lds0 = lds_addr(lds);
+    auto step = [&](const int kt, const int set) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(0x0070);   // vmcnt(0) lgkmcnt(0): this step's rows are here, the other buffer has been read
+        if (kt + 1 < nk) {
+            request(BK * (kt + 1), lds0 + (set ^ 1) * STEP);
+            request_h(set ^ 1, BK * (kt + 1));
+        } else {   // (an odd number of steps is rounded up: the extra one multiplies zeros)
+#pragma unroll
+            for (int b = 0; b < NB; b++)
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                    for (int j = 0; j < 8; j++) h[set ^ 1][b][ks][j] = (__bf16)0.f;
+        }
+        const char* buf = lds + (kt < nk ? set : 0) * STEP;   // (of one step only one buffer was ever filled)
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+            for (int a = 0; a < 4; a++) {
+                const bf16x8 wv = *(const bf16x8*)(buf + piece[ks] + a * 32 * BK * 2);
+#pragma unroll
+                for (int b = 0; b < NB; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, h[set][b][ks], acc[a][b], 0, 0, 0);
+            }
+    };
+    request(0, lds0);
+    request_h(0, 0);
+    for (int kt = 0; kt < nk; kt += 2) {
+        step(kt, 0);
+        step(kt + 1, 1);
+    }
+    leave_tile<NB, CAPPED, BF16>(p, acc, vw0, rw0, blockIdx.x, (float*)lds, lane);
 }
 
 template <bool CAPPED, bool BF16>
@@ -81,9 +269,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     for (int i = 0; i < 8; i++) {
         const int row = (tid >> 3) + 32 * i;
         const int rr = r0 + row < p.rows ? r0 + row : p.rows - 1;
-        long hr = p.sel ? p.sel[rr] : rr;           // an entry of the row list counts from the end when negative, as tensor indexing does
-        hr = hr < 0 ? hr + p.h_rows : hr;
-        row_h[i] = hr >= 0 && hr < p.h_rows ? (int)hr : 0;   // (an entry outside h reads row 0; the finishing kernel turns its row into NaN)
+        row_h[i] = (int)row_of_h(p, rr);
     }
     // The row list's loads end here: a value that still counts as "in flight" when the loop is entered makes the compiler wait
     // for it at every use, and such a wait also waits for every tile load issued before it.
@@ -196,81 +382,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
     }
     __syncthreads();   // everyone is done with the staging buffers: the waves' output blocks go there
 
-    // ---- the capped logits, in place.  Register i of block (a, b) holds vocabulary row vw0 + 32 a + 8 (i / 4) + 4 g + i % 4
-    // for read row rw0 + 32 b + m.
-    const int vw0 = v0 + wv * WT, rw0 = r0 + wr * WT;
-#pragma unroll
-    for (int a = 0; a < 4; a++)
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                float x = acc[a][b][i];
-                if (BF16) x = to_bf16(x);
-                if (CAPPED) x = softcap<BF16>(x, p.cap, p.inv_cap);
-                acc[a][b][i] = x;
-            }
-    // ---- per read row one (reference, sum) pair over the wave's 128 vocabulary rows: 64 values in this lane, 64 in lane ^ 32
-    const bool tail = vw0 + WT > p.vocab;   // wave-uniform: some of the wave's vocabulary rows do not exist
-#pragma unroll
-    for (int b = 0; b < 4; b++) {
-        float ref = CAPPED ? p.cap : -INFINITY;
-        if (!CAPPED) {
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int i = 0; i < 16; i++)
-                    if (!tail || vw0 + 32 * a + 8 * (i >> 2) + 4 * g + (i & 3) < p.vocab) ref = fmaxf(ref, acc[a][b][i]);
-            ref = fmaxf(ref, __shfl_xor(ref, 32));
-        }
-        float sum = 0.f;
-        if (ref != -INFINITY) {
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-#pragma unroll
-                for (int i = 0; i < 16; i++)
-                    if (!tail || vw0 + 32 * a + 8 * (i >> 2) + 4 * g + (i & 3) < p.vocab) sum += __builtin_amdgcn_exp2f((acc[a][b][i] - ref) * LOG2E);
-        }
-        const float other = __shfl_xor(sum, 32);
-        sum = g == 0 ? sum + other : other + sum;   // both halves add in the same order
-        const int row = rw0 + 32 * b + m;
-        if (g == 0 && row < p.rows) p.part[(long)row * p.n_part + 2 * vtile + wv] = make_float2(ref, sum);
-    }
-    // ---- what leaves the tile: a 32 x 32 block goes through the wave's LDS tile, vocabulary-major
-    float* blk = (float*)lds + w * 32 * BP;
-    auto put = [&](const f32x16& x) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < 16; i++) blk[(8 * (i >> 2) + 4 * g + (i & 3)) * BP + m] = x[i];
-    };
-    if (p.cols) {   // the selected columns: rarely one of them lies in this wave's 128 vocabulary rows
-        for (int c = 0; c < p.n_cols; c++) {
-            const long col = p.cols[c];
-            if (col < vw0 || col >= vw0 + WT) continue;   // wave-uniform
-            const int ca = (int)(col - vw0) >> 5, cv = (int)(col - vw0) & 31;
-#pragma unroll
-            for (int a = 0; a < 4; a++) {
-                if (a != ca) continue;
-#pragma unroll
-                for (int b = 0; b < 4; b++) {
-                    put(acc[a][b]);
-                    const int row = rw0 + 32 * b + m;
-                    if (g == 0 && row < p.rows) p.out[(long)row * p.out_ld + c] = blk[cv * BP + m];
-                }
-            }
-        }
-    } else {        // the extraction rows: every block, a read row's 32 values of the block as one 128-byte run
-#pragma unroll
-        for (int a = 0; a < 4; a++)
-#pragma unroll
-            for (int b = 0; b < 4; b++) {
-                put(acc[a][b]);
-                const int vb = vw0 + 32 * a + m;
-                for (int r = g; r < 32; r += 2) {
-                    const int row = rw0 + 32 * b + r;
-                    if (row < p.rows && vb < p.vocab) p.out[(long)row * p.out_ld + vb] = blk[m * BP + r];
-                }
-            }
-    }
+    leave_tile<4, CAPPED, BF16>(p, acc, v0 + wv * WT, r0 + wr * WT, 2 * vtile + wv, (float*)lds + w * 32 * BP, lane);
 }
 
 // per read row: merge the pairs in their fixed order, subtract the log-sum-exp
@@ -305,7 +417,8 @@ __global__ __launch_bounds__(256) void lm_head_finish_kernel(const HeadParams p)
     const long hr = p.sel ? p.sel[row] : row;
     const bool row_known = hr >= -p.h_rows && hr < p.h_rows;   // a row list entry that names no row of h
     for (int i = threadIdx.x; i < n; i += 256) {
-        const bool known = row_known && (!p.cols || (p.cols[i] >= 0 && p.cols[i] < p.vocab));   // no tile wrote a column outside the vocabulary
+        const long col = p.cols ? column(p, i) : i;
+        const bool known = row_known && col >= 0 && col < p.vocab;   // no tile wrote a column outside the vocabulary
         out[i] = known ? out[i] - lse : __builtin_nanf("");
     }
 }
@@ -349,17 +462,29 @@ extern "C" int spinf_lm_head_fwd(const spinf_lm_head_args* a, void* stream) {
     p.h = (const __bf16*)a->h; p.h_ld = a->h_ld; p.sel = a->sel; p.rows = (int)a->rows; p.h_rows = a->h_rows;
     p.w = (const __bf16*)a->w; p.w_ld = a->w_ld; p.vocab = (int)a->vocab; p.hidden = (int)a->hidden;
     p.cap = a->softcap; p.inv_cap = a->softcap > 0.f ? 1.0f / a->softcap : 0.f;
-    p.cols = a->cols; p.n_cols = (int)a->n_cols; p.out = a->out; p.out_ld = a->out_ld;
+    p.cols = a->cols; p.n_cols = (int)a->n_cols; p.cols_wrap = a->cols_wrap != 0; p.out = a->out; p.out_ld = a->out_ld;
     p.part = (float2*)a->workspace; p.n_part = (int)parts_of(a);
     p.row_tiles = (int)((a->rows + TR - 1) / TR);
     const int64_t vtiles = (a->vocab + TV - 1) / TV;
     const dim3 grid((unsigned)(p.row_tiles * ((vtiles + 7) / 8 * 8)));
     hipStream_t s = (hipStream_t)stream;
     const bool capped = a->softcap > 0.f, bf = a->logits_dtype == 1;
-    if (capped && bf) hipLaunchKernelGGL((lm_head_tile_kernel<true, true>), grid, dim3(256), 0, s, p);
-    else if (capped) hipLaunchKernelGGL((lm_head_tile_kernel<true, false>), grid, dim3(256), 0, s, p);
-    else if (bf) hipLaunchKernelGGL((lm_head_tile_kernel<false, true>), grid, dim3(256), 0, s, p);
-    else hipLaunchKernelGGL((lm_head_tile_kernel<false, false>), grid, dim3(256), 0, s, p);
+    auto with = [&](auto launch) {   // launch(capped, bf16) with the two as compile-time values
+        if (capped && bf) launch(std::true_type{}, std::true_type{});
+        else if (capped) launch(std::true_type{}, std::false_type{});
+        else if (bf) launch(std::false_type{}, std::true_type{});
+        else launch(std::false_type{}, std::false_type{});
+    };
+    if (a->rows <= ROWS_MAX) {
+        const dim3 few((unsigned)p.n_part, 1);
+        with([&](auto c, auto b) {
+            switch ((a->rows + 31) / 32) {
+                case 1: hipLaunchKernelGGL((lm_head_rows_kernel<1, c, b>), few, dim3(64), 0, s, p); break;
+                case 2: hipLaunchKernelGGL((lm_head_rows_kernel<2, c, b>), few, dim3(64), 0, s, p); break;
+                default: hipLaunchKernelGGL((lm_head_rows_kernel<3, c, b>), few, dim3(64), 0, s, p);
+            }
+        });
+    } else with([&](auto c, auto b) { hipLaunchKernelGGL((lm_head_tile_kernel<c, b>), grid, dim3(256), 0, s, p); });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "lm_head: launch: %s", hipGetErrorString(e));
     hipLaunchKernelGGL(lm_head_finish_kernel, dim3((unsigned)a->rows), dim3(256), 0, s, p);

@@ -17,7 +17,7 @@ namespace {
 
 struct LmParams {
     const void* logits; long ld;      // [rows, >= vocab], row stride in elements
-    const long* cols; int n_cols;     // selected columns (NULL: every column)
+    const long* cols; int n_cols; bool cols_wrap;   // selected columns (NULL: every column)
     float* out; long out_ld;
     int rows, vocab;
     float cap, inv_cap;               // soft-capping (0: none)
@@ -112,7 +112,8 @@ __global__ __launch_bounds__(256) void lm_logprobs_kernel(const LmParams p) {
     float* out = p.out + (long)row * p.out_ld;
     if (p.cols) {
         for (int c = threadIdx.x; c < p.n_cols; c += 256) {   // a column outside the vocabulary is not read: NaN
-            const long col = p.cols[c];
+            long col = p.cols[c];
+            if (p.cols_wrap && col < 0) col += p.vocab;
             out[c] = col >= 0 && col < p.vocab ? softcap(load1<BF16>(base, col), p.cap, p.inv_cap) - lse : __builtin_nanf("");
         }
     } else {
@@ -134,7 +135,7 @@ extern "C" int spinf_lm_logprobs(const spinf_lm_args* a, void* stream) {
     if (a->out_ld < (a->cols ? a->n_cols : a->vocab)) return spinf_fail(SPINF_E_ARG, "lm_logprobs: output rows too short");
     if (a->softcap < 0.f || a->softcap > 40.f) return spinf_fail(SPINF_E_ARG, "lm_logprobs: softcap %g outside 0 .. 40", (double)a->softcap);
     LmParams p;
-    p.logits = a->logits; p.ld = a->ld; p.cols = a->cols; p.n_cols = (int)a->n_cols; p.out = a->out; p.out_ld = a->out_ld;
+    p.logits = a->logits; p.ld = a->ld; p.cols = a->cols; p.n_cols = (int)a->n_cols; p.cols_wrap = a->cols_wrap != 0; p.out = a->out; p.out_ld = a->out_ld;
     p.rows = (int)a->rows; p.vocab = (int)a->vocab; p.cap = a->softcap; p.inv_cap = a->softcap > 0.f ? 1.0f / a->softcap : 0.f;
     if (a->dtype) hipLaunchKernelGGL(lm_logprobs_kernel<true>, dim3(p.rows), dim3(256), 0, (hipStream_t)stream, p);
     else hipLaunchKernelGGL(lm_logprobs_kernel<false>, dim3(p.rows), dim3(256), 0, (hipStream_t)stream, p);

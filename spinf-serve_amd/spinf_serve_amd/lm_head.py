@@ -20,8 +20,7 @@ import torch
 from . import _lib
 
 
-@torch.library.custom_op("spinf::lm_logprobs", mutates_args=())
-def _lm_op(logits: torch.Tensor, cols: Optional[torch.Tensor], softcap: float) -> torch.Tensor:
+def _lm(logits: torch.Tensor, cols: Optional[torch.Tensor], softcap: float) -> torch.Tensor:
     if not logits.is_cuda:
         raise RuntimeError("spinf::lm_logprobs runs on ROCm device tensors only (no CPU path)")
     if logits.dim() != 2 or logits.stride(1) != 1 or logits.dtype not in (torch.float32, torch.bfloat16):
@@ -38,10 +37,12 @@ def _lm_op(logits: torch.Tensor, cols: Optional[torch.Tensor], softcap: float) -
     if cols is not None:
         a.cols, a.n_cols = cols.data_ptr(), cols.numel()
     a.out, a.out_ld = out.data_ptr(), out.stride(0)
-    lib = _lib.load_library()
-    with torch.cuda.device(logits.device):
-        _lib.check(lib.spinf_lm_logprobs(C.byref(a), C.c_void_p(torch.cuda.current_stream(logits.device).cuda_stream)), "spinf_lm_logprobs")
+    a.cols_wrap = 1
+    _lib.launch(_lib.load_library().spinf_lm_logprobs, a, logits.device, "spinf_lm_logprobs")
     return out
+
+
+_lm_op = torch.library.custom_op("spinf::lm_logprobs", _lm, mutates_args=())
 
 
 @_lm_op.register_fake
@@ -52,13 +53,10 @@ def _(logits, cols, softcap):
 def lm_logprobs(logits, cols=None, softcap=None):
     """logits [rows, vocab] fp32 / bf16 -> log_softmax(softcap * tanh(logits / softcap)) fp32, the columns ``cols`` of it
     (int64 device vector; negative = from the end, outside the vocabulary = NaN) or with cols None all of it"""
-    if cols is not None:
-        cols = torch.where(cols < 0, cols + logits.shape[1], cols)
-    return _lm_op(logits, cols, float(softcap) if softcap else 0.0)
+    return (_lm if _lib.eager(logits, cols) else _lm_op)(logits, cols, float(softcap) if softcap else 0.0)
 
 
-@torch.library.custom_op("spinf::lm_head_logprobs", mutates_args=())
-def _head_op(h: torch.Tensor, sel: Optional[torch.Tensor], w: torch.Tensor, cols: Optional[torch.Tensor], softcap: float, bf16_logits: bool) -> torch.Tensor:
+def _head(h: torch.Tensor, sel: Optional[torch.Tensor], w: torch.Tensor, cols: Optional[torch.Tensor], softcap: float, bf16_logits: bool) -> torch.Tensor:
     if not (h.is_cuda and w.is_cuda):
         raise RuntimeError("spinf::lm_head_logprobs runs on ROCm device tensors only (no CPU path)")
     if h.dim() != 2 or w.dim() != 2 or h.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or h.stride(1) != 1 or w.stride(1) != 1:
@@ -88,9 +86,12 @@ def _head_op(h: torch.Tensor, sel: Optional[torch.Tensor], w: torch.Tensor, cols
     _lib.check(lib.spinf_lm_head_workspace(C.byref(a), C.byref(need)), "spinf_lm_head_workspace")
     work = torch.empty(max(need.value, 8), dtype=torch.uint8, device=h.device)
     a.workspace, a.workspace_bytes = work.data_ptr(), work.numel()
-    with torch.cuda.device(h.device):
-        _lib.check(lib.spinf_lm_head_fwd(C.byref(a), C.c_void_p(torch.cuda.current_stream(h.device).cuda_stream)), "spinf_lm_head_fwd")
+    a.cols_wrap = 1
+    _lib.launch(lib.spinf_lm_head_fwd, a, h.device, "spinf_lm_head_fwd")
     return out
+
+
+_head_op = torch.library.custom_op("spinf::lm_head_logprobs", _head, mutates_args=())
 
 
 @_head_op.register_fake
@@ -108,6 +109,4 @@ def lm_head_logprobs(h, sel, w, cols=None, softcap=None, logits="fp32"):
     torch's indexing would raise: the list is a device tensor, and checking it on the host would cost a synchronisation)."""
     if logits not in ("fp32", "bf16"):
         raise ValueError(f"logits mode {logits!r}")
-    if cols is not None:
-        cols = torch.where(cols < 0, cols + w.shape[0], cols)
-    return _head_op(h, sel, w, cols, float(softcap) if softcap else 0.0, logits == "bf16")
+    return (_head if _lib.eager(h, sel, w, cols) else _head_op)(h, sel, w, cols, float(softcap) if softcap else 0.0, logits == "bf16")

@@ -222,3 +222,20 @@ def test_fused_head_columns_at_tile_and_wave_boundaries(dev):
     want = olm.head_logprobs(h.float().numpy(), w.float().numpy(), None, None, 30.0)
     assert np.abs(whole.cpu().numpy() - want).max() <= TOL
     assert np.abs(np.exp(whole.double().cpu().numpy()).sum(1) - 1.0).max() < 1e-5
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 31, 32, 33, 64, 65, 96, 97])
+@pytest.mark.parametrize("vocab,hidden", [(127, 64), (385, 192), (1000, 128)])
+def test_few_read_rows_give_the_bits_they_have_among_many(dev, rows, vocab, hidden):
+    """the kernel for few read rows (32, 64 or 96 of them per wave) and the tile kernel behind it, at the edges of both, on vocabularies that
+    end inside a wave's 128 rows and with an odd number of 64-dim steps: the oracle's values, and the bits of the same rows among 300"""
+    rng = np.random.default_rng(rows + vocab)
+    h, w = _bf16_values(rng, (300, hidden), 1.0), _bf16_values(rng, (vocab, hidden), 1.0)
+    sel, cols = rng.integers(0, 300, rows), np.concatenate([rng.integers(0, vocab, 70), [-1, 0, vocab - 1]])
+    hd, wd, seld, colsd = h.to(dev), w.to(dev), torch.from_numpy(sel).to(dev), torch.from_numpy(cols).to(dev)
+    for cap in (30.0, None):
+        whole = sa.lm_head_logprobs(hd, seld, wd, None, cap)
+        assert np.abs(whole.cpu().numpy() - olm.head_logprobs(h.float().numpy(), w.float().numpy(), sel, None, cap)).max() <= TOL
+        assert torch.equal(sa.lm_head_logprobs(hd, seld, wd, colsd, cap), whole[:, colsd])
+        assert torch.equal(sa.lm_head_logprobs(hd, None, wd, None, cap)[seld], whole)
