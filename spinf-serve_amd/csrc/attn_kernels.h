@@ -38,11 +38,11 @@ struct AttnParams {
 
 // Softmax reference point.  The fast pass fixes each row's reference at the maximum of the first 32-key block in which
 // the row sees a key and never rescales the accumulators: probabilities are exp2(t - ref) and stay below 2^TAU_FAST, well
-// inside fp32 / bf16 range.  If any row of a tile meets scores so far above its reference that a lane's 16 probabilities of a
-// block sum to more than 2^TAU_FAST (at the latest when one score lies TAU_FAST above the reference), the whole tile is
+// inside fp32 / bf16 range.  If any of a wave's 32 rows meets scores so far above its reference that a lane's 16 probabilities of a
+// block sum to more than 2^TAU_FAST (at the latest when one score lies TAU_FAST above the reference), those 32 rows of that head are
 // recomputed by the exact pass: classic online softmax, reference raised and accumulators rescaled whenever a block
-// maximum exceeds the reference by more than TAU_LAZY.  Which pass produced a row depends on the rows of its own
-// 128-token tile only, so it does not depend on what the job is packed with.
+// maximum exceeds the reference by more than TAU_LAZY.  Which pass produced a row depends on the rows of its own aligned 32-row
+// group only, so it does not depend on what the job is packed with, nor on which kernel computed it.
 constexpr float TAU_FAST = 60.f;
 constexpr float VIOL_SUM = 1152921504606846976.f;   // 2^TAU_FAST: a lane's 16 probabilities of a block summing above it send the tile to the exact pass
 constexpr float TAU_LAZY = 8.f;
@@ -194,3 +194,5 @@ __device__ __forceinline__ int fresh_lane_id() {
 // tree_attn_ring.hip: the pass with decoupled waves over a static schedule (p.list_ptr delimits n_wg item lists, one per
 // workgroup; plan entries of 32 keys), the exact recomputation of the items that need it included.  Stream-ordered launch on `stream`.
 int spinf_launch_ring(const AttnParams& p, int d, bool win, int n_wg, hipStream_t stream);
+// tree_attn_spread.hip: a workgroup per 32-row group and `heads` heads over the eight lists of a schedule with that many heads per item.
+int spinf_launch_spread(const AttnParams& p, int d, int heads, bool win, int ktile, long n_items, hipStream_t stream);

@@ -37,10 +37,10 @@
 #include "attn_kernels.h"
 
 // normalise O^T and store it as rows: each wave stages 32 rows x 64 head dims at a time in its own LDS slice (144-byte
-// rows) and writes them out as 16-byte pieces, 8 lanes per 128-byte row segment
+// rows) and writes them out as 16-byte pieces, 8 lanes per 128-byte row segment; heads without `keep` are left alone
 template <int D, int RT, bool ROWS = false, class LaneT>
 __device__ __forceinline__ void store_rows(const AttnParams& p, const LaneT& L, char* stage, const f32x16 (&o)[RT][D / 32], const float (&l)[RT],
-                                           int t, int h0) {
+                                           const bool (&keep)[RT], int t, int h0) {
     constexpr int NDT = D / 32;
     constexpr int SROW = 128 + 16;
     const int tok0 = t * SPINF_QTILE + 32 * L.wr;
@@ -55,6 +55,7 @@ __device__ __forceinline__ void store_rows(const AttnParams& p, const LaneT& L, 
     }
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
+        if (!keep[rt]) continue;   // (wave-uniform)
         const float inv = 1.0f / lane32_sum(l[rt]);
         __bf16* ob = p.o + (long)(h0 + rt) * p.o_head;
 #pragma unroll
@@ -111,11 +112,13 @@ __device__ __forceinline__ void attn_item_exact(const AttnParams& p, const int4 
     const int pos_q = WIN ? p.pos[tok_c] : 0;
     const int grp_q = GRP && tok < p.n ? p.grp[tok_c] : -1;
     f32x16 o[RT][NDT];
-    float M[RT], l[RT];
+    float M[RT], l[RT], Mf[RT];
+    bool far[RT];   // did the fast pass find this row (these rows) too far above its reference?  The same test on the same numbers
 #pragma unroll
     for (int rt = 0; rt < RT; rt++) {
-        M[rt] = -INFINITY;
+        M[rt] = Mf[rt] = -INFINITY;
         l[rt] = 0.f;
+        far[rt] = false;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
@@ -174,6 +177,12 @@ __device__ __forceinline__ void attn_item_exact(const AttnParams& p, const int4 
                 for (int i2 = 1; i2 < 16; i2++) mx = fmaxf(mx, s_acc[rt][i2]);
                 mx = lane32_max(mx);
                 const float tm = mx * p.c;
+                Mf[rt] = Mf[rt] == -INFINITY ? tm : Mf[rt];
+                const float msf = Mf[rt] == -INFINITY ? 0.f : Mf[rt];
+                float sumf = 0.f;
+#pragma unroll
+                for (int i2 = 0; i2 < 16; i2++) sumf += __builtin_amdgcn_exp2f(__builtin_fmaf(s_acc[rt][i2], p.c, -msf));
+                far[rt] = far[rt] | !(sumf <= VIOL_SUM);
                 const bool up = tm > M[rt] + TAU_LAZY;
                 const float mn = up ? tm : M[rt];
                 const float alpha = up ? __builtin_amdgcn_exp2f(M[rt] - mn) : 1.0f;
@@ -210,7 +219,9 @@ __device__ __forceinline__ void attn_item_exact(const AttnParams& p, const int4 
             }
         }
     }
-    store_rows<DV, RT, ROWS>(p, L, stage, o, l, t, h0);
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) far[rt] = __builtin_amdgcn_ballot_w64(far[rt]) != 0;
+    store_rows<DV, RT, ROWS>(p, L, stage, o, l, far, t, h0);   // (the other rows of the item have the fast pass's output)
 }
 
 // An item of HPI heads is recomputed RT heads at a time.
@@ -310,7 +321,7 @@ __global__ __launch_bounds__(256 * NHW) void tree_attn_kernel(const AttnParams p
     int art_q = -1, pos_q = 0, grp_q = -1;
     f32x16 o[RT][NDT];
     float M[RT], l[RT];
-    bool viol = false;
+    bool viol[RT];
     int2* ent_cur = ent_a;
     int2* ent_nxt = ent_b;
     int* entr_cur = entr_a;
@@ -357,12 +368,12 @@ __global__ __launch_bounds__(256 * NHW) void tree_attn_kernel(const AttnParams p
         for (int rt = 0; rt < RT; rt++) {
             M[rt] = -INFINITY;
             l[rt] = 0.f;
+            viol[rt] = false;
 #pragma unroll
             for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
                 for (int i = 0; i < 16; i++) o[rt][dt][i] = 0.f;
         }
-        viol = false;
     };
 
     // ---- compute pieces
@@ -445,7 +456,7 @@ __global__ __launch_bounds__(256 * NHW) void tree_attn_kernel(const AttnParams p
 #pragma unroll
                 for (int i2 = 0; i2 < 16; i2++) sm_elem(sa[rt], i2, ms, sum, pa[rt]);
                 l[rt] += sum;
-                viol = viol | !(sum <= VIOL_SUM);   // (a NaN counts as too far as well)
+                viol[rt] = viol[rt] | !(sum <= VIOL_SUM);   // (a NaN counts as too far as well)
             }
             pv_phase(vb + sub * G::VSUB, pa);
         };
@@ -529,15 +540,17 @@ __global__ __launch_bounds__(256 * NHW) void tree_attn_kernel(const AttnParams p
             const int2 en = ent_cur[i - base];
             compute_tile(buf, __builtin_amdgcn_readfirstlane(en.x), (unsigned)__builtin_amdgcn_readfirstlane(en.y) >> (2 * L.wr));
         }
-        // ---- item finished: output (or hand the item to the exact pass), switch to the next item
-        const int any_viol = __builtin_amdgcn_readfirstlane(__syncthreads_or(viol));
-        if (any_viol) {
-            if (threadIdx.x == 0) p.redo[atomicAdd(&p.counters[NLIST + 1], 1)] = cur_idx;
-        } else {
-            // (the loop has already flipped par: the last tile came from buffer par ^ 1)
-            char* const stage = STAGE_IN_TILE ? bufs + (par ^ 1) * G::BUFB + L.w * 32 * 144 : stage_own;
-            store_rows<DV, RT, ROWS>(p, L, stage, o, l, item_t(cur), item_hp(cur) * HPI + L.wh * RT);
+        // ---- item finished: output (rows and heads with too wide a range of scores are left to the exact pass), next item
+        bool keep[RT], any = false;
+#pragma unroll
+        for (int rt = 0; rt < RT; rt++) {
+            keep[rt] = __builtin_amdgcn_ballot_w64(viol[rt]) == 0;
+            any = any | !keep[rt];
         }
+        if (__builtin_amdgcn_readfirstlane(__syncthreads_or(any)) && threadIdx.x == 0) p.redo[atomicAdd(&p.counters[NLIST + 1], 1)] = cur_idx;
+        // (the loop has already flipped par: the last tile came from buffer par ^ 1)
+        char* const stage = STAGE_IN_TILE ? bufs + (par ^ 1) * G::BUFB + L.w * 32 * 144 : stage_own;
+        store_rows<DV, RT, ROWS>(p, L, stage, o, l, keep, item_t(cur), item_hp(cur) * HPI + L.wh * RT);
         cur_ok = nxt_ok;
         if (!cur_ok) break;
         // finish whatever of the next item's prefetch has not happened yet (one-tile items), then switch
@@ -709,10 +722,12 @@ int launch(const AttnParams& p, int blocks, hipStream_t stream) {
 //   variant 0: eight waves (nhw = 2) wherever a group has an even number of heads, else one head per item
 //   variant 1: one head per item, four waves
 //   variant 2: four waves with two heads each where their registers fit (head dim <= 128), else as 1
+//   variant 4: the spread kernel (tree_attn_spread.hip), two heads of a group per item where it has an even number
 void pick_kernel(int hq, int hkv, int d, int variant, int* rt, int* nhw) {
     const bool pairs = (hq / hkv) % 2 == 0;
     *rt = 1;
     *nhw = 1;
+    if (variant == 4) { *nhw = pairs ? 2 : 1; return; }
     if (d > 256) return;   // head dim 512: one head per item, the single-pass kernel
     if ((variant == 0 || variant == 3) && pairs) *nhw = 2;
     if (variant == 2 && pairs && d <= 128) *rt = 2;
@@ -766,6 +781,16 @@ int launch_ring(const AttnParams& p, int d, bool win, int n_wg, hipStream_t stre
         if (e0 != hipSuccess) return spinf_fail(SPINF_E_HIP, "tree_attn: launch (clear): %s", hipGetErrorString(e0));
     }
     return spinf_launch_ring(p, d, win, n_wg, stream);
+}
+
+// The spread kernel (tree_attn_spread.hip): one launch, no cursors, no second kernel either.
+int launch_spread(const AttnParams& p, int d, int heads, bool win, int ktile, long n_items, hipStream_t stream) {
+    if (p.clear_first) {
+        hipLaunchKernelGGL(attn_clear_counters_kernel, dim3(1), dim3(64), 0, stream, p.counters);
+        hipError_t e0 = hipGetLastError();
+        if (e0 != hipSuccess) return spinf_fail(SPINF_E_HIP, "tree_attn: launch (clear): %s", hipGetErrorString(e0));
+    }
+    return spinf_launch_spread(p, d, heads, win, ktile, n_items, stream);
 }
 
 int launch_d512(const AttnParams& p, bool win, int grp_mode, int blocks, hipStream_t s) {
@@ -843,6 +868,10 @@ static int attn_fwd(const spinf_attn_args* a, void* stream, bool no_alloc) {
     // the ring kernel: a static schedule over 32-key entries (head dim 256 and 512), or variant 3 at head dim 128 (64-key entries)
     const bool ring128 = a->variant == 3;
     const bool ring = a->n_lists > 0 && (a->ktile == 32 || ring128);
+    const bool spread = a->variant == 4;
+    if (spread && (a->n_lists > 0 || a->grp || (a->ktile != 0 && a->ktile != 32 && a->ktile != 64) || (a->row_of && a->ktile == 32 && a->d != 512)))
+        return spinf_fail(SPINF_E_ARG, "tree_attn: variant 4 (the spread kernel) takes the eight shared lists, no image groups, and plan entries of 64 or 32 keys (compact "
+                                       "rows: of 32 at head dim 512 only)");
     if (ring128 && !(a->d == 128 && a->n_lists > 0 && (a->ktile == 0 || a->ktile == 64) && nhw == 2 && rt == 1 && !a->row_of && !a->grp))
         return spinf_fail(SPINF_E_ARG, "tree_attn: variant 3 (the kernel with decoupled waves at head dim 128) takes head dim 128, an even number of query heads per "
                                        "key / value head, a static schedule over 64-key entries, the stream layout and no image groups");
@@ -850,7 +879,7 @@ static int attn_fwd(const spinf_attn_args* a, void* stream, bool no_alloc) {
         if (!((a->d == 256 && nhw == 2 && rt == 1) || a->d == 512) || a->row_of || a->grp)
             return spinf_fail(SPINF_E_ARG, "tree_attn: a static schedule over 32-key entries goes with head dim 512, or head dim 256 with an even number of query heads "
                                            "per key / value head and variant 0; with the stream layout and no image groups");
-    } else if ((a->d == 512) != (a->ktile == 32) || (a->ktile != 0 && a->ktile != 32 && a->ktile != 64))
+    } else if (!spread && ((a->d == 512) != (a->ktile == 32) || (a->ktile != 0 && a->ktile != 32 && a->ktile != 64)))
         return spinf_fail(SPINF_E_ARG, "tree_attn: plan entries of %d keys with head dim %d (32 goes with 512, 64 with the others)", a->ktile ? a->ktile : 64, a->d);
     if (a->grp && (a->grp_mode != 1 && a->grp_mode != 2)) return spinf_fail(SPINF_E_ARG, "tree_attn: group mode %d not in {1, 2}", a->grp_mode);
     if (a->grp && a->grp_mode == 2 && a->window <= 0)
@@ -889,8 +918,8 @@ static int attn_fwd(const spinf_attn_args* a, void* stream, bool no_alloc) {
     // A block's cursors are zero: it was cleared when allocated, and every call's exact-pass kernel, which runs after the fast pass,
     // puts them back.  Only a block whose last call failed to get its kernels onto the stream is cleared first; so is the scratch
     // array of the entry point that allocates nothing, which every caller on the GPU shares.
-    // (the ring kernel uses no cursors: only a block left dirty is cleared in front of it, for the calls that follow)
-    p.clear_first = ring ? dirty : no_alloc || dirty;
+    // (the ring kernel and the spread kernel use no cursors: only a block left dirty is cleared in front of it, for the calls that follow)
+    p.clear_first = ring || spread ? dirty : no_alloc || dirty;
     p.static_lists = a->n_lists > 0;
     p.q = (const __bf16*)a->q; p.k = (const __bf16*)a->k; p.v = (const __bf16*)a->v; p.o = (__bf16*)a->out;
     p.q_tok = a->q_tok; p.q_head = a->q_head; p.k_tok = a->k_tok; p.k_head = a->k_head;
@@ -910,6 +939,7 @@ static int attn_fwd(const spinf_attn_args* a, void* stream, bool no_alloc) {
     const bool win = p.window > 0;
     int rc;
     if (ring) rc = launch_ring(p, a->d, win, a->n_lists, s);
+    else if (spread) rc = launch_spread(p, a->d, hpi, win, a->ktile ? a->ktile : 64, (long)a->n_items, s);
     else switch (a->d) {
         case 64: rc = launch_d<64>(p, rt, nhw, win, a->grp_mode, blocks, s); break;
         case 128: rc = launch_d<128>(p, rt, nhw, win, a->grp_mode, blocks, s); break;

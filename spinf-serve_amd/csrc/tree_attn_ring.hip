@@ -276,8 +276,8 @@ __device__ __forceinline__ void ring_paced_pass(const AttnParams& p, char* const
         const int tz = it_t | (int)((unsigned)it_z >> 20 << 20);
         const int kvh = (int)((unsigned)it_z >> 20) * HPI / p.group;
         ring_load_q<D, WIN>(p, wr, wh, tz, qf, art_q, pos_q);
-        float M = -INFINITY, l = 0.f;
-        bool viol = false;
+        float M = -INFINITY, l = 0.f, Mf = -INFINITY;
+        bool viol = false;   // (in the exact recomputation too: the ring pass's test on its numbers says which waves' rows are done again)
         acc_zero<NDT>();
 #pragma unroll 1
         for (int e = 0; e < ne; e++) {
@@ -332,6 +332,12 @@ __device__ __forceinline__ void ring_paced_pass(const AttnParams& p, char* const
                 for (int i2 = 1; i2 < 16; i2++) mx = fmaxf(mx, sa[i2]);
                 mx = lane32_max(mx);
                 const float tm = mx * p.c;
+                Mf = Mf == -INFINITY ? tm : Mf;
+                const float msf = Mf == -INFINITY ? 0.f : Mf;
+                float sumf = 0.f;
+#pragma unroll
+                for (int i2 = 0; i2 < 16; i2++) sumf += __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i2], p.c, -msf));
+                viol = viol | !(sumf <= VIOL_SUM);
                 const bool up = tm > M + TAU_LAZY;
                 const float mn = up ? tm : M;
                 const float alpha = up ? __builtin_amdgcn_exp2f(M - mn) : 1.0f;
@@ -385,9 +391,10 @@ __device__ __forceinline__ void ring_paced_pass(const AttnParams& p, char* const
             pv_steps<NVF>(step);
             }
         }
-        if (!exact && __builtin_amdgcn_ballot_w64(viol) != 0) {   // scores ranged too widely somewhere in these 32 rows: the item is done again, exactly
+        const bool far = __builtin_amdgcn_ballot_w64(viol) != 0;   // scores ranged too widely somewhere in these 32 rows: done again, exactly
+        if (!exact && far) {
             if (fresh_lane_id() == 0) __hip_atomic_store(sy_vote, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        } else {
+        } else if (!exact || far) {   // (the item's other rows keep the fast pass's output)
             ring_store_rows<D>(p, wr, wh, stage, tz, l);
         }
         if (exact) {

@@ -35,6 +35,10 @@ RING_MAX_ITEMS_PER_WG = 8
 # head dim 128: the kernel with decoupled waves over 64-key tiles (the library's variant 3) where the geometry allows
 RING_128 = False
 
+# the kernel that spreads a row group over a workgroup (variant 4), for short streams (0: never, 1: wherever it takes the call)
+SPREAD = int(os.environ.get("SPINF_ATTN_SPREAD", "-1"))  # -1 = auto
+SPREAD_MAX_ITEMS_PER_CU = 0.625
+
 # test hook (spinf_attn_args.debug_expire): k > 0 = polls after which a wave of the decoupled kernel gives up a wait (2^18 otherwise)
 DEBUG_EXPIRE = 0
 
@@ -85,6 +89,24 @@ def _ring_lists(device, hq, hkv, d, variant, compact, mask):
     if ring or static:
         return n_wg, ring
     return 0, False
+
+
+def _spread(device, hq, hkv, d, variant, mask) -> bool:
+    """does the call go to the spread kernel?  It shortens the chain of key blocks a row waits for, at about half the other kernels'
+    throughput: a gain while the GPU has idle compute units.  Measured on MI355X (GPU time per call, spread against the kernel that took
+    the call before; a work item = 128 rows x 2 heads, 256 compute units): head dim 256, 40 items 17.3 / 36.4 us, 88 items 37.4 / 75.3, 168
+    items 48.3 / 50.1, 336 items 94 / 66; compact rows, 132 items 59.7 / 83.6, 252 items 80.6 / 61.9; head dim 128, 96 items 17.9 / 31.2, 176
+    items 45.3 / 64.4, 320 items 59.5 / 53.3; head dim 64, 88 items 27.3 / 54.0, 168 items 31.6 / 35.4, 336 items 53 / 49."""
+    if variant == 4:
+        return True
+    if variant != 0 or d == 512 or mask.grp is not None or not SPREAD or RING >= 0 or STATIC >= 0:
+        return False
+    if SPREAD > 0:
+        return True
+    from .masks import _static_lists
+
+    per_item = 2 if (hq // hkv) % 2 == 0 else 1
+    return mask.n_qtiles * (hq // per_item) <= SPREAD_MAX_ITEMS_PER_CU * _static_lists(device)
 
 
 def _attn_args(q, k, v, out, n, art, end, pos, kv_idx, kv_bits, items, list_ptr, n_items, scale, window, variant, row_of, kv_row0, grp, grp_mode, ktile, n_lists=0):
@@ -153,7 +175,10 @@ class _Layer:
     that does not belong to one layer's tensors (the mask owns the memory it points to)"""
 
     def __init__(self, mask, hq, hkv, d, variant, compact, device):
-        n_lists, ring = _ring_lists(device, hq, hkv, d, variant, compact, mask)
+        if _spread(device, hq, hkv, d, variant, mask):
+            variant, n_lists, ring = 4, 0, False
+        else:
+            n_lists, ring = _ring_lists(device, hq, hkv, d, variant, compact, mask)
         if ring and d == 128:
             variant = 3   # (64-key plan entries, as the lockstep kernels take)
         self.ring = ring and d != 128
@@ -174,7 +199,7 @@ class _Layer:
     @classmethod
     def of(cls, mask, q, k, variant, compact):
         hq, hkv, d = q.shape[1], k.shape[1], q.shape[2]
-        key = (hq, hkv, d, variant, compact, RING, STATIC, RING_128)
+        key = (hq, hkv, d, variant, compact, RING, STATIC, RING_128, SPREAD)
         got = mask._layers.get(key)
         if got is None:
             got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, q.device)

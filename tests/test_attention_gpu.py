@@ -770,3 +770,58 @@ def test_a_wave_that_gives_up_a_wait_costs_time_not_rows(dev, d, limit, wide, mo
         again = sa.tree_attn(q, k, v, mask, cfg.scale)   # and the next launch starts clean
         torch.cuda.synchronize()
         assert torch.equal(again, want) and _ring_aborts() == before + (_ring_aborts() - before)
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(64, 4, 1), (128, 4, 2), (256, 4, 2), (256, 6, 2), (256, 3, 3), (128, 3, 1)])
+@pytest.mark.parametrize("window", [None, 150])
+def test_spread_kernel_gives_the_lockstep_bits(dev, d, hq, hkv, window, monkeypatch):
+    """the kernel that spreads a row group over a workgroup against the lockstep kernel, bit for bit: a trunk longer than one segment of
+    its block list would need 16,384 keys, so the list is exercised by ragged ends (a stream that ends inside a query tile and a key block,
+    jobs packed without alignment, an odd number of key blocks), with wide scores in a stretch of keys (its own exact recomputation), in
+    stream layout and over compact rows"""
+    from spinf_serve_amd import attention
+
+    rng = np.random.default_rng(17)
+    trees = [synth._tree(rng, 333, [30, 11, 64, 5]), synth._tree(rng, 1, [3]), synth._tree(rng, 150, [9, 40]), synth._tree(rng, 70, [])]
+    for align, cut in ((True, 0), (True, 37), (False, 21)):
+        cfg = synth.AttnConfig("spread", hq, hkv, d, d ** -0.5, 1.0, None, trees)
+        b = synth.pack(trees, align=align)[0]
+        n = b.length - cut
+        q, k, v = (t[:n].contiguous() for t in synth.qkv(cfg, b, seed=6, device=dev))
+        mask = sa.TreeMask.build(b.art[:n], np.minimum(b.end[:n], n), b.pos[:n], window=window, device=dev)
+        sidx = torch.from_numpy(np.flatnonzero(b.art[:n] >= 0)).to(dev)
+        for wide in (1.0, 60.0):
+            kw = k.clone()
+            kw[200:280] *= wide
+            outs = []
+            for ring, spread in ((0, 0), (-1, 1)):
+                monkeypatch.setattr(attention, "RING", ring)
+                monkeypatch.setattr(attention, "SPREAD", spread)
+                print(f"case spread d={d} {hq}/{hkv} n={n} wide={wide} spread={spread}", flush=True)
+                before = _exact_items()
+                outs.append((sa.tree_attn(q, kw, v, mask, cfg.scale), sa.tree_attn(*(t[sidx].contiguous() for t in (q, kw, v)), mask, cfg.scale, sidx=sidx)))
+                torch.cuda.synchronize()
+                assert (_exact_items() > before) == (wide > 1)
+            assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+def test_spread_kernel_on_a_list_of_several_segments(dev, monkeypatch):
+    """16,600 keys: more key blocks than the spread kernel lists at a time; against the lockstep kernel, with and without wide scores"""
+    from spinf_serve_amd import attention
+
+    rng = np.random.default_rng(18)
+    trees = [synth._tree(rng, 16600, [5, 40])]
+    cfg = synth.AttnConfig("long", 2, 1, 64, 0.125, 1.0, None, trees)
+    b = synth.pack(trees)[0]
+    q, k, v = synth.qkv(cfg, b, seed=2, device=dev)
+    mask = sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
+    for wide in (1.0, 60.0):
+        kw = k.clone()
+        kw[16430:16450] *= wide
+        outs = []
+        for spread in (0, 1):
+            monkeypatch.setattr(attention, "SPREAD", spread)
+            print(f"case spread segments wide={wide} spread={spread}", flush=True)
+            outs.append(sa.tree_attn(q, kw, v, mask, cfg.scale))
+            torch.cuda.synchronize()
+        assert torch.equal(outs[0], outs[1])
