@@ -371,28 +371,26 @@ extern "C" int spinf_tileplan_schedule_static(const spinf_tileplan* p, int32_t h
         }
         // the workgroup of a list that is free first (the lowest numbered of equals) takes its next item: a heap per list
         const int nl = std::min<int32_t>(8, n_lists);
-        std::vector<std::vector<int32_t>> mine((size_t)n_lists);
+        std::vector<int32_t> owner((size_t)std::max<int64_t>(1, nqt * head_groups));
         std::vector<std::vector<std::pair<float, int>>> free_at((size_t)nl);
+        for (auto& f : free_at) f.reserve((size_t)n_lists / nl + 1);
         for (int w = 0; w < n_lists; w++) free_at[w % nl].emplace_back(0.f, w);
+        for (int w = 0; w <= n_lists; w++) list_ptr[w] = 0;
         const auto later = std::greater<std::pair<float, int>>();
         for (auto& f : free_at) std::make_heap(f.begin(), f.end(), later);
         for (int l = 0; l < 8; l++)
             for (int64_t i = lp[l]; i < lp[l + 1]; i++) {
                 auto& f = free_at[l % nl];
                 std::pop_heap(f.begin(), f.end(), later);
-                mine[f.back().second].push_back((int32_t)i);
+                owner[i] = f.back().second;
+                list_ptr[owner[i] + 1]++;
                 f.back().first += cost[base[4 * i]];
                 std::push_heap(f.begin(), f.end(), later);
             }
-        int64_t k = 0;
-        for (int w = 0; w < n_lists; w++) {
-            list_ptr[w] = (int32_t)k;
-            for (int32_t i : mine[w]) {
-                std::memcpy(items + 4 * k, base.data() + 4 * (int64_t)i, 4 * sizeof(int32_t));
-                k++;
-            }
-        }
-        list_ptr[n_lists] = (int32_t)k;
+        for (int w = 0; w < n_lists; w++) list_ptr[w + 1] += list_ptr[w];
+        std::vector<int32_t> fill(list_ptr, list_ptr + n_lists);
+        for (int l = 0; l < 8; l++)
+            for (int64_t i = lp[l]; i < lp[l + 1]; i++) std::memcpy(items + 4 * (int64_t)fill[owner[i]]++, base.data() + 4 * i, 4 * sizeof(int32_t));
     } catch (const std::bad_alloc&) {
         return spinf_fail(SPINF_E_NOMEM, "tileplan_schedule_static: out of memory");
     }

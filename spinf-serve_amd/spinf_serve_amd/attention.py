@@ -186,35 +186,66 @@ class _Layer:
         per_item = _lib.load_library().spinf_attn_heads_per_item(hq, hkv, d, variant)
         if per_item <= 0:
             raise ValueError(f"{hq} query heads do not group over {hkv} key / value heads")
-        self.items, self.list_ptr, self.n_items = m.schedule(hq // per_item, n_lists)
-        self.variant, self.n_lists = variant, n_lists
+        self.head_groups, self.variant, self.n_lists = hq // per_item, variant, n_lists
         a = self.args = _lib.AttnArgs()
         a.n, a.hq, a.hkv, a.d, a.window = m.n, hq, hkv, d, m.window
         a.art, a.end, a.pos = m.art.data_ptr(), m.end.data_ptr(), m.pos.data_ptr()
-        a.kv_idx, a.kv_bits, a.items, a.list_ptr = m.kv_idx.data_ptr(), m.kv_bits.data_ptr(), self.items.data_ptr(), self.list_ptr.data_ptr()
-        a.n_items, a.variant, a.ktile, a.n_lists = self.n_items, variant, m._ktile, n_lists
+        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items = m.pointers(self.head_groups, n_lists)
+        a.variant, a.ktile, a.n_lists = variant, m._ktile, n_lists
         if m.grp is not None:
             a.grp, a.grp_mode = m.grp.data_ptr(), m.grp_mode
 
     @classmethod
-    def of(cls, mask, q, k, variant, compact):
-        hq, hkv, d = q.shape[1], k.shape[1], q.shape[2]
+    def of(cls, mask, hq, hkv, d, variant, compact, device):
         key = (hq, hkv, d, variant, compact, RING, STATIC, RING_128, SPREAD)
         got = mask._layers.get(key)
         if got is None:
-            got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, q.device)
+            got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, device)
         return got
 
-    def bound(self, q, k, v, out, scale):
-        """the argument block of one call (a block of its own: calls may come from several threads)"""
+    def bound(self, q, qs, k, ks, v, vs, out, os, scale):
+        """the argument block of one call (a block of its own: calls may come from several threads); qs, ..: token and head stride"""
         a = _lib.AttnArgs.from_buffer_copy(self.args)
         a.q, a.k, a.v, a.out = q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr()
-        a.q_tok, a.q_head, _ = q.stride()
-        a.k_tok, a.k_head, _ = k.stride()
-        a.v_tok, a.v_head, _ = v.stride()
-        a.o_tok, a.o_head, _ = out.stride()
+        a.q_tok, a.q_head = qs
+        a.k_tok, a.k_head = ks
+        a.v_tok, a.v_head = vs
+        a.o_tok, a.o_head = os
         a.scale, a.debug_expire = scale, DEBUG_EXPIRE
         return a
+
+
+def _heads_first(q, k, v, mask, scale, sidx):
+    """tree_attn for the model layers' layout: q [1, hq, rows, d], k / v [1, hkv, rows, d] -> [1, rows, hq, d], or None for anything that is not
+    plain (then the general path takes the call, and names what is wrong with it).  The views into token-major layout and the general
+    path's checks were 8 of a call's 17 us of host time."""
+    bf16 = torch.bfloat16
+    if not (type(mask) is TreeMask and q.dtype is bf16 and k.dtype is bf16 and v.dtype is bf16 and q.dim() == 4 and _lib.eager(q, k, v, sidx)):
+        return None
+    one, hq, rows, d = q.shape
+    ks, dev = k.shape, q.device
+    if not (one == 1 and len(ks) == 4 and ks[0] == 1 and ks[2] == rows and ks[3] == d and v.shape == ks and hq % ks[1] == 0
+            and k.device == dev and v.device == dev and mask.art.device == dev and dev.type == "cuda"):
+        return None
+    qs, kst, vs = q.stride(), k.stride(), v.stride()
+    if qs[3] != 1 or kst[3] != 1 or vs[3] != 1:
+        return None
+    if sidx is None:
+        if rows != mask.n:
+            return None
+    elif mask.grp is not None or sidx.shape[0] > rows or sidx.device != dev:
+        return None
+    variant = VARIANT if VARIANT != 2 or (sidx is None and mask.grp is None) else 0
+    layer = _Layer.of(mask, hq, ks[1], d, variant, sidx is not None, dev)
+    out = torch.empty((1, rows, hq, d), dtype=bf16, device=dev)
+    a = layer.bound(q, (qs[2], qs[1]), k, (kst[2], kst[1]), v, (vs[2], vs[1]), out, (hq * d, d), float(d ** -0.5 if scale is None else scale))
+    if sidx is not None:
+        if sidx.shape[0] < rows:
+            out[0, sidx.shape[0] :].zero_()
+        row_of, kv_row0 = mask.for_head_dim(d, ring=layer.ring).rows(sidx)
+        a.row_of, a.kv_row0 = row_of.data_ptr(), kv_row0.data_ptr()
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, dev, "spinf_tree_attn_fwd")
+    return out
 
 
 def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
@@ -232,15 +263,16 @@ def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
         variant = 0   # the two-heads-per-wave kernels take neither compact rows nor image groups
     if sidx is not None and mask.grp is not None:
         raise ValueError("image groups go with the stream layout (no sidx)")
-    layer = _Layer.of(mask, q, k, variant, sidx is not None)
+    layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], variant, sidx is not None, q.device)
     m = mask.for_head_dim(q.shape[2], ring=layer.ring)   # the plan of the kernel's key-tile size
     row_of, kv_row0 = m.rows(sidx) if sidx is not None else (None, None)
     if not _lib.eager(q, k, v, sidx):
-        return _tree_attn_op(q, k, v, m.art, m.end, m.pos, m.kv_idx, m.kv_bits, layer.items, layer.list_ptr, layer.n_items,
+        items, list_ptr, n_items = m.schedule(layer.head_groups, layer.n_lists)
+        return _tree_attn_op(q, k, v, m.art, m.end, m.pos, m.kv_idx, m.kv_bits, items, list_ptr, n_items,
                              scale, int(m.window), layer.variant, row_of, kv_row0, 0 if sidx is None else int(sidx.shape[0]),
                              m.grp, int(m.grp_mode), int(m._ktile), layer.n_lists)
     out = torch.empty(q.shape, dtype=torch.bfloat16, device=q.device)
-    a = layer.bound(q, k, v, out, scale)
+    a = layer.bound(q, q.stride()[:2], k, k.stride()[:2], v, v.stride()[:2], out, out.stride()[:2], scale)
     if sidx is not None:
         if sidx.shape[0] < q.shape[0]:
             out[sidx.shape[0] :].zero_()
@@ -259,7 +291,8 @@ def tree_attn_noalloc(q, k, v, mask: TreeMask, out, scale=None):
     if out.shape != q.shape or out.dtype != torch.bfloat16 or not out.is_contiguous():
         raise ValueError("out must be a contiguous bf16 tensor of q's shape")
     _check_tensors(q, k, v, mask.n, False, (out, mask.art))
-    a = _Layer.of(mask, q, k, 0, False).bound(q, k, v, out, float(q.shape[-1] ** -0.5 if scale is None else scale))
+    layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], 0, False, q.device)
+    a = layer.bound(q, q.stride()[:2], k, k.stride()[:2], v, v.stride()[:2], out, out.stride()[:2], float(q.shape[-1] ** -0.5 if scale is None else scale))
     _lib.launch(_lib.load_library().spinf_tree_attn_fwd_noalloc, a, q.device, "spinf_tree_attn_fwd_noalloc")
     return out
 
@@ -318,6 +351,9 @@ def tree_flex_forward(module, query, key, value, attention_mask, scaling=None, s
             cap["kv"].setdefault(name, {})[module.layer_idx] = (key[:, :, a : start + n].clone(), value[:, :, a : start + n].clone())
     if query.shape[0] != 1:
         raise ValueError("the packed stream is one sequence: batch size must be 1")
+    out = _heads_first(query, key, value, attention_mask, scaling, None)
+    if out is not None:
+        return out, None
     out = tree_attn(query[0].transpose(0, 1), key[0].transpose(0, 1), value[0].transpose(0, 1), attention_mask, scaling)
     return out[None], None
 
@@ -340,6 +376,9 @@ def tree_attention(q, k, v, mask, scale, sidx=None, plan=None, mod=None):
     if cap is not None:
         for r0, n, name in cap["ranges"]:
             cap["out"]["kv"].setdefault(name, {})[mod.li] = (k[:, :, r0 : r0 + n].clone(), v[:, :, r0 : r0 + n].clone())
+    out = _heads_first(q, k, v, mask, scale, sidx)
+    if out is not None:
+        return out.transpose(1, 2)
     if sidx is None:
         o = tree_attn(q[0].transpose(0, 1), k[0].transpose(0, 1), v[0].transpose(0, 1), mask, scale)
         return o.transpose(0, 1)[None]

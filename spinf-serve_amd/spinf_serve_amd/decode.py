@@ -84,11 +84,9 @@ class GroupKV:
     def update(self, key_states, value_states, layer_idx, *args, **kwargs):
         c = self.caches  # key_states [G, h, Q, d] -> entry step of every query's generated K/V
         gk, gv = c.gk[layer_idx], c.gv[layer_idx]
-        if _puttable(key_states, value_states, gk, gv, c.step_t):   # one launch for both
-            G, h, Q, S, d = gk.shape
-            _lib.launch(_lib.load_library().spinf_xdecode_put,
-                        (key_states.data_ptr(), *key_states.stride()[:3], value_states.data_ptr(), *value_states.stride()[:3], gk.data_ptr(), gv.data_ptr(),
-                         c.step_t.data_ptr(), G, h, Q, S, d), gk.device, "spinf_xdecode_put")
+        put = _put_args(key_states, value_states, gk, gv, c.step_t)
+        if put is not None:   # one launch for both
+            _lib.launch(_lib.load_library().spinf_xdecode_put, put, gk.device, "spinf_xdecode_put")
             return ("x", layer_idx), ("x", layer_idx)
         c.gk[layer_idx].index_copy_(3, c.step_t, key_states.unsqueeze(3))
         c.gv[layer_idx].index_copy_(3, c.step_t, value_states.unsqueeze(3))
@@ -98,14 +96,19 @@ class GroupKV:
         return 0
 
 
-def _puttable(k, v, gk, gv, step) -> bool:
-    """does spinf_xdecode_put take these tensors?  (bf16 with 16-byte rows, contiguous caches; anything else goes through index_copy_)"""
-    shape = gk.shape[:3] + gk.shape[4:]
-    if not (_lib.eager(k, v, gk, gv, step) and k.shape == shape and v.shape == shape and gk.shape == gv.shape and gk.is_cuda and shape[3] % 8 == 0 and step.numel() == 1):
-        return False
-    if any(t.dtype != torch.bfloat16 or t.device != gk.device or t.data_ptr() % 16 for t in (k, v, gk, gv)) or step.dtype != torch.int64 or step.device != gk.device:
-        return False
-    return gk.is_contiguous() and gv.is_contiguous() and all(t.stride(3) == 1 and not any(x % 8 for x in t.stride()[:3]) for t in (k, v))
+def _put_args(k, v, gk, gv, step):
+    """the arguments of spinf_xdecode_put for these tensors, or None where it does not take them (it wants bf16, 16-byte rows, contiguous
+    caches; anything else goes through index_copy_)"""
+    bf16, dev = torch.bfloat16, gk.device
+    if not (k.dtype is bf16 and v.dtype is bf16 and gk.dtype is bf16 and gv.dtype is bf16 and step.dtype is torch.int64 and step.numel() == 1
+            and gk.dim() == 5 and _lib.eager(k, v, gk, gv, step) and dev.type == "cuda"):
+        return None
+    G, h, Q, S, d = shape = gk.shape
+    ks, vs, ptrs = k.stride(), v.stride(), (k.data_ptr(), v.data_ptr(), gk.data_ptr(), gv.data_ptr())
+    if (gv.shape != shape or k.shape != (G, h, Q, d) or v.shape != k.shape or d % 8 or ks[3] != 1 or vs[3] != 1 or (ks[0] | ks[1] | ks[2] | vs[0] | vs[1] | vs[2]) % 8
+            or (ptrs[0] | ptrs[1] | ptrs[2] | ptrs[3]) % 16 or not (gk.is_contiguous() and gv.is_contiguous()) or k.device != dev or v.device != dev or gv.device != dev or step.device != dev):
+        return None
+    return (ptrs[0], *ks[:3], ptrs[1], *vs[:3], ptrs[2], ptrs[3], step.data_ptr(), G, h, Q, S, d)
 
 
 def _i32(t: Optional[torch.Tensor], what: str) -> Optional[torch.Tensor]:

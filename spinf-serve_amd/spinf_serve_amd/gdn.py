@@ -72,6 +72,23 @@ def _launch(mode, q, k, v, g, beta, scale, cu, n, h0, h0_idx, ht, ht_idx, idx, o
     return o
 
 
+def level_args(q, k, v, g, beta, o, scale):
+    """the argument block that the launches over one layer's tensors share (q, k [T, H, K], v, o [T, HV, V], g, beta [T, HV]), or None for
+    tensors that are not plain or not as the kernels take them (the call by call path names what is wrong)"""
+    bf16 = torch.bfloat16
+    if not (_lib.eager(q, k, v, g, beta) and q.is_cuda and q.dtype is bf16 and k.dtype is bf16 and v.dtype is bf16 and g.dtype is torch.float32 and beta.dtype is bf16):
+        return None
+    (T, H, K), (_, HV, V), qs, vs, gs = k.shape, v.shape, q.stride(), v.stride(), g.stride()
+    if not (q.shape == k.shape and v.shape[0] == T and g.shape == beta.shape == (T, HV) and k.stride() == qs and qs[1:] == (K, 1) and vs[1:] == (V, 1)
+            and o.stride()[1:] == (V, 1) and gs[1] == 1 and beta.stride() == gs and all(t.device == q.device for t in (k, v, g, beta))):
+        return None
+    a = _lib.GdnArgs()
+    a.q, a.k, a.v, a.g, a.beta, a.o = q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), o.data_ptr()
+    a.q_tok, a.v_tok, a.g_tok, a.o_tok = qs[0], vs[0], gs[0], o.stride(0)
+    a.h, a.hv, a.dk, a.dv, a.scale = H, HV, K, V, float(scale)
+    return a
+
+
 def recurrent(q, k, v, g, beta, scale, cu, n, h0=None, h0_idx=None, ht=None, ht_idx=None, idx=None, o=None):
     """q, k [1, rows, H, K], v [1, rows, HV, V], g / beta [1, rows, HV], cu [n + 1] int64 (device) -> o [1, rows, HV, V].
     idx [sum of lengths] int64: the call's tokens are these rows of the tensors and the outputs go to the same rows of `o`

@@ -144,7 +144,7 @@ class TreeMask:
         self.seq_lengths = (self.n, self.n)
         self.device = device
         self.art, self.end, self.pos = meta
-        self._kv = None                     # device copies of the plan's kv_idx, kv_bits
+        self._kv = None                     # the buffer with the device copies of the plan's kv_idx, kv_bits, and where they lie in it
         self._sched = {}
         self._layers = {}                   # prepared calls by head geometry (attention.py)
         self._rows = None
@@ -171,7 +171,8 @@ class TreeMask:
     def _entries(self):
         if self._kv is None:
             self._upload(1, 0)
-        return self._kv
+        dev, at = self._kv
+        return dev[at[2] : at[3]], dev[at[3] : at[4]]
 
     def for_head_dim(self, d: int, ring: bool = False) -> "TreeMask":
         """the mask with the plan granularity the kernel takes: 32-key entries at head dim 512 and for the kernel with decoupled
@@ -212,23 +213,31 @@ class TreeMask:
         from pinned memory of its own, was 11 copies and 150 us of a new stream's two masks.)"""
         plan, first = self.plan, self._kv is None
         ni, nl, ne, nq = 4 * max(plan.n_qtiles * head_groups, 1), (n_lists or 8) + 1, max(plan.n_entries, 1), plan.n_qtiles
-        at = [0, ni, ni + nl, ni + nl + ne, ni + nl + 2 * ne]   # items (16-byte aligned), list_ptr, kv_idx, kv_bits, host only: qt_ptr, order
-        used = at[4] if first else at[2]
+        at = (0, ni, ni + nl, ni + nl + ne, ni + nl + 2 * ne)   # items (16-byte aligned), list_ptr, kv_idx, kv_bits, host only: qt_ptr, order
         buf = _staging(at[4] + 2 * nq + 1 if first else at[2], self.device)
         p = buf.data_ptr()
         plan.schedule_into(head_groups, n_lists, p, p + 4 * at[1])
         if first:
             plan.export(p + 4 * at[4], p + 4 * at[2], p + 4 * at[3], p + 4 * (at[4] + nq + 1))
-        dev = buf[:used].to(self.device, non_blocking=True)
+            buf = buf[: at[4]]
+        dev = buf.to(self.device, non_blocking=True)
         if first:
-            self._kv = dev[at[2] : at[3]], dev[at[3] : at[4]]
-        got = self._sched[(head_groups, n_lists)] = (dev[:ni].view(-1, 4), dev[ni : at[2]], plan.n_qtiles * head_groups)
+            self._kv = dev, at
+        got = self._sched[(head_groups, n_lists)] = dev, at, plan.n_qtiles * head_groups
         return got
 
     def schedule(self, head_groups: int, n_lists: int = 0):
         """device copy of the work lists for this many head groups (built on first use, then kept); n_lists > 0: the static
         schedule for that many workgroups"""
-        return self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
+        dev, at, n_items = self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
+        return dev[: at[1]].view(-1, 4), dev[at[1] : at[2]], n_items
+
+    def pointers(self, head_groups: int, n_lists: int):
+        """-> device addresses of items, list_ptr, kv_idx, kv_bits, and the number of items"""
+        dev, at, n_items = self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
+        items, (kv, kv_at) = dev.data_ptr(), self._kv
+        kv = kv.data_ptr()
+        return items, items + 4 * at[1], kv + 4 * kv_at[2], kv + 4 * kv_at[3], n_items
 
     @classmethod
     def build(cls, art, end, pos, window=None, device="cuda", meta=None, grp=None, grp_windowed=False, grp_dev=None):

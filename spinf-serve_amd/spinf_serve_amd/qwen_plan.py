@@ -43,7 +43,7 @@ class TreePlan:
     seg_slot: object | None = None
     cap: dict | None = None
     pad_rows: object | None = None   # [pads] int64 (device): rows of the tensors no segment covers; their outputs are zero
-    launches: list | None = None     # indexed path: per level the kernel launches (tuples for gdn.launch), neighbouring calls of one kind as one
+    launches: list | None = None     # indexed path: per level the kernel launches (mode, segments, longest, addresses of cu, idx, h0_idx, ht_idx), neighbouring calls of one kind as one
 
 
 _PATHS = {"indexed": 0, "levels": 1}
@@ -132,11 +132,11 @@ def tree_plan(prev, real, device, max_init: int = 96, path: str = "indexed", sho
                 calls.append(Call(idx, cu, cu_cpu, starts, bool(call_keep[c])))
         levels.append(calls)
         merged = []
-        for i, j in lv:
-            idx, cu, _, starts, ends = cut(i, j) if indexed else (None,) * 5
-            if indexed:
-                lens = seg_len[seg_ptr[i] : seg_ptr[j]]
-                merged.append((int(call_kind[i]), cu, len(lens), starts if d else None, ends if call_keep[i:j].any() else None, idx, int(lens.max()) if call_kind[i] else 0))
+        for i, j in lv if indexed else ():
+            idx, cu, _, starts, ends = cut(i, j)
+            lens = seg_len[seg_ptr[i] : seg_ptr[j]]
+            merged.append((int(call_kind[i]), len(lens), int(lens.max()) if call_kind[i] else 0, cu.data_ptr(), idx.data_ptr(), starts.data_ptr() if d else None,
+                           ends.data_ptr() if call_keep[i:j].any() else None))   # (views of on_dev, which plan.conv keeps alive)
         launches.append(merged)
     seg_of_row = a["seg_of_row"]
     return TreePlan(conv.view(-1, 4), levels, a["n_segments"], path, a["n_keep"].tolist() if indexed else None, rows, sidx if rows is not None else None, seg_of_row,
@@ -182,15 +182,18 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
     g32 = g if g.dtype == torch.float32 else g.float()
     b16 = beta if beta.dtype == torch.bfloat16 else beta.to(torch.bfloat16)
     indexed = plan.path == "indexed"
-    direct = indexed and plan.launches is not None and _lib.eager(q, k, v, g, beta)
+    args = gdn.level_args(q, k, v, g32, b16, o, scale) if indexed and plan.launches is not None else None
     above = None   # the states the level above left
     for d, calls in enumerate(plan.levels):
         n_slots = plan.n_keep[d] if indexed else sum(len(c.cu_cpu) - 1 for c in calls if c.keep)
         states = q.new_empty((n_slots, v.shape[1], q.shape[-1], v.shape[-1]), dtype=torch.float32) if n_slots else None
         next_slot = 0
-        if direct:
-            for mode, cu, n_seg, h0_idx, ht_idx, idx, longest in plan.launches[d]:
-                gdn._launch(mode, q[None], k[None], v[None], g32[None], b16[None], scale, cu, n_seg, above, h0_idx, states, ht_idx, idx, o[None], longest)
+        if args is not None:
+            h0, ht = None if above is None else above.data_ptr(), None if states is None else states.data_ptr()
+            for args.mode, args.n_seg, args.max_len, args.cu, args.idx, h0_idx, ht_idx in plan.launches[d]:
+                args.h0, args.h0_idx = (h0, h0_idx) if h0_idx is not None else (None, None)
+                args.ht, args.ht_idx = (ht, ht_idx) if ht_idx is not None else (None, None)
+                _lib.launch(_lib.load_library().spinf_gdn_fwd, args, q.device, "spinf_gdn_fwd")
             calls = ()
         for c in calls:
             n_seg = len(c.cu_cpu) - 1
