@@ -311,6 +311,9 @@ typedef struct spinf_xdec_args {
 } spinf_xdec_args;
 /* suggested nsplit for these sizes (enough workgroups to fill the GPU) and the workspace it needs (0 for nsplit 1) */
 int spinf_xdecode_plan(const spinf_xdec_args* args, int32_t* nsplit, int64_t* workspace_bytes);
+/* split size and count for groups whose prefix / template ranges reach len_p[g] / len_t[g] entries (host arrays [G]): the pair for
+ * spinf_xdec_args.nsplit and tiles_per_split.  From G, H, h, Q, S, Lp, Tt, d, beam alone; host only. */
+int spinf_xdecode_plan_ragged(const spinf_xdec_args* args, const int32_t* len_p, const int32_t* len_t, int32_t* nsplit, int32_t* tiles_per_split);
 /* tiles of the longest list of these sizes (a group whose prefix and template ranges are full) */
 int spinf_xdecode_tiles(const spinf_xdec_args* args, int32_t* tiles);
 int spinf_xdecode_attn_fwd(const spinf_xdec_args* args, void* stream);

@@ -23,11 +23,16 @@
 // ds_read_b64_tr_b16.  A list longer than one split (XdecParams::per tiles) leaves (O, reference, sum) per row and split in a
 // workspace and xdec_combine_kernel merges them; a list that fits one split is written out by its one workgroup.
 //
-// Head dim 512: the output is computed 256 head dims at a time, in two launches (see launch_d).
+// Head dim 512: a workgroup computes 256 of the output's head dims (see launch_d).
 //
 // A row's result depends on its own keys only (fixed tile order, masked entries are exact zeros), so a group's outputs do
 // not depend on which other groups share the call.
 #include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <functional>
+#include <new>
+#include <vector>
 
 #include "spinf_tree.h"
 #include "common.h"
@@ -56,7 +61,6 @@ struct XdecParams {
     float* part_o; float* part_ml;
     int G, H, h, r, Q, Lp, Tt, S, beam, window;
     int R, nchunk, nsplit, per;
-    int vcol;   // first of the DV value / output head dims this launch computes (head dim 512: two launches of 256)
     float c, cap_in, cap_out;
 };
 
@@ -113,6 +117,7 @@ __global__ __launch_bounds__(256, D <= 256 ? 2 : 1) void xdec_kernel(const XdecP
     const int chunk = blockIdx.x / per_chunk;
     const int rest = blockIdx.x - chunk * per_chunk;
     const int split = rest % p.nsplit, gh = rest / p.nsplit;
+    const int vcol = DV < D ? blockIdx.y * DV : 0;   // first of the DV value / output head dims of this workgroup
     const int g = gh / p.h, hh = gh - g * p.h;
 
     const int row0 = chunk * XROWS + 32 * w;
@@ -171,7 +176,7 @@ __global__ __launch_bounds__(256, D <= 256 ? 2 : 1) void xdec_kernel(const XdecP
         if (which >= 0) {   // the usual case: a wave-uniform base, no vector arithmetic on addresses
             const long first = which == 0 ? (long)gh * p.Lp + k0 : which == 1 ? (long)gh * p.Tt + (k0 - p.Lp) : (long)gh * p.Q * p.S + (k0 - lk);
             const char* kb = (const char*)(which == 0 ? p.kp : which == 1 ? p.kt : p.gk) + first * (D * 2);
-            const char* vb = (const char*)(which == 0 ? p.vp : which == 1 ? p.vt : p.gv) + first * (D * 2) + p.vcol * 2;
+            const char* vb = (const char*)(which == 0 ? p.vp : which == 1 ? p.vt : p.gv) + first * (D * 2) + vcol * 2;
 #pragma unroll
             for (int i = 0; i < IPWK; i++) {
                 const int reg = w * IPWK + i;
@@ -200,7 +205,7 @@ __global__ __launch_bounds__(256, D <= 256 ? 2 : 1) void xdec_kernel(const XdecP
             for (int i = 0; i < IPWV; i++) {
                 const int reg = w * IPWV + i;
                 int wh;
-                const long off = locate(k0 + reg + GV::NREG * (lane / GV::CPR), wh) + (lane % GV::CPR) * 8 + p.vcol;
+                const long off = locate(k0 + reg + GV::NREG * (lane / GV::CPR), wh) + (lane % GV::CPR) * 8 + vcol;
                 dma16_lane((wh == 0 ? vp_s : wh == 1 ? vt_s : gv_s) + off * 2, buf + KTILEB + reg * GV::VRS);
             }
         }
@@ -348,7 +353,7 @@ __global__ __launch_bounds__(256, D <= 256 ? 2 : 1) void xdec_kernel(const XdecP
     if (!valid) return;
     if (p.nsplit == 1 || tl.nt <= p.per) {   // the list's only split: the output itself (lists longer than p.per leave partial results)
         const float inv = 1.0f / lsum;
-        __bf16* ob = p.out + (((long)g * p.Q + qi) * p.H + head) * D + p.vcol;
+        __bf16* ob = p.out + (((long)g * p.Q + qi) * p.H + head) * D + vcol;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
@@ -360,22 +365,22 @@ __global__ __launch_bounds__(256, D <= 256 ? 2 : 1) void xdec_kernel(const XdecP
             }
     } else {
         const long prow = (((long)g * p.H + head) * p.Q + qi) * p.nsplit + split;
-        float* po = p.part_o + prow * DV;
+        float* po = p.part_o + prow * D + vcol;
 #pragma unroll
         for (int dt = 0; dt < NDT; dt++)
 #pragma unroll
             for (int i4 = 0; i4 < 4; i4++)
                 *(float4*)(po + 32 * dt + 8 * i4 + 4 * g2) = make_float4(o[dt][4 * i4], o[dt][4 * i4 + 1], o[dt][4 * i4 + 2], o[dt][4 * i4 + 3]);
-        if (g2 == 0) *(float2*)(p.part_ml + prow * 2) = make_float2(M, lsum);
+        if (g2 == 0 && vcol == 0) *(float2*)(p.part_ml + prow * 2) = make_float2(M, lsum);   // (the same in every workgroup of the row)
     }
 }
 
 // out = sum_s 2^(M_s - M*) O_s / sum_s 2^(M_s - M*) l_s over the splits of a row, splits in ascending order; one thread per 4 head dims
-template <int D, int DV>
+template <int D>
 __global__ __launch_bounds__(256) void xdec_combine_kernel(const XdecParams p, const long n_rows) {
     const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-    const long rowid = idx / (DV / 4);
-    const int d4 = (int)(idx - rowid * (DV / 4));
+    const long rowid = idx / (D / 4);
+    const int d4 = (int)(idx - rowid * (D / 4));
     if (rowid >= n_rows) return;
     const long gg = rowid / ((long)p.H * p.Q);
     const int head = (int)((rowid / p.Q) % p.H), qi = (int)(rowid % p.Q);
@@ -394,14 +399,14 @@ __global__ __launch_bounds__(256) void xdec_combine_kernel(const XdecParams p, c
         const float ms = ml[2 * s];
         if (ms == -INFINITY) continue;
         const float wgt = __builtin_amdgcn_exp2f(ms - mstar);
-        const float4 x = *(const float4*)(p.part_o + (rowid * p.nsplit + s) * DV + 4 * d4);
+        const float4 x = *(const float4*)(p.part_o + (rowid * p.nsplit + s) * D + 4 * d4);
         acc.x += wgt * x.x; acc.y += wgt * x.y; acc.z += wgt * x.z; acc.w += wgt * x.w;
         lsum += wgt * ml[2 * s + 1];
     }
     const float inv = 1.0f / lsum;
     bf16x4 r;
     r[0] = (__bf16)(acc.x * inv); r[1] = (__bf16)(acc.y * inv); r[2] = (__bf16)(acc.z * inv); r[3] = (__bf16)(acc.w * inv);
-    *(bf16x4*)(p.out + ((gg * p.Q + qi) * p.H + head) * D + p.vcol + 4 * d4) = r;
+    *(bf16x4*)(p.out + ((gg * p.Q + qi) * p.H + head) * D + 4 * d4) = r;
 }
 
 // The new tokens' keys (blockIdx.y 0) and values (1) into entry `step` of the generated caches: one thread per 16 bytes.  Latency bound:
@@ -440,26 +445,24 @@ int check_args(const spinf_xdec_args* a) {
 int n_chunks(const spinf_xdec_args* a) { return (int)(((int64_t)a->Q * (a->H / a->h) + XROWS - 1) / XROWS); }
 
 // Head dim 512 (the Gemma-4 full-attention layers): O^T for 32 rows x 512 head dims would be 256 accumulator registers per lane
-// next to 128 of queries, so the output is computed 256 head dims at a time, in two launches: each computes the scores over all
-// 512 head dims and P V for one half of V's columns (DV = 256, XdecParams::vcol), in one workgroup per CU.
+// next to 128 of queries, so a workgroup computes 256 of them (DV = 256; the second half of the grid takes the others): each
+// computes the scores over all 512 head dims and P V for one half of V's columns, in one workgroup per CU.
 template <int D, int DV>
-int launch_d(XdecParams p, bool cap, int blocks, hipStream_t s) {
+int launch_d(const XdecParams& p, bool cap, int blocks, hipStream_t s) {
     const bool win = p.window > 0;
-    p.part_ml = p.part_o ? p.part_o + (long)p.G * p.H * p.Q * p.nsplit * DV : nullptr;
-    for (p.vcol = 0; p.vcol < D; p.vcol += DV) {
-        if (win && cap) hipLaunchKernelGGL((xdec_kernel<D, DV, true, true>), dim3(blocks), dim3(256), 0, s, p);
-        else if (win) hipLaunchKernelGGL((xdec_kernel<D, DV, true, false>), dim3(blocks), dim3(256), 0, s, p);
-        else if (cap) hipLaunchKernelGGL((xdec_kernel<D, DV, false, true>), dim3(blocks), dim3(256), 0, s, p);
-        else hipLaunchKernelGGL((xdec_kernel<D, DV, false, false>), dim3(blocks), dim3(256), 0, s, p);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "xdecode_attn: launch: %s", hipGetErrorString(e));
-        if (p.nsplit > 1) {
-            const long n_rows = (long)p.G * p.H * p.Q;
-            const long threads = n_rows * (DV / 4);
-            hipLaunchKernelGGL((xdec_combine_kernel<D, DV>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p, n_rows);
-            e = hipGetLastError();
-            if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "xdecode_attn: launch (combine): %s", hipGetErrorString(e));
-        }
+    const dim3 grid(blocks, D / DV);
+    if (win && cap) hipLaunchKernelGGL((xdec_kernel<D, DV, true, true>), grid, dim3(256), 0, s, p);
+    else if (win) hipLaunchKernelGGL((xdec_kernel<D, DV, true, false>), grid, dim3(256), 0, s, p);
+    else if (cap) hipLaunchKernelGGL((xdec_kernel<D, DV, false, true>), grid, dim3(256), 0, s, p);
+    else hipLaunchKernelGGL((xdec_kernel<D, DV, false, false>), grid, dim3(256), 0, s, p);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "xdecode_attn: launch: %s", hipGetErrorString(e));
+    if (p.nsplit > 1) {
+        const long n_rows = (long)p.G * p.H * p.Q;
+        const long threads = n_rows * (D / 4);
+        hipLaunchKernelGGL((xdec_combine_kernel<D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p, n_rows);
+        e = hipGetLastError();
+        if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "xdecode_attn: launch (combine): %s", hipGetErrorString(e));
     }
     return SPINF_OK;
 }
@@ -506,6 +509,75 @@ extern "C" int spinf_xdecode_plan(const spinf_xdec_args* a, int32_t* nsplit, int
         if (best < 0 || cost < best) { best = cost; *nsplit = ns; }
     }
     if (*nsplit > 1) *workspace_bytes = (int64_t)a->G * a->H * a->Q * *nsplit * (a->d + 2) * 4;
+    return SPINF_OK;
+}
+
+// Split size for groups of these lengths: the one with the shortest estimated step.  The estimate is the longer of (a) the schedule
+// (workgroups in launch order onto the places the GPU has; one costs FIX + its tiles +, of a split list, writing its partial results)
+// and (b) the step's bytes at what the memory delivers; a split step adds the merge launch and its reads.  The constants are a least-squares
+// fit to 400 measured steps (4 head geometries, 1 .. 48 groups, prefixes of 64 .. 4,000, splits of 1 .. 140 tiles; the choice is within 5 %
+// of the best measured split on average, the first version's was 20 % off: it charged a piece of a lone list the traffic of a full GPU and
+// cut nothing below 8 tiles.  One group with a 301-token prefix: head dim 256 33 -> 20 us, 128 25 -> 19, 512 131 -> 26, with both halves in one launch).
+extern "C" int spinf_xdecode_plan_ragged(const spinf_xdec_args* a, const int32_t* len_p, const int32_t* len_t, int32_t* nsplit, int32_t* tiles_per_split) {
+    const int rc = check_args(a);
+    if (rc) return rc;
+    if (!nsplit || !tiles_per_split || (a->G > 0 && (!len_p || !len_t))) return spinf_fail(SPINF_E_ARG, "xdecode_plan_ragged: null pointer");
+    *nsplit = 1;
+    const int nt_max = max_tiles(a);
+    *tiles_per_split = nt_max;
+    if (a->G == 0 || a->Q == 0 || nt_max == 0) return SPINF_OK;
+    const double FIX = 5.0, PART = 3.0, COMBINE = 3.7, BYTES_PER_US = 4.87e6, MERGE_BYTES_PER_US = 3.0e6;
+    const double tile_us = a->d == 512 ? 2.6 : a->d == 256 ? 2.2 : 1.6;
+    const int places = a->d == 512 ? 256 : a->d == 256 ? 512 : 1024, halves = a->d == 512 ? 2 : 1;
+    const int r = a->H / a->h;
+    const long R = (long)a->Q * r;
+    try {
+        struct List { int tiles; double part_bytes; };
+        std::vector<List> lists;
+        double mean = 0;
+        for (long row0 = 0; row0 < R; row0 += XROWS) {
+            const long last = row0 + XROWS - 1 < R ? row0 + XROWS - 1 : R - 1;
+            for (int g = 0; g < a->G; g++) {
+                const int lp = len_p[g] < 0 ? 0 : len_p[g] < a->Lp ? len_p[g] : a->Lp, lt = len_t[g] < 0 ? 0 : len_t[g] < a->Tt ? len_t[g] : a->Tt;
+                const TileList tl(a->Lp, a->Tt, a->S, lp, lt, (int)(row0 / r), (int)(last / r));
+                lists.push_back({tl.nt, (double)(last - row0 + 1) * (a->d < 256 ? a->d : 256) * 4});
+                mean += tl.nt;
+            }
+        }
+        mean /= (double)lists.size();
+        std::vector<int> sizes{nt_max};
+        for (int c : {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48}) sizes.push_back(c);
+        for (int k = 2; k <= 8; k++) sizes.push_back((nt_max + k - 1) / k);
+        for (double f : {1.0, 1.15, 1.3, 1.5}) sizes.push_back((int)(mean * f) + 1);
+        std::sort(sizes.begin(), sizes.end());
+        sizes.erase(std::unique(sizes.begin(), sizes.end()), sizes.end());
+        const double tile_bytes = 32.0 * a->d * 4 * (a->d == 512 ? 0.75 : 1.0);
+        double best = -1;
+        std::vector<double> free_at;
+        for (int per : sizes) {
+            if (per > nt_max || (per < 8 && nt_max >= 64) || (nt_max + per - 1) / per > 64) continue;   // (long lists: below 8 tiles a piece is mostly overhead)
+            free_at.assign((size_t)places, 0.0);
+            double end = 0, bytes = 0, part_bytes = 0;
+            for (int half = 0; half < halves; half++)
+                for (const List& l : lists) {
+                    const bool cut = l.tiles > per;
+                    for (int hh = 0; hh < a->h; hh++)
+                        for (int t0 = 0; t0 < l.tiles; t0 += per) {
+                            const int t = l.tiles - t0 < per ? l.tiles - t0 : per;
+                            std::pop_heap(free_at.begin(), free_at.end(), std::greater<double>());
+                            end = std::max(end, free_at.back() += FIX + tile_us * t + (cut ? PART : 0));
+                            std::push_heap(free_at.begin(), free_at.end(), std::greater<double>());
+                            bytes += t * tile_bytes;
+                            if (cut) part_bytes += l.part_bytes;
+                        }
+                }
+            const double est = std::max(end, (bytes + part_bytes) / BYTES_PER_US) + (part_bytes > 0 ? COMBINE + part_bytes / MERGE_BYTES_PER_US : 0);
+            if (best < 0 || est < best) { best = est; *tiles_per_split = per; }
+        }
+    } catch (const std::bad_alloc&) {
+        return spinf_fail(SPINF_E_NOMEM, "xdecode_plan_ragged: out of memory");
+    }
+    *nsplit = (nt_max + *tiles_per_split - 1) / *tiles_per_split;
     return SPINF_OK;
 }
 

@@ -188,7 +188,7 @@ def plan_splits(G: int, H: int, h: int, Q: int, S: int, Lp: int, Tt: int, d: int
     return ns.value, wb.value
 
 
-_TILE, _ROWS = 32, 128   # keys per tile, rows per workgroup (csrc/xdecode_attn.hip)
+_TILE = 32   # keys per tile (csrc/xdecode_attn.hip)
 
 
 def _list_tiles(Lp: int, Tt: int, S: int, len_p: int, len_t: int, qlo: int, qhi: int) -> int:
@@ -203,49 +203,13 @@ def _list_tiles(Lp: int, Tt: int, S: int, len_p: int, len_t: int, qlo: int, qhi:
 
 
 def plan_ragged(G: int, H: int, h: int, Q: int, S: int, Lp: int, Tt: int, d: int, beam: int, len_p, len_t) -> tuple[int, int]:
-    """-> (nsplit, tiles per split) for groups whose prefix / template ranges reach len_p[g] / len_t[g] entries: the split size
-    with the shortest estimated step: the longer of (a) the simulated schedule (workgroups in launch order onto the places the
-    GPU runs at a time; a workgroup costs its tiles + 2, a list that is split also its partial results' traffic, 7 tiles a piece
-    at 128 rows x 256 head dims) at 2 us a tile and (b) all the tiles of the step at the rate the memory delivers them (6.5 ns a
-    tile), plus 10 us for the merge launch of a split step.  The two rates are measured ones (XDEC, XDEC_long, XDEC_qwen of bench.py)."""
-    import heapq
-
-    r = H // h
-    R = Q * r
+    """-> (nsplit, tiles per split) for groups whose prefix / template ranges reach len_p[g] / len_t[g] entries (spinf_xdecode_plan_ragged)"""
     a = _lib.XdecArgs()
     a.G, a.H, a.h, a.Q, a.S, a.Lp, a.Tt, a.d, a.beam = G, H, h, Q, S, Lp, Tt, d, beam
-    nt_max = C.c_int32(0)
-    _lib.check(_lib.load_library().spinf_xdecode_tiles(C.byref(a), C.byref(nt_max)), "spinf_xdecode_tiles")
-    nt_max = nt_max.value
-    chunks = [(c * _ROWS // r, (min(c * _ROWS + _ROWS, R) - 1) // r, min(_ROWS, R - c * _ROWS)) for c in range(-(-R // _ROWS))]
-    lists = [[_list_tiles(Lp, Tt, S, min(len_p[g], Lp), min(len_t[g], Tt), lo, hi) for g in range(G)] for lo, hi, _ in chunks]
-    mean = sum(map(sum, lists)) / (G * len(chunks))
-    places = 256 if d == 512 else 512
-    cands = {nt_max} | {-(-nt_max // k) for k in range(2, 9)} | {int(mean * f) + 1 for f in (1.0, 1.15, 1.3, 1.5)}
-    best = None
-    for per in sorted(c for c in cands if 8 <= c <= nt_max or c == nt_max):
-        ns_max = -(-nt_max // per)
-        if ns_max > 16:
-            continue
-        free = [0.0] * places
-        heapq.heapify(free)
-        end = total = 0.0
-        for (lo, hi, rows), nts in zip(chunks, lists):
-            part = 7.0 * rows * (min(d, 256) + 2) / (_ROWS * 258)
-            for nt in nts:
-                ns = -(-nt // per)
-                for _ in range(h):
-                    for sp in range(ns_max):
-                        t = min(per, nt - sp * per)
-                        cost = 0.2 if t <= 0 else t + 2 + (part if ns > 1 else 0.0)
-                        t0 = heapq.heappop(free)
-                        heapq.heappush(free, t0 + cost)
-                        end = max(end, t0 + cost)
-                        total += cost
-        est = max(end * 2.0, total * 0.0065) + (10.0 if ns_max > 1 else 0.0)   # microseconds
-        if best is None or est < best[0]:
-            best = (est, ns_max, per)
-    return best[1], best[2]
+    lens = [(C.c_int32 * max(G, 1))(*x) for x in (len_p, len_t)]
+    ns, per = C.c_int32(1), C.c_int32(0)
+    _lib.check(_lib.load_library().spinf_xdecode_plan_ragged(C.byref(a), lens[0], lens[1], C.byref(ns), C.byref(per)), "spinf_xdecode_plan_ragged")
+    return ns.value, per.value
 
 
 def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None, softcap=None, nsplit=None):

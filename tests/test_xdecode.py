@@ -316,3 +316,16 @@ def test_cache_update_equals_index_copy(dev, G, h, Q, S, d):
     c.gk[0], c.gv[0] = c.gk[0].float(), c.gv[0].float()
     decode.GroupKV(c).update(v.float(), k.float(), 0)
     assert torch.equal(c.gk[0][:, :, :, S - 1], v.float()) and torch.equal(c.gv[0][:, :, :, S - 1], k.float())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,h,d,slots,prefix", [(16, 1, 512, 4, (301, 301)), (16, 1, 512, 1, (5, 40)), (24, 4, 256, 2, (64, 64)), (32, 16, 128, 3, (20, 130)), (4, 2, 64, 1, (1, 9))])
+def test_small_steps_cut_into_short_splits(dev, H, h, d, slots, prefix):
+    """one or two groups: the planned splits go down to single tiles, head dim 512 computes both halves of the output in one launch and merges
+    them in one; against the oracle, and against the unsplit step"""
+    q, c = synth.xdecode_case(2, H, h, d, slots, 6, 17, prefix, (4, 12), None, 9, seed=3, device=dev)
+    got = sa.xdecode_attn(q, c, 0, d**-0.5)
+    (ns, per), = c._plans.values()
+    assert 1 <= per < 8 and (ns > 1 or prefix[1] < 10)
+    assert np.abs(_np(got) - _oracle(q, c, d**-0.5)).max() <= TOL
+    assert np.abs(_np(got) - _np(sa.xdecode_attn(q, c, 0, d**-0.5, nsplit=1))).max() <= TOL
