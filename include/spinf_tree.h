@@ -163,7 +163,9 @@ int spinf_attn_ring_aborts(int64_t* total);
  *   cu, idx, h0_idx, ht_idx: int64 device arrays.  mode 0 = the recurrent entry point (short
  *   segments; consecutive segments of at most 16 tokens that start from the same state and leave none behind are taken
  *   two to a chunk), 1 = the chunked entry point (one workgroup per segment and head, 32-token chunks); both are the WY
- *   form of the same recurrence and either mode accepts any segment length.
+ *   form of the same recurrence and either mode accepts any segment length.  mode 2 = forests of short segments (a plan's program,
+ *   spinf_gdn_plan_program): cu [n_seg + 1] counts the blocks of n_seg units, idx is the table of these blocks (int32), h0_idx [n_seg]
+ *   the state above each unit; no state is left (ht is not used).
  *   v and o must be 16-byte aligned with row strides that are multiples of 8 elements.
  */
 typedef struct spinf_gdn_args {
@@ -203,6 +205,12 @@ int spinf_gdn_plan_counts(const spinf_gdn_plan* plan, int64_t counts[6]);
 int spinf_gdn_plan_export(const spinf_gdn_plan* plan, int64_t* level_ptr, int32_t* call_kind, int32_t* call_keep, int64_t* call_seg_ptr,
                           int64_t* call_row_ptr, int64_t* seg_len, int64_t* h0_idx, int64_t* ht_idx, int64_t* idx, int64_t* n_keep,
                           int64_t* conv, int64_t* seg_of_row, int64_t* seg_level, int64_t* seg_slot);
+/* The same scan as a program of spinf_gdn_fwd launches (path 0 only): small subtrees of short segments (segments of at most short_len
+ * tokens, 64 tokens along any path, 1,024 in all, none in `keep`) become mode 2 launches of their own where that pays, everything else stays
+ * one launch per level and kind.  No launches at all: the calls are as good.  counts[0] launches, [1] int64 values of `data`.  launches [counts[0], 8]: level, mode, n_seg, max_len, and the
+ * offsets into data of cu, idx, h0_idx (-1: zero states), ht_idx (-1: no state is left), in the order they must run; data goes to the device as it
+ * is (its parts are 16-byte aligned).  States are slots of the plan's levels (n_keep), as in the calls.  NULL arrays: only the counts. */
+int spinf_gdn_plan_program(const spinf_gdn_plan* plan, int64_t counts[2], int64_t* launches, int64_t* data);
 void spinf_gdn_plan_free(spinf_gdn_plan* plan);
 
 /* ------------------------------------------------------------------------------------------------ Gated DeltaNet layer, around the scan

@@ -220,6 +220,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 3))) void
 }
 
 int gdn_wy_launch(GdnParams p, bool pairs, hipStream_t stream);   // gdn_chunk.hip
+int gdn_forest_launch(const GdnParams& p, hipStream_t stream);    // gdn_forest.hip
 
 extern "C" int spinf_gdn_fwd(const spinf_gdn_args* a, void* stream) {
     if (!a) return spinf_fail(SPINF_E_ARG, "gdn: null args");
@@ -246,6 +247,7 @@ extern "C" int spinf_gdn_fwd(const spinf_gdn_args* a, void* stream) {
     p.run = 1;
     hipStream_t s = (hipStream_t)stream;
     if (a->mode == 1) return gdn_wy_launch(p, false, s);
+    if (a->mode == 2) return gdn_forest_launch(p, s);
     if (a->mode != 0) return spinf_fail(SPINF_E_ARG, "gdn: unknown mode %d", a->mode);
     if (a->dv == 128) return gdn_wy_launch(p, true, s);   // the workgroup kernel shares the per-head work of the four 32-column waves
     const long blocks = a->n_seg * a->hv * (a->dv / 32);

@@ -12,6 +12,7 @@
 // their depth at once; a counting sort by depth keeps stream order inside a level; calls are cut from the sorted array.
 #include "spinf_tree.h"
 #include "common.h"
+#include "gdn_forest.h"
 
 #include <algorithm>
 #include <cstring>
@@ -30,6 +31,7 @@ struct spinf_gdn_plan {
     std::vector<int64_t> n_keep;         // slots per level
     std::vector<int64_t> conv;           // [conv_rows, 4]
     std::vector<int64_t> seg_of_row, seg_level, seg_slot;
+    std::vector<int64_t> prog, prog_data;   // launches [*, 8] and what they read (spinf_gdn_plan_program)
 };
 
 namespace {
@@ -38,7 +40,153 @@ struct Seg {
     int64_t first, len, parent;
     int32_t depth;
     bool keeps;
+    bool wanted;   // the caller asked for its state
 };
+
+// ---- the program: forests apart (see gdn_forest.hip), the rest level by level
+constexpr int64_t FOREST_TREE = 1024;   // tokens of one tree, at most: a tree is one workgroup's work, and it should not outlast the level
+// A unit's tokens, at most (a larger tree is a unit of its own).  Fixed, and a unit never spans two parents, so that a content's blocks, and with
+// them the bits of its outputs, do not depend on what else is in the stream.  Four blocks: the state a unit loads first costs about as much
+// as one block, and a small stream needs its units side by side.  One layer with units of 32 / 64 / 128 / 256 / 512 tokens: 22 tries of 480 tokens
+// 522 / 487 / 475 / 464 / 484 us, one of them 76 / 75 / 82 / 98 / 127, 54 of 200 949 / 921 / 899 / 907 / 904.
+constexpr int64_t FOREST_UNIT = 128;
+
+template <class Row>
+void build_program(spinf_gdn_plan* p, const std::vector<Seg>& seg, int32_t n_levels, const std::vector<int64_t>& by_level, const std::vector<int64_t>& at, int32_t short_len, Row row) {
+    const int64_t ns = (int64_t)seg.size();
+    // per segment: can its subtree be (part of) a forest's tree; the subtree's tokens and its longest path
+    std::vector<char> fits(ns, 1), inside(ns, 0);
+    std::vector<int64_t> tokens(ns, 0), path(ns, 0);
+    for (int64_t s = ns - 1; s >= 0; s--) {
+        tokens[s] += seg[s].len;
+        path[s] += seg[s].len;
+        if (seg[s].len > short_len || seg[s].wanted || path[s] > GDN_FOREST_DEPTH || tokens[s] > FOREST_TREE) fits[s] = 0;
+        const int64_t up = seg[s].parent;
+        if (up >= 0) {
+            fits[up] &= fits[s];
+            tokens[up] += tokens[s];
+            path[up] = std::max(path[up], path[s]);
+        }
+    }
+    // children (in stream order) of every segment, and of none (index ns)
+    std::vector<int64_t> ptr(ns + 2, 0), kid(ns);
+    for (const Seg& s : seg) ptr[(s.parent >= 0 ? s.parent : ns) + 1]++;
+    for (int64_t s = 0; s <= ns; s++) ptr[s + 1] += ptr[s];
+    {
+        std::vector<int64_t> fill(ptr.begin(), ptr.end() - 1);
+        for (int64_t s = 0; s < ns; s++) kid[fill[seg[s].parent >= 0 ? seg[s].parent : ns]++] = s;
+    }
+    // A parent's children are taken as a forest if one of them forks.  Leaves alone leave no state that could be saved, only fuller blocks, and
+    // the recurrent entry point's smaller workgroups start sooner: a layer over 6 leaves of 8 tokens takes 55.0 us against 57.3, 108 such
+    // leaves 139 / 146, 168 of 7 125.6 / 124.9, 320 of 6.5 369 / 355, 325 of 14 253 / 236.
+    std::vector<char> forks(ns, 0);
+    for (int64_t s = 0; s < ns; s++)
+        if (fits[s] && ptr[s + 1] > ptr[s] && seg[s].parent >= 0) forks[seg[s].parent] = 1;
+    bool any = false;
+    for (int64_t s = 0; s < ns; s++) {
+        const int64_t up = seg[s].parent;
+        inside[s] = (up >= 0 && inside[up]) || (fits[s] && (up >= 0 ? forks[up] : ptr[s + 1] > ptr[s]));
+        any |= inside[s];
+    }
+    if (!any) return;
+    const int64_t B = GDN_FOREST_BLOCK;
+
+    // units, by the level that runs them
+    struct Level { std::vector<int64_t> cu{0}, h0; std::vector<int32_t> table; };
+    std::vector<Level> lev(n_levels);
+    std::vector<int64_t> stack;
+    std::vector<int32_t> where, up, dep, rowv;    // of a unit's tokens: parent token in the unit (-1 none), depth, tensor row; last token of a segment
+    where.assign(ns, -1);
+    auto flush = [&](Level& L, int64_t slot) {
+        const int64_t n = (int64_t)rowv.size();
+        if (!n) return;
+        std::vector<uint32_t> mask(n, 0);
+        std::vector<int32_t> from(n, 0);
+        for (int64_t f = 0; f < n; f += B) {
+            const int64_t e = std::min(n, f + B), next = f + B < n ? dep[f + B] : 0;
+            int32_t save[GDN_FOREST_BLOCK] = {};
+            for (int64_t i = f; i < e; i++) {
+                const int64_t a = up[i];
+                if (a >= f) { mask[i] = mask[a] | 1u << (a - f); from[i] = from[a]; }
+                else from[i] = a >= 0 ? dep[a] + 1 : 0;    // (pre-order: a token above i in an earlier block is above the block's first token)
+            }
+            if (f + B < n)
+                for (int64_t a = up[f + B]; a >= f; a = up[a]) save[a - f] = dep[a] + 1;
+            for (int64_t i = f; i < f + B; i++) L.table.push_back(i < e ? rowv[i] : -1);
+            for (int64_t i = f; i < f + B; i++) L.table.push_back(i < e ? (int32_t)mask[i] : 0);
+            for (int64_t i = f; i < f + B; i++)
+                L.table.push_back((int32_t)((uint32_t)(i < e ? from[i] : 0) | (uint32_t)(i < e ? save[i - f] : 0) << 8 | (uint32_t)dep[f] << 16 | (uint32_t)next << 24));
+        }
+        L.cu.push_back(L.cu.back() + (n + B - 1) / B);
+        L.h0.push_back(slot);
+        rowv.clear(); up.clear(); dep.clear();
+    };
+    for (int64_t u = -1; u < ns; u++) {      // the trees below segment u (-1: below none)
+        const int64_t of = u < 0 ? ns : u;
+        if (u >= 0 && inside[u]) continue;
+        Level* L = nullptr;
+        const int64_t slot = u >= 0 ? p->seg_slot[u] : -1;
+        for (int64_t k = ptr[of]; k < ptr[of + 1]; k++) {
+            const int64_t head = kid[k];
+            if (!inside[head]) continue;
+            L = &lev[seg[head].depth];
+            if (!rowv.empty() && (u < 0 || (int64_t)rowv.size() + tokens[head] > FOREST_UNIT)) flush(*L, slot);
+            stack.assign(1, head);
+            while (!stack.empty()) {
+                const int64_t s = stack.back();
+                stack.pop_back();
+                int32_t last = s == head ? -1 : where[seg[s].parent];
+                for (int64_t t = 0; t < seg[s].len; t++) {
+                    up.push_back(last);
+                    dep.push_back(last >= 0 ? dep[last] + 1 : 0);
+                    last = (int32_t)rowv.size();
+                    rowv.push_back((int32_t)row(seg[s].first + t));
+                }
+                where[s] = last;
+                for (int64_t j = ptr[s + 1] - 1; j >= ptr[s]; j--) stack.push_back(kid[j]);
+            }
+        }
+        if (L) flush(*L, slot);
+    }
+
+    // what is left of each level, then its units
+    auto put = [&](const int64_t* x, size_t n) {
+        if (p->prog_data.size() % 2) p->prog_data.push_back(0);
+        const int64_t o = (int64_t)p->prog_data.size();
+        p->prog_data.insert(p->prog_data.end(), x, x + n);
+        return o;
+    };
+    std::vector<int64_t> cu, h0, ht, idx;
+    for (int32_t d = 0; d < n_levels; d++) {
+        for (int kind = 1; kind >= 0; kind--) {
+            cu.assign(1, 0); h0.clear(); ht.clear(); idx.clear();
+            int64_t longest = 0;
+            bool keeps = false;
+            for (int64_t i = at[d]; i < at[d + 1]; i++) {
+                const Seg& s = seg[by_level[i]];
+                if (inside[by_level[i]] || (s.len > short_len) != (kind == 1)) continue;
+                cu.push_back(cu.back() + s.len);
+                h0.push_back(d > 0 ? p->seg_slot[s.parent] : -1);
+                ht.push_back(s.keeps ? p->seg_slot[by_level[i]] : -1);
+                keeps |= s.keeps;
+                longest = std::max(longest, s.len);
+                for (int64_t t = 0; t < s.len; t++) idx.push_back(row(s.first + t));
+            }
+            if (h0.empty()) continue;
+            const int64_t rec[8] = {d, kind, (int64_t)h0.size(), kind ? longest : 0, put(cu.data(), cu.size()), put(idx.data(), idx.size()),
+                                    d > 0 ? put(h0.data(), h0.size()) : -1, keeps ? put(ht.data(), ht.size()) : -1};
+            p->prog.insert(p->prog.end(), rec, rec + 8);
+        }
+        const Level& L = lev[d];
+        if (L.h0.empty()) continue;
+        const int64_t words = (int64_t)L.table.size() / 2;   // (GDN_FOREST_INTS is even)
+        std::vector<int64_t> table(words);
+        std::memcpy(table.data(), L.table.data(), words * 8);
+        const int64_t rec[8] = {d, 2, (int64_t)L.h0.size(), 0, put(L.cu.data(), L.cu.size()), put(table.data(), table.size()),
+                                d > 0 ? put(L.h0.data(), L.h0.size()) : -1, -1};
+        p->prog.insert(p->prog.end(), rec, rec + 8);
+    }
+}
 
 }  // namespace
 
@@ -88,7 +236,7 @@ extern "C" int spinf_gdn_plan_build(const int64_t* prev, const uint8_t* real, in
                 s.len = 0;
                 s.parent = b >= 0 ? seg_at[b] : -1;
                 s.depth = s.parent >= 0 ? seg[s.parent].depth + 1 : 0;
-                s.keeps = false;
+                s.keeps = s.wanted = false;
                 if (s.parent >= 0) seg[s.parent].keeps = true;   // somebody continues from it
                 seg.push_back(s);
             }
@@ -97,7 +245,7 @@ extern "C" int spinf_gdn_plan_build(const int64_t* prev, const uint8_t* real, in
         }
         for (int64_t j = 0; j < n_keep; j++) {
             const int64_t i = keep[j];
-            if (i >= 0 && i < n && real[i]) seg[seg_at[i]].keeps = true;   // the caller wants this segment's state
+            if (i >= 0 && i < n && real[i]) seg[seg_at[i]].keeps = seg[seg_at[i]].wanted = true;   // the caller wants this segment's state
         }
         const int64_t ns = (int64_t)seg.size();
         p->n_segments = ns;
@@ -192,6 +340,8 @@ extern "C" int spinf_gdn_plan_build(const int64_t* prev, const uint8_t* real, in
             p->level_ptr.push_back((int64_t)p->call_kind.size());
         }
 
+        if (path == 0) build_program(p, seg, n_levels, by_level, at, short_len, row);
+
         // ---- convolution taps: the three tokens before a token on its path, oldest first, then the token itself
         const int64_t none = compact ? rows : n;
         p->conv_rows = compact ? rows : n;
@@ -242,6 +392,15 @@ extern "C" int spinf_gdn_plan_export(const spinf_gdn_plan* p, int64_t* level_ptr
                     put(call_row_ptr, p->call_row_ptr) && put(seg_len, p->len) && put(h0_idx, p->h0) && put(ht_idx, p->ht) && put(idx, p->idx) &&
                     put(n_keep, p->n_keep) && put(conv, p->conv) && put(seg_of_row, p->seg_of_row) && put(seg_level, p->seg_level) && put(seg_slot, p->seg_slot);
     if (!ok) return spinf_fail(SPINF_E_ARG, "gdn_plan_export: null array for a non-empty part of the plan");
+    return SPINF_OK;
+}
+
+extern "C" int spinf_gdn_plan_program(const spinf_gdn_plan* p, int64_t counts[2], int64_t* launches, int64_t* data) {
+    if (!p || !counts) return spinf_fail(SPINF_E_ARG, "gdn_plan_program: null argument");
+    counts[0] = (int64_t)p->prog.size() / 8;
+    counts[1] = (int64_t)p->prog_data.size();
+    if (launches && !p->prog.empty()) std::memcpy(launches, p->prog.data(), p->prog.size() * 8);
+    if (data && !p->prog_data.empty()) std::memcpy(data, p->prog_data.data(), p->prog_data.size() * 8);
     return SPINF_OK;
 }
 

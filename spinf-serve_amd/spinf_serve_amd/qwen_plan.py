@@ -44,6 +44,7 @@ class TreePlan:
     cap: dict | None = None
     pad_rows: object | None = None   # [pads] int64 (device): rows of the tensors no segment covers; their outputs are zero
     launches: list | None = None     # indexed path: per level the kernel launches (mode, segments, longest, addresses of cu, idx, h0_idx, ht_idx), neighbouring calls of one kind as one
+    program: list | None = None      # the same with the small subtrees as forests of their own (mode 2, csrc/gdn_forest.hip); None without any
 
 
 _PATHS = {"indexed": 0, "levels": 1}
@@ -69,6 +70,10 @@ def _compile(prev, real, path, short, call_tokens, max_init, rows, keep):
         _lib.check(lib.spinf_gdn_plan_export(handle, *(out[name].ctypes.data for name in shapes)), "tree_plan")
         out = {name: out[name][: shapes[name][0]] for name in shapes}
         out["n_segments"] = n_seg
+        counts = (C.c_int64 * 2)()
+        _lib.check(lib.spinf_gdn_plan_program(handle, counts, None, None), "tree_plan")
+        out["program"], out["program_data"] = np.zeros((counts[0], 8), np.int64), np.zeros(counts[1], np.int64)
+        _lib.check(lib.spinf_gdn_plan_program(handle, counts, out["program"].ctypes.data, out["program_data"].ctypes.data), "tree_plan")
         return out
     finally:
         lib.spinf_gdn_plan_free(handle)
@@ -104,14 +109,14 @@ def tree_plan(prev, real, device, max_init: int = 96, path: str = "indexed", sho
     cu_at = np.concatenate([[0], np.cumsum([seg_ptr[j] - seg_ptr[i] + 1 for i, j in spans])]).astype(np.int64).tolist()
     # everything the kernels read, in one copy
     sidx_host = np.flatnonzero(real) if rows is not None else np.zeros(0, np.int64)
-    parts = [a["conv"], a["idx"], a["h0_idx"], a["ht_idx"], cu_host.numpy(), sidx_host, np.flatnonzero(a["seg_of_row"] < 0)]
+    parts = [a["conv"], a["idx"], a["h0_idx"], a["ht_idx"], cu_host.numpy(), sidx_host, np.flatnonzero(a["seg_of_row"] < 0), a["program_data"]]
     at = np.concatenate([[0], np.cumsum([-(-len(x) // 2) * 2 for x in parts])]).tolist()   # (each part 16-byte aligned)
     stage = torch.empty(at[-1], dtype=torch.int64, pin_memory=dev.type == "cuda")
     host = stage.numpy()
     for x, o in zip(parts, at):
         host[o : o + len(x)] = x
     on_dev = stage.to(dev, non_blocking=True)
-    conv, idx_all, h0_all, ht_all, cu_all, sidx, pad_rows = (on_dev[o : o + len(x)] for x, o in zip(parts, at))
+    conv, idx_all, h0_all, ht_all, cu_all, sidx, pad_rows, program_data = (on_dev[o : o + len(x)] for x, o in zip(parts, at))
     cu_of = {span: k for k, span in enumerate(spans)}
 
     def cut(i, j):
@@ -138,9 +143,15 @@ def tree_plan(prev, real, device, max_init: int = 96, path: str = "indexed", sho
             merged.append((int(call_kind[i]), len(lens), int(lens.max()) if call_kind[i] else 0, cu.data_ptr(), idx.data_ptr(), starts.data_ptr() if d else None,
                            ends.data_ptr() if call_keep[i:j].any() else None))   # (views of on_dev, which plan.conv keeps alive)
         launches.append(merged)
+    program = None
+    if len(a["program"]):
+        program = [[] for _ in levels]
+        base = program_data.data_ptr()
+        for d, mode, n, longest, *offsets in a["program"].tolist():
+            program[d].append((mode, n, longest, *(base + 8 * o if o >= 0 else None for o in offsets)))
     seg_of_row = a["seg_of_row"]
     return TreePlan(conv.view(-1, 4), levels, a["n_segments"], path, a["n_keep"].tolist() if indexed else None, rows, sidx if rows is not None else None, seg_of_row,
-                    a["seg_level"], a["seg_slot"], pad_rows=pad_rows, launches=launches if indexed else None)
+                    a["seg_level"], a["seg_slot"], pad_rows=pad_rows, launches=launches if indexed else None, program=program)
 
 
 def _kept_state_requests(plan: TreePlan, cap):
@@ -183,14 +194,19 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
     b16 = beta if beta.dtype == torch.bfloat16 else beta.to(torch.bfloat16)
     indexed = plan.path == "indexed"
     args = gdn.level_args(q, k, v, g32, b16, o, scale) if indexed and plan.launches is not None else None
+    # a forest's nodes leave no states (and its kernel is built for 128 value dims): a caller that asks for states gets every level's
+    launches = plan.launches if wanted or plan.program is None or v.shape[-1] != 128 else plan.program
     above = None   # the states the level above left
     for d, calls in enumerate(plan.levels):
-        n_slots = plan.n_keep[d] if indexed else sum(len(c.cu_cpu) - 1 for c in calls if c.keep)
+        if args is not None and launches is plan.program:
+            n_slots = plan.n_keep[d] if any(launch[-1] is not None for launch in launches[d]) else 0
+        else:
+            n_slots = plan.n_keep[d] if indexed else sum(len(c.cu_cpu) - 1 for c in calls if c.keep)
         states = q.new_empty((n_slots, v.shape[1], q.shape[-1], v.shape[-1]), dtype=torch.float32) if n_slots else None
         next_slot = 0
         if args is not None:
             h0, ht = None if above is None else above.data_ptr(), None if states is None else states.data_ptr()
-            for args.mode, args.n_seg, args.max_len, args.cu, args.idx, h0_idx, ht_idx in plan.launches[d]:
+            for args.mode, args.n_seg, args.max_len, args.cu, args.idx, h0_idx, ht_idx in launches[d]:
                 args.h0, args.h0_idx = (h0, h0_idx) if h0_idx is not None else (None, None)
                 args.ht, args.ht_idx = (ht, ht_idx) if ht_idx is not None else (None, None)
                 _lib.launch(_lib.load_library().spinf_gdn_fwd, args, q.device, "spinf_gdn_fwd")

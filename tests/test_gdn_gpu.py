@@ -191,6 +191,57 @@ def test_deep_trie(dev):
     _within(o, want, TOL, "deep tree")
 
 
+def _chain_tree(rng, trunk, nodes):
+    """nodes [(length, parent)] below a trunk"""
+    return synth._tree(rng, trunk, [n for n, _ in nodes], [p for _, p in nodes])
+
+
+@pytest.mark.parametrize("h, hv", [(2, 4), (3, 3)])
+@pytest.mark.parametrize("kind", ["path64", "path65", "straddle", "single", "deep", "large", "trunkless", "compact"])
+def test_forests(dev, kind, h, hv):
+    """small subtrees taken whole (csrc/gdn_forest.hip) at the edges of its blocks, stack and trees, against the float64 recurrence and no
+    further from it than the level by level launches (per output the largest error, with 1.5 for the order of the roundings)"""
+    rng = np.random.default_rng(4)
+    star = [(n, -1) for n in (1, 31, 32, 33, 16, 16, 17, 64, 2)]
+    trees = {
+        "path64": [_chain_tree(rng, 100, [(32, -1), (16, 0), (15, 1), (1, 2), (1, 1), (33, 0)])],
+        "path65": [_chain_tree(rng, 100, [(32, -1), (16, 0), (16, 1), (1, 2), (1, 1), (33, 0)])],
+        "straddle": [_chain_tree(rng, 70, star), _chain_tree(rng, 200, [(20, -1), (20, 0), (20, 1), (3, 2), (3, 2), (40, 0), (30, -1), (9, 6)])],
+        "single": [_chain_tree(rng, 65, [(1, -1), (1, -1), (1, 1), (1, 1)]), _chain_tree(rng, 1, [(1, -1), (1, -1)])],
+        "deep": [_chain_tree(rng, 80, [(2, b - 1 if b % 2 else b - 2 if b else -1) for b in range(62)])],
+        "large": [_chain_tree(rng, 90, [(4, -1)] + [(int(rng.integers(4, 9)), int(rng.integers(max(0, b - 12), b))) for b in range(1, 180)])],
+        "trunkless": [_chain_tree(rng, 8, [(3, -1), (4, 0), (5, 0)]), _chain_tree(rng, 40, [(3, -1)] * 3)],
+        "compact": [_chain_tree(rng, 130, star + [(5, 0), (7, 0)])] * 3,
+    }[kind]
+    cfg = synth.GdnConfig(kind, h, hv, 128, 128, trees)
+    cfg.batch = b = synth.pack(trees)[0]
+    t = synth.gdn_inputs(cfg, seed=3, device=dev)
+    real = b.art >= 0
+    want = ogdn.tree_scan(*(_np(t[x]) for x in ("q", "k", "v", "g", "beta")), b.prev, real)
+    if kind == "compact":
+        t = {x: y[torch.from_numpy(real).to(dev)] for x, y in t.items()}
+        want = want[real]
+        plan = sa.tree_plan(b.prev, real, dev, rows=b.n_tokens)
+    else:
+        plan = cfg.plan(dev)
+    assert plan.program is not None and any(launch[0] == 2 for level in plan.program for launch in level)
+    args = [t[x] for x in ("q", "k", "v", "g", "beta")]
+    print(f"case forest {kind} {h} {hv}", flush=True)
+    o = sa.gdn_tree(*args, plan)
+    torch.cuda.synchronize()
+    err = _within(o, want, TOL, f"forest {kind}")
+    plan.program = None
+    by_level = _within(sa.gdn_tree(*args, plan), want, TOL, f"levels {kind}")
+    if kind in ("straddle", "single", "trunkless"):    # a content's outputs do not depend on what else is in the stream
+        one = synth.GdnConfig("one", h, hv, 128, 128, trees[1:2])
+        one.batch = synth.pack(trees[1:2])[0]
+        s0, n = b.jobs[1][0], trees[1].n_tokens
+        pad = lambda x: torch.cat([x[s0 : s0 + n], x.new_zeros((one.batch.length - n, *x.shape[1:]))])  # noqa: E731
+        assert torch.equal(sa.gdn_tree(*(pad(x) for x in args), one.plan(dev))[:n], o[s0 : s0 + n])
+    print(f"  forest {kind}: max abs err {err:.3e}, level by level {by_level:.3e}", flush=True)
+    assert err <= 1.5 * by_level + 1e-5
+
+
 def test_decoder_steps_rerun_the_recurrence_from_the_prefix_state(dev):
     """the extraction decoder's call (spinf_serve/models/qwen35/qwen_decode.py:305-318): every step each slot re-runs the recurrence
     from its group's prefix state over its template rows plus the tokens generated so far, read out of row caches through idx,

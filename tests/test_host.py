@@ -496,6 +496,68 @@ def test_tree_plan_matches_reference_and_oracle(golden):
                         assert (None if c.ht_idx is None else c.ht_idx.tolist()) == wc["ht_idx"]
 
 
+def _program(plan):
+    """a CPU plan's program as (level, mode, cu, idx or block table, h0_idx, ht_idx) with the arrays read back from their addresses"""
+    at = lambda p, n, t=ctypes.c_int64: np.ctypeslib.as_array((t * n).from_address(p)).copy() if n else np.zeros(0, np.int64)  # noqa: E731
+    for d, launches in enumerate(plan.program):
+        for mode, n, _, cu, idx, h0, ht in launches:
+            cu = at(cu, n + 1)
+            table = at(idx, 96 * int(cu[-1]), ctypes.c_int32).reshape(-1, 3, 32) if mode == 2 else at(idx, int(cu[-1]))
+            yield d, mode, cu, table, at(h0, n) if h0 else None, at(ht, n) if ht else None
+
+
+@pytest.mark.parametrize("seed", range(12))
+def test_tree_plan_program_is_the_forest(seed):
+    """the program's launches over random tries (path lengths around 64, trees around 1,024 tokens, empty trunk states, wanted states):
+    every real row once, and for every token of a forest exactly its ancestors, through the in-block masks and the stack of the path"""
+    rng = np.random.default_rng(seed)
+    trees = []
+    for _ in range(int(rng.integers(1, 5))):
+        n = int(rng.integers(1, 120))
+        parents = [int(rng.integers(max(-1, b - 9), b)) for b in range(n)]
+        lens = rng.integers(1, int(rng.choice([2, 9, 30, 70])), n)
+        trees.append(TokenTree([5] * int(rng.choice([1, 20, 63, 64, 65, 300])), [[7] * int(x) for x in lens], parents))
+    s = sa.pack_stream(trees)
+    real = s.art >= 0
+    keep = rng.choice(np.flatnonzero(real), 2).tolist() if seed % 3 == 0 else None
+    plan = sa.tree_plan(s.prev, real, "cpu", keep=keep)
+    if plan.program is None:
+        pytest.skip("no forest in this stream")
+    done, slot_tail, forests = np.zeros(len(real), int), [dict() for _ in plan.levels], 0
+    for d, mode, cu, table, h0, ht in _program(plan):
+        for u in range(len(cu) - 1):
+            start = -1 if h0 is None or h0[u] < 0 else slot_tail[d - 1][h0[u]]   # the token whose state the unit starts from
+            if mode != 2:
+                rows = table[cu[u] : cu[u + 1]]
+                done[rows] += 1
+                assert s.prev[rows[0]] == start and (s.prev[rows[1:]] == rows[:-1]).all() and (len(rows) > 64) == (mode == 1)
+                if ht is not None and ht[u] >= 0:
+                    slot_tail[d][ht[u]] = int(rows[-1])
+                continue
+            forests += 1
+            stack = np.full(64, -1)
+            for b in range(cu[u], cu[u + 1]):
+                rows, masks, meta = table[b]
+                depth, following = (meta[0] >> 16) & 255, (meta[0] >> 24) & 255
+                for i in np.flatnonzero(rows >= 0):
+                    above = set(stack[: meta[i] & 255]) | {int(rows[j]) for j in range(32) if (int(masks[i]) >> j) & 1}
+                    a, want = int(s.prev[rows[i]]), set()
+                    while a != start:
+                        want.add(a)
+                        a = int(s.prev[a])
+                    assert above == want and (meta[i] & 255) <= depth and not int(masks[i]) & 0xFFFFFFFF & -(1 << int(i))
+                    done[rows[i]] += 1
+                for i in np.flatnonzero((meta >> 8) & 255):
+                    stack[((meta[i] >> 8) & 255) - 1] = rows[i]
+                assert (b + 1 < cu[u + 1]) or following == 0
+                assert b + 1 >= cu[u + 1] or following == (table[b + 1][2][0] >> 16) & 255
+    assert forests and (done == real).all()
+    if keep is not None:
+        for i in keep:   # a wanted state is left by a launch of its level
+            sg = plan.seg_of_row[i]
+            assert int(plan.seg_slot[sg]) in slot_tail[int(plan.seg_level[sg])]
+
+
 def test_tree_plan_compact_rows_keep_and_levels():
     """tests/test_qwen_plan.py:102-164 and tests/test_stacks.py:67-75 against the mirror"""
     plan = sa.tree_plan(np.array([-1, 0, 1, 1, 3]), np.ones(5, bool), "cpu")
