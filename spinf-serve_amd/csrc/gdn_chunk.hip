@@ -8,11 +8,13 @@
 // fp32 accumulator registers.  Per chunk, with G = cumsum(g), D_ij = e^{G_i - G_j}:
 //     A   = -strict_tril(beta_i (K K^T)_ij D_ij)         T = (I - A)^-1      (fp32: 16 x 16 blocks solved by substitution in
 //                                                                             registers, merged with fp32 MFMAs)
-//     U   = T diag(beta) V          -W = -T diag(beta e^G) K                 (bf16 MFMA, fp32 accumulate)
-//     V'  = U - W S                 O = s e^{G_i} (Q S)_i + tril(s (Q K^T) D) V'
+//     R   = -e^G (K S)              V'  = T diag(beta) (V + R)                (bf16 MFMA, fp32 accumulate)
+//     O   = s e^{G_i} (Q S)_i + tril(s (Q K^T) D) V'
 //     S  <- e^{G_L} S + (K e^{G_L - G})^T V'
-// The token x token and token x key quantities (A, P, T, W) are the same for all value columns: the waves split them (one
-// 16 x 16 tile of A and P per wave, the triangular solve on wave 0, two key tiles of W per wave) and exchange them through
+// (K S and Q S need no T: the waves compute them beside the solve, and there is no product W = T diag(beta e^G) K and no barrier for it.
+// 2,048-token trunks, 1,024 workgroups: 639 us against 656 with W and V' = U - W S; the error against 64 bits is the same.)
+// The token x token quantities (A, P, T) are the same for all value columns: the waves split them (one
+// 16 x 16 tile of A and P per wave, the triangular solve on one wave) and exchange them through
 // LDS; everything that touches value columns is private to a wave, and every product leaves its result in the register
 // layout the next product takes as an operand (see gdn_tiles.h), so of those only the output rows pass through LDS (for
 // 16-byte stores).  The kernels are bound by instruction issue, not by the matrix cores: what is shared is not recomputed.
@@ -28,7 +30,7 @@ namespace {
 
 constexpr int KD = 128;        // key head dim
 constexpr int VD = 128;        // value head dim
-// Row strides of the LDS tiles, chosen by how a tile is read most.  A tile read row-wise in 8- or 16-byte pieces (Q, -W: lane c
+// Row strides of the LDS tiles, chosen by how a tile is read most.  A tile read row-wise in 8- or 16-byte pieces (Q: lane c
 // takes row c) wants a stride of 4 banks (mod 64): 16 rows then start in 16 different groups of four banks.  A tile read through
 // ds_read_b64_tr_b16 (K, V: 16 lanes take a 4 rows x 32 bytes block, the next 16 lanes the four rows below) wants 8 banks
 // (mod 64): eight rows x 32 bytes then cover the 64 banks once.  Measured LDS clocks per instruction of a workgroup (stride in
@@ -36,8 +38,7 @@ constexpr int VD = 128;        // value head dim
 // 16-byte row reads 4.0 at 8, 8.0 at 4, 20, 36.
 constexpr int LD = 136;        // row stride (elements) of the Q tile: 68 banks
 constexpr int LDT = 144;       // row stride of the K and V tiles: 72 banks
-constexpr int LW = 136;        // row stride of the -W tile
-constexpr int LP = 40;         // row stride of the token x token bf16 tiles (P, T diag(beta), -T diag(beta e^G))
+constexpr int LP = 40;         // row stride of the token x token bf16 tiles (P, T diag(beta))
 constexpr int LA = 36;         // row stride (floats) of A
 constexpr int LX = 20;         // row stride (floats) of the 16 x 16 blocks of T and of the merge scratch
 
@@ -51,7 +52,9 @@ __device__ __forceinline__ bf16x4 zero_bf4() {
 }
 }  // namespace
 
-template <bool PAIRS>
+// SOLVER: a fifth wave has the gates and the solve, and no value columns.  TIGHT: fewer registers, by computing LDS addresses anew in every
+// phase and, without SOLVER, reading A as the solve goes.
+template <bool PAIRS, bool SOLVER, bool TIGHT>
 __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
     constexpr int NT = 2;                           // 16-token tiles per chunk
     constexpr int CH = 16 * NT;
@@ -62,21 +65,24 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
     __shared__ __attribute__((aligned(16))) __bf16 Ks[CH * LDT];
     __shared__ __attribute__((aligned(16))) __bf16 Qs[CH * LD];
     __shared__ __attribute__((aligned(16))) __bf16 Vs[CH * LDT];     // V; later the waves' output tiles
-    __shared__ __attribute__((aligned(16))) char solve[32 * LA * 4 + 32 * LX * 4 + 16 * LX * 4 + 256];   // A, T blocks, merge scratch; later -W
+    __shared__ __attribute__((aligned(16))) float As[32 * LA];
+    __shared__ __attribute__((aligned(16))) float Ts[32 * LX];       // T_00 in rows 0..15, T_11 in rows 16..31
+    __shared__ __attribute__((aligned(16))) float Xs[16 * LX];       // merge scratch
     __shared__ __attribute__((aligned(16))) __bf16 Ps[CH * LP];
     __shared__ __attribute__((aligned(16))) __bf16 Tus[CH * LP];
-    __shared__ __attribute__((aligned(16))) __bf16 Tws[CH * LP];
     __shared__ __attribute__((aligned(16))) float Gs[CH];
     __shared__ __attribute__((aligned(16))) float Bs[CH];
     __shared__ int Rs[CH];
-    float* As = (float*)solve;
-    float* Ts = As + 32 * LA;          // T_00 in rows 0..15, T_11 in rows 16..31
-    float* Xs = Ts + 32 * LX;
-    __bf16* Wn = (__bf16*)solve;       // -W [CH][LW], written when A and T are dead
-    static_assert(32 * LW * 2 <= (int)sizeof(solve), "-W must fit the region it shares");
     static_assert(4 * 32 * LO <= CH * LDT, "the output tiles must fit the V tile");
 
-    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, q4 = lane >> 4;
+    int tid = threadIdx.x, lane = tid & 63, c = lane & 15, q4 = lane >> 4;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto fresh = [&]() __attribute__((always_inline)) {
+        if (TIGHT) asm volatile("" : "+v"(tid));
+        lane = tid & 63;
+        c = lane & 15;
+        q4 = lane >> 4;
+    };
     // Workgroups go round the 8 XCDs (each with its own L2) in launch order.  Two value heads that share a key head read the
     // same q and k rows: they get launch slots 8 apart, i.e. the same XCD at about the same time, so the second read hits L2.
     long slot = blockIdx.x;
@@ -137,8 +143,101 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             len = max(0, min(16, T - j * CH - 16 * cc));
         }
     };
-    __bf16* Ow = Vs + w * 32 * LO;
+    __bf16* Ow = Vs + (w & 3) * 32 * LO;
 
+    const bool keep = p.ht != nullptr && p.ht_idx != nullptr && p.ht_idx[seg] >= 0;
+
+    // The next chunk's rows are fetched into registers while the current chunk is computed, and the stream rows (idx) of
+    // the chunk after that one chunk earlier still, so that no load ever waits for the load of its own address.
+    // Thread -> 16-byte piece tid%16 of chunk rows tid/16 (+ 16).
+    // Only the low half of an index is loaded: the register of an unused high half would be handed out again at once, and
+    // whoever writes it first has to wait for the load (and with it for every load in flight).
+    const int* idx_lo = (const int*)p.idx;
+    // ---- g, beta and the stream rows of the chunk (lane = chunk row), G, and T: wave 0, or a fifth wave
+    int rb = -1, pr32 = -1;
+    float pg = 0.f;
+    __bf16 pbeta = (__bf16)0.f;   // (kept as loaded: converting here would make the wave wait for the load at once)
+    auto fetch_gate_row = [&](const int j) __attribute__((always_inline)) {
+        long base[NT];
+        int len[NT];
+#pragma unroll
+        for (int cc = 0; cc < NT; cc++) tile_of(j, cc, base[cc], len[cc]);
+        rb = -1;
+        const bool hi = (lane & 16) != 0;     // chunk row lane % 32 = row lane % 16 of tile (lane / 16) % 2
+        if (c < (hi ? len[NT - 1] : len[0])) {
+            const long t = (hi ? base[NT - 1] : base[0]) + c;
+            rb = p.idx ? idx_lo[2 * t] : (int)t;
+        }
+    };
+    auto fetch_gates = [&]() __attribute__((always_inline)) {
+        pr32 = rb;
+        pg = 0.f;
+        pbeta = (__bf16)0.f;
+        if (rb >= 0) {
+            pg = p.g[row_offset(rb, p.g_tok) + hv];
+            pbeta = p.beta[row_offset(rb, p.g_tok) + hv];
+        }
+    };
+    auto stage_gates = [&]() __attribute__((always_inline)) {
+        float x = row_prefix_sum(pg);
+        // row_bcast:15 -> lanes 16..31 (not for a pair: the second tile is another segment)
+        if (!run_mode) x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x142, 0xa, 0xf, false));
+        if (lane < CH) {
+            Gs[lane] = x;
+            Bs[lane] = (float)pbeta;
+            Rs[lane] = pr32;
+        }
+    };
+    // T = (I - A)^-1: rows of the diagonal blocks by substitution in registers (lane groups 0 and 2 the upper-left block, 1 and 3 the
+    // lower-right one, in the same instructions), then the lower-left block T_lo = T_11 A_lo T_00, computed transposed
+    // (T_lo^T = T_00^T (A_lo^T T_11^T)) so that the lane again holds a row.  Leaves T diag(beta) in LDS as bf16, tile by tile.
+    // The others wait for this wave: it goes first.
+    auto solve = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_s_setprio(3);
+        float t[16];
+        const int blk = q4 & 1;
+        unit_lower_inverse_row<SOLVER || !TIGHT>(As + blk * (16 * LA + 16), LA, c, t);
+        // the rows pass through LDS to reach the lanes in operand order (row c, columns 4 q4 ..+3)
+#pragma unroll
+        for (int j4 = 0; j4 < 4; j4++) *(f32x4*)(Ts + (16 * blk + c) * LX + 4 * j4) = f32x4{t[4 * j4], t[4 * j4 + 1], t[4 * j4 + 2], t[4 * j4 + 3]};
+        wave_lds_order();
+        const float* T1s = Ts + 16 * LX;
+        const f32x4 B0 = *(const f32x4*)(Bs + 4 * q4), B1 = *(const f32x4*)(Bs + 16 + 4 * q4);
+        const f32x4 t00 = *(const f32x4*)(Ts + c * LX + 4 * q4), t11 = *(const f32x4*)(T1s + c * LX + 4 * q4);
+        *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
+        *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
+        f32x4 tlo = zero4();
+        if (!run_mode) {      // (a pair's tiles are different segments: A_lo = 0, so is T_lo)
+            f32x4 x = zero4();
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++)        // X[j][i] = sum_m A_lo[m][j] T_11[i][m]
+                x = mfma4(As[(16 + 4 * s4 + q4) * LA + c], T1s[c * LX + 4 * s4 + q4], x);
+#pragma unroll
+            for (int r = 0; r < 4; r++) Xs[(4 * q4 + r) * LX + c] = x[r];
+            wave_lds_order();
+#pragma unroll
+            for (int s4 = 0; s4 < 4; s4++)        // T_lo[16 + i][j'] = sum_j T_00[j][j'] X[j][i]
+                tlo = mfma4(Ts[(4 * s4 + q4) * LX + c], Xs[(4 * s4 + q4) * LX + c], tlo);
+        }
+        *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = round4(tlo * B0);
+        __builtin_amdgcn_s_setprio(0);
+    };
+    if (SOLVER && w == 4) {
+        fetch_gate_row(0);
+        fetch_gates();
+        fetch_gate_row(1);
+        for (int j = 0; j < n_chunks; j++) {      // (the barriers of the other waves' loop below)
+            lds_barrier();
+            stage_gates();
+            lds_barrier();
+            fetch_gates();
+            fetch_gate_row(j + 2);
+            lds_barrier();
+            solve();
+            lds_barrier();
+        }
+        continue;
+    }
     // ---- state: S[kt][vt][r] = S[16 kt + 4 q4 + r][32 w + 16 vt + c]
     f32x4 S[8][2];
 #pragma unroll
@@ -157,20 +256,8 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
                     for (int vt = 0; vt < 2; vt++) S[kt][vt][r] = hp[(16 * kt + r) * VD + 16 * vt];
         }
     }
-    const bool keep = p.ht != nullptr && p.ht_idx != nullptr && p.ht_idx[seg] >= 0;
-
-    // The next chunk's rows are fetched into registers while the current chunk is computed, and the stream rows (idx) of
-    // the chunk after that one chunk earlier still, so that no load ever waits for the load of its own address.
-    // Thread -> 16-byte piece tid%16 of chunk rows tid/16 (+ 16); threads 0..CH-1 also -> g, beta and the stream row of chunk
-    // row tid.
     bf16x8 pk[NT], pq[NT], pv[NT];
-    int pr32 = -1;
-    float pg = 0.f;
-    __bf16 pbeta = (__bf16)0.f;   // (kept as loaded: converting here would make the wave wait for the load at once)
-    int ra[NT], rb = -1;          // stream rows (< 2^31) of the chunk fetched next: this thread's K / Q / V rows; chunk row tid
-    // Only the low half of an index is loaded: the register of an unused high half would be handed out again at once, and
-    // whoever writes it first has to wait for the load (and with it for every load in flight).
-    const int* idx_lo = (const int*)p.idx;
+    int ra[NT];                   // stream rows (< 2^31) of the chunk fetched next: this thread's K / Q / V rows
     auto fetch_rows = [&](const int j) __attribute__((always_inline)) {
         long base[NT];
         int len[NT];
@@ -181,15 +268,6 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             if ((tid >> 4) < len[cc]) {       // this thread's row of tile cc
                 const long t = base[cc] + (tid >> 4);
                 ra[cc] = p.idx ? idx_lo[2 * t] : (int)t;
-            }
-        }
-        rb = -1;
-        if (tid < CH) {                       // chunk row tid = row tid % 16 of tile tid / 16
-            const bool hi = tid >= 16;
-            const int r = tid & 15;
-            if (r < (hi ? len[NT - 1] : len[0])) {
-                const long t = (hi ? base[NT - 1] : base[0]) + r;
-                rb = p.idx ? idx_lo[2 * t] : (int)t;
             }
         }
     };
@@ -205,29 +283,21 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
                 pv[cc] = *(const bf16x8*)(p.v + row_offset(ra[cc], p.v_tok) + hv * VD + col);
             }
         }
-        pr32 = rb;
-        pg = 0.f;
-        pbeta = (__bf16)0.f;
-        if (rb >= 0) {
-            pg = p.g[row_offset(rb, p.g_tok) + hv];
-            pbeta = p.beta[row_offset(rb, p.g_tok) + hv];
-        }
     };
+    if (!SOLVER && w == 0) {
+        fetch_gate_row(0);
+        fetch_gates();
+        fetch_gate_row(1);
+    }
     fetch_rows(0);
     fetch_data();
     fetch_rows(1);
 
     for (int j = 0; j < n_chunks; j++) {
         lds_barrier();   // every wave is done with the previous chunk's tiles
+        fresh();
         // ---- stage the chunk from the prefetch registers (rows >= L are zero): cumulative g, beta, stream rows, K / Q / V
-        if (tid < CH) {
-            float x = row_prefix_sum(pg);
-            // row_bcast:15 -> lanes 16..31 (not for a pair: the second tile is another segment)
-            if (!run_mode) x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x142, 0xa, 0xf, false));
-            Gs[tid] = x;
-            Bs[tid] = (float)pbeta;
-            Rs[tid] = pr32;
-        }
+        if (!SOLVER && w == 0) stage_gates();
         {
             const int col = (tid & 15) * 8;
 #pragma unroll
@@ -239,6 +309,7 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             }
         }
         lds_barrier();
+        fresh();
 
         // Token tiles: tile t = chunk rows 16 t .. 16 t + 15.  In a transposed token x token result the lane owns row
         // i = 16 it + c and its registers hold columns j = 16 jt + 4 q4 + r.
@@ -272,111 +343,31 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             *(bf16x4*)(Ps + i * LP + 16 * jt + 4 * q4) = p4;
         }
         lds_barrier();
-
-        // ---- T = (I - A)^-1 on wave 0: rows of the diagonal blocks by substitution in registers (lane groups 0 and 2 the
-        // upper-left block, 1 and 3 the lower-right one, in the same instructions), then the lower-left block
-        // T_lo = T_11 A_lo T_00, computed transposed (T_lo^T = T_00^T (A_lo^T T_11^T)) so that the lane again holds a row.
-        // Leaves T diag(beta) and -T diag(beta e^G) in LDS as bf16, tile by tile.
-        if (w == 0) {
-            float t[16];
-            const int blk = q4 & 1;
-            unit_lower_inverse_row<true>(As + blk * (16 * LA + 16), LA, c, t);
-            // the rows pass through LDS to reach the lanes in operand order (row c, columns 4 q4 ..+3)
-#pragma unroll
-            for (int j4 = 0; j4 < 4; j4++) *(f32x4*)(Ts + (16 * blk + c) * LX + 4 * j4) = f32x4{t[4 * j4], t[4 * j4 + 1], t[4 * j4 + 2], t[4 * j4 + 3]};
-            wave_lds_order();
-            const f32x4 G0 = *(const f32x4*)(Gs + 4 * q4), B0 = *(const f32x4*)(Bs + 4 * q4);
-            const f32x4 t00 = *(const f32x4*)(Ts + c * LX + 4 * q4);
-            f32x4 e0;
-            bf16x4 u4, w4;
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                e0[r] = B0[r] * __expf(G0[r]);
-                u4[r] = (__bf16)(t00[r] * B0[r]);
-                w4[r] = (__bf16)(-t00[r] * e0[r]);
-            }
-            *(bf16x4*)(Tus + c * LP + 4 * q4) = u4;
-            *(bf16x4*)(Tws + c * LP + 4 * q4) = w4;
-            {
-                const float* T1s = Ts + 16 * LX;
-                const f32x4 G1 = *(const f32x4*)(Gs + 16 + 4 * q4), B1 = *(const f32x4*)(Bs + 16 + 4 * q4);
-                const f32x4 t11 = *(const f32x4*)(T1s + c * LX + 4 * q4);
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    u4[r] = (__bf16)(t11[r] * B1[r]);
-                    w4[r] = (__bf16)(-t11[r] * B1[r] * __expf(G1[r]));
-                }
-                *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = u4;
-                *(bf16x4*)(Tws + (16 + c) * LP + 16 + 4 * q4) = w4;
-                f32x4 tlo = zero4();
-                if (!run_mode) {      // (a pair's tiles are different segments: A_lo = 0, so is T_lo)
-                    f32x4 x = zero4();
-#pragma unroll
-                    for (int s4 = 0; s4 < 4; s4++)        // X[j][i] = sum_m A_lo[m][j] T_11[i][m]
-                        x = mfma4(As[(16 + 4 * s4 + q4) * LA + c], T1s[c * LX + 4 * s4 + q4], x);
-#pragma unroll
-                    for (int r = 0; r < 4; r++) Xs[(4 * q4 + r) * LX + c] = x[r];
-                    wave_lds_order();
-#pragma unroll
-                    for (int s4 = 0; s4 < 4; s4++)        // T_lo[16 + i][j'] = sum_j T_00[j][j'] X[j][i]
-                        tlo = mfma4(Ts[(4 * s4 + q4) * LX + c], Xs[(4 * s4 + q4) * LX + c], tlo);
-                }
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    u4[r] = (__bf16)(tlo[r] * B0[r]);
-                    w4[r] = (__bf16)(-tlo[r] * e0[r]);
-                }
-                *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = u4;
-                *(bf16x4*)(Tws + (16 + c) * LP + 4 * q4) = w4;
-            }
-        }
-        lds_barrier();   // T visible; A and the T blocks are dead, -W may take their place
-
-        // ---- U[i][v] = sum_j Tu[i][j] V[j][v] for this wave's columns (lane = column v, registers = rows i), and this wave's
-        // share of -W^T[k][i] = sum_j K[j][k] Tw[i][j]: key tiles 2w and 2w + 1, stored as -W[i][k]
-        f32x4 vp[NT][2], qs[NT][2];
-        {
-            tok_op tu[NT], tw[NT];
-#pragma unroll
-            for (int it = 0; it < NT; it++) {
-                const __bf16* up = Tus + (16 * it + c) * LP + 4 * q4;
-                const __bf16* wp = Tws + (16 * it + c) * LP + 4 * q4;
-                tu[it] = join(*(const bf16x4*)up, it ? *(const bf16x4*)(up + 16) : zero_bf4());
-                tw[it] = join(*(const bf16x4*)wp, it ? *(const bf16x4*)(wp + 16) : zero_bf4());
-            }
-#pragma unroll
-            for (int vt = 0; vt < 2; vt++) {
-                const tok_op vB = join(frag_tr4(Vs, LDT, 0, 32 * w + 16 * vt, lane), frag_tr4(Vs, LDT, 16, 32 * w + 16 * vt, lane));
-#pragma unroll
-                for (int it = 0; it < NT; it++) {
-                    vp[it][vt] = mfma32(tu[it], vB, zero4());
-                    qs[it][vt] = zero4();
-                }
-            }
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int kt = 2 * w + h;
-                const tok_op kT = join(frag_tr4(Ks, LDT, 0, 16 * kt, lane), frag_tr4(Ks, LDT, 16, 16 * kt, lane));
-#pragma unroll
-                for (int it = 0; it < NT; it++) *(bf16x4*)(Wn + (16 * it + c) * LW + 16 * kt + 4 * q4) = round4(mfma32(kT, tw[it], zero4()));
-            }
-        }
-        lds_barrier();   // -W visible; every wave has read its V columns
-        // The next chunk's rows are requested here: the registers they land in are free since the staging, and from here no phase
-        // needs more registers than there are (one phase earlier the solve spills).  They have the three value-column phases
-        // (about 4 k cycles) to arrive; requested after the V' phase (2 k cycles) the next chunk's staging waited for them.
+        fresh();
+        if (!SOLVER && w == 0) solve();
+        // The next chunk's rows are requested here, behind the solve (which needs their registers): they have the rest of the chunk to arrive.
         fetch_data();          // chunk j + 1, whose rows are known since the previous chunk
         fetch_rows(j + 2);
-
-        // ---- V' = U + (-W) S and Q S over the 128 key rows, 32 at a time (the state tiles 2s and 2s + 1 are the B operand)
+        if (!SOLVER && w == 0) {
+            fetch_gates();
+            fetch_gate_row(j + 2);
+        }
+        f32x4 vp[NT][2], qs[NT][2], Gj[NT], eG[NT];
+        tok_op vin[2], rin[2];     // V (as it came) and R = -e^G (K S), rounded by itself
+        // ---- K S and Q S over the 128 key rows, 32 at a time (the state tiles 2s and 2s + 1 are the B operand): they do not need T, so
+        // waves 0 - 3 do them beside the solve
+#pragma unroll
+        for (int it = 0; it < NT; it++)
+#pragma unroll
+            for (int vt = 0; vt < 2; vt++) vp[it][vt] = qs[it][vt] = zero4();
 #pragma unroll
         for (int s = 0; s < KD / 32; s++) {
-            bf16x8 wA[NT], qA[NT];
+            bf16x8 kA[NT], qA[NT];
 #pragma unroll
             for (int it = 0; it < NT; it++) {
-                const __bf16* wp = Wn + (16 * it + c) * LW + 32 * s + 4 * q4;
+                const __bf16* kp = Ks + (16 * it + c) * LDT + 32 * s + 4 * q4;
                 const __bf16* qp = Qs + (16 * it + c) * LD + 32 * s + 4 * q4;
-                wA[it] = join(*(const bf16x4*)wp, *(const bf16x4*)(wp + 16));
+                kA[it] = join(*(const bf16x4*)kp, *(const bf16x4*)(kp + 16));
                 qA[it] = join(*(const bf16x4*)qp, *(const bf16x4*)(qp + 16));
             }
 #pragma unroll
@@ -384,15 +375,36 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
                 const bf16x8 sb = join(round4(S[2 * s][vt]), round4(S[2 * s + 1][vt]));
 #pragma unroll
                 for (int it = 0; it < NT; it++) {
-                    vp[it][vt] = mfma32(wA[it], sb, vp[it][vt]);
+                    vp[it][vt] = mfma32(kA[it], sb, vp[it][vt]);
                     qs[it][vt] = mfma32(qA[it], sb, qs[it][vt]);
                 }
             }
         }
-        // ---- O[i][v] = s e^{G_i} (Q S)[i][v] + sum_j P[i][j] V'[j][v], rows i = 16 it + 4 q4 + r; through LDS for 16-byte stores
-        f32x4 Gj[NT];
 #pragma unroll
-        for (int it = 0; it < NT; it++) Gj[it] = *(const f32x4*)(Gs + 16 * it + 4 * q4);
+        for (int it = 0; it < NT; it++) {
+            Gj[it] = *(const f32x4*)(Gs + 16 * it + 4 * q4);
+#pragma unroll
+            for (int r = 0; r < 4; r++) eG[it][r] = __expf(Gj[it][r]);
+        }
+#pragma unroll
+        for (int vt = 0; vt < 2; vt++) {
+            vin[vt] = join(frag_tr4(Vs, LDT, 0, 32 * w + 16 * vt, lane), frag_tr4(Vs, LDT, 16, 32 * w + 16 * vt, lane));
+            rin[vt] = join(round4(-eG[0] * vp[0][vt]), round4(-eG[1] * vp[1][vt]));
+        }
+        lds_barrier();   // T visible; every wave has read its V columns
+        fresh();
+
+        // ---- V' = T diag(beta) (V + R)
+        {
+#pragma unroll
+            for (int it = 0; it < NT; it++) {
+                const __bf16* up = Tus + (16 * it + c) * LP + 4 * q4;
+                const tok_op tu = join(*(const bf16x4*)up, it ? *(const bf16x4*)(up + 16) : zero_bf4());
+#pragma unroll
+                for (int vt = 0; vt < 2; vt++) vp[it][vt] = mfma32(tu, rin[vt], mfma32(tu, vin[vt], zero4()));
+            }
+        }
+        // ---- O[i][v] = s e^{G_i} (Q S)[i][v] + sum_j P[i][j] V'[j][v], rows i = 16 it + 4 q4 + r; through LDS for 16-byte stores
         {
             tok_op pA[NT];
 #pragma unroll
@@ -407,7 +419,7 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
                 for (int it = 0; it < NT; it++) {
                     f32x4 o = mfma32(pA[it], vb, zero4());
 #pragma unroll
-                    for (int r = 0; r < 4; r++) o[r] = __builtin_fmaf(p.scale * __expf(Gj[it][r]), qs[it][vt][r], o[r]);
+                    for (int r = 0; r < 4; r++) o[r] = __builtin_fmaf(p.scale * eG[it][r], qs[it][vt][r], o[r]);
                     *(bf16x4*)(Ow + (16 * vt + c) * LO + 16 * it + 4 * q4) = round4(o);      // O^T[v][i]
                 }
             }
@@ -462,9 +474,26 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
   }
 }
 
-// 32-token chunks, 254 registers, two workgroups per compute unit; the recurrent entry point's kernel also pairs up leaves.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_wy32_kernel(const GdnParams p) { gdn_wy_body<false>(p); }
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_wy_pairs_kernel(const GdnParams p) { gdn_wy_body<true>(p); }
+// 32-token chunks.  Three kernels of the same bits for long segments; a launch takes one by the number of its workgroups:
+// * at most one per compute unit: with a solving wave.  Of a chunk's 7.9 k clocks the other waves wait 2.0 k for wave 0, which has the solve
+//   and its columns.  A trunk of 301 tokens, 32 workgroups: 34.8 us against 38.1.  A compute unit does not take two such workgroups
+//   (2,048-token trunks, 1,024 workgroups: 817 us against 639).
+// * two per compute unit (248 registers) or three (168): a workgroup alone takes 1, two together 1.42 and three 1.96 times as long, so three
+//   win unless the last round leaves them behind: 704 workgroups of about 300 tokens 90.2 us against 106.4, but 1,024 of 2,048 tokens
+//   669 against 639 (a round of 768 and one of 256, against two full ones).
+// The recurrent entry point's kernel, which also pairs up leaves, is the tight one: 24 leaves of a request 12.0 us against 15.5, 1,024 leaves
+// of 12 tokens 154 against 162.
+__global__ __launch_bounds__(320) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_wy32_solver_kernel(const GdnParams p) { gdn_wy_body<false, true, true>(p); }
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void gdn_wy32_kernel(const GdnParams p) { gdn_wy_body<false, false, false>(p); }
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void gdn_wy32_tight_kernel(const GdnParams p) { gdn_wy_body<false, false, true>(p); }
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void gdn_wy_pairs_kernel(const GdnParams p) { gdn_wy_body<true, false, true>(p); }
+
+// rounds of n workgroups, `fit` to each of 256 compute units, in units of one workgroup alone
+static float scan_rounds(long n, int fit) {
+    const float together[4] = {0.f, 1.f, 1.42f, 1.96f};
+    const long full = n / (256 * fit), rest = n % (256 * fit);
+    return (float)full * together[fit] + together[(rest + 255) / 256];
+}
 
 // pairs: the recurrent entry point (short segments, leaves two to a chunk)
 int gdn_wy_launch(GdnParams p, bool pairs, hipStream_t stream) {
@@ -474,8 +503,11 @@ int gdn_wy_launch(GdnParams p, bool pairs, hipStream_t stream) {
     while (pairs && p.run < 16 && (p.n_seg + 2 * p.run - 1) / (2 * p.run) * p.hv >= 2048) p.run *= 2;
     const long blocks = (p.n_seg + p.run - 1) / p.run * p.hv;
     if (blocks > INT32_MAX) return spinf_fail(SPINF_E_ARG, "gdn: too many segments");
-    if (!pairs) hipLaunchKernelGGL(gdn_wy32_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL(gdn_wy_pairs_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, p);
+    const dim3 grid((unsigned)blocks);
+    if (pairs) hipLaunchKernelGGL(gdn_wy_pairs_kernel, grid, dim3(256), 0, stream, p);
+    else if (blocks <= 256) hipLaunchKernelGGL(gdn_wy32_solver_kernel, grid, dim3(320), 0, stream, p);
+    else if (scan_rounds(blocks, 3) < scan_rounds(blocks, 2)) hipLaunchKernelGGL(gdn_wy32_tight_kernel, grid, dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL(gdn_wy32_kernel, grid, dim3(256), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "gdn: launch: %s", hipGetErrorString(e));
     return SPINF_OK;

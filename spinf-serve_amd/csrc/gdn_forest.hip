@@ -252,6 +252,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
         // ---- T diag(beta) on wave 0 (gdn_chunk.hip explains the solve), while the other waves go on with their columns
         if (w == 0) {
+            __builtin_amdgcn_s_setprio(3);
             float t[16];
             const int blk = q4 & 1;
             unit_lower_inverse_row<true>(As + blk * (16 * LA + 16), LA, c, t);
@@ -272,6 +273,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
             *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
             *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = round4(tlo * B0);
+            __builtin_amdgcn_s_setprio(0);
         }
         // Block j + 1 is requested here, behind the solve, which needs the registers; it has the rest of this block to arrive.
         fetch_data();

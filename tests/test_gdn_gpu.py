@@ -191,6 +191,30 @@ def test_deep_trie(dev):
     _within(o, want, TOL, "deep tree")
 
 
+@pytest.mark.parametrize("n", [100, 130])
+def test_scan_kernels_agree_bit_for_bit(dev, n):
+    """the chunked entry point's three kernels (by the number of workgroups: up to 256, rounds of 512, rounds of 768; n segments x 4 heads
+    take two of them, a call over 5 of the segments the third) leave the same outputs and states"""
+    H, HV, lens = 2, 4, [1 + (7 * i) % 70 for i in range(n)]
+    cu_cpu = np.concatenate([[0], np.cumsum(lens)])
+    t = _inputs(int(cu_cpu[-1]), H, HV, dev, seed=n)
+    args = [t[x][None] for x in ("q", "k", "v", "g", "beta")]
+    ht, few = (torch.full((n, HV, 128, 128), float("nan"), device=dev) for _ in range(2))
+    idx = torch.arange(n, device=dev)
+    o = sa.chunked(*args, 128 ** -0.5, torch.from_numpy(cu_cpu).to(dev), cu_cpu, ht=ht, ht_idx=idx)
+    o_few = torch.zeros_like(o)
+    for a in range(0, n, 5):
+        cu = cu_cpu[a : a + 6]
+        rows = torch.arange(int(cu[0]), int(cu[-1]), device=dev)
+        sa.chunked(*args, 128 ** -0.5, torch.from_numpy(cu - cu[0]).to(dev), cu - cu[0], ht=few, ht_idx=idx[a : a + 5].contiguous(), idx=rows, o=o_few)
+    torch.cuda.synchronize()
+    assert torch.equal(o, o_few) and torch.equal(ht, few)
+    for i in (0, 9, n - 1):
+        want, S = ogdn.recurrent(*(_np(t[x][cu_cpu[i] : cu_cpu[i + 1]]) for x in ("q", "k", "v", "g", "beta")))
+        _within(o[0, cu_cpu[i] : cu_cpu[i + 1]], want, TOL, f"segment {i} of {n}")
+        _within(ht[i], S, STATE_TOL, f"state {i} of {n}")
+
+
 def _chain_tree(rng, trunk, nodes):
     """nodes [(length, parent)] below a trunk"""
     return synth._tree(rng, trunk, [n for n, _ in nodes], [p for _, p in nodes])
