@@ -375,38 +375,61 @@ __global__ __launch_bounds__(256, D <= 256 ? 2 : 1) void xdec_kernel(const XdecP
     }
 }
 
-// out = sum_s 2^(M_s - M*) O_s / sum_s 2^(M_s - M*) l_s over the splits of a row, splits in ascending order; one thread per 4 head dims
+// out = sum_s 2^(M_s - M*) O_s / sum_s 2^(M_s - M*) l_s over the splits of a row, splits in ascending order; one wave per row, so that the
+// row's place, its tile list and the loop are scalar and lane s has split s's weight (64 splits at most).  A thread per four head dims did
+// all of that by itself, one load after the other: 24 groups x 48 queries x 16 heads x 256, two splits, 13.9 -> 12.3 us (3.8 TB/s); one group at
+// head dim 512, 7.5 us of a step of 29.4, which now takes 25.6.
 template <int D>
-__global__ __launch_bounds__(256) void xdec_combine_kernel(const XdecParams p, const long n_rows) {
-    const long idx = (long)blockIdx.x * 256 + threadIdx.x;
-    const long rowid = idx / (D / 4);
-    const int d4 = (int)(idx - rowid * (D / 4));
+__global__ __launch_bounds__(256) void xdec_combine_kernel(const XdecParams p, const int n_rows) {
+    constexpr int VEC = D / 64;    // head dims per lane
+    typedef __attribute__((ext_vector_type(VEC))) float vec;
+    typedef __attribute__((ext_vector_type(VEC))) __bf16 bvec;
+    const int lane = threadIdx.x & 63;
+    const int rowid = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
     if (rowid >= n_rows) return;
-    const long gg = rowid / ((long)p.H * p.Q);
-    const int head = (int)((rowid / p.Q) % p.H), qi = (int)(rowid % p.Q);
+    const int gg = rowid / (p.H * p.Q), in_group = rowid - gg * (p.H * p.Q), head = in_group / p.Q, qi = in_group - head * p.Q;
     // the splits that exist for this row: those of its row chunk's tile list
     const int chunk = (qi * p.r + head % p.r) / XROWS;
     const int last_row = chunk * XROWS + XROWS - 1 < p.R ? chunk * XROWS + XROWS - 1 : p.R - 1;
     const TileList tl(p.Lp, p.Tt, p.S, group_len(p.len_p, gg, p.Lp), group_len(p.len_t, gg, p.Tt), (chunk * XROWS) / p.r, last_row / p.r);
     const int ns = (tl.nt + p.per - 1) / p.per;
     if (ns == 1) return;   // written by the one workgroup itself
-    const float* ml = p.part_ml + rowid * p.nsplit * 2;
-    float mstar = -INFINITY;
-    for (int s = 0; s < ns; s++) mstar = fmaxf(mstar, ml[2 * s]);
-    float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+    float2 ml = make_float2(-INFINITY, 0.f);
+    if (lane < ns) ml = ((const float2*)p.part_ml)[(long)rowid * p.nsplit + lane];
+    float mstar = ml.x;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) mstar = fmaxf(mstar, __shfl_xor(mstar, d));
+    const float weight = __builtin_amdgcn_exp2f(ml.x - mstar);
+    unsigned long long left = __builtin_amdgcn_ballot_w64(ml.x != -INFINITY);   // (the others wrote nothing)
+    const float* part = p.part_o + (long)rowid * p.nsplit * D + VEC * lane;
+    vec acc = (vec)(0.f);
     float lsum = 0.f;
-    for (int s = 0; s < ns; s++) {
-        const float ms = ml[2 * s];
-        if (ms == -INFINITY) continue;
-        const float wgt = __builtin_amdgcn_exp2f(ms - mstar);
-        const float4 x = *(const float4*)(p.part_o + (rowid * p.nsplit + s) * D + 4 * d4);
-        acc.x += wgt * x.x; acc.y += wgt * x.y; acc.z += wgt * x.z; acc.w += wgt * x.w;
-        lsum += wgt * ml[2 * s + 1];
+    while (left) {
+        int split[4], n = 0;
+        vec x[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (left) {
+                split[k] = __builtin_ctzll(left);
+                left &= left - 1;
+                x[k] = *(const vec*)(part + (long)split[k] * D);
+                n = k + 1;
+            }
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            if (k < n) {
+                const float wgt = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), split[k]));
+                const float l = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ml.y), split[k]));
+#pragma unroll
+                for (int i = 0; i < VEC; i++) acc[i] += wgt * x[k][i];
+                lsum += wgt * l;
+            }
     }
     const float inv = 1.0f / lsum;
-    bf16x4 r;
-    r[0] = (__bf16)(acc.x * inv); r[1] = (__bf16)(acc.y * inv); r[2] = (__bf16)(acc.z * inv); r[3] = (__bf16)(acc.w * inv);
-    *(bf16x4*)(p.out + ((gg * p.Q + qi) * p.H + head) * D + 4 * d4) = r;
+    bvec r;
+#pragma unroll
+    for (int i = 0; i < VEC; i++) r[i] = (__bf16)(acc[i] * inv);
+    *(bvec*)(p.out + (((long)gg * p.Q + qi) * p.H + head) * D + VEC * lane) = r;
 }
 
 // The new tokens' keys (blockIdx.y 0) and values (1) into entry `step` of the generated caches: one thread per 16 bytes.  Latency bound:
@@ -458,9 +481,9 @@ int launch_d(const XdecParams& p, bool cap, int blocks, hipStream_t s) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "xdecode_attn: launch: %s", hipGetErrorString(e));
     if (p.nsplit > 1) {
-        const long n_rows = (long)p.G * p.H * p.Q;
-        const long threads = n_rows * (D / 4);
-        hipLaunchKernelGGL((xdec_combine_kernel<D>), dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, p, n_rows);
+        const long n_rows = (long)p.G * p.H * p.Q;   // (2^31 rows would be a workspace of over 1 TB)
+        if (n_rows > INT32_MAX) return spinf_fail(SPINF_E_ARG, "xdecode_attn: %ld rows in splits", n_rows);
+        hipLaunchKernelGGL((xdec_combine_kernel<D>), dim3((unsigned)((n_rows + 3) / 4)), dim3(256), 0, s, p, (int)n_rows);
         e = hipGetLastError();
         if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "xdecode_attn: launch (combine): %s", hipGetErrorString(e));
     }
