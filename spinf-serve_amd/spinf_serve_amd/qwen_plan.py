@@ -43,8 +43,9 @@ class TreePlan:
     seg_slot: object | None = None
     cap: dict | None = None
     pad_rows: object | None = None   # [pads] int64 (device): rows of the tensors no segment covers; their outputs are zero
-    launches: list | None = None     # indexed path: per level the kernel launches (mode, segments, longest, addresses of cu, idx, h0_idx, ht_idx), neighbouring calls of one kind as one
+    launches: list | None = None     # indexed path: per level the kernel launches (mode, segments, longest, places of cu, idx, h0_idx, ht_idx in data, -1 none), neighbouring calls of one kind as one
     program: list | None = None      # the same with the small subtrees as forests of their own (mode 2, csrc/gdn_forest.hip); None without any
+    data: object | None = None       # [*] int64 (device): what the launches read (places, not addresses: a copied or reloaded plan has its own)
 
 
 _PATHS = {"indexed": 0, "levels": 1}
@@ -140,18 +141,18 @@ def tree_plan(prev, real, device, max_init: int = 96, path: str = "indexed", sho
         for i, j in lv if indexed else ():
             idx, cu, _, starts, ends = cut(i, j)
             lens = seg_len[seg_ptr[i] : seg_ptr[j]]
-            merged.append((int(call_kind[i]), len(lens), int(lens.max()) if call_kind[i] else 0, cu.data_ptr(), idx.data_ptr(), starts.data_ptr() if d else None,
-                           ends.data_ptr() if call_keep[i:j].any() else None))   # (views of on_dev, which plan.conv keeps alive)
+            merged.append((int(call_kind[i]), len(lens), int(lens.max()) if call_kind[i] else 0, cu.storage_offset(), idx.storage_offset(),
+                           starts.storage_offset() if d else -1, ends.storage_offset() if call_keep[i:j].any() else -1))   # (views of on_dev)
         launches.append(merged)
     program = None
     if len(a["program"]):
         program = [[] for _ in levels]
-        base = program_data.data_ptr()
-        for d, mode, n, longest, *offsets in a["program"].tolist():
-            program[d].append((mode, n, longest, *(base + 8 * o if o >= 0 else None for o in offsets)))
+        first = program_data.storage_offset()
+        for d, mode, n, longest, *places in a["program"].tolist():
+            program[d].append((mode, n, longest, *(first + o if o >= 0 else -1 for o in places)))
     seg_of_row = a["seg_of_row"]
     return TreePlan(conv.view(-1, 4), levels, a["n_segments"], path, a["n_keep"].tolist() if indexed else None, rows, sidx if rows is not None else None, seg_of_row,
-                    a["seg_level"], a["seg_slot"], pad_rows=pad_rows, launches=launches if indexed else None, program=program)
+                    a["seg_level"], a["seg_slot"], pad_rows=pad_rows, launches=launches if indexed else None, program=program, data=on_dev if indexed else None)
 
 
 def _kept_state_requests(plan: TreePlan, cap):
@@ -196,19 +197,21 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
     args = gdn.level_args(q, k, v, g32, b16, o, scale) if indexed and plan.launches is not None else None
     # a forest's nodes leave no states (and its kernel is built for 128 value dims): a caller that asks for states gets every level's
     launches = plan.launches if wanted or plan.program is None or v.shape[-1] != 128 else plan.program
+    base = plan.data.data_ptr() if args is not None else 0
     above = None   # the states the level above left
     for d, calls in enumerate(plan.levels):
         if args is not None and launches is plan.program:
-            n_slots = plan.n_keep[d] if any(launch[-1] is not None for launch in launches[d]) else 0
+            n_slots = plan.n_keep[d] if any(launch[-1] >= 0 for launch in launches[d]) else 0
         else:
             n_slots = plan.n_keep[d] if indexed else sum(len(c.cu_cpu) - 1 for c in calls if c.keep)
         states = q.new_empty((n_slots, v.shape[1], q.shape[-1], v.shape[-1]), dtype=torch.float32) if n_slots else None
         next_slot = 0
         if args is not None:
             h0, ht = None if above is None else above.data_ptr(), None if states is None else states.data_ptr()
-            for args.mode, args.n_seg, args.max_len, args.cu, args.idx, h0_idx, ht_idx in launches[d]:
-                args.h0, args.h0_idx = (h0, h0_idx) if h0_idx is not None else (None, None)
-                args.ht, args.ht_idx = (ht, ht_idx) if ht_idx is not None else (None, None)
+            for args.mode, args.n_seg, args.max_len, cu, idx, h0_idx, ht_idx in launches[d]:
+                args.cu, args.idx = base + 8 * cu, base + 8 * idx
+                args.h0, args.h0_idx = (h0, base + 8 * h0_idx) if h0_idx >= 0 else (None, None)
+                args.ht, args.ht_idx = (ht, base + 8 * ht_idx) if ht_idx >= 0 else (None, None)
                 _lib.launch(_lib.load_library().spinf_gdn_fwd, args, q.device, "spinf_gdn_fwd")
             calls = ()
         for c in calls:

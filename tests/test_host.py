@@ -1,6 +1,7 @@
 """Host side of the path (no GPU): the stream layout, the tile-plan compiler (C ABI, host code), the recurrent-layer planner,
 and that the shared library loads and exports every symbol include/spinf_tree.h declares."""
 
+import copy
 import ctypes
 import gzip
 import json
@@ -497,13 +498,14 @@ def test_tree_plan_matches_reference_and_oracle(golden):
 
 
 def _program(plan):
-    """a CPU plan's program as (level, mode, cu, idx or block table, h0_idx, ht_idx) with the arrays read back from their addresses"""
-    at = lambda p, n, t=ctypes.c_int64: np.ctypeslib.as_array((t * n).from_address(p)).copy() if n else np.zeros(0, np.int64)  # noqa: E731
+    """a CPU plan's program as (level, mode, cu, idx or block table, h0_idx, ht_idx) with the arrays cut out of plan.data"""
+    data = plan.data.numpy()
+    at = lambda place, n: data[place : place + n].copy() if place >= 0 else None  # noqa: E731
     for d, launches in enumerate(plan.program):
         for mode, n, _, cu, idx, h0, ht in launches:
             cu = at(cu, n + 1)
-            table = at(idx, 96 * int(cu[-1]), ctypes.c_int32).reshape(-1, 3, 32) if mode == 2 else at(idx, int(cu[-1]))
-            yield d, mode, cu, table, at(h0, n) if h0 else None, at(ht, n) if ht else None
+            table = at(idx, 48 * int(cu[-1])).view(np.int32).reshape(-1, 3, 32) if mode == 2 else at(idx, int(cu[-1]))
+            yield d, mode, cu, table, at(h0, n), at(ht, n)
 
 
 @pytest.mark.parametrize("seed", range(12))
@@ -523,6 +525,7 @@ def test_tree_plan_program_is_the_forest(seed):
     plan = sa.tree_plan(s.prev, real, "cpu", keep=keep)
     if plan.program is None:
         pytest.skip("no forest in this stream")
+    plan = copy.deepcopy(plan)     # (places in its own data, no addresses)
     done, slot_tail, forests = np.zeros(len(real), int), [dict() for _ in plan.levels], 0
     for d, mode, cu, table, h0, ht in _program(plan):
         for u in range(len(cu) - 1):
