@@ -189,6 +189,7 @@ class _Layer:
         self.head_groups, self.variant, self.n_lists = hq // per_item, variant, n_lists
         a = self.args = _lib.AttnArgs()
         a.n, a.hq, a.hkv, a.d, a.window = m.n, hq, hkv, d, m.window
+        self.owned = (m.art, m.end, m.pos, m.grp)   # (alive for as long as the block points to them)
         a.art, a.end, a.pos = m.art.data_ptr(), m.end.data_ptr(), m.pos.data_ptr()
         a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items = m.pointers(self.head_groups, n_lists)
         a.variant, a.ktile, a.n_lists = variant, m._ktile, n_lists

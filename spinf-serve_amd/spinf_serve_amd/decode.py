@@ -13,7 +13,6 @@ over workgroups): nothing is copied per slot or per beam, no mask tensor is buil
 from __future__ import annotations
 
 import ctypes as C
-import weakref
 from dataclasses import dataclass, field
 from typing import Optional
 
@@ -223,12 +222,12 @@ def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None
     eager = _lib.eager(query, *tensors) and query.dtype == torch.bfloat16 and query.is_cuda and query.device == gk.device and query.stride(3) == 1
     key = (li, query.shape, nsplit, c.beam)
     if eager:   # a decoder's later steps: the same caches, another query tensor
-        where = tuple(t if t is None else t.data_ptr() for t in tensors)
+        where = [t if t is None else (t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tensors]
         got = c._calls.get(key)
-        if got is not None and got[1] == where and all(x is None if y is None else x is y() for x, y in zip(tensors, got[0])):
-            a = _lib.XdecArgs.from_buffer_copy(got[2])
+        if got is not None and got[0] == where:
+            a = _lib.XdecArgs.from_buffer_copy(got[1])
             a.scale, a.window, a.softcap = scale, window, softcap
-            return _xdecode_run(a, query, c.workspace(query.device, got[3]) if got[3] else None)
+            return _xdecode_run(a, query, c.workspace(query.device, got[2]) if got[2] else None)
     per = 0
     if nsplit is None and li in c._host_len:   # the groups' own lengths are known: split sizes that balance them
         geo = (G, H, gk.shape[1], Q, gk.shape[3], kp.shape[2], c.kt[li].shape[2], d, c.beam)
@@ -242,7 +241,7 @@ def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None
     work = c.workspace(query.device, nbytes) if nbytes else None
     if eager:
         a = _xdecode_args(query, *tensors, int(nsplit), int(per), int(c.beam))
-        c._calls[key] = (tuple(t if t is None else weakref.ref(t) for t in tensors), where, _lib.XdecArgs.from_buffer_copy(a), nbytes)
+        c._calls[key] = (where, _lib.XdecArgs.from_buffer_copy(a), nbytes)
         a.scale, a.window, a.softcap = scale, window, softcap
         return _xdecode_run(a, query, work)
     return _xdecode_op(query, *tensors, work, int(nsplit), int(per), int(c.beam), scale, window, softcap)
