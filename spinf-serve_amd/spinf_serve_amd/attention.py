@@ -172,7 +172,8 @@ def _(q, k, v, art, end, pos, kv_idx, kv_bits, items, list_ptr, n_items, scale, 
 
 class _Layer:
     """what the calls of one mask at one head geometry share: the schedule on the device and the argument block with everything in it
-    that does not belong to one layer's tensors (the mask owns the memory it points to)"""
+    that does not belong to one layer's tensors.  It owns every tensor its block points into: the mask it is kept in may be the one with
+    the other key-tile size, and outlive the one the tensors came from."""
 
     def __init__(self, mask, hq, hkv, d, variant, compact, device):
         if _spread(device, hq, hkv, d, variant, mask):
@@ -189,9 +190,9 @@ class _Layer:
         self.head_groups, self.variant, self.n_lists = hq // per_item, variant, n_lists
         a = self.args = _lib.AttnArgs()
         a.n, a.hq, a.hkv, a.d, a.window = m.n, hq, hkv, d, m.window
-        self.owned = (m.art, m.end, m.pos, m.grp)   # (alive for as long as the block points to them)
         a.art, a.end, a.pos = m.art.data_ptr(), m.end.data_ptr(), m.pos.data_ptr()
-        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items = m.pointers(self.head_groups, n_lists)
+        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items, uploads = m.pointers(self.head_groups, n_lists)
+        self.owned = (m.art, m.end, m.pos, m.grp, *uploads)
         a.variant, a.ktile, a.n_lists = variant, m._ktile, n_lists
         if m.grp is not None:
             a.grp, a.grp_mode = m.grp.data_ptr(), m.grp_mode
@@ -201,7 +202,10 @@ class _Layer:
         key = (hq, hkv, d, variant, compact, RING, STATIC, RING_128, SPREAD)
         got = mask._layers.get(key)
         if got is None:
-            got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, device)
+            with mask._lock:
+                got = mask._layers.get(key)
+                if got is None:
+                    got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, device)
         return got
 
     def bound(self, q, qs, k, ks, v, vs, out, os, scale):

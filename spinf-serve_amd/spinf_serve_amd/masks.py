@@ -10,6 +10,7 @@ whose global layers have 512-dim heads never compiles the 64-key plan of its glo
 from __future__ import annotations
 
 import ctypes as C
+import threading
 import weakref
 
 import numpy as np
@@ -129,10 +130,12 @@ def _staging(n: int, device):
 
 class TreeMask:
     """Device-side handle: the stream's metadata, and per key-tile size a plan compiled when the first call that takes it comes (a
-    forward's layers share it).  ``seq_lengths`` mirrors BlockMask.seq_lengths (spinf_serve/models/qwen35/qwen.py:615 reads it)."""
+    forward's layers share it).  ``seq_lengths`` mirrors BlockMask.seq_lengths (spinf_serve/models/qwen35/qwen.py:615 reads it).
+    Host threads may share a mask: what a first call makes (plan, uploads, prepared calls) is made once, under a lock."""
 
-    def __init__(self, plan, meta, device, grp=None, host=None, window=None, ktile=64):
+    def __init__(self, plan, meta, device, grp=None, host=None, window=None, ktile=64, lock=None):
         """plan: a compiled plan, or None: compiled from host = (art, end, pos, grp or None, grp_windowed) for this window and ktile"""
+        self._lock = lock or threading.RLock()   # (one for both key-tile sizes: they refer to each other)
         self._host = host
         self._plan = plan
         self._ktile = plan.ktile if plan is not None else ktile
@@ -142,8 +145,8 @@ class TreeMask:
         self.n = plan.n if plan is not None else len(host[0])
         self.window = plan.window if plan is not None else int(window) if window else 0
         self.seq_lengths = (self.n, self.n)
-        self.device = device
         self.art, self.end, self.pos = meta
+        self.device = self.art.device       # (of "cuda" the GPU that was current at the build, whatever is current at the first call)
         self._kv = None                     # the buffer with the device copies of the plan's kv_idx, kv_bits, and where they lie in it
         self._sched = {}
         self._layers = {}                   # prepared calls by head geometry (attention.py)
@@ -152,8 +155,10 @@ class TreeMask:
     @property
     def plan(self) -> TilePlan:
         if self._plan is None:
-            art, end, pos, grp, grp_windowed = self._host
-            self._plan = TilePlan.build(art, end, pos, self.window, grp, grp_windowed, self._ktile)
+            with self._lock:
+                if self._plan is None:
+                    art, end, pos, grp, grp_windowed = self._host
+                    self._plan = TilePlan.build(art, end, pos, self.window, grp, grp_windowed, self._ktile)
         return self._plan
 
     @property
@@ -170,7 +175,7 @@ class TreeMask:
 
     def _entries(self):
         if self._kv is None:
-            self._upload(1, 0)
+            self._schedule(1, 0)
         dev, at = self._kv
         return dev[at[2] : at[3]], dev[at[3] : at[4]]
 
@@ -180,12 +185,17 @@ class TreeMask:
         ktile = 32 if d == 512 or ring else 64
         if ktile == self._ktile:
             return self
-        other = self._other() if isinstance(self._other, weakref.ref) else self._other
+        other = self._other
+        other = other() if isinstance(other, weakref.ref) else other
         if other is None:
             if self._host is None:
                 raise ValueError(f"this mask was built for key tiles of {self._ktile}; head dim {d} takes {ktile}")
-            other = self._other = TreeMask(None, (self.art, self.end, self.pos), self.device, self.grp, self._host, self.window, ktile)
-            other._other = weakref.ref(self)   # (no cycle: a pass's masks go, and give their device memory back, with the last reference)
+            with self._lock:
+                other = self._other() if isinstance(self._other, weakref.ref) else self._other
+                if other is None:
+                    other = TreeMask(None, (self.art, self.end, self.pos), self.device, self.grp, self._host, self.window, ktile, self._lock)
+                    other._other = weakref.ref(self)   # (no cycle: a pass's masks go, and give their device memory back, with the last reference)
+                    self._other = other
         return other
 
     def rows(self, sidx):
@@ -226,18 +236,26 @@ class TreeMask:
         got = self._sched[(head_groups, n_lists)] = dev, at, plan.n_qtiles * head_groups
         return got
 
+    def _schedule(self, head_groups: int, n_lists: int):
+        got = self._sched.get((head_groups, n_lists))
+        if got is None:
+            with self._lock:   # (two first calls at a time: the second one's buffers would replace the ones the first is about to read)
+                got = self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
+        return got
+
     def schedule(self, head_groups: int, n_lists: int = 0):
         """device copy of the work lists for this many head groups (built on first use, then kept); n_lists > 0: the static
         schedule for that many workgroups"""
-        dev, at, n_items = self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
+        dev, at, n_items = self._schedule(head_groups, n_lists)
         return dev[: at[1]].view(-1, 4), dev[at[1] : at[2]], n_items
 
     def pointers(self, head_groups: int, n_lists: int):
-        """-> device addresses of items, list_ptr, kv_idx, kv_bits, and the number of items"""
-        dev, at, n_items = self._sched.get((head_groups, n_lists)) or self._upload(head_groups, n_lists)
-        items, (kv, kv_at) = dev.data_ptr(), self._kv
-        kv = kv.data_ptr()
-        return items, items + 4 * at[1], kv + 4 * kv_at[2], kv + 4 * kv_at[3], n_items
+        """-> device addresses of items, list_ptr, kv_idx, kv_bits, the number of items, and the tensors the addresses lie in (whoever
+        keeps an address keeps its tensor)"""
+        dev, at, n_items = self._schedule(head_groups, n_lists)
+        kv, kv_at = self._kv
+        items, entries = dev.data_ptr(), kv.data_ptr()
+        return items, items + 4 * at[1], entries + 4 * kv_at[2], entries + 4 * kv_at[3], n_items, (dev, kv)
 
     @classmethod
     def build(cls, art, end, pos, window=None, device="cuda", meta=None, grp=None, grp_windowed=False, grp_dev=None):

@@ -3,6 +3,8 @@ recurrent-layer interfaces (spinf_serve/models/gemma4.py:98-119, spinf_serve/mod
 with transformers (gemma4.py:121-122), the plan compilers under threads, and the CPU baseline's fp32 arithmetic against the
 float64 oracle."""
 
+import gc
+import sys
 import threading
 import types
 
@@ -15,7 +17,7 @@ from oracle import attention as oattn
 from oracle import cpu_baseline
 from oracle import gdn as ogdn
 from oracle import mask as omask
-from spinf_serve_amd import attention, synth
+from spinf_serve_amd import attention, masks, synth
 
 
 # ----------------------------------------------------------------------------------------------------------------- CPU
@@ -68,6 +70,55 @@ def test_plan_compilers_from_two_threads():
             t.join()
         for a, b in zip(serial, got):
             assert all(np.array_equal(np.asarray(x), np.asarray(y)) for x, y in zip(a, b))
+
+
+def _fresh_mask(seed=0):
+    b = synth.attention_config("C2", seed=seed, contents=3).batches[0]
+    return sa.TreeMask.build(b.art, b.end, b.pos, device="cpu")
+
+
+def _owns_what_it_points_to(layer):
+    spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for t in layer.owned if t is not None]
+    return all(any(a <= getattr(layer.args, f) < a + n for a, n in spans) for f in ("art", "end", "pos", "items", "list_ptr", "kv_idx", "kv_bits"))
+
+
+def test_first_calls_of_two_threads_on_one_mask_share_what_they_make(monkeypatch):
+    """calls from different host threads may overlap, also the first ones on a mask: one upload, one prepared call, and the call holds
+    every buffer its argument block names"""
+    monkeypatch.setattr(masks, "_static_lists", lambda device: 256)
+    cpu, before = torch.device("cpu"), sys.getswitchinterval()
+    sys.setswitchinterval(1e-5)
+    try:
+        for r in range(20):
+            mask, start, got = _fresh_mask(), threading.Barrier(3), [None] * 3
+
+            def run(i):
+                start.wait()
+                got[i] = attention._Layer.of(mask, 16, 8, (256, 256, 512)[i], 0, i == 2, cpu)
+
+            threads = [threading.Thread(target=run, args=(i,)) for i in range(3)]
+            for t in threads:
+                t.start()
+            for t in threads:
+                t.join()
+            assert got[0] is got[1] and all(_owns_what_it_points_to(x) for x in got), r
+            assert all(x in mask._layers.values() for x in got) and mask.for_head_dim(512) is mask.for_head_dim(512)
+    finally:
+        sys.setswitchinterval(before)
+
+
+@pytest.mark.parametrize("d, other", [(256, 512), (512, 256)])
+def test_a_prepared_call_outlives_the_mask_its_buffers_came_from(monkeypatch, d, other):
+    """a call through the mask of the other key-tile size reads this one's buffers: it keeps them when this one goes"""
+    monkeypatch.setattr(masks, "_static_lists", lambda device: 256)
+    mask = _fresh_mask()
+    wide = mask.for_head_dim(other)
+    layer = attention._Layer.of(wide, 4, 2, d, 0, False, torch.device("cpu"))
+    want = mask.for_head_dim(d).pointers(layer.head_groups, layer.n_lists)
+    assert layer.args.items == want[0] and layer.args.kv_bits == want[3] and not layer.ring
+    del mask, want
+    gc.collect()
+    assert attention._Layer.of(wide, 4, 2, d, 0, False, torch.device("cpu")) is layer and _owns_what_it_points_to(layer)
 
 
 def test_c1_in_fp32_on_the_cpu_against_the_oracle():
