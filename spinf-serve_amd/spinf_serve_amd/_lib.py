@@ -202,6 +202,13 @@ def eager(*tensors) -> bool:
     return True
 
 
+def raw_stream(device):
+    """the current stream of `device` as the library takes it; None where there are no streams"""
+    import torch
+
+    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else None
+
+
 def launch(fn, args, device, what: str) -> None:
     """fn(args, current stream of `device`) with `device` current; args: an argument block, or a tuple of plain arguments"""
     import torch

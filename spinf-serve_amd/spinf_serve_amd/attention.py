@@ -191,8 +191,11 @@ class _Layer:
         a = self.args = _lib.AttnArgs()
         a.n, a.hq, a.hkv, a.d, a.window = m.n, hq, hkv, d, m.window
         a.art, a.end, a.pos = m.art.data_ptr(), m.end.data_ptr(), m.pos.data_ptr()
-        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items, uploads = m.pointers(self.head_groups, n_lists)
-        self.owned = (m.art, m.end, m.pos, m.grp, *uploads)
+        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items, self.shared = m.pointers(self.head_groups, n_lists)
+        if m._meta is not None:
+            self.shared += (m._meta,)
+        self.owned = (m.art, m.end, m.pos, m.grp)
+        self.streams = set()   # those that have reached the shared tensors
         a.variant, a.ktile, a.n_lists = variant, m._ktile, n_lists
         if m.grp is not None:
             a.grp, a.grp_mode = m.grp.data_ptr(), m.grp_mode
@@ -207,6 +210,12 @@ class _Layer:
                 if got is None:
                     got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, device)
         return got
+
+    def reach(self, device):
+        """ahead of a launch: the current stream of `device` may read what the block points into"""
+        stream = _lib.raw_stream(device)
+        if stream not in self.streams and all([x.reach(stream) for x in self.shared]):
+            self.streams.add(stream)
 
     def bound(self, q, qs, k, ks, v, vs, out, os, scale):
         """the argument block of one call (a block of its own: calls may come from several threads); qs, ..: token and head stride"""
@@ -242,6 +251,7 @@ def _heads_first(q, k, v, mask, scale, sidx):
         return None
     variant = VARIANT if VARIANT != 2 or (sidx is None and mask.grp is None) else 0
     layer = _Layer.of(mask, hq, ks[1], d, variant, sidx is not None, dev)
+    layer.reach(dev)
     out = torch.empty((1, rows, hq, d), dtype=bf16, device=dev)
     a = layer.bound(q, (qs[2], qs[1]), k, (kst[2], kst[1]), v, (vs[2], vs[1]), out, (hq * d, d), float(d ** -0.5 if scale is None else scale))
     if sidx is not None:
@@ -269,6 +279,7 @@ def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
     if sidx is not None and mask.grp is not None:
         raise ValueError("image groups go with the stream layout (no sidx)")
     layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], variant, sidx is not None, q.device)
+    layer.reach(q.device)
     m = mask.for_head_dim(q.shape[2], ring=layer.ring)   # the plan of the kernel's key-tile size
     row_of, kv_row0 = m.rows(sidx) if sidx is not None else (None, None)
     if not _lib.eager(q, k, v, sidx):
@@ -297,6 +308,7 @@ def tree_attn_noalloc(q, k, v, mask: TreeMask, out, scale=None):
         raise ValueError("out must be a contiguous bf16 tensor of q's shape")
     _check_tensors(q, k, v, mask.n, False, (out, mask.art))
     layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], 0, False, q.device)
+    layer.reach(q.device)
     a = layer.bound(q, q.stride()[:2], k, k.stride()[:2], v, v.stride()[:2], out, out.stride()[:2], float(q.shape[-1] ** -0.5 if scale is None else scale))
     _lib.launch(_lib.load_library().spinf_tree_attn_fwd_noalloc, a, q.device, "spinf_tree_attn_fwd_noalloc")
     return out

@@ -128,10 +128,63 @@ def _staging(n: int, device):
     return torch.empty(n, dtype=torch.int32, pin_memory=device.type == "cuda")
 
 
+def _mark(device):
+    """an event behind what the current stream of `device` has been given (None under capture: a graph's nodes are ordered by the graph)"""
+    import torch
+
+    with torch.cuda.device(device):
+        if torch.cuda.is_current_stream_capturing():
+            return None
+        event = torch.cuda.Event()
+        event.record()
+        return event
+
+
+def _join(made, tensors, device) -> bool:
+    """the current stream of `device` waits for the event `made` (None: no wait) and is named to the allocator as a reader of the tensors;
+    False under capture, where neither can be done"""
+    import torch
+
+    with torch.cuda.device(device):
+        if torch.cuda.is_current_stream_capturing():
+            return False
+        stream = torch.cuda.current_stream()
+        if made is not None:
+            stream.wait_event(made)
+        for t in tensors:
+            t.record_stream(stream)
+        return True
+
+
+class _Shared:
+    """Device tensors that one stream made and calls on any stream may read.  Another stream's first call waits for what made them, and
+    tells the allocator of its stream: a buffer that goes with the last reference is then not handed out while that stream
+    still reads it.  The caller cannot do either, as the buffers are made behind its back by whichever call comes first."""
+
+    __slots__ = ("tensors", "device", "made", "streams")
+
+    def __init__(self, *tensors, wait=True):
+        self.tensors, self.device = tensors, tensors[0].device
+        on = _lib.raw_stream(self.device)
+        self.made = _mark(self.device) if wait and on is not None else None
+        self.streams = {on}
+
+    def reach(self, stream) -> bool:
+        """makes the tensors safe to read for the current stream (`stream`: its raw handle)"""
+        if stream in self.streams:
+            return True
+        if not _join(self.made, self.tensors, self.device):
+            return False
+        self.streams.add(stream)
+        return True
+
+
 class TreeMask:
     """Device-side handle: the stream's metadata, and per key-tile size a plan compiled when the first call that takes it comes (a
     forward's layers share it).  ``seq_lengths`` mirrors BlockMask.seq_lengths (spinf_serve/models/qwen35/qwen.py:615 reads it).
-    Host threads may share a mask: what a first call makes (plan, uploads, prepared calls) is made once, under a lock."""
+    Host threads and streams may share a mask: what a first call makes (plan, uploads, prepared calls) is made once, under a lock, and a
+    call on another stream waits for its copies.  (The metadata is copied at the build: as with any tensor, a stream that is to use
+    the mask waits for the one it was built on.)"""
 
     def __init__(self, plan, meta, device, grp=None, host=None, window=None, ktile=64, lock=None):
         """plan: a compiled plan, or None: compiled from host = (art, end, pos, grp or None, grp_windowed) for this window and ktile"""
@@ -147,6 +200,7 @@ class TreeMask:
         self.seq_lengths = (self.n, self.n)
         self.art, self.end, self.pos = meta
         self.device = self.art.device       # (of "cuda" the GPU that was current at the build, whatever is current at the first call)
+        self._meta = None                   # art, end, pos, grp as shared tensors, where the build copied them
         self._kv = None                     # the buffer with the device copies of the plan's kv_idx, kv_bits, and where they lie in it
         self._sched = {}
         self._layers = {}                   # prepared calls by head geometry (attention.py)
@@ -176,7 +230,8 @@ class TreeMask:
     def _entries(self):
         if self._kv is None:
             self._schedule(1, 0)
-        dev, at = self._kv
+        dev, at, shared = self._kv
+        shared.reach(_lib.raw_stream(self.device))
         return dev[at[2] : at[3]], dev[at[3] : at[4]]
 
     def for_head_dim(self, d: int, ring: bool = False) -> "TreeMask":
@@ -194,6 +249,7 @@ class TreeMask:
                 other = self._other() if isinstance(self._other, weakref.ref) else self._other
                 if other is None:
                     other = TreeMask(None, (self.art, self.end, self.pos), self.device, self.grp, self._host, self.window, ktile, self._lock)
+                    other._meta = self._meta
                     other._other = weakref.ref(self)   # (no cycle: a pass's masks go, and give their device memory back, with the last reference)
                     self._other = other
         return other
@@ -205,8 +261,10 @@ class TreeMask:
         sidx tensor it was built from (one forward: every layer passes the same tensor)."""
         import torch
 
-        if self._rows is not None and self._rows[0] is sidx:
-            return self._rows[1], self._rows[2]
+        got = self._rows   # (read once: another thread's rows may replace them)
+        if got is not None and got[0] is sidx:
+            got[3].reach(_lib.raw_stream(self.device))
+            return got[1], got[2]
         n = self.n
         row_of = torch.full((n + 63,), -1, dtype=torch.int32, device=self.device)   # padded: every key tile is 64 long
         row_of[sidx.to(self.device, torch.long)] = torch.arange(sidx.shape[0], dtype=torch.int32, device=self.device)
@@ -215,8 +273,9 @@ class TreeMask:
         run = (tiles - tiles[:, :1]) == torch.arange(kt, dtype=torch.int32, device=self.device)
         tile_row0 = torch.where((tiles[:, 0] >= 0) & run.all(1), tiles[:, 0], torch.full_like(tiles[:, 0], -1))
         kv_row0 = tile_row0[self.kv_idx.long()].contiguous()
-        self._rows = (sidx, row_of[:n].contiguous(), kv_row0)
-        return self._rows[1], self._rows[2]
+        row_of = row_of[:n].contiguous()
+        self._rows = (sidx, row_of, kv_row0, _Shared(row_of, kv_row0))
+        return row_of, kv_row0
 
     def _upload(self, head_groups: int, n_lists: int):
         """one staging buffer, one copy: items | list_ptr and, with the plan's first schedule, kv_idx | kv_bits.  (A copy per array, each
@@ -231,9 +290,10 @@ class TreeMask:
             plan.export(p + 4 * at[4], p + 4 * at[2], p + 4 * at[3], p + 4 * (at[4] + nq + 1))
             buf = buf[: at[4]]
         dev = buf.to(self.device, non_blocking=True)
+        shared = _Shared(dev)
         if first:
-            self._kv = dev, at
-        got = self._sched[(head_groups, n_lists)] = dev, at, plan.n_qtiles * head_groups
+            self._kv = dev, at, shared
+        got = self._sched[(head_groups, n_lists)] = dev, at, plan.n_qtiles * head_groups, shared
         return got
 
     def _schedule(self, head_groups: int, n_lists: int):
@@ -246,16 +306,17 @@ class TreeMask:
     def schedule(self, head_groups: int, n_lists: int = 0):
         """device copy of the work lists for this many head groups (built on first use, then kept); n_lists > 0: the static
         schedule for that many workgroups"""
-        dev, at, n_items = self._schedule(head_groups, n_lists)
+        dev, at, n_items, shared = self._schedule(head_groups, n_lists)
+        shared.reach(_lib.raw_stream(self.device))
         return dev[: at[1]].view(-1, 4), dev[at[1] : at[2]], n_items
 
     def pointers(self, head_groups: int, n_lists: int):
-        """-> device addresses of items, list_ptr, kv_idx, kv_bits, the number of items, and the tensors the addresses lie in (whoever
-        keeps an address keeps its tensor)"""
-        dev, at, n_items = self._schedule(head_groups, n_lists)
-        kv, kv_at = self._kv
+        """-> device addresses of items, list_ptr, kv_idx, kv_bits, the number of items, and the shared tensors the addresses lie in
+        (whoever keeps an address keeps its tensor, and a stream that reads it reaches it)"""
+        dev, at, n_items, shared = self._schedule(head_groups, n_lists)
+        kv, kv_at, kv_shared = self._kv
         items, entries = dev.data_ptr(), kv.data_ptr()
-        return items, items + 4 * at[1], entries + 4 * kv_at[2], entries + 4 * kv_at[3], n_items, (dev, kv)
+        return items, items + 4 * at[1], entries + 4 * kv_at[2], entries + 4 * kv_at[3], n_items, (shared, kv_shared)
 
     @classmethod
     def build(cls, art, end, pos, window=None, device="cuda", meta=None, grp=None, grp_windowed=False, grp_dev=None):
@@ -267,6 +328,7 @@ class TreeMask:
         host = _host_arrays(art, end, pos, grp)
         n = len(host[0])
         given = [i for i in range(4) if host[i] is not None and not (grp_dev is not None if i == 3 else meta is not None)]
+        shared = None
         if given:
             buf = _staging(len(given) * n, device).view(len(given), n)
             rows = buf.numpy()
@@ -274,11 +336,14 @@ class TreeMask:
                 rows[r] = host[i]
             host = tuple(rows[given.index(i)] if i in given else h for i, h in enumerate(host))   # (the caller may reuse its arrays)
             dev = buf.to(device, non_blocking=True)
+            shared = _Shared(dev, wait=False)
             if meta is None:
                 meta = tuple(dev[:3])
             if 3 in given:
                 grp_dev = dev[-1]
-        return cls(None, meta, device, grp_dev if grp is not None else None, (*host, grp_windowed), window)
+        mask = cls(None, meta, device, grp_dev if grp is not None else None, (*host, grp_windowed), window)
+        mask._meta = shared
+        return mask
 
 
 def block_masks(batch, sliding_window=None, device="cuda", grp=None, bidir_all=True):
@@ -294,6 +359,7 @@ def block_masks(batch, sliding_window=None, device="cuda", grp=None, bidir_all=T
     meta = (full.art, full.end, full.pos)
     if grp is None or bidir_all:
         slid = TreeMask(None, meta, full.device, full.grp, full._host, sliding_window)
+        slid._meta = full._meta
     else:
         slid = TreeMask.build(*full._host[:3], sliding_window, device, meta=meta, grp=grp, grp_windowed=True)
     return {"full_attention": full, "sliding_attention": slid}

@@ -78,7 +78,8 @@ def _fresh_mask(seed=0):
 
 
 def _owns_what_it_points_to(layer):
-    spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for t in layer.owned if t is not None]
+    owned = [t for t in layer.owned if t is not None] + [t for x in layer.shared for t in x.tensors]
+    spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for t in owned]
     return all(any(a <= getattr(layer.args, f) < a + n for a, n in spans) for f in ("art", "end", "pos", "items", "list_ptr", "kv_idx", "kv_bits"))
 
 
@@ -118,6 +119,51 @@ def test_a_prepared_call_outlives_the_mask_its_buffers_came_from(monkeypatch):
     del mask, want
     gc.collect()
     assert attention._Layer.of(wide, 4, 2, 256, 0, False, torch.device("cpu")) is layer and _owns_what_it_points_to(layer)
+
+
+def test_a_call_on_another_stream_waits_for_what_the_first_one_uploaded(monkeypatch):
+    """a mask's schedules, entries and row maps are uploaded by whichever call comes first, on its stream: every other stream waits for
+    the copy of each buffer it reads, once, and the allocator hears of it; the stream that copied does not wait"""
+    now, log, marks = ["a"], [], []
+
+    def mark(device):
+        marks.append((len(marks), now[0]))
+        return marks[-1]
+
+    def join(made, tensors, device):
+        log.append((now[0], made, tuple(t.data_ptr() for t in tensors)))
+        return now[0] != "capture"
+
+    monkeypatch.setattr(masks, "_static_lists", lambda device: 256)
+    monkeypatch.setattr(masks._lib, "raw_stream", lambda device: now[0])
+    monkeypatch.setattr(masks, "_mark", mark)
+    monkeypatch.setattr(masks, "_join", join)
+    cpu, mask = torch.device("cpu"), _fresh_mask()   # built on "a": the metadata is there, and no event for it
+
+    def call(stream, hq, sidx=None):
+        now[0] = stream
+        del log[:]
+        layer = attention._Layer.of(mask, hq, 2, 256, 0, sidx is not None, cpu)
+        layer.reach(cpu)
+        if sidx is not None:
+            mask.rows(sidx)
+        return layer, [(s, made) for s, made, _ in log]
+
+    assert not marks
+    layer, seen = call("b", 4)                     # uploads entries and its schedule on b
+    assert marks == [(0, "b")] and seen == [("b", None)] and log[0][2][0] == mask.art.data_ptr()   # (the metadata: named to the allocator only)
+    assert call("b", 4)[1] == []
+    _, seen = call("c", 8)                         # another geometry on c: its schedule on c, the entries are b's
+    assert marks[1:] == [(1, "c")] and seen == [("c", (0, "b")), ("c", None)]
+    assert call("c", 8)[1] == [] and call("c", 4)[1] == []     # (what b made has been waited for)
+    assert call("b", 8)[1] == [("b", (1, "c"))]
+    assert call("a", 4)[1] == [("a", (0, "b"))]
+    for _ in range(2):                             # nothing can be waited for under capture, and it is not taken for done
+        assert [s for s, _ in call("capture", 4)[1]] == ["capture"] * 3 and "capture" not in layer.streams
+    sidx = torch.from_numpy(np.flatnonzero(mask.art.numpy() >= 0))
+    _, seen = call("b", 4, sidx)
+    assert marks[2:] == [(2, "b")] and seen == []
+    assert call("d", 4, sidx)[1] == [("d", (0, "b")), ("d", None), ("d", (2, "b"))]
 
 
 def test_c1_in_fp32_on_the_cpu_against_the_oracle():
@@ -253,3 +299,33 @@ def test_every_c3_pass(dev):
             want = oattn.tree_attention(*(_np(x) for x in sub), b.art[s0:e0], b.end[s0:e0] - s0, b.pos[s0:e0], window=window, scale=cfg.scale)
             real = b.art[s0:e0] >= 0
             assert np.abs(_np(out[s0:e0])[real] - want[real]).max() <= 2e-2
+
+
+@pytest.mark.gpu
+def test_layers_of_one_mask_on_two_streams(dev):
+    """the first call's stream is busy, so its uploads are late; a call on another stream gives the bits of one that has waited for
+    everything, and what it reads is not handed out again when the mask goes while it is still to run"""
+    cfg = synth.attention_config("C2", contents=2)
+    b = cfg.batches[0]
+    q, k, v = synth.qkv(cfg, b, seed=5, device=dev)
+    few = [t[:, :n].contiguous() for t, n in ((q, 8), (k, 4), (v, 4))]
+    ref = sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
+    want = [sa.tree_attn(q, k, v, ref, cfg.scale), sa.tree_attn(*few, ref, cfg.scale)]
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    mask = sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(streams[0]):
+        torch.cuda._sleep(20_000_000)
+        one = sa.tree_attn(q, k, v, mask, cfg.scale)
+    with torch.cuda.stream(streams[1]):
+        two = [sa.tree_attn(*few, mask, cfg.scale), sa.tree_attn(q, k, v, mask, cfg.scale)]
+        torch.cuda._sleep(20_000_000)
+        two.append(sa.tree_attn(*few, mask, cfg.scale))
+    buffers = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for x in (*mask._sched.values(), mask._kv) for t in x[-1].tensors}
+    streams[0].synchronize()
+    del mask
+    with torch.cuda.stream(streams[0]):   # (the stream whose pool they came from)
+        fresh = [torch.empty(n, dtype=torch.uint8, device=dev) for n in buffers.values() for _ in range(4)]
+    assert not streams[1].query() and not any(t.data_ptr() in buffers for t in fresh)
+    torch.cuda.synchronize()
+    assert torch.equal(one, want[0]) and torch.equal(two[0], want[1]) and torch.equal(two[1], want[0]) and torch.equal(two[2], want[1])
