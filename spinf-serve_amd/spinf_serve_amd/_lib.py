@@ -202,6 +202,13 @@ def eager(*tensors) -> bool:
     return True
 
 
+def same_device(device, *tensors) -> None:
+    """raises unless every tensor lies on `device`: a kernel that is handed an address of another memory faults"""
+    for t in tensors:
+        if t is not None and t.device != device:
+            raise ValueError(f"all tensors of the call must be on {device}, one is on {t.device}")
+
+
 def raw_stream(device):
     """the current stream of `device` as the library takes it; None where there are no streams"""
     import torch

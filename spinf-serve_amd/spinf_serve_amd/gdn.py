@@ -58,6 +58,7 @@ def _launch(mode, q, k, v, g, beta, scale, cu, n, h0, h0_idx, ht, ht_idx, idx, o
     for t, name in ((h0, "h0"), (ht, "ht")):
         if t is not None and (t.dtype != torch.float32 or not t.is_contiguous() or t.shape[1:] != (HV, K, V)):
             raise ValueError(f"{name} must be contiguous fp32 [*, {HV}, {K}, {V}]")
+    _lib.same_device(q.device, k, v, g, beta, o, cu, idx, h0, h0_idx, ht, ht_idx)
     a = _lib.GdnArgs()
     a.q, a.k, a.v, a.g, a.beta, a.o = q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), o.data_ptr()
     a.q_tok, a.v_tok, a.g_tok, a.o_tok = q.stride(1), v.stride(1), g.stride(1), o.stride(1)
@@ -72,15 +73,16 @@ def _launch(mode, q, k, v, g, beta, scale, cu, n, h0, h0_idx, ht, ht_idx, idx, o
     return o
 
 
-def level_args(q, k, v, g, beta, o, scale):
+def level_args(q, k, v, g, beta, o, scale, plan_data):
     """the argument block that the launches over one layer's tensors share (q, k [T, H, K], v, o [T, HV, V], g, beta [T, HV]), or None for
-    tensors that are not plain or not as the kernels take them (the call by call path names what is wrong)"""
+    tensors that are not plain or not as the kernels take them, or a plan (plan_data) on another device (the call by call path names
+    what is wrong)"""
     bf16 = torch.bfloat16
     if not (_lib.eager(q, k, v, g, beta) and q.is_cuda and q.dtype is bf16 and k.dtype is bf16 and v.dtype is bf16 and g.dtype is torch.float32 and beta.dtype is bf16):
         return None
     (T, H, K), (_, HV, V), qs, vs, gs = k.shape, v.shape, q.stride(), v.stride(), g.stride()
     if not (q.shape == k.shape and v.shape[0] == T and g.shape == beta.shape == (T, HV) and k.stride() == qs and qs[1:] == (K, 1) and vs[1:] == (V, 1)
-            and o.stride()[1:] == (V, 1) and gs[1] == 1 and beta.stride() == gs and all(t.device == q.device for t in (k, v, g, beta))):
+            and o.stride()[1:] == (V, 1) and gs[1] == 1 and beta.stride() == gs and all(t.device == q.device for t in (k, v, g, beta, o, plan_data))):
         return None
     a = _lib.GdnArgs()
     a.q, a.k, a.v, a.g, a.beta, a.o = q.data_ptr(), k.data_ptr(), v.data_ptr(), g.data_ptr(), beta.data_ptr(), o.data_ptr()

@@ -194,7 +194,7 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
     g32 = g if g.dtype == torch.float32 else g.float()
     b16 = beta if beta.dtype == torch.bfloat16 else beta.to(torch.bfloat16)
     indexed = plan.path == "indexed"
-    args = gdn.level_args(q, k, v, g32, b16, o, scale) if indexed and plan.launches is not None else None
+    args = gdn.level_args(q, k, v, g32, b16, o, scale, plan.data) if indexed and plan.launches is not None else None
     # a forest's nodes leave no states (and its kernel is built for 128 value dims): a caller that asks for states gets every level's
     launches = plan.launches if wanted or plan.program is None or v.shape[-1] != 128 else plan.program
     base = plan.data.data_ptr() if args is not None else 0

@@ -298,6 +298,20 @@ def test_decoder_steps_rerun_the_recurrence_from_the_prefix_state(dev):
     assert torch.isnan(o_buf[0, untouched].float()).all()                         # rows of no slot are never written
 
 
+@pytest.mark.parametrize("path", ["indexed", "levels"])
+def test_a_plan_on_another_device_is_refused_before_any_launch(dev, path):
+    """compact rows without pads, so nothing stumbles over the plan ahead of the kernels: its rows and slots are host addresses"""
+    tree = sa.TokenTree([1] * 100, [[2] * 5, [2] * 9, [2] * 70], [-1, -1, 0])
+    b = sa.pack_stream([tree])
+    plan = sa.tree_plan(b.prev, b.art >= 0, "cpu", path=path, rows=b.n_tokens)
+    assert plan.pad_rows.numel() == 0 and plan.conv.device.type == "cpu"
+    t = b.n_tokens
+    q, v = torch.zeros(t, 2, 128, dtype=torch.bfloat16, device=dev), torch.zeros(t, 4, 128, dtype=torch.bfloat16, device=dev)
+    g = torch.zeros(t, 4, device=dev)
+    with pytest.raises((ValueError, RuntimeError), match="device"):
+        sa.gdn_tree(q, q, v, g, g.bfloat16(), plan)
+
+
 def test_zz_report_worst_errors():
     """(runs last in this file) the largest errors the tests above measured, for the record"""
     print(f"gdn kernels against the float64 recurrence: worst max abs error outputs {WORST['out']:.3e} (tolerance {TOL:.0e}), "
