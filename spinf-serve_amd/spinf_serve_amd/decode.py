@@ -145,6 +145,7 @@ def _xdecode_args(query, kp, vp, pos_p, kt, vt, pos_t, own_t, gk, gv, qpos, step
         raise ValueError("pos_p [G, Lp], pos_t and own_t [G, Tt] expected")
     if qpos.dtype != torch.int64 or tuple(qpos.shape) != (G, Q) or not qpos.is_contiguous() or step_t.dtype != torch.int64:
         raise ValueError("qpos [G, Q] and step_t [1] must be int64")
+    _lib.same_device(query.device, kp, vp, pos_p, kt, vt, pos_t, own_t, gk, gv, qpos, step_t, len_p, len_t)
     a = _lib.XdecArgs()
     a.kp, a.vp, a.pos_p = kp.data_ptr(), vp.data_ptr(), _i32(pos_p, "pos_p").data_ptr()
     a.kt, a.vt, a.pos_t, a.own_t = kt.data_ptr(), vt.data_ptr(), _i32(pos_t, "pos_t").data_ptr(), _i32(own_t, "own_t").data_ptr()

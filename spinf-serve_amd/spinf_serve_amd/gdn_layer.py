@@ -29,6 +29,9 @@ def _prologue(y: torch.Tensor, conv: torch.Tensor, conv_w: torch.Tensor, a_log: 
         raise ValueError("conv must be int64 [T, 4]")
     if conv_w.shape != (2 * kd + vd, 4):
         raise ValueError(f"conv_w must be [{2 * kd + vd}, 4]")
+    if a_log.numel() < hv or dt_bias.numel() < hv:
+        raise ValueError(f"A_log and dt_bias must hold a value for each of the {hv} value heads")
+    _lib.same_device(y.device, conv, conv_w, a_log, dt_bias)
     conv = conv.contiguous()
     conv_w = conv_w.float().contiguous()
     a_log = a_log.float().contiguous()
@@ -73,6 +76,9 @@ def _gate(o: torch.Tensor, z: torch.Tensor, norm_w: torch.Tensor, eps: float) ->
     T, hv, dv = o.shape
     if z.shape != (T, hv * dv) or z.stride(1) != 1 or o.stride(2) != 1 or o.stride(1) != dv:
         raise ValueError("z must be [T, hv dv] with contiguous rows, o dense inside a row")
+    if norm_w.numel() < dv:
+        raise ValueError(f"norm_w must hold {dv} values")
+    _lib.same_device(o.device, z, norm_w)
     norm_w = norm_w.to(torch.bfloat16).contiguous()
     out = torch.empty((T, hv * dv), dtype=torch.bfloat16, device=o.device)
     a = _lib.GdnGateArgs()

@@ -29,6 +29,7 @@ def _lm(logits: torch.Tensor, cols: Optional[torch.Tensor], softcap: float) -> t
     if cols is not None:
         if cols.dtype != torch.int64 or cols.dim() != 1 or cols.numel() == 0:
             raise ValueError("cols must be a non-empty int64 vector")
+        _lib.same_device(logits.device, cols)
         cols = cols.contiguous()
     out = torch.empty((rows, vocab if cols is None else cols.numel()), dtype=torch.float32, device=logits.device)
     a = _lib.LmArgs()
@@ -63,6 +64,7 @@ def _head(h: torch.Tensor, sel: Optional[torch.Tensor], w: torch.Tensor, cols: O
         raise ValueError("h [*, hidden] and W [vocab, hidden] must be bf16 matrices with contiguous rows")
     if h.shape[1] != w.shape[1]:
         raise ValueError(f"hidden sizes differ: h {h.shape[1]}, W {w.shape[1]}")
+    _lib.same_device(h.device, w, sel, cols)
     if sel is not None:
         if sel.dtype != torch.int64 or sel.dim() != 1:
             raise ValueError("sel must be an int64 vector")

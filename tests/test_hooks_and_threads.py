@@ -302,6 +302,40 @@ def test_every_c3_pass(dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("call", ["prologue", "gate", "logprobs", "head", "xdecode"])
+def test_tensors_of_another_device_are_refused_before_any_launch(dev, call):
+    """each tensor of a call in turn on the host: its address would go to the kernel"""
+    bf = dict(dtype=torch.bfloat16, device=dev)
+    if call == "prologue":
+        plan = sa.tree_plan(np.arange(-1, 39), np.ones(40, bool), dev)
+        args = [torch.zeros(40, 2 * 256 + 2 * 512 + 8, **bf), plan.conv, torch.zeros(1024, 4, device=dev), torch.zeros(4, device=dev), torch.zeros(4, device=dev)]
+        run = lambda *t: sa.gdn_prologue(*t, 2, 4, 128, 128)  # noqa: E731
+    elif call == "gate":
+        args = [torch.zeros(40, 4, 128, **bf), torch.zeros(40, 512, **bf), torch.zeros(128, **bf)]
+        run = lambda *t: sa.gdn_gate(*t, 1e-6)  # noqa: E731
+    elif call == "logprobs":
+        args = [torch.zeros(3, 64, device=dev), torch.tensor([1, 5], device=dev)]
+        run = sa.lm_logprobs
+    elif call == "head":
+        args = [torch.zeros(9, 64, **bf), torch.tensor([0, 8], device=dev), torch.zeros(128, 64, **bf), torch.tensor([1, 5], device=dev)]
+        run = sa.lm_head_logprobs
+    else:
+        q, c = synth.xdecode_case(G=1, H=2, h=1, d=64, slots=1, beam=2, S=2, prefix=(4, 4), template=(2, 2), device=dev)
+        for name in ("kp", "vp", "pos_p", "kt", "vt", "gk", "gv", "pos_t", "own_t", "qpos", "step_t"):
+            whole = getattr(c, name)
+            setattr(c, name, {0: whole[0].cpu()} if isinstance(whole, dict) else whole.cpu())
+            with pytest.raises((ValueError, RuntimeError), match="device|must be on"):
+                sa.xdecode_attn(q, c, 0)
+            setattr(c, name, whole)
+        sa.xdecode_attn(q, c, 0)
+        return
+    for i in range(len(args)):
+        with pytest.raises((ValueError, RuntimeError), match="device|must be on"):
+            run(*args[:i], args[i].cpu(), *args[i + 1 :])
+    run(*args)
+
+
+@pytest.mark.gpu
 def test_layers_of_one_mask_on_two_streams(dev):
     """the first call's stream is busy, so its uploads are late; a call on another stream gives the bits of one that has waited for
     everything, and what it reads is not handed out again when the mask goes while it is still to run"""

@@ -116,6 +116,17 @@ def test_ops_have_no_cpu_path(lib):
         sa.tree_attn(q, k, k, mask, cfg.scale)
 
 
+def test_same_device_names_the_stray_tensor():
+    import torch
+
+    from spinf_serve_amd import _lib
+
+    here, there = torch.zeros(2), torch.zeros(2, device="meta")
+    _lib.same_device(here.device, here, None, here)
+    with pytest.raises(ValueError, match="must be on cpu, one is on meta"):
+        _lib.same_device(here.device, here, there)
+
+
 @pytest.mark.parametrize("entry", ["tree_attn", "tree_attn_noalloc"])
 def test_both_attention_entry_points_check_their_tensors_before_any_launch(lib, entry):
     """one shared check in front of spinf_tree_attn_fwd and spinf_tree_attn_fwd_noalloc: a wrong dtype, shape, head grouping,
