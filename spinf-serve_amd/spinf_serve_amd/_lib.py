@@ -5,6 +5,8 @@ from __future__ import annotations
 import ctypes as C
 import os
 
+import torch
+
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
 
@@ -176,26 +178,16 @@ def check(code: int, what: str) -> None:
         raise (ValueError if code == -1 else RuntimeError)(f"{what}: {msg} (code {code})")
 
 
-_KINDS = None
-_RAW = None
-
-
-def _bind_torch():
-    global _KINDS, _RAW
-    import torch
-
-    _KINDS = (torch.Tensor, torch.nn.Parameter)
-    _RAW = (torch.is_grad_enabled, torch._C._len_torch_dispatch_stack, torch.compiler.is_compiling)
+_KINDS = (torch.Tensor, torch.nn.Parameter)
+_compiling, _grad_enabled, _dispatch_modes = torch.compiler.is_compiling, torch.is_grad_enabled, torch._C._len_torch_dispatch_stack
 
 
 def eager(*tensors) -> bool:
     """May this call go straight to the library?  Yes for plain tensors outside any tracing, dispatch mode or autograd recording; anything
     else takes the registered torch.library operator, which costs 15 - 25 us of host time per call more."""
-    if _RAW is None:
-        _bind_torch()
-    grad = _RAW[0]()
-    if _RAW[1]() or _RAW[2]():
+    if _compiling() or _dispatch_modes():   # (the compiler folds the first to True and must not meet the others)
         return False
+    grad = _grad_enabled()
     for t in tensors:
         if t is not None and (type(t) not in _KINDS or (grad and t.requires_grad)):
             return False
@@ -211,15 +203,11 @@ def same_device(device, *tensors) -> None:
 
 def raw_stream(device):
     """the current stream of `device` as the library takes it; None where there are no streams"""
-    import torch
-
     return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else None
 
 
 def launch(fn, args, device, what: str) -> None:
     """fn(args, current stream of `device`) with `device` current; args: an argument block, or a tuple of plain arguments"""
-    import torch
-
     args = args if type(args) is tuple else (C.byref(args),)
     if torch._C._cuda_getDevice() == device.index:
         rc = fn(*args, torch._C._cuda_getCurrentRawStream(device.index))

@@ -42,6 +42,39 @@ def test_ops_are_registered_with_torch_library():
                          torch.zeros(1, 4, 2), torch.zeros(1, 4, 2, dtype=torch.bfloat16), 1.0, torch.tensor([0, 4]), 1)
 
 
+def _wrapped_calls():
+    """the calls a compiled or traced program may hold: (name, function of plain tensors, tensors)"""
+    bf = torch.bfloat16
+    plan = sa.tree_plan(np.arange(-1, 7), np.ones(8, bool), "cpu")
+    q, caches = synth.xdecode_case(G=1, H=2, h=1, d=64, slots=1, beam=2, S=2, prefix=(4, 4), template=(2, 2), device="cpu")
+    return [
+        ("lm_logprobs", lambda x: sa.lm_logprobs(x, None, 30.0), (torch.zeros(3, 64),)),
+        ("lm_head_logprobs", lambda h, w: sa.lm_head_logprobs(h, None, w, None, 30.0), (torch.zeros(3, 64, dtype=bf), torch.zeros(16, 64, dtype=bf))),
+        ("gdn_prologue", lambda y, c, w, a, b: sa.gdn_prologue(y, c, w, a, b, 2, 4, 128, 128), (torch.zeros(8, 1544, dtype=bf), plan.conv, torch.zeros(1024, 4), torch.zeros(4), torch.zeros(4))),
+        ("gdn_gate", lambda o, z, n: sa.gdn_gate(o, z, n, 1e-6), (torch.zeros(8, 4, 128, dtype=bf), torch.zeros(8, 512, dtype=bf), torch.ones(128, dtype=bf))),
+        ("xdecode_attn", lambda x: sa.xdecode_attn(x, caches, 0, nsplit=1), (q,)),
+    ]
+
+
+@pytest.mark.parametrize("which", range(5))
+def test_a_compiled_program_holds_the_registered_operator(which):
+    """torch.compile(fullgraph=True) over the public calls: one opaque node each (the graph is looked at, not run: there is no CPU path)"""
+    name, call, args = _wrapped_calls()[which]
+    seen = []
+
+    def backend(gm, example):
+        seen.extend(str(n.target) for n in gm.graph.nodes if n.op == "call_function")
+        return lambda *a: (torch.zeros(()),) * 8
+
+    torch._dynamo.reset()
+    compiled = torch.compile(call, fullgraph=True, backend=backend)
+    try:
+        compiled(*args)
+    finally:
+        torch._dynamo.reset()
+    assert any(f"spinf.{name}" in t for t in seen), seen
+
+
 def test_plan_compilers_from_two_threads():
     """tile plans, their schedules and recurrent-layer plans built at the same time on different streams equal the ones built
     one after the other"""
