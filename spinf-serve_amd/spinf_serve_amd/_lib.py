@@ -6,6 +6,8 @@ import ctypes as C
 import os
 
 import torch
+from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _LIB = None
@@ -179,16 +181,28 @@ def check(code: int, what: str) -> None:
 
 
 _KINDS = (torch.Tensor, torch.nn.Parameter)
-_compiling, _grad_enabled, _dispatch_modes = torch.compiler.is_compiling, torch.is_grad_enabled, torch._C._len_torch_dispatch_stack
+_compiling, _grad_enabled = torch.compiler.is_compiling, torch.is_grad_enabled
+_dispatch_modes, _function_modes, _function_mode = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._get_function_stack_at
+_tracer, _functorch_level = torch._C._get_tracing_state, torch._C._functorch.maybe_current_level
 
 
-def eager(*tensors) -> bool:
-    """May this call go straight to the library?  Yes for plain tensors outside any tracing, dispatch mode or autograd recording; anything
-    else takes the registered torch.library operator, which costs 15 - 25 us of host time per call more."""
-    if _compiling() or _dispatch_modes():   # (the compiler folds the first to True and must not meet the others)
+def watched() -> bool:
+    """Is something looking at the operators that run: a compiler, a tracer, a function transform (vmap, jvp, ..), forward-mode autograd,
+    a dispatch or function mode?  A default device is a function mode too, one that looks at factory calls only."""
+    if _compiling():   # (first: the compiler folds it to True and cannot trace the others)
+        return True
+    return bool(_dispatch_modes() or _tracer() is not None or _functorch_level() is not None or forward_ad._current_level >= 0
+                or (n := _function_modes()) and any(type(_function_mode(i)) is not DeviceContext for i in range(n)))
+
+
+def eager(first, *tensors) -> bool:
+    """May this call go straight to the library?  Yes for plain tensors on a GPU (of ``first``; a launch compares the others with it) that
+    nothing watches and autograd does not record; anything else takes the registered torch.library operator, which costs 15 - 25 us
+    of host time per call more."""
+    if watched() or not first.is_cuda:
         return False
     grad = _grad_enabled()
-    for t in tensors:
+    for t in (first, *tensors):
         if t is not None and (type(t) not in _KINDS or (grad and t.requires_grad)):
             return False
     return True

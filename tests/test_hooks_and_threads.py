@@ -75,6 +75,58 @@ def test_a_compiled_program_holds_the_registered_operator(which):
     assert any(f"spinf.{name}" in t for t in seen), seen
 
 
+def test_what_watches_operators_is_seen():
+    """vmap, jvp, forward-mode duals, jit.trace, function and dispatch modes get the registered operator, a default device does not"""
+    import torch.autograd.forward_ad as fwd
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from spinf_serve_amd import _lib
+
+    class Functions(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatches(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    x, seen = torch.ones(3), {}
+
+    def look(name, y):
+        seen[name] = _lib.watched()
+        return y * 2
+
+    look("plain", x)
+    with torch.device("cpu"):
+        look("device", x)
+    with torch.inference_mode():
+        look("inference", x)
+    assert seen == {"plain": False, "device": False, "inference": False}
+    torch.vmap(lambda y: look("vmap", y))(x)
+    torch.func.jvp(lambda y: look("jvp", y), (x,), (x,))
+    torch.func.grad(lambda y: look("grad", y).sum())(x)
+    torch.func.functionalize(lambda y: look("functionalize", y))(x)
+    torch.jit.trace(lambda y: look("trace", y), (x,), check_trace=False)
+    with fwd.dual_level():
+        look("dual", fwd.make_dual(x, x))
+    for name, mode in (("functions", Functions()), ("dispatches", Dispatches())):
+        with mode:
+            look(name, x)
+        with torch.device("cpu"), mode:
+            look(name + " on a default device", x)
+    assert all(seen[n] for n in seen if n not in ("plain", "device", "inference")) and len(seen) == 13, seen
+    assert not _lib.watched()
+
+
+def test_shapes_without_memory_go_through_the_operators():
+    """meta tensors have no memory to read: the operators give the outputs' shapes, types and device"""
+    for name, call, args in _wrapped_calls()[:4]:
+        out = call(*(a.to("meta") for a in args))
+        out = out if isinstance(out, tuple) else (out,)
+        assert all(o.device.type == "meta" and o.shape[0] == len(args[0]) for o in out), name
+
+
 def test_plan_compilers_from_two_threads():
     """tile plans, their schedules and recurrent-layer plans built at the same time on different streams equal the ones built
     one after the other"""
@@ -396,3 +448,14 @@ def test_layers_of_one_mask_on_two_streams(dev):
     assert not streams[1].query() and not any(t.data_ptr() in buffers for t in fresh)
     torch.cuda.synchronize()
     assert torch.equal(one, want[0]) and torch.equal(two[0], want[1]) and torch.equal(two[1], want[0]) and torch.equal(two[2], want[1])
+
+
+@pytest.mark.gpu
+def test_a_traced_program_holds_the_operator(dev):
+    """torch.jit.trace records the operator: the trace gives the next input's result, not the first one's"""
+    gen = torch.Generator(device=dev).manual_seed(0)
+    a, b = (torch.randn(5, 128, generator=gen, device=dev) for _ in range(2))
+    traced = torch.jit.trace(lambda x: sa.lm_logprobs(x, None, 30.0), (a,), check_trace=False)
+    assert "spinf::lm_logprobs" in str(traced.graph)
+    for x in (a, b):
+        assert torch.equal(traced(x), sa.lm_logprobs(x, None, 30.0))
