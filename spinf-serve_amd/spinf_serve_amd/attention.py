@@ -229,6 +229,21 @@ class _Layer:
         return a
 
 
+def _variant(variant, mask, compact) -> int:
+    """the kernel variant of a call: the two-heads-per-wave kernels take neither compact rows nor image groups"""
+    return 0 if variant == 2 and (compact or mask.grp is not None) else variant
+
+
+def prepare_calls(mask, heads, sidx) -> None:
+    """TreeMask.prepare: the prepared calls of these head geometries, and the row map of sidx"""
+    if sidx is not None and mask.grp is not None:
+        raise ValueError("image groups go with the stream layout (no sidx)")
+    for hq, hkv, d in heads:
+        layer = _Layer.of(mask, hq, hkv, d, _variant(VARIANT, mask, sidx is not None), sidx is not None, mask.device)
+        if sidx is not None:
+            mask.for_head_dim(d, ring=layer.ring).rows(sidx)
+
+
 def _heads_first(q, k, v, mask, scale, sidx):
     """tree_attn for the model layers' layout: q [1, hq, rows, d], k / v [1, hkv, rows, d] -> [1, rows, hq, d], or None for anything that is not
     plain (then the general path takes the call, and names what is wrong with it).  The views into token-major layout and the general
@@ -249,8 +264,7 @@ def _heads_first(q, k, v, mask, scale, sidx):
             return None
     elif mask.grp is not None or sidx.shape[0] > rows or sidx.device != dev:
         return None
-    variant = VARIANT if VARIANT != 2 or (sidx is None and mask.grp is None) else 0
-    layer = _Layer.of(mask, hq, ks[1], d, variant, sidx is not None, dev)
+    layer = _Layer.of(mask, hq, ks[1], d, _variant(VARIANT, mask, sidx is not None), sidx is not None, dev)
     layer.reach(dev)
     out = torch.empty((1, rows, hq, d), dtype=bf16, device=dev)
     a = layer.bound(q, (qs[2], qs[1]), k, (kst[2], kst[1]), v, (vs[2], vs[1]), out, (hq * d, d), float(d ** -0.5 if scale is None else scale))
@@ -273,9 +287,7 @@ def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
     if sidx is not None and sidx.shape[0] > q.shape[0]:
         raise ValueError(f"sidx names {sidx.shape[0]} rows, q has {q.shape[0]}")
     scale = float(q.shape[-1] ** -0.5 if scale is None else scale)
-    variant = int(VARIANT if variant is None else variant)
-    if (sidx is not None or mask.grp is not None) and variant == 2:
-        variant = 0   # the two-heads-per-wave kernels take neither compact rows nor image groups
+    variant = _variant(int(VARIANT if variant is None else variant), mask, sidx is not None)
     if sidx is not None and mask.grp is not None:
         raise ValueError("image groups go with the stream layout (no sidx)")
     layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], variant, sidx is not None, q.device)

@@ -4,7 +4,8 @@
 A TreeMask holds the stream's art / end / pos on the device and, instead of FlexAttention's nb x nb block tables
 (spinf_serve/packer.py:426-491), a compact per-query-tile list of visible key tiles compiled on the host by the
 library's tile-plan compiler: for the window and the key-tile size the layers ask for, at the first layer that asks (a pass
-whose global layers have 512-dim heads never compiles the 64-key plan of its global mask).  No dense mask is built anywhere.
+whose global layers have 512-dim heads never compiles the 64-key plan of its global mask) or ahead of it (TreeMask.prepare).
+No dense mask is built anywhere.
 """
 
 from __future__ import annotations
@@ -254,6 +255,16 @@ class TreeMask:
                     self._other = other
         return other
 
+    def prepare(self, *heads, sidx=None) -> "TreeMask":
+        """makes now, on the current stream, what the first calls of layers with these heads would make: heads = (query heads, key / value
+        heads, head dim) per kind of layer, sidx as the calls will pass it.  For a program that builds its masks on a thread or a
+        stream of its own: plans are compiled and uploaded there, what the compiler refuses is raised there, and a call on any
+        stream waits for the uploads.  Without it the first call of a kind does it, on its thread and its stream."""
+        from . import attention
+
+        attention.prepare_calls(self, heads, sidx)
+        return self
+
     def rows(self, sidx):
         """compact rows (spinf_serve/models/qwen35/qwen.py:613-622): sidx [R] = stream position of each real row (a device
         tensor) -> (row_of [n], kv_row0 [entries]) int32 device tensors for the kernel: the row of each stream position (-1:
@@ -325,6 +336,8 @@ class TreeMask:
         import torch
 
         device = torch.device(device)
+        if len(art) > 1 << 30:   # (what the plan compiler, which comes later, would refuse)
+            raise ValueError(f"a stream of {len(art)} tokens is too long")
         host = _host_arrays(art, end, pos, grp)
         n = len(host[0])
         given = [i for i in range(4) if host[i] is not None and not (grp_dev is not None if i == 3 else meta is not None)]

@@ -206,6 +206,39 @@ def test_a_prepared_call_outlives_the_mask_its_buffers_came_from(monkeypatch):
     assert attention._Layer.of(wide, 4, 2, 256, 0, False, torch.device("cpu")) is layer and _owns_what_it_points_to(layer)
 
 
+@pytest.mark.parametrize("compact", [False, True])
+def test_a_prepared_mask_leaves_nothing_to_its_first_calls(monkeypatch, compact):
+    """TreeMask.prepare compiles, schedules and uploads for the layers it is told of; a layer it was not told of still comes"""
+    monkeypatch.setattr(masks, "_static_lists", lambda device: 256)
+    cpu, mask = torch.device("cpu"), _fresh_mask()
+    sidx = torch.from_numpy(np.flatnonzero(mask.art.numpy() >= 0)) if compact else None
+    heads = [(16, 8, 256), (4, 2, 128), (8, 1, 512)]
+    assert mask.prepare(*heads, sidx=sidx) is mask
+
+    def more(*a, **k):
+        raise AssertionError("a prepared mask makes something at a call")
+
+    with monkeypatch.context() as m:
+        m.setattr(sa.TilePlan, "build", more)
+        m.setattr(sa.TreeMask, "_upload", more)
+        m.setattr(masks, "_Shared", more)
+        for hq, hkv, d in heads:
+            layer = attention._Layer.of(mask, hq, hkv, d, 0, compact, cpu)
+            assert _owns_what_it_points_to(layer)
+            if compact:
+                mask.for_head_dim(d, ring=layer.ring).rows(sidx)
+        with pytest.raises(AssertionError):
+            attention._Layer.of(mask, 6, 2, 64, 0, compact, cpu)
+    with pytest.raises(ValueError, match="do not group"):
+        mask.prepare((5, 2, 64))
+
+
+def test_a_stream_the_compiler_refuses_is_refused_at_the_build():
+    long = np.broadcast_to(np.int32(0), ((1 << 30) + 1,))
+    with pytest.raises(ValueError, match="too long"):
+        sa.TreeMask.build(long, long, long, device="cpu")
+
+
 def test_a_call_on_another_stream_waits_for_what_the_first_one_uploaded(monkeypatch):
     """a mask's schedules, entries and row maps are uploaded by whichever call comes first, on its stream: every other stream waits for
     the copy of each buffer it reads, once, and the allocator hears of it; the stream that copied does not wait"""
@@ -459,3 +492,28 @@ def test_a_traced_program_holds_the_operator(dev):
     assert "spinf::lm_logprobs" in str(traced.graph)
     for x in (a, b):
         assert torch.equal(traced(x), sa.lm_logprobs(x, None, 30.0))
+
+
+@pytest.mark.gpu
+def test_masks_prepared_on_a_thread_and_stream_of_their_own(dev):
+    """a producer thread builds and prepares a forward's masks on its stream; the layers run on another stream with no order between
+    the two but what the calls see to"""
+    cfg = synth.attention_config("C2", contents=2)
+    b = cfg.batches[0]
+    q, k, v = synth.qkv(cfg, b, seed=6, device=dev)
+    ref = sa.block_masks(b, sliding_window=100, device=dev)
+    want = {name: sa.tree_attn(q, k, v, m, cfg.scale) for name, m in ref.items()}
+    stream, made = torch.cuda.Stream(), {}
+    torch.cuda.synchronize()
+
+    def produce():
+        with torch.cuda.device(dev), torch.cuda.stream(stream):
+            torch.cuda._sleep(20_000_000)
+            made.update({name: m.prepare((cfg.hq, cfg.hkv, cfg.d)) for name, m in sa.block_masks(b, sliding_window=100, device=dev).items()})
+
+    t = threading.Thread(target=produce)
+    t.start()
+    t.join()
+    got = {name: sa.tree_attn(q, k, v, m, cfg.scale) for name, m in made.items()}
+    made.clear()
+    assert all(torch.equal(got[name], want[name]) for name in want)
