@@ -21,6 +21,11 @@
 // left: 4 barriers a block against 6 of the chunk kernel.  A block of 32 is also fuller than the chunk kernel's pairs of leaves
 // (two times 16 rows, whatever the leaves use of them).
 //
+// What is not finite in one option must not reach the others of its blocks, as every product above meets it with a coefficient of zero.
+// The entries of A, beta and g are cleared where they are computed or staged, and their token noted; V' is looked at (a product with zeros) and, where it is not finite, computed again with such entries of V + R cleared.  Noted tokens and all below them come out
+// as NaN, per value column; a stack row carries its note in a bit mask beside V'.  Outputs of all other tokens keep their bits.  The look
+// costs 1 % of a layer over a stream of tries (409 -> 413 us).
+//
 // What it measured (the stream above, 10.6 k tokens in tries, 32 value heads): 167 us in one launch for 0.70 ms in six; 0.4 GB of rows
 // and states, 2.5 TB/s.  Bound by a block's chain of phases: 11 k clocks, of them 2.7 k the solve on wave 0, 1.6 k A and P, 1.25 k staging
 // and G, 1.7 k R, 2.6 k V' / O and the stores, two workgroups per compute unit (LDS 79 KB, 256 registers).  Eight waves of 16 columns
@@ -42,7 +47,7 @@ constexpr int LD = 136;                  // row strides (elements) as in gdn_chu
 constexpr int LDT = 144;                 // V (transposing reads) 72,
 constexpr int LP = 40, LA = 36, LX = 20; // token x token tiles, A (floats), blocks of T (floats)
 constexpr int LO = CH + 4;               // a wave's transposed output tile
-constexpr int LS = ST + 4;               // the stack's V', by value column: 34 banks
+constexpr int LS = ST + 4;               // the stack's V', by value column: 34 banks.  The last four are a bit mask of the rows that are not finite
 __device__ __forceinline__ long row_offset(int row, long stride) { return (long)((unsigned long)(unsigned)row * (unsigned)stride); }
 __device__ __forceinline__ bf16x4 zero_bf4() {
     bf16x4 z;
@@ -50,6 +55,8 @@ __device__ __forceinline__ bf16x4 zero_bf4() {
     for (int r = 0; r < 4; r++) z[r] = (__bf16)0.f;
     return z;
 }
+__device__ __forceinline__ bool not_finite(float x) { return (__builtin_bit_cast(unsigned, x) & 0x7f800000u) == 0x7f800000u; }
+__device__ __forceinline__ bool not_finite(__bf16 x) { return (__builtin_bit_cast(unsigned short, x) & 0x7f80u) == 0x7f80u; }
 __device__ __forceinline__ bf16x8 join_rows(const __bf16* p) { return join(*(const bf16x4*)p, *(const bf16x4*)(p + 16)); }
 }  // namespace
 
@@ -72,6 +79,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     __shared__ __attribute__((aligned(16))) int Ds[CH];              // 1 + depth of a token the next block's path holds, 0 for others
     __shared__ __attribute__((aligned(16))) float Gr[CH];
     __shared__ int Rs[CH], Ns[CH], Ms[CH];
+    __shared__ unsigned odd_rows;                                    // tokens of the block with a beta, a g or a row of A that is not finite
     static_assert(4 * 32 * LO <= CH * LDT, "the output tiles must fit the V tile");
 
     const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15, q4 = lane >> 4;
@@ -150,15 +158,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
         for (int vt = 0; vt < 2; vt++) sb[s][vt] = join(round4(S0[2 * s][vt]), round4(S0[2 * s + 1][vt]));
 
+    bool noted = false;    // does a row of the stack carry a note in one of this wave's columns?
     for (int j = 0; j < n_blocks; j++) {
         lds_barrier();   // every wave is done with the previous block's tiles; the stack holds this block's path
         if (tid < CH) {
-            Gr[tid] = pg;
-            Bs[tid] = (float)pbeta;
-            Rs[tid] = pr;
-            Ms[tid] = pm;
-            Ns[tid] = pn;
-            Ds[tid] = (pn >> 8) & 0xff;
+            const bool odd = not_finite(pg) || not_finite(pbeta);
+            const unsigned long odds = __builtin_amdgcn_ballot_w64(odd);
+            int at = tid;                  // (addresses are computed here, as further down: kept in registers they would push others out)
+            asm volatile("" : "+v"(at));
+            if (at == 0) odd_rows = (unsigned)odds;
+            Gr[at] = odd ? 0.f : pg;
+            Bs[at] = odd ? 0.f : (float)pbeta;
+            Rs[at] = pr;
+            Ms[at] = pm;
+            Ns[at] = pn;
+            Ds[at] = (pn >> 8) & 0xff;
         }
         {
             const int col = (tid & 15) * 8;
@@ -172,14 +186,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         if (w == 0) {    // G: the path's sum so far and the tokens above in this block; lanes 0..31 add rows 0..15, the others 16..31
             wave_lds_order();
-            const int row = lane & 31, half = lane >> 5;
+            int at = lane;
+            asm volatile("" : "+v"(at));
+            const int row = at & 31, half = at >> 5;
             const int above = (Ms[row] | (int)(1u << row)) >> (16 * half);
             float x = 0.f;
 #pragma unroll
             for (int m4 = 0; m4 < 4; m4++) {
                 const f32x4 gv = *(const f32x4*)(Gr + 16 * half + 4 * m4);
 #pragma unroll
-                for (int r = 0; r < 4; r++) {   // (a mask, not a product: a NaN stays with the tokens below it)
+                for (int r = 0; r < 4; r++) {
                     const float g = gv[r];
                     x += __builtin_bit_cast(float, __builtin_bit_cast(int, g) & -((above >> (4 * m4 + r)) & 1));
                 }
@@ -211,19 +227,24 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             const f32x4 Gj = *(const f32x4*)(Gs + 16 * jt + 4 * q4);
             f32x4 a4;
             bf16x4 p4;
+            bool odd = false;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const int jj = 16 * jt + 4 * q4 + r;
                 const bool up = (above >> r) & 1;
                 const float d = __expf(Gi - Gj[r]);
-                a4[r] = up ? -bi * kk[r] * d : 0.f;
+                const float a = up ? -bi * kk[r] * d : 0.f;
+                const bool o = not_finite(a);
+                a4[r] = o ? 0.f : a;
+                odd |= o;
                 p4[r] = (__bf16)(up || jj == i ? p.scale * qk[r] * d : 0.f);
             }
+            if (odd) atomicOr(&odd_rows, 1u << i);
             *(f32x4*)(As + i * LA + 16 * jt + 4 * q4) = a4;
             *(bf16x4*)(Ps + i * LP + 16 * jt + 4 * q4) = p4;
         }
         // C and E over 32 rows of the stack: tile (jt, it) of wave w
-        auto against_path = [&](const int first) __attribute__((always_inline)) {
+        auto against_path = [&](const int first, const int c, const int q4) __attribute__((always_inline)) {
             const int jt = w >> 1, it = w & 1;
             f32x4 kk = zero4(), qk = zero4();
 #pragma unroll
@@ -247,7 +268,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             *(bf16x4*)(Cs + i * LP + 16 * jt + 4 * q4) = c4;
             *(bf16x4*)(Es + i * LP + 16 * jt + 4 * q4) = e4;
         };
-        if (depth > 0) against_path(0);
+        if (depth > 0) against_path(0, c, q4);
         lds_barrier();
 
         // ---- T diag(beta) on wave 0 (gdn_chunk.hip explains the solve), while the other waves go on with their columns
@@ -311,8 +332,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         for (int first = 0; first < depth; first += 32) {
             if (first > 0) {
+                int at = lane;
+                asm volatile("" : "+v"(at));
                 lds_barrier();
-                against_path(first);
+                against_path(first, at & 15, at >> 4);
                 lds_barrier();
             }
 #pragma unroll
@@ -339,11 +362,47 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 tA[it] = join(*(const bf16x4*)tp, it ? *(const bf16x4*)(tp + 16) : zero_bf4());
                 pA[it] = join(*(const bf16x4*)pp, it ? *(const bf16x4*)(pp + 16) : zero_bf4());
             }
+            bf16x8 rB[2];
+            bf16x4 vs[2][2];
 #pragma unroll
             for (int vt = 0; vt < 2; vt++) {
-                const bf16x8 rB = join(round4(R[0][vt]), round4(R[1][vt]));
-                const bf16x4 v0 = round4(mfma32(tA[0], rB, mfma32(tA[0], vin[vt], zero4()))), v1 = round4(mfma32(tA[1], rB, mfma32(tA[1], vin[vt], zero4())));
-                const bf16x8 vB = join(v0, v1);
+                rB[vt] = join(round4(R[0][vt]), round4(R[1][vt]));
+#pragma unroll
+                for (int it = 0; it < 2; it++) {
+                    vs[it][vt] = round4(mfma32(tA[it], rB[vt], mfma32(tA[it], vin[vt], zero4())));
+                }
+            }
+            const bf16x8 none = join(zero_bf4(), zero_bf4());
+            const float z = mfma32(none, join(vs[0][1], vs[1][1]), mfma32(none, join(vs[0][0], vs[1][0]), zero4()))[0];   // NaN if a column of V' is not finite
+            const bool look = noted || __builtin_amdgcn_ballot_w64(z != z || odd_rows != 0) != 0;
+            unsigned of_column[2] = {0, 0};       // the tokens to note, by this lane's columns
+            if (look) {
+#pragma unroll
+                for (int vt = 0; vt < 2; vt++) {
+                    unsigned m = 0;
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        if (not_finite((__bf16)rB[vt][e]) || not_finite((__bf16)vin[vt][e])) {
+                            rB[vt][e] = vin[vt][e] = (__bf16)0.f;
+                            m |= 1u << (16 * (e >> 2) + 4 * q4 + (e & 3));
+                        }
+#pragma unroll
+                    for (int it = 0; it < 2; it++) {
+                        vs[it][vt] = round4(mfma32(tA[it], rB[vt], mfma32(tA[it], vin[vt], zero4())));
+#pragma unroll
+                        for (int r = 0; r < 4; r++)      // (sums of finite numbers past the range)
+                            if (not_finite((__bf16)vs[it][vt][r])) {
+                                vs[it][vt][r] = (__bf16)0.f;
+                                m |= 1u << (16 * it + 4 * q4 + r);
+                            }
+                    }
+                    m |= __shfl_xor(m, 16);
+                    of_column[vt] = odd_rows | m | __shfl_xor(m, 32);
+                }
+            }
+#pragma unroll
+            for (int vt = 0; vt < 2; vt++) {
+                const bf16x8 vB = join(vs[0][vt], vs[1][vt]);
 #pragma unroll
                 for (int it = 0; it < 2; it++)
                     *(bf16x4*)(Ow + (16 * vt + c) * LO + 16 * it + 4 * q4) = round4(mfma32(pA[it], vB, O[it][vt]));      // O^T[v][i]
@@ -353,8 +412,39 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 #pragma unroll
                         for (int r = 0; r < 4; r++) {
                             const int d = Ds[16 * it + 4 * q4 + r];
-                            if (d > 0) Vst[(32 * w + 16 * vt + c) * LS + d - 1] = it ? v1[r] : v0[r];
+                            if (d > 0) Vst[(32 * w + 16 * vt + c) * LS + d - 1] = vs[it][vt][r];
                         }
+                }
+            }
+            if (look) {      // the noted tokens and those below them
+                int at = lane;         // (addresses of this path only: not to be kept in registers beside the other one's)
+                asm volatile("" : "+v"(at));
+                noted = false;
+                wave_lds_order();
+#pragma unroll 1
+                for (int vt = 0; vt < 2; vt++) {
+                    const int col = 16 * vt + (at & 15), row = 4 * (at >> 4);
+                    const unsigned of = vt ? of_column[1] : of_column[0];
+                    unsigned long* const notes = (unsigned long*)(Vst + (32 * w + col) * LS + ST);
+                    unsigned long on_stack = *notes;
+                    unsigned hit = 0;
+#pragma unroll 1
+                    for (int e = 0; e < 8; e++) {
+                        const int i = 16 * (e >> 2) + row + (e & 3), n = Ns[i] & 0xff;
+                        if ((((unsigned)Ms[i] | (1u << i)) & of) != 0 || (n > 0 && on_stack << (64 - n) != 0)) {
+                            hit |= 1u << i;
+                            Ow[col * LO + i] = (__bf16)__builtin_nanf("");
+                        }
+                    }
+                    hit |= __shfl_xor(hit, 16);
+                    hit |= __shfl_xor(hit, 32);
+                    if (next_depth > 0) {
+#pragma unroll 1
+                        for (int i = 0; i < CH; i++)
+                            if (const int d = Ds[i]; d > 0) on_stack = (on_stack & ~(1ul << (d - 1))) | ((unsigned long)((hit >> i) & 1u) << (d - 1));
+                        *notes = on_stack;
+                    }
+                    noted |= __builtin_amdgcn_ballot_w64(on_stack != 0) != 0;
                 }
             }
         }
@@ -370,12 +460,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         // ---- the path's K and G rows (read by every wave after the next two barriers; this block's readers are behind the last one)
         if (next_depth > 0) {
+            int at = tid;
+            asm volatile("" : "+v"(at));
 #pragma unroll
             for (int cc = 0; cc < 2; cc++) {
-                const int row = (tid >> 4) + 16 * cc, d = Ds[row], col = (tid & 15) * 8;
+                const int row = (at >> 4) + 16 * cc, d = Ds[row], col = (at & 15) * 8;
                 if (d > 0) *(bf16x8*)(Kst + (d - 1) * LD + col) = *(const bf16x8*)(Ks + row * LD + col);
             }
-            if (tid < CH && Ds[tid] > 0) Gst[Ds[tid] - 1] = Gs[tid];
+            if (at < CH && Ds[at] > 0) Gst[Ds[at] - 1] = Gs[at];
         }
     }
 }

@@ -266,6 +266,47 @@ def test_forests(dev, kind, h, hv):
     assert err <= 1.5 * by_level + 1e-5
 
 
+@pytest.mark.parametrize("what", ["v", "v inf", "k", "k inf", "q", "beta", "beta inf", "g", "g -inf", "two"])
+@pytest.mark.parametrize("at", ["leaf", "node", "deep"])
+def test_what_is_not_finite_in_a_forest_stays_at_and_below_its_token(dev, what, at):
+    """one option of a forest with a NaN or an infinity: it and the options below it come out as such, all others with the bits they have
+    without it, in its block, in the blocks below and in the blocks that only share the stack with it; a value's column is its own"""
+    rng = np.random.default_rng(8)
+    nodes = [(3, -1), (20, -1), (20, 1), (12, 2), (2, 3), (2, 3), (3, 2), (9, 1), (2, -1), (30, -1), (6, 9), (6, 9), (40, 0), (1, 12), (1, 12), (4, -1)]
+    trees = [_chain_tree(rng, 70, nodes), _chain_tree(rng, 40, nodes[::-1][:1] + [(5, -1), (7, 1)])]
+    cfg = synth.GdnConfig("poison", 2, 4, 128, 128, trees)
+    cfg.batch = b = synth.pack(trees)[0]
+    t = synth.gdn_inputs(cfg, seed=3, device=dev)
+    plan = cfg.plan(dev)
+    assert any(launch[0] == 2 for level in plan.program for launch in level)
+    first = np.cumsum([0] + [n for n, _ in nodes]) + 70
+    poisoned = {"leaf": [int(first[6]) + 1], "node": [int(first[1]) + 2], "deep": [int(first[3]) + 11]}[at] + ([int(first[10])] if what == "two" else [])
+    below = np.zeros(b.length, bool)
+    below[poisoned] = True
+    for i in range(b.length):
+        below[i] |= b.art[i] >= 0 and b.prev[i] >= 0 and below[b.prev[i]]
+    assert below.sum() < 80 and all(b.art[p] >= 0 for p in poisoned)
+    clean = sa.gdn_tree(*(t[x] for x in ("q", "k", "v", "g", "beta")), plan)
+    name, value = {"two": ("v", float("nan"))}.get(what, (what.split()[0], {"": float("nan"), "inf": float("inf"), "-inf": -float("inf")}[what[len(what.split()[0]):].strip()]))
+    for p in poisoned:
+        if name in ("beta", "g"):
+            t[name][p, 1] = value
+            hit_heads = [1]
+        else:
+            t[name][p, 1, 77] = value
+            hit_heads = [1] if name == "v" else [2, 3]
+    got = sa.gdn_tree(*(t[x] for x in ("q", "k", "v", "g", "beta")), plan)
+    torch.cuda.synchronize()
+    g, c = _np(got), _np(clean)
+    if name == "q":
+        below[:] = False
+        below[poisoned] = True
+    touched = np.zeros(g.shape, bool)
+    touched[np.ix_(np.flatnonzero(below), hit_heads, [77] if name == "v" else range(128))] = True
+    assert np.array_equal(g[~touched], c[~touched])
+    assert not np.isfinite(g[touched]).any()
+
+
 def test_decoder_steps_rerun_the_recurrence_from_the_prefix_state(dev):
     """the extraction decoder's call (spinf_serve/models/qwen35/qwen_decode.py:305-318): every step each slot re-runs the recurrence
     from its group's prefix state over its template rows plus the tokens generated so far, read out of row caches through idx,
