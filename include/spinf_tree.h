@@ -327,7 +327,8 @@ int spinf_xdecode_tiles(const spinf_xdec_args* args, int32_t* tiles);
 int spinf_xdecode_attn_fwd(const spinf_xdec_args* args, void* stream);
 /* Replaces the two index_copy_ of GroupKV.update (spinf_serve/decode.py:51-68): the new tokens' keys and values [G, h, Q, d] (bf16,
  * head dim contiguous, element strides *_g, *_h, *_q, multiples of 8) become entry *step (device scalar) of gk / gv [G, h, Q, S, d].
- * A step outside 0 .. S - 1 writes nothing.  d a multiple of 8, everything 16-byte aligned. */
+ * A step outside 0 .. S - 1 (index_copy_'s device assertion) puts NaN into the entry nearest to it: the step's attention comes out as NaN
+ * instead of an answer without its own token.  d a multiple of 8, everything 16-byte aligned. */
 int spinf_xdecode_put(const void* k, int64_t k_g, int64_t k_h, int64_t k_q, const void* v, int64_t v_g, int64_t v_h, int64_t v_q,
                       void* gk, void* gv, const int64_t* step, int32_t G, int32_t h, int32_t Q, int32_t S, int32_t d, void* stream);
 

@@ -443,13 +443,18 @@ struct PutParams {
 };
 __global__ __launch_bounds__(256) void xdec_put_kernel(const PutParams p) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
-    const long step = *p.step;
-    if (i >= p.n || step < 0 || step >= p.S) return;
+    if (i >= p.n) return;
+    // A step outside the caches, which only the device can see: NaN goes into the entry nearest to it, so the step's outputs say so.
+    const long want = *p.step, step = want < 0 ? 0 : want < p.S ? want : p.S - 1;
     const int c = blockIdx.y;
     const long row = i / p.d8, gh = row / p.Q, g = gh / p.h;
     const int piece = (int)(i - row * p.d8), q = (int)(row - gh * p.Q), hh = (int)(gh - g * p.h);
     const __bf16* from = p.src[c] + g * p.s_g[c] + hh * p.s_h[c] + q * p.s_q[c] + piece * 8;
-    *(bf16x8*)(p.dst[c] + (row * p.S + step) * (p.d8 * 8) + piece * 8) = *(const bf16x8*)from;
+    bf16x8 x = *(const bf16x8*)from;
+    if (step != want)
+#pragma unroll
+        for (int e = 0; e < 8; e++) x[e] = (__bf16)__builtin_nanf("");
+    *(bf16x8*)(p.dst[c] + (row * p.S + step) * (p.d8 * 8) + piece * 8) = x;
 }
 
 int check_args(const spinf_xdec_args* a) {

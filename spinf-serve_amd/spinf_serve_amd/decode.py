@@ -73,7 +73,9 @@ class XCaches:
 
 
 class GroupKV:
-    """stores the new tokens' K/V at the current step and hands the layer index to the attention (decode.py:51-68)"""
+    """stores the new tokens' K/V at the current step and hands the layer index to the attention (decode.py:51-68).  The step is a device
+    scalar: one outside the caches' 0 .. S - 1 cannot be refused here without a synchronisation; it puts NaN into the entry nearest
+    to it, and the step's outputs are NaN."""
 
     is_compileable = False
 

@@ -319,6 +319,24 @@ def test_cache_update_equals_index_copy(dev, G, h, Q, S, d):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 512])
+@pytest.mark.parametrize("step", [-(1 << 40), -1, 4, 5, 1 << 33])
+def test_a_step_outside_the_caches_does_not_go_unnoticed(dev, step, d):
+    """the entry nearest to it holds NaN, nothing else changes, and the step's attention is NaN throughout"""
+    q, c = synth.xdecode_case(2, 4, 2, d, 2, 3, 4, (40, 80), (3, 6), None, 0, seed=5, device=dev)
+    before = c.gk[0].clone(), c.gv[0].clone()
+    c.step_t.fill_(step)
+    new = torch.ones(2, 2, 6, d, dtype=torch.bfloat16, device=dev)
+    decode.GroupKV(c).update(new, new, 0)
+    at = 0 if step < 0 else 3
+    for t, old in zip((c.gk[0], c.gv[0]), before):
+        assert torch.isnan(t[:, :, :, at]).all()
+        keep = [s for s in range(4) if s != at]
+        assert torch.equal(t[:, :, :, keep], old[:, :, :, keep])
+    assert torch.isnan(sa.xdecode_attn(q, c, 0, d**-0.5)).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,h,d,slots,prefix", [(16, 1, 512, 4, (301, 301)), (16, 1, 512, 1, (5, 40)), (24, 4, 256, 2, (64, 64)), (32, 16, 128, 3, (20, 130)), (4, 2, 64, 1, (1, 9))])
 def test_small_steps_cut_into_short_splits(dev, H, h, d, slots, prefix):
     """one or two groups: the planned splits go down to single tiles, head dim 512 computes both halves of the output in one launch and merges
