@@ -100,22 +100,24 @@ void build_program(spinf_gdn_plan* p, const std::vector<Seg>& seg, int32_t n_lev
     auto flush = [&](Level& L, int64_t slot) {
         const int64_t n = (int64_t)rowv.size();
         if (!n) return;
-        std::vector<uint32_t> mask(n, 0);
-        std::vector<int32_t> from(n, 0);
-        for (int64_t f = 0; f < n; f += B) {
+        size_t o = L.table.size();
+        L.table.resize(o + (size_t)((n + B - 1) / B) * GDN_FOREST_INTS);
+        for (int64_t f = 0; f < n; f += B, o += GDN_FOREST_INTS) {
             const int64_t e = std::min(n, f + B), next = f + B < n ? dep[f + B] : 0;
-            int32_t save[GDN_FOREST_BLOCK] = {};
+            int32_t* const rows_out = L.table.data() + o;
+            uint32_t* const mask = (uint32_t*)rows_out + B;        // (signed and unsigned of one type may alias)
+            uint32_t* const packed = mask + B;
+            const uint32_t both = (uint32_t)dep[f] << 16 | (uint32_t)next << 24;
             for (int64_t i = f; i < e; i++) {
                 const int64_t a = up[i];
-                if (a >= f) { mask[i] = mask[a] | 1u << (a - f); from[i] = from[a]; }
-                else from[i] = a >= 0 ? dep[a] + 1 : 0;    // (pre-order: a token above i in an earlier block is above the block's first token)
+                rows_out[i - f] = rowv[i];
+                mask[i - f] = a >= f ? mask[a - f] | 1u << (a - f) : 0;
+                // (pre-order: a token above i in an earlier block is above the block's first token)
+                packed[i - f] = a >= f ? packed[a - f] : (a >= 0 ? (uint32_t)dep[a] + 1 : 0u) | both;
             }
+            for (int64_t i = e; i < f + B; i++) { rows_out[i - f] = -1; mask[i - f] = 0; packed[i - f] = both; }
             if (f + B < n)
-                for (int64_t a = up[f + B]; a >= f; a = up[a]) save[a - f] = dep[a] + 1;
-            for (int64_t i = f; i < f + B; i++) L.table.push_back(i < e ? rowv[i] : -1);
-            for (int64_t i = f; i < f + B; i++) L.table.push_back(i < e ? (int32_t)mask[i] : 0);
-            for (int64_t i = f; i < f + B; i++)
-                L.table.push_back((int32_t)((uint32_t)(i < e ? from[i] : 0) | (uint32_t)(i < e ? save[i - f] : 0) << 8 | (uint32_t)dep[f] << 16 | (uint32_t)next << 24));
+                for (int64_t a = up[f + B]; a >= f; a = up[a]) packed[a - f] |= (uint32_t)(dep[a] + 1) << 8;
         }
         L.cu.push_back(L.cu.back() + (n + B - 1) / B);
         L.h0.push_back(slot);
@@ -150,11 +152,11 @@ void build_program(spinf_gdn_plan* p, const std::vector<Seg>& seg, int32_t n_lev
     }
 
     // what is left of each level, then its units
-    auto put = [&](const int64_t* x, size_t n) {
-        if (p->prog_data.size() % 2) p->prog_data.push_back(0);
-        const int64_t o = (int64_t)p->prog_data.size();
-        p->prog_data.insert(p->prog_data.end(), x, x + n);
-        return o;
+    auto put = [&](const void* x, size_t n) {     // n pieces of 8 bytes
+        const size_t o = (p->prog_data.size() + 1) / 2 * 2;
+        p->prog_data.resize(o + n);
+        if (n) std::memcpy(p->prog_data.data() + o, x, n * 8);
+        return (int64_t)o;
     };
     std::vector<int64_t> cu, h0, ht, idx;
     for (int32_t d = 0; d < n_levels; d++) {
@@ -179,10 +181,7 @@ void build_program(spinf_gdn_plan* p, const std::vector<Seg>& seg, int32_t n_lev
         }
         const Level& L = lev[d];
         if (L.h0.empty()) continue;
-        const int64_t words = (int64_t)L.table.size() / 2;   // (GDN_FOREST_INTS is even)
-        std::vector<int64_t> table(words);
-        std::memcpy(table.data(), L.table.data(), words * 8);
-        const int64_t rec[8] = {d, 2, (int64_t)L.h0.size(), 0, put(L.cu.data(), L.cu.size()), put(table.data(), table.size()),
+        const int64_t rec[8] = {d, 2, (int64_t)L.h0.size(), 0, put(L.cu.data(), L.cu.size()), put(L.table.data(), L.table.size() / 2),   // (GDN_FOREST_INTS is even)
                                 d > 0 ? put(L.h0.data(), L.h0.size()) : -1, -1};
         p->prog.insert(p->prog.end(), rec, rec + 8);
     }

@@ -67,13 +67,13 @@ def _compile(prev, real, path, short, call_tokens, max_init, rows, keep):
                       call_row_ptr=(n_call + 1, np.int64), seg_len=(n_cseg, np.int64), h0_idx=(n_cseg, np.int64), ht_idx=(n_cseg, np.int64),
                       idx=(n_rows, np.int64), n_keep=(n_lev, np.int64), conv=(n_conv * 4, np.int64), seg_of_row=(n_conv, np.int64),
                       seg_level=(n_seg, np.int64), seg_slot=(n_seg, np.int64))
-        out = {name: np.zeros(max(size, 1), dtype) for name, (size, dtype) in shapes.items()}
+        out = {name: np.empty(max(size, 1), dtype) for name, (size, dtype) in shapes.items()}
         _lib.check(lib.spinf_gdn_plan_export(handle, *(out[name].ctypes.data for name in shapes)), "tree_plan")
         out = {name: out[name][: shapes[name][0]] for name in shapes}
         out["n_segments"] = n_seg
         counts = (C.c_int64 * 2)()
         _lib.check(lib.spinf_gdn_plan_program(handle, counts, None, None), "tree_plan")
-        out["program"], out["program_data"] = np.zeros((counts[0], 8), np.int64), np.zeros(counts[1], np.int64)
+        out["program"], out["program_data"] = np.empty((counts[0], 8), np.int64), np.empty(counts[1], np.int64)
         _lib.check(lib.spinf_gdn_plan_program(handle, counts, out["program"].ctypes.data, out["program_data"].ctypes.data), "tree_plan")
         return out
     finally:
@@ -117,37 +117,28 @@ def tree_plan(prev, real, device, max_init: int = 96, path: str = "indexed", sho
     for x, o in zip(parts, at):
         host[o : o + len(x)] = x
     on_dev = stage.to(dev, non_blocking=True)
-    conv, idx_all, h0_all, ht_all, cu_all, sidx, pad_rows, program_data = (on_dev[o : o + len(x)] for x, o in zip(parts, at))
+    conv, idx_all, h0_all, ht_all, cu_all, sidx, pad_rows, _ = (on_dev[o : o + len(x)] for x, o in zip(parts, at))
     cu_of = {span: k for k, span in enumerate(spans)}
-
-    def cut(i, j):
-        """calls i .. j - 1 as one: rows, cumulative lengths (device, host), start and end slots"""
-        k = cu_of[(i, j)]
-        seg, row = slice(seg_ptr[i], seg_ptr[j]), slice(row_ptr[i], row_ptr[j])
-        return idx_all[row], cu_all[cu_at[k] : cu_at[k + 1]], cu_host[cu_at[k] : cu_at[k + 1]], h0_all[seg], ht_all[seg]
 
     levels, launches = [], []
     for d, lv in enumerate(runs):
         calls = []
         for c in range(level_ptr[d], level_ptr[d + 1]):
-            idx, cu, cu_cpu, starts, ends = cut(c, c + 1)
-            starts = None if d == 0 else starts
+            seg, k = slice(seg_ptr[c], seg_ptr[c + 1]), slice(cu_at[c], cu_at[c + 1])     # (the first spans are the calls)
+            idx, cu, cu_cpu, ends = idx_all[row_ptr[c] : row_ptr[c + 1]], cu_all[k], cu_host[k], ht_all[seg]
+            starts = None if d == 0 else h0_all[seg]
             if indexed:
                 calls.append(Call(idx, cu, cu_cpu, None, False, "chunked" if call_kind[c] else "recurrent", starts, ends if call_keep[c] else None))
             else:
                 calls.append(Call(idx, cu, cu_cpu, starts, bool(call_keep[c])))
         levels.append(calls)
-        merged = []
-        for i, j in lv if indexed else ():
-            idx, cu, _, starts, ends = cut(i, j)
-            lens = seg_len[seg_ptr[i] : seg_ptr[j]]
-            merged.append((int(call_kind[i]), len(lens), int(lens.max()) if call_kind[i] else 0, cu.storage_offset(), idx.storage_offset(),
-                           starts.storage_offset() if d else -1, ends.storage_offset() if call_keep[i:j].any() else -1))   # (views of on_dev)
-        launches.append(merged)
+        launches.append([(int(call_kind[i]), seg_ptr[j] - seg_ptr[i], int(seg_len[seg_ptr[i] : seg_ptr[j]].max()) if call_kind[i] else 0,
+                          at[4] + cu_at[cu_of[(i, j)]], at[1] + row_ptr[i], at[2] + seg_ptr[i] if d else -1, at[3] + seg_ptr[i] if call_keep[i:j].any() else -1)
+                         for i, j in (lv if indexed else ())])
     program = None
     if len(a["program"]):
         program = [[] for _ in levels]
-        first = program_data.storage_offset()
+        first = at[7]
         for d, mode, n, longest, *places in a["program"].tolist():
             program[d].append((mode, n, longest, *(first + o if o >= 0 else -1 for o in places)))
     seg_of_row = a["seg_of_row"]
