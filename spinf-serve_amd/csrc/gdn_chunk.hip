@@ -38,18 +38,6 @@ constexpr int VD = 128;        // value head dim
 // 16-byte row reads 4.0 at 8, 8.0 at 4, 20, 36.
 constexpr int LD = 136;        // row stride (elements) of the Q tile: 68 banks
 constexpr int LDT = 144;       // row stride of the K and V tiles: 72 banks
-constexpr int LP = 40;         // row stride of the token x token bf16 tiles (P, T diag(beta))
-constexpr int LA = 36;         // row stride (floats) of A
-constexpr int LX = 20;         // row stride (floats) of the 16 x 16 blocks of T and of the merge scratch
-
-// element offset of a row: one 32 x 32 -> 64 bit multiply (rows and strides are below 2^31; the launch checks the strides)
-__device__ __forceinline__ long row_offset(int row, long stride) { return (long)((unsigned long)(unsigned)row * (unsigned)stride); }
-__device__ __forceinline__ bf16x4 zero_bf4() {
-    bf16x4 z;
-#pragma unroll
-    for (int r = 0; r < 4; r++) z[r] = (__bf16)0.f;
-    return z;
-}
 }  // namespace
 
 // SOLVER: a fifth wave has the gates and the solve, and no value columns.  TIGHT: fewer registers, by computing LDS addresses anew in every
@@ -58,8 +46,6 @@ template <bool PAIRS, bool SOLVER, bool TIGHT>
 __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
     constexpr int NT = 2;                           // 16-token tiles per chunk
     constexpr int CH = 16 * NT;
-    constexpr int LO = CH + 4;                      // row stride (elements) of a wave's transposed output tile [32 values][CH tokens]; 64-byte rows
-                                                    // put the 8-byte stores of 16 lanes into four banks (32 clocks per store instead of 7)
     constexpr int NTILES = NT * (NT + 1) / 2;       // 16 x 16 tiles of A / P on or below the diagonal
     typedef bf16x8 tok_op;                          // operand of a product that contracts over the chunk's 32 tokens
     __shared__ __attribute__((aligned(16))) __bf16 Ks[CH * LDT];
@@ -188,40 +174,7 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             Rs[lane] = pr32;
         }
     };
-    // T = (I - A)^-1: rows of the diagonal blocks by substitution in registers (lane groups 0 and 2 the upper-left block, 1 and 3 the
-    // lower-right one, in the same instructions), then the lower-left block T_lo = T_11 A_lo T_00, computed transposed
-    // (T_lo^T = T_00^T (A_lo^T T_11^T)) so that the lane again holds a row.  Leaves T diag(beta) in LDS as bf16, tile by tile.
-    // The others wait for this wave: it goes first.
-    auto solve = [&]() __attribute__((always_inline)) {
-        __builtin_amdgcn_s_setprio(3);
-        float t[16];
-        const int blk = q4 & 1;
-        unit_lower_inverse_row<SOLVER || !TIGHT>(As + blk * (16 * LA + 16), LA, c, t);
-        // the rows pass through LDS to reach the lanes in operand order (row c, columns 4 q4 ..+3)
-#pragma unroll
-        for (int j4 = 0; j4 < 4; j4++) *(f32x4*)(Ts + (16 * blk + c) * LX + 4 * j4) = f32x4{t[4 * j4], t[4 * j4 + 1], t[4 * j4 + 2], t[4 * j4 + 3]};
-        wave_lds_order();
-        const float* T1s = Ts + 16 * LX;
-        const f32x4 B0 = *(const f32x4*)(Bs + 4 * q4), B1 = *(const f32x4*)(Bs + 16 + 4 * q4);
-        const f32x4 t00 = *(const f32x4*)(Ts + c * LX + 4 * q4), t11 = *(const f32x4*)(T1s + c * LX + 4 * q4);
-        *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
-        *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
-        f32x4 tlo = zero4();
-        if (!run_mode) {      // (a pair's tiles are different segments: A_lo = 0, so is T_lo)
-            f32x4 x = zero4();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; s4++)        // X[j][i] = sum_m A_lo[m][j] T_11[i][m]
-                x = mfma4(As[(16 + 4 * s4 + q4) * LA + c], T1s[c * LX + 4 * s4 + q4], x);
-#pragma unroll
-            for (int r = 0; r < 4; r++) Xs[(4 * q4 + r) * LX + c] = x[r];
-            wave_lds_order();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; s4++)        // T_lo[16 + i][j'] = sum_j T_00[j][j'] X[j][i]
-                tlo = mfma4(Ts[(4 * s4 + q4) * LX + c], Xs[(4 * s4 + q4) * LX + c], tlo);
-        }
-        *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = round4(tlo * B0);
-        __builtin_amdgcn_s_setprio(0);
-    };
+    auto solve = [&]() __attribute__((always_inline)) { solve_tile<SOLVER || !TIGHT>(As, Bs, Ts, Xs, Tus, c, q4, run_mode); };   // (a pair's tiles are different segments)
     if (SOLVER && w == 4) {
         fetch_gate_row(0);
         fetch_gates();
@@ -425,16 +378,7 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             }
         }
         wave_lds_order();
-        // row i = 16 it + lane%16, values 8 (lane/16) ..+7 of this wave's 32: two transposing reads, one 16-byte store
-#pragma unroll
-        for (int it = 0; it < NT; it++) {
-            const int row = 16 * it + c;
-            const __bf16* op = Ow + (8 * q4 + (c >> 2)) * LO + 16 * it + 4 * (c & 3);
-            const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)op));
-            const bf16x4 hi = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(op + 4 * LO)));
-            const int orow = Rs[row];      // -1: no such row in this chunk
-            if (orow >= 0) *(bf16x8*)(p.o + row_offset(orow, p.o_tok) + hv * VD + 32 * w + 8 * q4) = join(lo, hi);
-        }
+        store_tile(Ow, Rs, p.o, p.o_tok, hv * VD + 32 * w, c, q4);
         // ---- S[k][v] = e^{G_L} S[k][v] + sum_j K[j][k] (V' e^{G_L - G_j})[j][v]; skipped when nothing reads the state again
         if (!run_mode && (j + 1 < n_chunks || keep)) {
             const float GL = Gs[CH - 1];

@@ -45,16 +45,7 @@ constexpr int CH = GDN_FOREST_BLOCK;     // tokens per block
 constexpr int ST = GDN_FOREST_DEPTH;     // rows of the stack
 constexpr int LD = 136;                  // row strides (elements) as in gdn_chunk.hip: K, Q and the stack's K (row-wise reads) 68 banks,
 constexpr int LDT = 144;                 // V (transposing reads) 72,
-constexpr int LP = 40, LA = 36, LX = 20; // token x token tiles, A (floats), blocks of T (floats)
-constexpr int LO = CH + 4;               // a wave's transposed output tile
 constexpr int LS = ST + 4;               // the stack's V', by value column: 34 banks.  The last four are a bit mask of the rows that are not finite
-__device__ __forceinline__ long row_offset(int row, long stride) { return (long)((unsigned long)(unsigned)row * (unsigned)stride); }
-__device__ __forceinline__ bf16x4 zero_bf4() {
-    bf16x4 z;
-#pragma unroll
-    for (int r = 0; r < 4; r++) z[r] = (__bf16)0.f;
-    return z;
-}
 __device__ __forceinline__ bool not_finite(float x) { return (__builtin_bit_cast(unsigned, x) & 0x7f800000u) == 0x7f800000u; }
 __device__ __forceinline__ bool not_finite(__bf16 x) { return (__builtin_bit_cast(unsigned short, x) & 0x7f80u) == 0x7f80u; }
 __device__ __forceinline__ bf16x8 join_rows(const __bf16* p) { return join(*(const bf16x4*)p, *(const bf16x4*)(p + 16)); }
@@ -271,31 +262,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (depth > 0) against_path(0, c, q4);
         lds_barrier();
 
-        // ---- T diag(beta) on wave 0 (gdn_chunk.hip explains the solve), while the other waves go on with their columns
-        if (w == 0) {
-            __builtin_amdgcn_s_setprio(3);
-            float t[16];
-            const int blk = q4 & 1;
-            unit_lower_inverse_row<true>(As + blk * (16 * LA + 16), LA, c, t);
-#pragma unroll
-            for (int j4 = 0; j4 < 4; j4++) *(f32x4*)(Ts + (16 * blk + c) * LX + 4 * j4) = f32x4{t[4 * j4], t[4 * j4 + 1], t[4 * j4 + 2], t[4 * j4 + 3]};
-            wave_lds_order();
-            const f32x4 B0 = *(const f32x4*)(Bs + 4 * q4), B1 = *(const f32x4*)(Bs + 16 + 4 * q4);
-            const float* T1s = Ts + 16 * LX;
-            const f32x4 t00 = *(const f32x4*)(Ts + c * LX + 4 * q4), t11 = *(const f32x4*)(T1s + c * LX + 4 * q4);
-            f32x4 x = zero4(), tlo = zero4();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; s4++) x = mfma4(As[(16 + 4 * s4 + q4) * LA + c], T1s[c * LX + 4 * s4 + q4], x);
-#pragma unroll
-            for (int r = 0; r < 4; r++) Xs[(4 * q4 + r) * LX + c] = x[r];
-            wave_lds_order();
-#pragma unroll
-            for (int s4 = 0; s4 < 4; s4++) tlo = mfma4(Ts[(4 * s4 + q4) * LX + c], Xs[(4 * s4 + q4) * LX + c], tlo);
-            *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
-            *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
-            *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = round4(tlo * B0);
-            __builtin_amdgcn_s_setprio(0);
-        }
+        // ---- T diag(beta) on wave 0, while the other waves go on with their columns
+        if (w == 0) solve_tile<true>(As, Bs, Ts, Xs, Tus, c, q4, false);
         // Block j + 1 is requested here, behind the solve, which needs the registers; it has the rest of this block to arrive.
         fetch_data();
         fetch_rows(j + 2);
@@ -449,15 +417,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
             }
         }
         wave_lds_order();
-        // row i = 16 it + lane%16, values 8 (lane/16) ..+7 of this wave's 32: two transposing reads, one 16-byte store
-#pragma unroll
-        for (int it = 0; it < 2; it++) {
-            const __bf16* op = Ow + (8 * q4 + (c >> 2)) * LO + 16 * it + 4 * (c & 3);
-            const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)op));
-            const bf16x4 hi = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(op + 4 * LO)));
-            const int orow = Rs[16 * it + c];
-            if (orow >= 0) *(bf16x8*)(p.o + row_offset(orow, p.o_tok) + hv * VD + 32 * w + 8 * q4) = join(lo, hi);
-        }
+        store_tile(Ow, Rs, p.o, p.o_tok, hv * VD + 32 * w, c, q4);
         // ---- the path's K and G rows (read by every wave after the next two barriers; this block's readers are behind the last one)
         if (next_depth > 0) {
             int at = tid;

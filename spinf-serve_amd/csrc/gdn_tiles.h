@@ -109,4 +109,71 @@ __device__ __forceinline__ void lds_barrier() {
     asm volatile("" ::: "memory");
 }
 
+// element offset of a row: one 32 x 32 -> 64 bit multiply (rows and strides are below 2^31; the launch checks the strides)
+__device__ __forceinline__ long row_offset(int row, long stride) { return (long)((unsigned long)(unsigned)row * (unsigned)stride); }
+__device__ __forceinline__ bf16x4 zero_bf4() {
+    bf16x4 z;
+#pragma unroll
+    for (int r = 0; r < 4; r++) z[r] = (__bf16)0.f;
+    return z;
+}
+
+// ---- what the chunk kernel (gdn_chunk.hip) and the forest kernel (gdn_forest.hip) do alike with their 32 tokens
+constexpr int LP = 40;         // row stride of the token x token bf16 tiles (P, T diag(beta), ..)
+constexpr int LA = 36;         // row stride (floats) of A
+constexpr int LX = 20;         // row stride (floats) of the 16 x 16 blocks of T and of the merge scratch
+constexpr int LO = 32 + 4;     // row stride (elements) of a wave's transposed output tile [32 values][32 tokens]; 64-byte rows
+                               // would put the 8-byte stores of 16 lanes into four banks (32 clocks per store instead of 7)
+
+// T = (I - A)^-1 by one wave: rows of the diagonal blocks by substitution in registers (lane groups 0 and 2 the upper-left block, 1 and 3
+// the lower-right one, in the same instructions), then the lower-left block T_lo = T_11 A_lo T_00, computed transposed
+// (T_lo^T = T_00^T (A_lo^T T_11^T)) so that the lane again holds a row; apart: the two tiles do not see each other, T_lo = 0.  Leaves
+// T diag(beta) in Tus as bf16, tile by tile.  Ts (T_00 in rows 0..15, T_11 in 16..31) and Xs are scratch.  The others wait for this
+// wave: it goes first.  c = lane % 16, q4 = lane / 16; by reference, which leaves their reading where the kernels' own code would (by value
+// the kernels of 168 registers spill).
+template <bool PRELOAD>
+__device__ __forceinline__ void solve_tile(const float* As, const float* Bs, float* Ts, float* Xs, __bf16* Tus, const int& c, const int& q4, const bool& apart) {
+    __builtin_amdgcn_s_setprio(3);
+    float t[16];
+    const int blk = q4 & 1;
+    unit_lower_inverse_row<PRELOAD>(As + blk * (16 * LA + 16), LA, c, t);
+    // the rows pass through LDS to reach the lanes in operand order (row c, columns 4 q4 ..+3)
+#pragma unroll
+    for (int j4 = 0; j4 < 4; j4++) *(f32x4*)(Ts + (16 * blk + c) * LX + 4 * j4) = f32x4{t[4 * j4], t[4 * j4 + 1], t[4 * j4 + 2], t[4 * j4 + 3]};
+    wave_lds_order();
+    const float* T1s = Ts + 16 * LX;
+    const f32x4 B0 = *(const f32x4*)(Bs + 4 * q4), B1 = *(const f32x4*)(Bs + 16 + 4 * q4);
+    const f32x4 t00 = *(const f32x4*)(Ts + c * LX + 4 * q4), t11 = *(const f32x4*)(T1s + c * LX + 4 * q4);
+    *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
+    *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
+    f32x4 tlo = zero4();
+    if (!apart) {
+        f32x4 x = zero4();
+#pragma unroll
+        for (int s4 = 0; s4 < 4; s4++)        // X[j][i] = sum_m A_lo[m][j] T_11[i][m]
+            x = mfma4(As[(16 + 4 * s4 + q4) * LA + c], T1s[c * LX + 4 * s4 + q4], x);
+#pragma unroll
+        for (int r = 0; r < 4; r++) Xs[(4 * q4 + r) * LX + c] = x[r];
+        wave_lds_order();
+#pragma unroll
+        for (int s4 = 0; s4 < 4; s4++)        // T_lo[16 + i][j'] = sum_j T_00[j][j'] X[j][i]
+            tlo = mfma4(Ts[(4 * s4 + q4) * LX + c], Xs[(4 * s4 + q4) * LX + c], tlo);
+    }
+    *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = round4(tlo * B0);
+    __builtin_amdgcn_s_setprio(0);
+}
+
+// A wave's transposed output tile to memory: row i = 16 it + lane % 16, values 8 (lane / 16) ..+7 of the wave's 32, the first of which is column col:
+// two transposing reads, one 16-byte store.  Rs: the tensor rows, -1 for none.
+__device__ __forceinline__ void store_tile(const __bf16* Ow, const int* Rs, __bf16* out, long o_tok, int col, int c, int q4) {
+#pragma unroll
+    for (int it = 0; it < 2; it++) {
+        const __bf16* op = Ow + (8 * q4 + (c >> 2)) * LO + 16 * it + 4 * (c & 3);
+        const bf16x4 lo = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)op));
+        const bf16x4 hi = __builtin_bit_cast(bf16x4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) s16x4*)(op + 4 * LO)));
+        const int orow = Rs[16 * it + c];
+        if (orow >= 0) *(bf16x8*)(out + row_offset(orow, o_tok) + col + 8 * q4) = join(lo, hi);
+    }
+}
+
 }  // namespace gdn_tiles
