@@ -183,16 +183,16 @@ def check(code: int, what: str) -> None:
 _KINDS = (torch.Tensor, torch.nn.Parameter)
 _compiling, _grad_enabled = torch.compiler.is_compiling, torch.is_grad_enabled
 _dispatch_modes, _function_modes, _function_mode = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack, torch._C._get_function_stack_at
-_tracer, _functorch_level = torch._C._get_tracing_state, torch._C._functorch.maybe_current_level
+_tracing, _functorch_level = torch._C._is_tracing, torch._C._functorch.maybe_current_level
 
 
 def watched() -> bool:
     """Is something looking at the operators that run: a compiler, a tracer, a function transform (vmap, jvp, ..), forward-mode autograd,
     a dispatch or function mode?  A default device is a function mode too, one that looks at factory calls only."""
-    if _compiling():   # (first: the compiler folds it to True and cannot trace the others)
-        return True
-    return bool(_dispatch_modes() or _tracer() is not None or _functorch_level() is not None or forward_ad._current_level >= 0
-                or (n := _function_modes()) and any(type(_function_mode(i)) is not DeviceContext for i in range(n)))
+    if _compiling() or _dispatch_modes() or _tracing() or _functorch_level() is not None or forward_ad._current_level >= 0:   # (a compiler
+        return True                                                # folds the first to True and cannot trace the others)
+    n = _function_modes()
+    return n > 0 and any(type(_function_mode(i)) is not DeviceContext for i in range(n))
 
 
 def eager(first, *tensors) -> bool:
@@ -215,18 +215,24 @@ def same_device(device, *tensors) -> None:
             raise ValueError(f"all tensors of the call must be on {device}, one is on {t.device}")
 
 
-def raw_stream(device):
-    """the current stream of `device` as the library takes it; None where there are no streams"""
-    return torch._C._cuda_getCurrentRawStream(device.index) if device.type == "cuda" else None
+_raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
-def launch(fn, args, device, what: str) -> None:
-    """fn(args, current stream of `device`) with `device` current; args: an argument block, or a tuple of plain arguments"""
+def raw_stream(index):
+    """the handle of the current stream of GPU `index`, as the library takes it; None where there is none (index None: the host)"""
+    return None if index is None else _raw(index)
+
+
+def launch(fn, args, device, what: str, stream=None) -> None:
+    """fn(args, current stream of `device`) with `device` current; args: an argument block, or a tuple of plain arguments; stream: that
+    stream's handle where the caller has it"""
     args = args if type(args) is tuple else (C.byref(args),)
+    if stream is None:
+        stream = _raw(device.index)
     if torch._C._cuda_getDevice() == device.index:
-        rc = fn(*args, torch._C._cuda_getCurrentRawStream(device.index))
+        rc = fn(*args, stream)
     else:
         with torch.cuda.device(device):
-            rc = fn(*args, torch._C._cuda_getCurrentRawStream(device.index))
+            rc = fn(*args, stream)
     if rc:
         check(rc, what)

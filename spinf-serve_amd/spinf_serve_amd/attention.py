@@ -195,7 +195,8 @@ class _Layer:
         if m._meta is not None:
             self.shared += (m._meta,)
         self.owned = (m.art, m.end, m.pos, m.grp)
-        self.streams = set()   # those that have reached the shared tensors
+        here = _lib.raw_stream(device.index)
+        self.streams = {here} if all([here in x.streams for x in self.shared]) else set()   # those that may read the shared tensors
         a.variant, a.ktile, a.n_lists = variant, m._ktile, n_lists
         if m.grp is not None:
             a.grp, a.grp_mode = m.grp.data_ptr(), m.grp_mode
@@ -211,10 +212,9 @@ class _Layer:
                     got = mask._layers[key] = cls(mask, hq, hkv, d, variant, compact, device)
         return got
 
-    def reach(self, device):
-        """ahead of a launch: the current stream of `device` may read what the block points into"""
-        stream = _lib.raw_stream(device)
-        if stream not in self.streams and all([x.reach(stream) for x in self.shared]):
+    def reach(self, stream):
+        """ahead of the first launch on a stream (the current one, by its handle): it may read what the block points into"""
+        if all([x.reach(stream) for x in self.shared]):
             self.streams.add(stream)
 
     def bound(self, q, qs, k, ks, v, vs, out, os, scale):
@@ -234,14 +234,19 @@ def _variant(variant, mask, compact) -> int:
     return 0 if variant == 2 and (compact or mask.grp is not None) else variant
 
 
-def prepare_calls(mask, heads, sidx) -> None:
-    """TreeMask.prepare: the prepared calls of these head geometries, and the row map of sidx"""
+def prepare_calls(mask, heads, sidx) -> list:
+    """TreeMask.prepare: the prepared calls of these head geometries, and the row map of sidx -> what they read"""
+    shared = []
     if sidx is not None and mask.grp is not None:
         raise ValueError("image groups go with the stream layout (no sidx)")
     for hq, hkv, d in heads:
         layer = _Layer.of(mask, hq, hkv, d, _variant(VARIANT, mask, sidx is not None), sidx is not None, mask.device)
+        shared += layer.shared
         if sidx is not None:
-            mask.for_head_dim(d, ring=layer.ring).rows(sidx)
+            m = mask.for_head_dim(d, ring=layer.ring)
+            m.rows(sidx)
+            shared.append(m._rows[3])
+    return shared
 
 
 def _heads_first(q, k, v, mask, scale, sidx):
@@ -265,7 +270,9 @@ def _heads_first(q, k, v, mask, scale, sidx):
     elif mask.grp is not None or sidx.shape[0] > rows or sidx.device != dev:
         return None
     layer = _Layer.of(mask, hq, ks[1], d, _variant(VARIANT, mask, sidx is not None), sidx is not None, dev)
-    layer.reach(dev)
+    stream = _lib.raw_stream(dev.index)
+    if stream not in layer.streams:
+        layer.reach(stream)
     out = torch.empty((1, rows, hq, d), dtype=bf16, device=dev)
     a = layer.bound(q, (qs[2], qs[1]), k, (kst[2], kst[1]), v, (vs[2], vs[1]), out, (hq * d, d), float(d ** -0.5 if scale is None else scale))
     if sidx is not None:
@@ -273,7 +280,7 @@ def _heads_first(q, k, v, mask, scale, sidx):
             out[0, sidx.shape[0] :].zero_()
         row_of, kv_row0 = mask.for_head_dim(d, ring=layer.ring).rows(sidx)
         a.row_of, a.kv_row0 = row_of.data_ptr(), kv_row0.data_ptr()
-    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, dev, "spinf_tree_attn_fwd")
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, dev, "spinf_tree_attn_fwd", stream)
     return out
 
 
@@ -291,7 +298,9 @@ def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
     if sidx is not None and mask.grp is not None:
         raise ValueError("image groups go with the stream layout (no sidx)")
     layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], variant, sidx is not None, q.device)
-    layer.reach(q.device)
+    stream = _lib.raw_stream(q.device.index)
+    if stream not in layer.streams:
+        layer.reach(stream)
     m = mask.for_head_dim(q.shape[2], ring=layer.ring)   # the plan of the kernel's key-tile size
     row_of, kv_row0 = m.rows(sidx) if sidx is not None else (None, None)
     if not _lib.eager(q, k, v, sidx):
@@ -305,7 +314,7 @@ def tree_attn(q, k, v, mask: TreeMask, scale=None, variant=None, sidx=None):
         if sidx.shape[0] < q.shape[0]:
             out[sidx.shape[0] :].zero_()
         a.row_of, a.kv_row0 = row_of.data_ptr(), kv_row0.data_ptr()
-    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, q.device, "spinf_tree_attn_fwd")
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd, a, q.device, "spinf_tree_attn_fwd", stream)
     return out
 
 
@@ -320,9 +329,11 @@ def tree_attn_noalloc(q, k, v, mask: TreeMask, out, scale=None):
         raise ValueError("out must be a contiguous bf16 tensor of q's shape")
     _check_tensors(q, k, v, mask.n, False, (out, mask.art))
     layer = _Layer.of(mask, q.shape[1], k.shape[1], q.shape[2], 0, False, q.device)
-    layer.reach(q.device)
+    stream = _lib.raw_stream(q.device.index)
+    if stream not in layer.streams:
+        layer.reach(stream)
     a = layer.bound(q, q.stride()[:2], k, k.stride()[:2], v, v.stride()[:2], out, out.stride()[:2], float(q.shape[-1] ** -0.5 if scale is None else scale))
-    _lib.launch(_lib.load_library().spinf_tree_attn_fwd_noalloc, a, q.device, "spinf_tree_attn_fwd_noalloc")
+    _lib.launch(_lib.load_library().spinf_tree_attn_fwd_noalloc, a, q.device, "spinf_tree_attn_fwd_noalloc", stream)
     return out
 
 

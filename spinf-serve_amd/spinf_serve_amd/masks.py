@@ -42,14 +42,17 @@ class TilePlan:
     def build(cls, art, end, pos, window=None, grp=None, grp_windowed=False, ktile=64) -> "TilePlan":
         """grp (image groups, spinf_serve/scorer.py:184-198): [n] int32, -1 none; the tokens of a group also see each other both
         ways, past the window unless grp_windowed.  ktile: keys per entry, 64, or 32 for the head dim 512 kernel."""
+        host = _host_arrays(art, end, pos, grp)
+        return cls.compile([None if a is None else a.ctypes.data for a in host], len(host[0]), window, grp_windowed, ktile)
+
+    @classmethod
+    def compile(cls, at, n, window, grp_windowed, ktile) -> "TilePlan":
+        """build from the addresses of art, end, pos and grp (None: no groups), int32 [n] each"""
         lib = _lib.load_library()
-        art, end, pos, grp = _host_arrays(art, end, pos, grp)
-        n = len(art)
         w = int(window) if window else 0
         h = C.c_void_p()
-        mode = 0 if grp is None else 2 if grp_windowed else 1
-        _lib.check(lib.spinf_tileplan_build_ktile(art.ctypes.data, end.ctypes.data, pos.ctypes.data, None if grp is None else grp.ctypes.data, mode, n, w,
-                                                  int(ktile), C.byref(h)), "tileplan_build")
+        mode = 0 if at[3] is None else 2 if grp_windowed else 1
+        _lib.check(lib.spinf_tileplan_build_ktile(*at, mode, n, w, int(ktile), C.byref(h)), "tileplan_build")
         counts = (C.c_int64 * 5)()
         _lib.check(lib.spinf_tileplan_counts(h, counts), "tileplan_counts")
         return cls(h, counts, n, w, mode, int(ktile))
@@ -130,29 +133,36 @@ def _staging(n: int, device):
 
 
 def _mark(device):
-    """an event behind what the current stream of `device` has been given (None under capture: a graph's nodes are ordered by the graph)"""
+    """an event behind what the current stream of `device` has been given"""
     import torch
 
     with torch.cuda.device(device):
-        if torch.cuda.is_current_stream_capturing():
-            return None
         event = torch.cuda.Event()
         event.record()
         return event
 
 
-def _join(made, tensors, device) -> bool:
-    """the current stream of `device` waits for the event `made` (None: no wait) and is named to the allocator as a reader of the tensors;
-    False under capture, where neither can be done"""
+def _join(shared) -> bool:
+    """the current stream waits for what made these tensors and is named to the allocator as a reader; False under capture, where neither
+    can be done"""
     import torch
 
-    with torch.cuda.device(device):
+    with torch.cuda.device(shared.device):
         if torch.cuda.is_current_stream_capturing():
             return False
         stream = torch.cuda.current_stream()
-        if made is not None:
-            stream.wait_event(made)
-        for t in tensors:
+        if shared.made is not None:
+            stream.wait_event(shared.made)
+        elif shared.home is not None:
+            home = torch.cuda.ExternalStream(shared.home)
+            try:
+                with torch.cuda.stream(home):
+                    done = torch.cuda.is_current_stream_capturing()   # (torch waits for the device before a capture begins)
+                if not done:
+                    stream.wait_stream(home)
+            except RuntimeError:   # a stream of the caller's own that is gone by now
+                torch.cuda.synchronize()
+        for t in shared.tensors:
             t.record_stream(stream)
         return True
 
@@ -160,21 +170,25 @@ def _join(made, tensors, device) -> bool:
 class _Shared:
     """Device tensors that one stream made and calls on any stream may read.  Another stream's first call waits for what made them, and
     tells the allocator of its stream: a buffer that goes with the last reference is then not handed out while that stream
-    still reads it.  The caller cannot do either, as the buffers are made behind its back by whichever call comes first."""
+    still reads it.  The caller cannot do either, as the buffers are made behind its back by whichever call comes first.
 
-    __slots__ = ("tensors", "device", "made", "streams")
+    The wait is for the event `made` where there is one (TreeMask.prepare), else for all that the stream `home` has been given by then: an
+    event behind every upload cost a new stream's two masks 54 us, on a path where hardly any program needs it."""
+
+    __slots__ = ("tensors", "device", "home", "made", "streams")
 
     def __init__(self, *tensors, wait=True):
-        self.tensors, self.device = tensors, tensors[0].device
-        on = _lib.raw_stream(self.device)
-        self.made = _mark(self.device) if wait and on is not None else None
+        self.tensors, self.made = tensors, None
+        self.device = device = tensors[0].device
+        on = _lib.raw_stream(device.index)
+        self.home = on if wait else None
         self.streams = {on}
 
     def reach(self, stream) -> bool:
         """makes the tensors safe to read for the current stream (`stream`: its raw handle)"""
         if stream in self.streams:
             return True
-        if not _join(self.made, self.tensors, self.device):
+        if not _join(self):
             return False
         self.streams.add(stream)
         return True
@@ -184,11 +198,12 @@ class TreeMask:
     """Device-side handle: the stream's metadata, and per key-tile size a plan compiled when the first call that takes it comes (a
     forward's layers share it).  ``seq_lengths`` mirrors BlockMask.seq_lengths (spinf_serve/models/qwen35/qwen.py:615 reads it).
     Host threads and streams may share a mask: what a first call makes (plan, uploads, prepared calls) is made once, under a lock, and a
-    call on another stream waits for its copies.  (The metadata is copied at the build: as with any tensor, a stream that is to use
+    call on another stream waits for the copies.  (The metadata is copied at the build: as with any tensor, a stream that is to use
     the mask waits for the one it was built on.)"""
 
     def __init__(self, plan, meta, device, grp=None, host=None, window=None, ktile=64, lock=None):
-        """plan: a compiled plan, or None: compiled from host = (art, end, pos, grp or None, grp_windowed) for this window and ktile"""
+        """plan: a compiled plan, or None: compiled from host = (art, end, pos, grp or None, grp_windowed, the four arrays' addresses) for
+        this window and ktile"""
         self._lock = lock or threading.RLock()   # (one for both key-tile sizes: they refer to each other)
         self._host = host
         self._plan = plan
@@ -212,8 +227,7 @@ class TreeMask:
         if self._plan is None:
             with self._lock:
                 if self._plan is None:
-                    art, end, pos, grp, grp_windowed = self._host
-                    self._plan = TilePlan.build(art, end, pos, self.window, grp, grp_windowed, self._ktile)
+                    self._plan = TilePlan.compile(self._host[5], self.n, self.window, self._host[4], self._ktile)
         return self._plan
 
     @property
@@ -232,7 +246,7 @@ class TreeMask:
         if self._kv is None:
             self._schedule(1, 0)
         dev, at, shared = self._kv
-        shared.reach(_lib.raw_stream(self.device))
+        shared.reach(_lib.raw_stream(self.device.index))
         return dev[at[2] : at[3]], dev[at[3] : at[4]]
 
     def for_head_dim(self, d: int, ring: bool = False) -> "TreeMask":
@@ -260,9 +274,16 @@ class TreeMask:
         heads, head dim) per kind of layer, sidx as the calls will pass it.  For a program that builds its masks on a thread or a
         stream of its own: plans are compiled and uploaded there, what the compiler refuses is raised there, and a call on any
         stream waits for the uploads.  Without it the first call of a kind does it, on its thread and its stream."""
+        import torch
+
         from . import attention
 
-        attention.prepare_calls(self, heads, sidx)
+        shared = attention.prepare_calls(self, heads, sidx)
+        if self.device.type == "cuda" and not torch.cuda.is_current_stream_capturing():
+            event, here = _mark(self.device), _lib.raw_stream(self.device.index)
+            for x in shared:
+                if x.home == here:
+                    x.made = event
         return self
 
     def rows(self, sidx):
@@ -274,7 +295,7 @@ class TreeMask:
 
         got = self._rows   # (read once: another thread's rows may replace them)
         if got is not None and got[0] is sidx:
-            got[3].reach(_lib.raw_stream(self.device))
+            got[3].reach(_lib.raw_stream(self.device.index))
             return got[1], got[2]
         n = self.n
         row_of = torch.full((n + 63,), -1, dtype=torch.int32, device=self.device)   # padded: every key tile is 64 long
@@ -318,7 +339,7 @@ class TreeMask:
         """device copy of the work lists for this many head groups (built on first use, then kept); n_lists > 0: the static
         schedule for that many workgroups"""
         dev, at, n_items, shared = self._schedule(head_groups, n_lists)
-        shared.reach(_lib.raw_stream(self.device))
+        shared.reach(_lib.raw_stream(self.device.index))
         return dev[: at[1]].view(-1, 4), dev[at[1] : at[2]], n_items
 
     def pointers(self, head_groups: int, n_lists: int):
@@ -339,22 +360,25 @@ class TreeMask:
         if len(art) > 1 << 30:   # (what the plan compiler, which comes later, would refuse)
             raise ValueError(f"a stream of {len(art)} tokens is too long")
         host = _host_arrays(art, end, pos, grp)
-        n = len(host[0])
+        n, at = len(host[0]), [None] * 4
         given = [i for i in range(4) if host[i] is not None and not (grp_dev is not None if i == 3 else meta is not None)]
         shared = None
         if given:
             buf = _staging(len(given) * n, device).view(len(given), n)
-            rows = buf.numpy()
+            rows, base, host = buf.numpy(), buf.data_ptr(), list(host)
             for r, i in enumerate(given):
                 rows[r] = host[i]
-            host = tuple(rows[given.index(i)] if i in given else h for i, h in enumerate(host))   # (the caller may reuse its arrays)
+                host[i], at[i] = rows[r], base + 4 * n * r   # (the caller may reuse its arrays)
             dev = buf.to(device, non_blocking=True)
             shared = _Shared(dev, wait=False)
             if meta is None:
                 meta = tuple(dev[:3])
             if 3 in given:
                 grp_dev = dev[-1]
-        mask = cls(None, meta, device, grp_dev if grp is not None else None, (*host, grp_windowed), window)
+        for i, h in enumerate(host):
+            if h is not None and at[i] is None:
+                at[i] = h.ctypes.data
+        mask = cls(None, meta, device, grp_dev if grp is not None else None, (*host, grp_windowed, at), window)
         mask._meta = shared
         return mask
 

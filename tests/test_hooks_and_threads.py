@@ -219,7 +219,7 @@ def test_a_prepared_mask_leaves_nothing_to_its_first_calls(monkeypatch, compact)
         raise AssertionError("a prepared mask makes something at a call")
 
     with monkeypatch.context() as m:
-        m.setattr(sa.TilePlan, "build", more)
+        m.setattr(sa.TilePlan, "compile", more)
         m.setattr(sa.TreeMask, "_upload", more)
         m.setattr(masks, "_Shared", more)
         for hq, hkv, d in heads:
@@ -242,46 +242,42 @@ def test_a_stream_the_compiler_refuses_is_refused_at_the_build():
 def test_a_call_on_another_stream_waits_for_what_the_first_one_uploaded(monkeypatch):
     """a mask's schedules, entries and row maps are uploaded by whichever call comes first, on its stream: every other stream waits for
     the copy of each buffer it reads, once, and the allocator hears of it; the stream that copied does not wait"""
-    now, log, marks = ["a"], [], []
+    now, log = ["a"], []
 
-    def mark(device):
-        marks.append((len(marks), now[0]))
-        return marks[-1]
-
-    def join(made, tensors, device):
-        log.append((now[0], made, tuple(t.data_ptr() for t in tensors)))
+    def join(shared):
+        log.append((now[0], shared))
         return now[0] != "capture"
 
     monkeypatch.setattr(masks, "_static_lists", lambda device: 256)
-    monkeypatch.setattr(masks._lib, "raw_stream", lambda device: now[0])
-    monkeypatch.setattr(masks, "_mark", mark)
+    monkeypatch.setattr(masks._lib, "raw_stream", lambda index: now[0])
     monkeypatch.setattr(masks, "_join", join)
-    cpu, mask = torch.device("cpu"), _fresh_mask()   # built on "a": the metadata is there, and no event for it
+    cpu, mask = torch.device("cpu"), _fresh_mask()
 
     def call(stream, hq, sidx=None):
         now[0] = stream
         del log[:]
         layer = attention._Layer.of(mask, hq, 2, 256, 0, sidx is not None, cpu)
-        layer.reach(cpu)
+        if stream not in layer.streams:
+            layer.reach(stream)
         if sidx is not None:
             mask.rows(sidx)
-        return layer, [(s, made) for s, made, _ in log]
+        return layer, [(s, shared.home) for s, shared in log]
 
-    assert not marks
-    layer, seen = call("b", 4)                     # uploads entries and its schedule on b
-    assert marks == [(0, "b")] and seen == [("b", None)] and log[0][2][0] == mask.art.data_ptr()   # (the metadata: named to the allocator only)
+    # the metadata, built on "a", is the caller's to wait for, as any tensor: other streams are named to the allocator only
+    assert mask._meta.home is None and mask._meta.streams == {"a"} and mask._meta.tensors[0].data_ptr() == mask.art.data_ptr()
+    assert call("b", 4)[1] == [("b", None)]        # uploads entries and its schedule on b
     assert call("b", 4)[1] == []
-    _, seen = call("c", 8)                         # another geometry on c: its schedule on c, the entries are b's
-    assert marks[1:] == [(1, "c")] and seen == [("c", (0, "b")), ("c", None)]
+    assert call("c", 8)[1] == [("c", "b"), ("c", None)]        # another geometry on c: its schedule on c, the entries are b's
     assert call("c", 8)[1] == [] and call("c", 4)[1] == []     # (what b made has been waited for)
-    assert call("b", 8)[1] == [("b", (1, "c"))]
-    assert call("a", 4)[1] == [("a", (0, "b"))]
+    assert call("b", 8)[1] == [("b", "c")]
+    layer, seen = call("a", 4)
+    assert seen == [("a", "b")] and all(x.made is None for x in layer.shared)
     for _ in range(2):                             # nothing can be waited for under capture, and it is not taken for done
-        assert [s for s, _ in call("capture", 4)[1]] == ["capture"] * 3 and "capture" not in layer.streams
+        layer, seen = call("capture", 4)
+        assert [s for s, _ in seen] == ["capture"] * 3 and "capture" not in layer.streams
     sidx = torch.from_numpy(np.flatnonzero(mask.art.numpy() >= 0))
-    _, seen = call("b", 4, sidx)
-    assert marks[2:] == [(2, "b")] and seen == []
-    assert call("d", 4, sidx)[1] == [("d", (0, "b")), ("d", None), ("d", (2, "b"))]
+    assert call("b", 4, sidx)[1] == [] and mask._rows[3].home == "b"
+    assert call("d", 4, sidx)[1] == [("d", "b"), ("d", None), ("d", "b")]
 
 
 def test_c1_in_fp32_on_the_cpu_against_the_oracle():
@@ -504,16 +500,22 @@ def test_masks_prepared_on_a_thread_and_stream_of_their_own(dev):
     ref = sa.block_masks(b, sliding_window=100, device=dev)
     want = {name: sa.tree_attn(q, k, v, m, cfg.scale) for name, m in ref.items()}
     stream, made = torch.cuda.Stream(), {}
+    sidx = torch.from_numpy(np.flatnonzero(b.art >= 0)).to(dev)
+    compact = [x[sidx].contiguous() for x in (q, k, v)]
     torch.cuda.synchronize()
 
     def produce():
         with torch.cuda.device(dev), torch.cuda.stream(stream):
             torch.cuda._sleep(20_000_000)
             made.update({name: m.prepare((cfg.hq, cfg.hkv, cfg.d)) for name, m in sa.block_masks(b, sliding_window=100, device=dev).items()})
+            made["full_attention"].prepare((cfg.hq, cfg.hkv, cfg.d), sidx=sidx)
 
     t = threading.Thread(target=produce)
     t.start()
     t.join()
     got = {name: sa.tree_attn(q, k, v, m, cfg.scale) for name, m in made.items()}
+    rows = sa.tree_attn(*compact, made["full_attention"], cfg.scale, sidx=sidx)
+    assert all(x.made is not None for m in made.values() for x in (m.for_head_dim(cfg.d, ring=l.ring)._kv[2] for l in m._layers.values()))
     made.clear()
+    assert torch.equal(rows, want["full_attention"][sidx])
     assert all(torch.equal(got[name], want[name]) for name in want)
