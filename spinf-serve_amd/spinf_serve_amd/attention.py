@@ -191,9 +191,8 @@ class _Layer:
         a = self.args = _lib.AttnArgs()
         a.n, a.hq, a.hkv, a.d, a.window = m.n, hq, hkv, d, m.window
         a.art, a.end, a.pos = m.art.data_ptr(), m.end.data_ptr(), m.pos.data_ptr()
-        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items, self.shared = m.pointers(self.head_groups, n_lists)
-        if m._meta is not None:
-            self.shared += (m._meta,)
+        a.items, a.list_ptr, a.kv_idx, a.kv_bits, a.n_items, shared = m.pointers(self.head_groups, n_lists)
+        self.shared = shared + m._meta
         self.owned = (m.art, m.end, m.pos, m.grp)
         here = _lib.raw_stream(device.index)
         self.streams = {here} if all([here in x.streams for x in self.shared]) else set()   # those that may read the shared tensors

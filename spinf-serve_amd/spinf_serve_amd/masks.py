@@ -216,7 +216,7 @@ class TreeMask:
         self.seq_lengths = (self.n, self.n)
         self.art, self.end, self.pos = meta
         self.device = self.art.device       # (of "cuda" the GPU that was current at the build, whatever is current at the first call)
-        self._meta = None                   # art, end, pos, grp as shared tensors, where the build copied them
+        self._meta = ()                     # art, end, pos, grp as shared tensors, where a build copied them
         self._kv = None                     # the buffer with the device copies of the plan's kv_idx, kv_bits, and where they lie in it
         self._sched = {}
         self._layers = {}                   # prepared calls by head geometry (attention.py)
@@ -362,7 +362,7 @@ class TreeMask:
         host = _host_arrays(art, end, pos, grp)
         n, at = len(host[0]), [None] * 4
         given = [i for i in range(4) if host[i] is not None and not (grp_dev is not None if i == 3 else meta is not None)]
-        shared = None
+        shared = ()
         if given:
             buf = _staging(len(given) * n, device).view(len(given), n)
             rows, base, host = buf.numpy(), buf.data_ptr(), list(host)
@@ -370,7 +370,7 @@ class TreeMask:
                 rows[r] = host[i]
                 host[i], at[i] = rows[r], base + 4 * n * r   # (the caller may reuse its arrays)
             dev = buf.to(device, non_blocking=True)
-            shared = _Shared(dev, wait=False)
+            shared = (_Shared(dev, wait=False),)
             if meta is None:
                 meta = tuple(dev[:3])
             if 3 in given:
@@ -399,4 +399,5 @@ def block_masks(batch, sliding_window=None, device="cuda", grp=None, bidir_all=T
         slid._meta = full._meta
     else:
         slid = TreeMask.build(*full._host[:3], sliding_window, device, meta=meta, grp=grp, grp_windowed=True)
+        slid._meta += full._meta
     return {"full_attention": full, "sliding_attention": slid}

@@ -233,6 +233,20 @@ def test_a_prepared_mask_leaves_nothing_to_its_first_calls(monkeypatch, compact)
         mask.prepare((5, 2, 64))
 
 
+@pytest.mark.parametrize("bidir_all", [False, True])
+def test_every_buffer_of_a_mask_with_images_is_shared(monkeypatch, bidir_all):
+    """what the allocator is told of when another stream reads a mask: the metadata of the mask it shares it with among them"""
+    monkeypatch.setattr(masks, "_static_lists", lambda device: 256)
+    b = synth.attention_config("C2", contents=2).batches[0]
+    grp = np.where(np.arange(b.length) % 300 < 20, np.arange(b.length) // 300, -1)
+    for mask in sa.block_masks(b, sliding_window=100, device="cpu", grp=grp, bidir_all=bidir_all).values():
+        layer = attention._Layer.of(mask, 4, 2, 128, 0, False, torch.device("cpu"))
+        layer.owned = ()   # (the shared ones alone)
+        assert _owns_what_it_points_to(layer)
+        spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for x in layer.shared for t in x.tensors]
+        assert mask.grp is None or any(a <= layer.args.grp < a + n for a, n in spans)
+
+
 def test_a_stream_the_compiler_refuses_is_refused_at_the_build():
     long = np.broadcast_to(np.int32(0), ((1 << 30) + 1,))
     with pytest.raises(ValueError, match="too long"):
@@ -264,7 +278,8 @@ def test_a_call_on_another_stream_waits_for_what_the_first_one_uploaded(monkeypa
         return layer, [(s, shared.home) for s, shared in log]
 
     # the metadata, built on "a", is the caller's to wait for, as any tensor: other streams are named to the allocator only
-    assert mask._meta.home is None and mask._meta.streams == {"a"} and mask._meta.tensors[0].data_ptr() == mask.art.data_ptr()
+    meta, = mask._meta
+    assert meta.home is None and meta.streams == {"a"} and meta.tensors[0].data_ptr() == mask.art.data_ptr()
     assert call("b", 4)[1] == [("b", None)]        # uploads entries and its schedule on b
     assert call("b", 4)[1] == []
     assert call("c", 8)[1] == [("c", "b"), ("c", None)]        # another geometry on c: its schedule on c, the entries are b's
