@@ -43,7 +43,7 @@ class XCaches:
     beam: int = 6
     len_p: dict = field(default_factory=dict)   # by layer: [G] int32, entries of each group's prefix that can hold keys (set_lengths)
     len_t: Optional[torch.Tensor] = None        # [G] int32, the same for the template range
-    _spaces: dict = field(default_factory=dict)   # workspace of the split launches, by device
+    _spaces: dict = field(default_factory=dict)   # workspaces of the split launches, by device, each twice the one before
     _host_len: dict = field(default_factory=dict)   # by layer: (len_p, len_t) as host tuples (set_lengths)
     _plans: dict = field(default_factory=dict)      # split plans by geometry and lengths (plan_ragged)
     _calls: dict = field(default_factory=dict)      # prepared calls by layer and query shape (xdecode_attn)
@@ -66,10 +66,10 @@ class XCaches:
         self._calls.clear()
 
     def workspace(self, device, nbytes: int) -> torch.Tensor:
-        w = self._spaces.get(device)
-        if w is None or w.numel() < nbytes:
-            w = self._spaces[device] = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        return w
+        kept = self._spaces.setdefault(device, [])
+        if not kept or kept[-1].numel() < nbytes:   # (a smaller one stays: a step in a captured graph may still write to it)
+            kept.append(torch.empty(max(nbytes, 2 * kept[-1].numel() if kept else 0), dtype=torch.uint8, device=device))
+        return kept[-1]
 
 
 class GroupKV:

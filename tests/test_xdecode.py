@@ -214,6 +214,14 @@ def test_a_group_alone_or_among_others_bit_for_bit(dev, nsplit):
         assert torch.equal(alone[0], full[g])
 
 
+def test_a_workspace_that_grows_leaves_the_smaller_one_to_the_graphs_that_write_to_it():
+    c, cpu = decode.XCaches(), torch.device("cpu")
+    one = c.workspace(cpu, 100)
+    assert c.workspace(cpu, 60) is one
+    two = c.workspace(cpu, 101)
+    assert two is not one and two.numel() >= 200 and c.workspace(cpu, 100) is two and any(w is one for w in c._spaces[cpu])
+
+
 @pytest.mark.gpu
 def test_the_interface_callable_and_the_cache_update(dev):
     """GroupKV.update writes the step's K/V, x_attention reads the running decoder's caches (decode.py:51-104); steps 0, 1, 2 in a row"""
