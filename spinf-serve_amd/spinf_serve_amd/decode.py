@@ -228,7 +228,7 @@ def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None
         where = [t if t is None else (t.data_ptr(), t.shape, t.stride(), t.dtype) for t in tensors]
         got = c._calls.get(key)
         if got is not None and got[0] == where:
-            a = _lib.XdecArgs.from_buffer_copy(got[1])
+            a = _lib.XdecArgs.from_buffer_copy(got[1])   # (kept as bytes: the caches can be copied and saved)
             a.scale, a.window, a.softcap = scale, window, softcap
             return _xdecode_run(a, query, c.workspace(query.device, got[2]) if got[2] else None)
     per = 0
@@ -244,7 +244,7 @@ def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None
     work = c.workspace(query.device, nbytes) if nbytes else None
     if eager:
         a = _xdecode_args(query, *tensors, int(nsplit), int(per), int(c.beam))
-        c._calls[key] = (where, _lib.XdecArgs.from_buffer_copy(a), nbytes)
+        c._calls[key] = (where, bytes(a), nbytes)
         a.scale, a.window, a.softcap = scale, window, softcap
         return _xdecode_run(a, query, work)
     return _xdecode_op(query, *tensors, work, int(nsplit), int(per), int(c.beam), scale, window, softcap)

@@ -1,7 +1,9 @@
 """The extraction decoder's attention step (spinf_serve/decode.py:71-104): the numpy oracle against torch's SDPA and against the
 tree-attention oracle, the host side, and (gpu) the HIP kernel through the C ABI against the oracle."""
 
+import copy
 import ctypes as C
+import pickle
 
 import numpy as np
 import pytest
@@ -220,6 +222,18 @@ def test_a_workspace_that_grows_leaves_the_smaller_one_to_the_graphs_that_write_
     assert c.workspace(cpu, 60) is one
     two = c.workspace(cpu, 101)
     assert two is not one and two.numel() >= 200 and c.workspace(cpu, 100) is two and any(w is one for w in c._spaces[cpu])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("how", [copy.deepcopy, lambda c: pickle.loads(pickle.dumps(c))])
+def test_caches_are_copied_and_saved_after_a_step(dev, how):
+    """a used decoder's caches: the copy's next step reads its own tensors"""
+    q, c = synth.xdecode_case(2, 8, 4, 128, 2, 6, 4, (40, 80), (3, 6), None, 2, seed=9, device=dev)
+    want = sa.xdecode_attn(q, c, 0, 0.09)
+    mine = how(c)
+    for t in (*c.kp.values(), *c.gk.values(), *c.vt.values()):
+        t.zero_()
+    assert torch.equal(sa.xdecode_attn(q, mine, 0, 0.09), want) and not torch.equal(sa.xdecode_attn(q, c, 0, 0.09), want)
 
 
 @pytest.mark.gpu
