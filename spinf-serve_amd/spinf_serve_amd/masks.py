@@ -222,6 +222,13 @@ class TreeMask:
         self._layers = {}                   # prepared calls by head geometry (attention.py)
         self._rows = None
 
+    def __reduce__(self):
+        """copied and saved as what it is built from: plans and uploads belong to one object"""
+        if self._host is None:
+            raise TypeError("a mask around a compiled plan cannot be copied or saved")
+        art, end, pos, grp, grp_windowed, _ = self._host
+        return _built, (art, end, pos, self.window, str(self.device), grp, grp_windowed, self._ktile)
+
     @property
     def plan(self) -> TilePlan:
         if self._plan is None:
@@ -381,6 +388,12 @@ class TreeMask:
         mask = cls(None, meta, device, grp_dev if grp is not None else None, (*host, grp_windowed, at), window)
         mask._meta = shared
         return mask
+
+
+def _built(art, end, pos, window, device, grp, grp_windowed, ktile):
+    mask = TreeMask.build(art, end, pos, window, device, grp=grp, grp_windowed=grp_windowed)
+    mask._ktile = ktile
+    return mask
 
 
 def block_masks(batch, sliding_window=None, device="cuda", grp=None, bidir_all=True):

@@ -3,7 +3,9 @@ recurrent-layer interfaces (spinf_serve/models/gemma4.py:98-119, spinf_serve/mod
 with transformers (gemma4.py:121-122), the plan compilers under threads, and the CPU baseline's fp32 arithmetic against the
 float64 oracle."""
 
+import copy
 import gc
+import pickle
 import sys
 import threading
 import types
@@ -245,6 +247,20 @@ def test_every_buffer_of_a_mask_with_images_is_shared(monkeypatch, bidir_all):
         assert _owns_what_it_points_to(layer)
         spans = [(t.untyped_storage().data_ptr(), t.untyped_storage().nbytes()) for x in layer.shared for t in x.tensors]
         assert mask.grp is None or any(a <= layer.args.grp < a + n for a, n in spans)
+
+
+@pytest.mark.parametrize("how", [copy.copy, copy.deepcopy, lambda m: pickle.loads(pickle.dumps(m))])
+def test_masks_are_copied_and_saved(how):
+    b = synth.attention_config("C2", contents=2).batches[0]
+    grp = np.where(np.arange(b.length) % 300 < 20, np.arange(b.length) // 300, -1)
+    for mask in sa.block_masks(b, sliding_window=100, device="cpu", grp=grp, bidir_all=False).values():
+        for used in (False, True):
+            for m in (mask, mask.for_head_dim(512)):
+                if used:
+                    m.kv_idx
+                mine = how(m)
+                assert (mine.window, mine.grp_mode, mine.n, mine._ktile) == (m.window, m.grp_mode, m.n, m._ktile) and torch.equal(mine.art, m.art)
+                assert torch.equal(mine.kv_idx, m.kv_idx) and torch.equal(mine.kv_bits, m.kv_bits) and mine.kv_idx.data_ptr() != m.kv_idx.data_ptr()
 
 
 def test_a_stream_the_compiler_refuses_is_refused_at_the_build():
