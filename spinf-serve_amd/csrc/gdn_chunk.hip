@@ -174,7 +174,7 @@ __device__ __forceinline__ void gdn_wy_body(const GdnParams& p) {
             Rs[lane] = pr32;
         }
     };
-    auto solve = [&]() __attribute__((always_inline)) { solve_tile<SOLVER || !TIGHT>(As, Bs, Ts, Xs, Tus, c, q4, run_mode); };   // (a pair's tiles are different segments)
+    auto solve = [&]() __attribute__((always_inline)) { solve_tile<SOLVER || !TIGHT, false>(As, Bs, Ts, Xs, Tus, c, q4, run_mode); };   // (a pair's tiles are different segments)
     if (SOLVER && w == 4) {
         fetch_gate_row(0);
         fetch_gates();

@@ -24,7 +24,7 @@
 // What is not finite in one option must not reach the others of its blocks, as every product above meets it with a coefficient of zero.
 // The entries of A, beta and g are cleared where they are computed or staged, and their token noted; V' is looked at (a product with zeros) and, where it is not finite, computed again with such entries of V + R cleared.  Noted tokens and all below them come out
 // as NaN, per value column; a stack row carries its note in a bit mask beside V'.  Outputs of all other tokens keep their bits.  The look
-// costs 1 % of a layer over a stream of tries (409 -> 413 us).
+// costs 2 % of a layer's scans over a stream of tries (203.8 -> 208.2 us), 1 % of the layer.
 //
 // What it measured (the stream above, 10.6 k tokens in tries, 32 value heads): 167 us in one launch for 0.70 ms in six; 0.4 GB of rows
 // and states, 2.5 TB/s.  Bound by a block's chain of phases: 11 k clocks, of them 2.7 k the solve on wave 0, 1.6 k A and P, 1.25 k staging
@@ -155,15 +155,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         if (tid < CH) {
             const bool odd = not_finite(pg) || not_finite(pbeta);
             const unsigned long odds = __builtin_amdgcn_ballot_w64(odd);
-            int at = tid;                  // (addresses are computed here, as further down: kept in registers they would push others out)
-            asm volatile("" : "+v"(at));
-            if (at == 0) odd_rows = (unsigned)odds;
-            Gr[at] = odd ? 0.f : pg;
-            Bs[at] = odd ? 0.f : (float)pbeta;
-            Rs[at] = pr;
-            Ms[at] = pm;
-            Ns[at] = pn;
-            Ds[at] = (pn >> 8) & 0xff;
+            if (tid == 0) odd_rows = (unsigned)odds;
+            Gr[tid] = odd ? 0.f : pg;
+            Bs[tid] = odd ? 0.f : (float)pbeta;
+            Rs[tid] = pr;
+            Ms[tid] = pm;
+            Ns[tid] = pn;
+            Ds[tid] = (pn >> 8) & 0xff;
         }
         {
             const int col = (tid & 15) * 8;
@@ -177,7 +175,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         }
         if (w == 0) {    // G: the path's sum so far and the tokens above in this block; lanes 0..31 add rows 0..15, the others 16..31
             wave_lds_order();
-            int at = lane;
+            int at = lane;                 // (addresses are computed here, as further down: kept in registers they would push others out)
             asm volatile("" : "+v"(at));
             const int row = at & 31, half = at >> 5;
             const int above = (Ms[row] | (int)(1u << row)) >> (16 * half);
@@ -263,7 +261,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         lds_barrier();
 
         // ---- T diag(beta) on wave 0, while the other waves go on with their columns
-        if (w == 0) solve_tile<true>(As, Bs, Ts, Xs, Tus, c, q4, false);
+        if (w == 0) solve_tile<true, true>(As, Bs, Ts, Xs, Tus, c, q4, false);
         // Block j + 1 is requested here, behind the solve, which needs the registers; it has the rest of this block to arrive.
         fetch_data();
         fetch_rows(j + 2);

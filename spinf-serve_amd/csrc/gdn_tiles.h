@@ -130,8 +130,9 @@ constexpr int LO = 32 + 4;     // row stride (elements) of a wave's transposed o
 // (T_lo^T = T_00^T (A_lo^T T_11^T)) so that the lane again holds a row; apart: the two tiles do not see each other, T_lo = 0.  Leaves
 // T diag(beta) in Tus as bf16, tile by tile.  Ts (T_00 in rows 0..15, T_11 in 16..31) and Xs are scratch.  The others wait for this
 // wave: it goes first.  c = lane % 16, q4 = lane / 16; by reference, which leaves their reading where the kernels' own code would (by value
-// the kernels of 168 registers spill).
-template <bool PRELOAD>
+// the kernels of 168 registers spill).  MERGE_FIRST: the diagonal blocks are stored behind T_lo (the forest kernel: a layer's scans
+// 210.4 -> 209.5 us over a stream of tries; the chunk kernels lose 0.5 - 1 % that way).
+template <bool PRELOAD, bool MERGE_FIRST>
 __device__ __forceinline__ void solve_tile(const float* As, const float* Bs, float* Ts, float* Xs, __bf16* Tus, const int& c, const int& q4, const bool& apart) {
     __builtin_amdgcn_s_setprio(3);
     float t[16];
@@ -144,8 +145,10 @@ __device__ __forceinline__ void solve_tile(const float* As, const float* Bs, flo
     const float* T1s = Ts + 16 * LX;
     const f32x4 B0 = *(const f32x4*)(Bs + 4 * q4), B1 = *(const f32x4*)(Bs + 16 + 4 * q4);
     const f32x4 t00 = *(const f32x4*)(Ts + c * LX + 4 * q4), t11 = *(const f32x4*)(T1s + c * LX + 4 * q4);
-    *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
-    *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
+    if (!MERGE_FIRST) {
+        *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
+        *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
+    }
     f32x4 tlo = zero4();
     if (!apart) {
         f32x4 x = zero4();
@@ -158,6 +161,10 @@ __device__ __forceinline__ void solve_tile(const float* As, const float* Bs, flo
 #pragma unroll
         for (int s4 = 0; s4 < 4; s4++)        // T_lo[16 + i][j'] = sum_j T_00[j][j'] X[j][i]
             tlo = mfma4(Ts[(4 * s4 + q4) * LX + c], Xs[(4 * s4 + q4) * LX + c], tlo);
+    }
+    if (MERGE_FIRST) {
+        *(bf16x4*)(Tus + c * LP + 4 * q4) = round4(t00 * B0);
+        *(bf16x4*)(Tus + (16 + c) * LP + 16 + 4 * q4) = round4(t11 * B1);
     }
     *(bf16x4*)(Tus + (16 + c) * LP + 4 * q4) = round4(tlo * B0);
     __builtin_amdgcn_s_setprio(0);
