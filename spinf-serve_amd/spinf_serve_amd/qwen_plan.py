@@ -189,6 +189,7 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
     # a forest's nodes leave no states (and its kernel is built for 128 value dims): a caller that asks for states gets every level's
     launches = plan.launches if wanted or plan.program is None or v.shape[-1] != 128 else plan.program
     base = plan.data.data_ptr() if args is not None else 0
+    run, stream = _lib.load_library().spinf_gdn_fwd, _lib.raw_stream(q.device.index)
     above = None   # the states the level above left
     for d, calls in enumerate(plan.levels):
         if args is not None and launches is plan.program:
@@ -203,7 +204,7 @@ def gdn_tree(q, k, v, g, beta, plan: TreePlan, mod=None):
                 args.cu, args.idx = base + 8 * cu, base + 8 * idx
                 args.h0, args.h0_idx = (h0, base + 8 * h0_idx) if h0_idx >= 0 else (None, None)
                 args.ht, args.ht_idx = (ht, base + 8 * ht_idx) if ht_idx >= 0 else (None, None)
-                _lib.launch(_lib.load_library().spinf_gdn_fwd, args, q.device, "spinf_gdn_fwd")
+                _lib.launch(run, args, q.device, "spinf_gdn_fwd", stream)
             calls = ()
         for c in calls:
             n_seg = len(c.cu_cpu) - 1
