@@ -15,6 +15,7 @@
 #include "gdn_forest.h"
 
 #include <algorithm>
+#include <exception>
 #include <cstring>
 #include <new>
 #include <vector>
@@ -196,6 +197,7 @@ extern "C" int spinf_gdn_plan_build(const int64_t* prev, const uint8_t* real, in
     if (n < 0 || (n > 0 && (!prev || !real))) return spinf_fail(SPINF_E_ARG, "gdn_plan_build: null stream arrays");
     if (path != 0 && path != 1) return spinf_fail(SPINF_E_ARG, "gdn_plan_build: unknown path %d (0 indexed, 1 levels)", path);
     if (n_keep < 0 || (n_keep > 0 && !keep)) return spinf_fail(SPINF_E_ARG, "gdn_plan_build: null keep list");
+    if (rows > INT32_MAX) return spinf_fail(SPINF_E_ARG, "gdn_plan_build: %lld compact rows (row indices are below 2^31)", (long long)rows);
     if (path == 1 && max_init <= 0) return spinf_fail(SPINF_E_ARG, "gdn_plan_build: max_init must be positive");
     for (int64_t i = 0; i < n; i++)
         if (prev[i] >= i || prev[i] < -1) return spinf_fail(SPINF_E_ARG, "gdn_plan_build: prev[%lld] = %lld does not point backwards", (long long)i, (long long)prev[i]);
@@ -228,7 +230,7 @@ extern "C" int spinf_gdn_plan_build(const int64_t* prev, const uint8_t* real, in
         for (int64_t i = 0; i < n; i++) {
             if (!real[i]) continue;
             const int64_t b = prev[i];
-            const bool opens = b < 0 || b != i - 1 || kids[b] > 1;
+            const bool opens = b < 0 || b != i - 1 || kids[b] > 1 || !real[b];   // (a pad is in no segment)
             if (opens) {
                 Seg s;
                 s.first = i;
@@ -358,7 +360,7 @@ extern "C" int spinf_gdn_plan_build(const int64_t* prev, const uint8_t* real, in
         p->seg_of_row.assign((size_t)p->conv_rows, -1);
         for (int64_t i = 0; i < n; i++)
             if (real[i]) p->seg_of_row[row(i)] = seg_at[i];
-    } catch (const std::bad_alloc&) {
+    } catch (const std::exception&) {
         delete p;
         return spinf_fail(SPINF_E_NOMEM, "gdn_plan_build: out of memory");
     }

@@ -6,6 +6,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <exception>
 #include <cstring>
 #include <functional>
 #include <new>
@@ -234,7 +235,7 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
             std::stable_sort(p->order.begin() + a, p->order.begin() + b, [&](int32_t x, int32_t y) { return weight[x] > weight[y]; });
             a = b;
         }
-    } catch (const std::bad_alloc&) {
+    } catch (const std::exception&) {
         delete p;
         return spinf_fail(SPINF_E_NOMEM, "tileplan_build: out of memory");
     }
@@ -332,7 +333,7 @@ extern "C" int spinf_tileplan_schedule(const spinf_tileplan* p, int32_t head_gro
             for (int64_t j = n_tail - 1; j >= 0; j--) tmp.insert(tmp.end(), items + 4 * (int64_t)idx[j], items + 4 * (int64_t)idx[j] + 4);
             std::memcpy(items + 4 * lo, tmp.data(), tmp.size() * sizeof(int32_t));
         }
-    } catch (const std::bad_alloc&) {
+    } catch (const std::exception&) {
         return spinf_fail(SPINF_E_NOMEM, "tileplan_schedule: out of memory");
     }
     return SPINF_OK;
@@ -391,7 +392,7 @@ extern "C" int spinf_tileplan_schedule_static(const spinf_tileplan* p, int32_t h
         std::vector<int32_t> fill(list_ptr, list_ptr + n_lists);
         for (int l = 0; l < 8; l++)
             for (int64_t i = lp[l]; i < lp[l + 1]; i++) std::memcpy(items + 4 * (int64_t)fill[owner[i]]++, base.data() + 4 * i, 4 * sizeof(int32_t));
-    } catch (const std::bad_alloc&) {
+    } catch (const std::exception&) {
         return spinf_fail(SPINF_E_NOMEM, "tileplan_schedule_static: out of memory");
     }
     return SPINF_OK;

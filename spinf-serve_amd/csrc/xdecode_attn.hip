@@ -30,6 +30,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <exception>
 #include <functional>
 #include <new>
 #include <vector>
@@ -602,7 +603,7 @@ extern "C" int spinf_xdecode_plan_ragged(const spinf_xdec_args* a, const int32_t
             const double est = std::max(end, (bytes + part_bytes) / BYTES_PER_US) + (part_bytes > 0 ? COMBINE + part_bytes / MERGE_BYTES_PER_US : 0);
             if (best < 0 || est < best) { best = est; *tiles_per_split = per; }
         }
-    } catch (const std::bad_alloc&) {
+    } catch (const std::exception&) {
         return spinf_fail(SPINF_E_NOMEM, "xdecode_plan_ragged: out of memory");
     }
     *nsplit = (nt_max + *tiles_per_split - 1) / *tiles_per_split;

@@ -710,6 +710,12 @@ def test_gdn_plan_compiler_edge_cases():
     assert lib.spinf_gdn_plan_build(prev.ctypes.data, real.ctypes.data, 3, 0, 64, 8192, 96, -1, None, 0, C.byref(handle)) == -1
     assert b"does not point backwards" in lib.spinf_last_error()
     prev = np.array([-1, 0, 1], np.int64)
+    for rows in (1 << 31, 1 << 61, 1 << 62):   # (four taps a row: the last one's table would be of size 0)
+        assert lib.spinf_gdn_plan_build(prev.ctypes.data, real.ctypes.data, 3, 0, 64, 8192, 96, rows, None, 0, C.byref(handle)) == -1
+        assert b"compact rows" in lib.spinf_last_error()
+    after_pad = sa.tree_plan(np.array([-1, 0, 1]), np.array([False, True, True]), "cpu")   # a token behind a pad starts a path
+    assert after_pad.n_segments == 1 and after_pad.levels[0][0].idx.tolist() == [1, 2] and after_pad.levels[0][0].h0_idx is None
+    prev = np.array([-1, 0, 1], np.int64)
     assert lib.spinf_gdn_plan_build(prev.ctypes.data, real.ctypes.data, 3, 7, 64, 8192, 96, -1, None, 0, C.byref(handle)) == -1
     assert lib.spinf_gdn_plan_build(prev.ctypes.data, real.ctypes.data, 3, 0, 64, 8192, 96, 2, None, 0, C.byref(handle)) == -1
     assert b"compact rows" in lib.spinf_last_error()
