@@ -297,11 +297,12 @@ class TreeMask:
         """compact rows (spinf_serve/models/qwen35/qwen.py:613-622): sidx [R] = stream position of each real row (a device
         tensor) -> (row_of [n], kv_row0 [entries]) int32 device tensors for the kernel: the row of each stream position (-1:
         pad) and, per plan entry, the row of its first key where its 64 keys are consecutive rows (else -1).  Kept for the
-        sidx tensor it was built from (one forward: every layer passes the same tensor)."""
+        sidx tensor it was built from, as it was then (one forward: every layer passes the same tensor)."""
         import torch
 
+        version = 0 if sidx.is_inference() else sidx._version   # (counts changes in place; tensors of inference mode keep none)
         got = self._rows   # (read once: another thread's rows may replace them)
-        if got is not None and got[0] is sidx:
+        if got is not None and got[0] is sidx and got[4] == version:
             got[3].reach(_lib.raw_stream(self.device.index))
             return got[1], got[2]
         n = self.n
@@ -313,7 +314,7 @@ class TreeMask:
         tile_row0 = torch.where((tiles[:, 0] >= 0) & run.all(1), tiles[:, 0], torch.full_like(tiles[:, 0], -1))
         kv_row0 = tile_row0[self.kv_idx.long()].contiguous()
         row_of = row_of[:n].contiguous()
-        self._rows = (sidx, row_of, kv_row0, _Shared(row_of, kv_row0))
+        self._rows = (sidx, row_of, kv_row0, _Shared(row_of, kv_row0), version)
         return row_of, kv_row0
 
     def _upload(self, head_groups: int, n_lists: int):

@@ -263,6 +263,20 @@ def test_masks_are_copied_and_saved(how):
                 assert torch.equal(mine.kv_idx, m.kv_idx) and torch.equal(mine.kv_bits, m.kv_bits) and mine.kv_idx.data_ptr() != m.kv_idx.data_ptr()
 
 
+def test_a_row_map_follows_its_row_list():
+    """kept for the tensor it was built from, and built again when that tensor was changed in place"""
+    mask = _fresh_mask()
+    sidx = torch.from_numpy(np.flatnonzero(mask.art.numpy() >= 0).copy())
+    one = mask.rows(sidx)
+    assert mask.rows(sidx)[0] is one[0]
+    sidx[:64] = sidx[:64].flip(0)
+    two = mask.rows(sidx)
+    assert two[0] is not one[0] and torch.equal(two[0][sidx], torch.arange(len(sidx), dtype=torch.int32))
+    with torch.inference_mode():
+        other = sidx + 0
+    assert mask.rows(other)[0] is mask.rows(other)[0]
+
+
 def test_a_stream_the_compiler_refuses_is_refused_at_the_build():
     long = np.broadcast_to(np.int32(0), ((1 << 30) + 1,))
     with pytest.raises(ValueError, match="too long"):
