@@ -257,7 +257,7 @@ def _heads_first(q, k, v, mask, scale, sidx):
         return None
     one, hq, rows, d = q.shape
     ks, dev = k.shape, q.device
-    if not (one == 1 and len(ks) == 4 and ks[0] == 1 and ks[2] == rows and ks[3] == d and v.shape == ks and hq % ks[1] == 0
+    if not (one == 1 and len(ks) == 4 and ks[0] == 1 and ks[2] == rows and ks[3] == d and v.shape == ks and ks[1] > 0 and hq % ks[1] == 0
             and k.device == dev and v.device == dev and mask.art.device == dev and dev.type == "cuda"):
         return None
     qs, kst, vs = q.stride(), k.stride(), v.stride()

@@ -564,3 +564,26 @@ def test_masks_prepared_on_a_thread_and_stream_of_their_own(dev):
     made.clear()
     assert torch.equal(rows, want["full_attention"][sidx])
     assert all(torch.equal(got[name], want[name]) for name in want)
+
+
+@pytest.mark.gpu
+def test_the_model_layers_layout_refuses_what_the_general_path_refuses(dev):
+    """tree_flex_forward and tree_attention take plain calls past the general path's checks: every refused form still ends there, and
+    every accepted stride gives its bits"""
+    cfg = synth.attention_config("C2", contents=1)
+    b = cfg.batches[0]
+    n, mask = b.length, sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
+    q, k, v = (t.transpose(0, 1)[None] for t in synth.qkv(cfg, b, seed=1, device=dev))
+    want = sa.tree_attn(*(t[0].transpose(0, 1) for t in (q, k, v)), mask, cfg.scale)
+    wide = torch.zeros(1, cfg.hkv, n, 2 * cfg.d, dtype=torch.bfloat16, device=dev)
+    wide[..., : cfg.d] = v
+    for qq, kk, vv in ((q, k, v), (q.contiguous(), k.contiguous(), v.contiguous()), (q, k.contiguous(), wide[..., : cfg.d])):
+        assert torch.equal(sa.tree_flex_forward(None, qq, kk, vv, mask, cfg.scale)[0][0], want)
+        assert torch.equal(sa.tree_attention(qq, kk, vv, mask, cfg.scale)[0].transpose(0, 1), want)
+    bad = [(q, k[:, :0], v[:, :0]), (q, k[:, :, :-1], v), (q, k, v[:, :1]), (q[..., :-1], k, v), (q[:, :3], k, v), (q.float(), k, v), (q, k, v.half()),
+           (q[:, :, :-128], k[:, :, :-128], v[:, :, :-128]), (q[..., ::2], k[..., ::2], v[..., ::2]), (q, k.cpu(), v)]
+    for i, args in enumerate(bad):
+        for call in (lambda *a: sa.tree_flex_forward(None, *a, mask, cfg.scale), lambda *a: sa.tree_attention(*a, mask, cfg.scale)):
+            with pytest.raises((ValueError, RuntimeError)):
+                call(*args)
+                pytest.fail(f"case {i} was taken")
