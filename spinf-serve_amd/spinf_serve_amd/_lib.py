@@ -199,10 +199,13 @@ def eager(first, *tensors) -> bool:
     """May this call go straight to the library?  Yes for plain tensors on a GPU (of ``first``; a launch compares the others with it) that
     nothing watches and autograd does not record; anything else takes the registered torch.library operator, which costs 15 - 25 us
     of host time per call more."""
-    if watched() or not first.is_cuda:
+    if (_compiling() or _dispatch_modes() or _tracing() or _functorch_level() is not None or forward_ad._current_level >= 0   # (watched(), in place)
+            or _function_modes() and watched() or not first.is_cuda or type(first) not in _KINDS):
         return False
     grad = _grad_enabled()
-    for t in (first, *tensors):
+    if grad and first.requires_grad:
+        return False
+    for t in tensors:
         if t is not None and (type(t) not in _KINDS or (grad and t.requires_grad)):
             return False
     return True
