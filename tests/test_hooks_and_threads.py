@@ -495,7 +495,8 @@ def test_tensors_of_another_device_are_refused_before_any_launch(dev, call):
 
 
 @pytest.mark.gpu
-def test_layers_of_one_mask_on_two_streams(dev):
+@pytest.mark.parametrize("default", [False, True])
+def test_layers_of_one_mask_on_two_streams(dev, default):
     """the first call's stream is busy, so its uploads are late; a call on another stream gives the bits of one that has waited for
     everything, and what it reads is not handed out again when the mask goes while it is still to run"""
     cfg = synth.attention_config("C2", contents=2)
@@ -504,7 +505,7 @@ def test_layers_of_one_mask_on_two_streams(dev):
     few = [t[:, :n].contiguous() for t, n in ((q, 8), (k, 4), (v, 4))]
     ref = sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
     want = [sa.tree_attn(q, k, v, ref, cfg.scale), sa.tree_attn(*few, ref, cfg.scale)]
-    streams = [torch.cuda.Stream() for _ in range(2)]
+    streams = [torch.cuda.default_stream() if default else torch.cuda.Stream(), torch.cuda.Stream()]
     mask = sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
     torch.cuda.synchronize()
     with torch.cuda.stream(streams[0]):
