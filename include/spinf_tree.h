@@ -111,7 +111,9 @@ typedef struct spinf_attn_args {
                           no compact rows); 3 = the kernel with decoupled waves at head dim 128 (items as for 0; needs an even
                           group, a static schedule (n_lists > 0) over 64-key entries, the stream layout, no image groups); 4 = the kernel
                           that spreads a 32-row group over a workgroup, for short streams (n_lists 0, no image groups; items of two heads
-                          where a group has an even number, at every head dim; plan entries of 64 or 32 keys) */
+                          where a group has an even number, at every head dim; plan entries of 64 or 32 keys); 5 = the pipelined kernel
+                          in place of the kernel with decoupled waves at head dim 512 (a static schedule over 32-key entries, the stream
+                          layout, no window; where it does not take the call, the kernel with decoupled waves does) */
     const int32_t* row_of; const int32_t* kv_row0;
     const int32_t* grp; int32_t grp_mode;   /* image groups, as given to spinf_tileplan_build_groups (device copy of grp), or NULL */
     int32_t ktile;                          /* keys per plan entry: 0 or 64; 32 with d = 512, and with a static schedule */

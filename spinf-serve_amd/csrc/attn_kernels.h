@@ -194,5 +194,8 @@ __device__ __forceinline__ int fresh_lane_id() {
 // tree_attn_ring.hip: the pass with decoupled waves over a static schedule (p.list_ptr delimits n_wg item lists, one per
 // workgroup; plan entries of 32 keys), the exact recomputation of the items that need it included.  Stream-ordered launch on `stream`.
 int spinf_launch_ring(const AttnParams& p, int d, bool win, int n_wg, hipStream_t stream);
+// tree_attn_pipe.hip: head dim 512 without a window, over the ring kernel's schedule; strides of k and v below PIPE_MAX_STRIDE elements.
+constexpr long PIPE_MAX_STRIDE = 1 << 26;   // (a wave's eight rows are reached by 32-bit byte offsets)
+int spinf_launch_pipe(const AttnParams& p, int n_wg, hipStream_t stream);
 // tree_attn_spread.hip: a workgroup per 32-row group and `heads` heads over the eight lists of a schedule with that many heads per item.
 int spinf_launch_spread(const AttnParams& p, int d, int heads, bool win, int ktile, long n_items, hipStream_t stream);

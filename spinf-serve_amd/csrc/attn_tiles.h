@@ -63,4 +63,9 @@ __device__ __forceinline__ void dma4_lane(const int* addr, unsigned lds) {
     lds = __builtin_amdgcn_readfirstlane(lds);
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(addr), "s"(lds) : "memory", "m0");
 }
+__device__ __forceinline__ void dma4_uniform(const char* base, unsigned lane_off, unsigned lds) {   // base is wave-uniform
+    base = uniform_ptr(base);
+    lds = __builtin_amdgcn_readfirstlane(lds);
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %1, %0" ::"s"(base), "v"(lane_off), "s"(lds) : "memory", "m0");
+}
 __device__ __forceinline__ unsigned lds_addr(const void* p) { return (unsigned)(size_t)(const __attribute__((address_space(3))) char*)p; }

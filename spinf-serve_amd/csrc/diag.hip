@@ -45,10 +45,10 @@ __global__ __launch_bounds__(512) void mfma_rate_kernel(const long iters, float*
 // instructions that depend on nothing the MFMA touches: v_fma_f32 (KIND 0) or v_exp_f32 (KIND 1) }, with one, two or four waves per
 // SIMD (KIND 2: rounds shaped like a 32 x 32 attention block at head dim 128: 8 chained MFMAs, 3 NV v_fma_f32 + NV v_exp_f32, 8 MFMAs
 // on four accumulators).  Every wave of workgroup 0 records the clock before and after its loop (s_memtime ticks, which count core clocks here: the bare
-// MFMA chain reads 32.3 per MFMA).  If the vector instructions ran under the MFMA a wave would need max(36, 4 + 4 NV) clocks per round;
-// measured on MI355X it needs 36 + 4 NV (8 NV for v_exp_f32): they do not, the two add up, and only ANOTHER wave of the SIMD can use
-// the vector ALU while an MFMA runs.  This is what bounds the attention kernels at head dim 128, where a 32 x 32 block is 16 MFMAs
-// (512 clocks) and about as many clocks of softmax per wave.
+// MFMA chain reads 32.3 per MFMA).  A round is an iteration of the loop and has the loop's branch in it: one wave per SIMD takes ~44 + 4 NV clocks per
+// round here, but 32.8 with 4 and 35.5 with 6 v_fma_f32 per MFMA when 16 rounds are unrolled into an iteration.  So a wave's vector
+// instructions do run under its own MFMAs, a branch does not; with two waves per SIMD the other wave covers the branch.  Beyond ~6
+// vector instructions per MFMA the vector ALU's issue port is the bound, which is where the attention kernels are at head dim 128.
 template <int NV, int KIND>
 __global__ __launch_bounds__(1024) void mfma_valu_kernel(const int iters, long long* out) {
     bf16x8 a, b;

@@ -774,12 +774,15 @@ int launch_512(const AttnParams& p, int blocks, hipStream_t s) {
 
 // The ring kernel (tree_attn_ring.hip) over a static schedule: one launch.  It takes no item from a shared list and recomputes
 // the items that need the exact arithmetic itself, so the call uses none of the block's cursors and no second kernel.
-int launch_ring(const AttnParams& p, int d, bool win, int n_wg, hipStream_t stream) {
+// With `pipe` the pipelined kernel (tree_attn_pipe.hip) in its place where it takes the call: same schedule, same bits.
+int launch_ring(const AttnParams& p, int d, bool win, bool pipe, int n_wg, hipStream_t stream) {
     if (p.clear_first) {
         hipLaunchKernelGGL(attn_clear_counters_kernel, dim3(1), dim3(64), 0, stream, p.counters);
         hipError_t e0 = hipGetLastError();
         if (e0 != hipSuccess) return spinf_fail(SPINF_E_HIP, "tree_attn: launch (clear): %s", hipGetErrorString(e0));
     }
+    const bool near = p.k_tok >= 0 && p.k_tok < PIPE_MAX_STRIDE && p.v_tok >= 0 && p.v_tok < PIPE_MAX_STRIDE;
+    if (pipe && d == 512 && !win && near) return spinf_launch_pipe(p, n_wg, stream);
     return spinf_launch_ring(p, d, win, n_wg, stream);
 }
 
@@ -938,7 +941,7 @@ static int attn_fwd(const spinf_attn_args* a, void* stream, bool no_alloc) {
     const int blocks = a->n_lists > 0 ? a->n_lists : (int)(a->n_items < cus ? a->n_items : cus);
     const bool win = p.window > 0;
     int rc;
-    if (ring) rc = launch_ring(p, a->d, win, a->n_lists, s);
+    if (ring) rc = launch_ring(p, a->d, win, a->variant == 5, a->n_lists, s);
     else if (spread) rc = launch_spread(p, a->d, hpi, win, a->ktile ? a->ktile : 64, (long)a->n_items, s);
     else switch (a->d) {
         case 64: rc = launch_d<64>(p, rt, nhw, win, a->grp_mode, blocks, s); break;

@@ -20,8 +20,8 @@ from . import _lib
 from .masks import TreeMask
 
 # kernel tuning variant handed to the library (0 = its default choice: eight waves, the two heads of a GQA pair per work item, where
-# a group is even; 1 = one head per work item, four waves; 2 = four waves with two heads each, head dim <= 128; 3 is set by
-# tree_attn itself where head dim 128 goes to the kernel with decoupled waves); results do not depend on it
+# a group is even; 1 = one head per work item, four waves; 2 = four waves with two heads each, head dim <= 128; 3, 4 and 5 are set by
+# tree_attn itself where a call goes to the decoupled kernel at head dim 128, the spread or the pipelined kernel); results do not depend on it
 VARIANT = int(os.environ.get("SPINF_ATTN_VARIANT", "0"))
 # the kernel with decoupled waves over a static schedule, where the library has one for the geometry (0: the lockstep kernels only)
 RING = int(os.environ.get("SPINF_ATTN_RING", "-1"))      # -1 = auto
@@ -32,6 +32,7 @@ STATIC = int(os.environ.get("SPINF_ATTN_STATIC", "-1"))  # -1 = auto
 
 
 RING_MAX_ITEMS_PER_WG = 8
+PIPE_MIN_ITEMS_PER_WG = 12
 # head dim 128: the kernel with decoupled waves over 64-key tiles (the library's variant 3) where the geometry allows
 RING_128 = False
 
@@ -89,6 +90,13 @@ def _ring_lists(device, hq, hkv, d, variant, compact, mask):
     if ring or static:
         return n_wg, ring
     return 0, False
+
+
+def _pipelined(hq, d, n_wg, mask) -> bool:
+    """does a call of head dim 512 that would go to the kernel with decoupled waves go to the pipelined one (variant 5; same bits)?  Measured
+    on MI355X, global layers of 16 query heads over one key / value head: 13.5 items per workgroup 554 us against 610 - 621, 32 items 2.06 ms
+    against 2.16 - 2.28.  Fewer items, and layers with a window, were not compared: they stay where they were."""
+    return d == 512 and RING < 0 and not mask.window and mask.n_qtiles * hq >= PIPE_MIN_ITEMS_PER_WG * n_wg
 
 
 def _spread(device, hq, hkv, d, variant, mask) -> bool:
@@ -182,6 +190,8 @@ class _Layer:
             n_lists, ring = _ring_lists(device, hq, hkv, d, variant, compact, mask)
         if ring and d == 128:
             variant = 3   # (64-key plan entries, as the lockstep kernels take)
+        elif ring and _pipelined(hq, d, n_lists, mask):
+            variant = 5   # on the decoupled kernel's schedule
         self.ring = ring and d != 128
         m = mask.for_head_dim(d, ring=self.ring)
         per_item = _lib.load_library().spinf_attn_heads_per_item(hq, hkv, d, variant)

@@ -609,6 +609,39 @@ def test_head_dim_512_kernel_choices_give_the_same_bits(dev, window, monkeypatch
     assert float(np.abs(outs[1][sl].float().cpu().numpy() - ref).max()) <= TOL
 
 
+@pytest.mark.parametrize("lists", [None, 3, 1])
+@pytest.mark.parametrize("cut,wide", [(0, 1.0), (108, 1.0), (37, 60.0)])
+def test_pipelined_kernel_gives_the_lockstep_bits(dev, lists, cut, wide, monkeypatch):
+    """head dim 512: the pipelined kernel (variant 5) against the lockstep kernel, bit for bit, where its walk over the work items can go
+    wrong: items of one tile (20 rows, cut 108) and of 80 (more than a chunk of entries), more items in a list than are held in LDS (192 in one), a stream
+    that ends inside a query tile and a key tile, and scores that send items to the exact recomputation"""
+    from spinf_serve_amd import attention
+
+    rng = np.random.default_rng(23)
+    trees = [synth._tree(rng, 2400, [30, 11]), synth._tree(rng, 1, [3]), synth._tree(rng, 150, [9, 40]), synth._tree(rng, 70, [])]
+    cfg = synth.AttnConfig("pipe", 8, 1, 512, 512 ** -0.5, 1.0, None, trees)
+    b = synth.pack(trees)[0]
+    n = b.length - cut
+    q, k, v = (t[:n].contiguous() for t in synth.qkv(cfg, b, seed=8, device=dev))
+    k[200:280] *= wide
+    mask = sa.TreeMask.build(b.art[:n], np.minimum(b.end[:n], n), b.pos[:n], device=dev)
+    print(f"case pipelined n={n} lists={lists} wide={wide}", flush=True)
+    monkeypatch.setattr(attention, "RING", 0)
+    want = sa.tree_attn(q, k, v, mask, cfg.scale)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(attention, "RING", -1)
+    before = _exact_items()
+    if lists is None:
+        got = sa.tree_attn(q, k, v, mask, cfg.scale, variant=5)
+    else:
+        m = mask.for_head_dim(512)
+        items, list_ptr, n_items = m.schedule(8, lists)
+        got = attention._tree_attn_op(q, k, v, m.art, m.end, m.pos, m.kv_idx, m.kv_bits, items, list_ptr, n_items, cfg.scale, 0, 5, None, None, 0, None, 0, 32, lists)
+    torch.cuda.synchronize()
+    assert (_exact_items() > before) == (wide > 1)
+    assert torch.equal(got, want), float((got.float() - want.float()).abs().max())
+
+
 def test_calls_on_two_streams_do_not_share_cursors(dev):
     """calls interleaved on two streams, not synchronised with each other, give the bits of the same calls one after the other"""
     cfgs = [synth.attention_config("C2", seed=s, contents=4 + 3 * s) for s in range(2)]
