@@ -659,6 +659,49 @@ def test_tileplan_is_exact_on_random_forests():
     run()
 
 
+@pytest.mark.parametrize("window", [None, 1, 64, 127, 128, 129, 190, 191, 192, 193, 255, 256, 320])
+def test_tile_pairs_settled_as_a_whole(window):
+    """trunks of several query tiles: pairs of tiles that are wholly visible, wholly hidden (ended subtrees, behind the window) or just not so
+    (windows around multiples of the tile sizes, a subtree that ends inside a query tile, a second job, a stream cut inside a tile), against
+    the dense mask at both key-tile sizes"""
+    s = pack_stream([Job([1] * 700, [[2] * 200, [3] * 130, [4] * 5]), Job([5] * 128, [[6] * 256]), Job([7] * 300, [])])
+    for n in (len(s.art), len(s.art) - 100):
+        art, end, pos = s.art[:n], np.minimum(s.end[:n], n), s.pos[:n]
+        p64 = _check_plan(art, end, pos, window)
+        p32 = sa.TilePlan.build(art, end, pos, window, ktile=32)
+        for t in range(p64.n_qtiles):
+            want = {}
+            for e in range(p64.qt_ptr[t], p64.qt_ptr[t + 1]):
+                for half in range(2):
+                    if int(p64.kv_bits[e]) >> half & 0x55:
+                        want[2 * int(p64.kv_idx[e]) + half] = int(p64.kv_bits[e]) >> half & 0x5555
+            assert {int(p32.kv_idx[e]): int(p32.kv_bits[e]) for e in range(p32.qt_ptr[t], p32.qt_ptr[t + 1])} == want
+
+
+@pytest.mark.parametrize("head_groups,n_lists", [(1, 1), (8, 5), (8, 8), (3, 20), (8, 256)])
+def test_static_schedule_is_the_simulation(head_groups, n_lists):
+    """an item goes to the workgroup of its XCD's list that is free first, the lowest numbered of equals, in single precision"""
+    import heapq
+
+    b = synth.attention_config("C2", contents=7).batches[0]
+    plan = sa.TilePlan.build(b.art, b.end, b.pos, None, ktile=32)
+    items, lp = plan.schedule(head_groups)
+    nl = min(8, n_lists)
+    free = [[(np.float32(0), w) for w in range(n_lists) if w % nl == l] for l in range(nl)]
+    want = [[] for _ in range(n_lists)]
+    for l in range(8):
+        for i in range(lp[l], lp[l + 1]):
+            bits = [int(x) for x in plan.kv_bits[items[i, 1] : items[i, 1] + (items[i, 2] & 0xFFFFF)]]
+            mask = [x & x >> 8 for x in bits]
+            most = max(sum(bin(x & pair).count("1") for x in mask) for pair in (0x41, 0x14))
+            cost = np.float32(np.float32(3.2) + np.float32(sum(x & 0x55 != 0 for x in bits)) + np.float32(0.3) * np.float32(most))
+            at, w = heapq.heappop(free[l % nl])
+            want[w].append(tuple(items[i]))
+            heapq.heappush(free[l % nl], (np.float32(at + cost), w))
+    got, ptr = plan.schedule_static(head_groups, n_lists)
+    assert [[tuple(r) for r in got[ptr[w] : ptr[w + 1]]] for w in range(n_lists)] == want
+
+
 def test_static_schedule_deals_every_item_out_once():
     """the static schedule: the same items as the queue's lists, regrouped into one list per workgroup; workgroup b serves XCD
     b % 8 (its items come from that XCD's list, in that list's order); lists are balanced under the cost model"""
