@@ -22,7 +22,7 @@
 // Nothing but products and their beside-work may stand in a phase: a scalar branch between two products costs ~30 clocks (requests handed out
 // by a branch per product: 2.79 ms against 2.12 on 65,536 tokens), and bookkeeping ahead of a phase's first product is not under anything.
 //
-// Measured: 24 contents of 470 tokens with 56 questions (28,672 tokens, 16 / 1 heads, 13.5 items a workgroup) 554 us, the ring kernel 610 - 621 in
+// Measured: 24 contents of 470 tokens with 56 questions (28,672 tokens, 16 / 1 heads, 14 items a workgroup) 554 us, the ring kernel 610 - 621 in
 // turns with it; 65,536 tokens (32 items a workgroup) 2.06 ms with clock stamps in, the ring kernel 2.16 - 2.28.  A tile takes 5.0 k clocks
 // of 2.05 k products: A 1.5, B 2.8, waits for the other waves 0.7.  What bounds it now: the issue of everything that stands behind the
 // products of one wave.  Timing-only builds on the 65,536 tokens: without exponentials 1.98 ms; an earlier form of this kernel 2.03 - 2.14, without

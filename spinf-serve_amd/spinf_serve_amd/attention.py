@@ -94,7 +94,7 @@ def _ring_lists(device, hq, hkv, d, variant, compact, mask):
 
 def _pipelined(hq, d, n_wg, mask) -> bool:
     """does a call of head dim 512 that would go to the kernel with decoupled waves go to the pipelined one (variant 5; same bits)?  Measured
-    on MI355X, global layers of 16 query heads over one key / value head: 13.5 items per workgroup 554 us against 610 - 621, 32 items 2.06 ms
+    on MI355X, global layers of 16 query heads over one key / value head: 14 items per workgroup 554 us against 610 - 621, 32 items 2.06 ms
     against 2.16 - 2.28.  Fewer items, and layers with a window, were not compared: they stay where they were."""
     return d == 512 and RING < 0 and not mask.window and mask.n_qtiles * hq >= PIPE_MIN_ITEMS_PER_WG * n_wg
 
