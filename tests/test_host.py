@@ -214,6 +214,16 @@ def test_build_scan_of_the_ring_assembly_catches_what_it_is_there_for():
     with pytest.raises(RuntimeError, match="spills 16"):
         ge._scan_ring_assembly(meta)
     ge._scan_ring_assembly([meta[0], "    .vgpr_spill_count: 2"])
+    # the pipelined kernel: no reload from scratch in a block with products, whichever comes first; a message names the file it is about
+    pipe = ["_ZN12_GLOBAL__N_121tree_attn_pipe_kernelILi512EEEv10AttnParams: ; @kernel", ".LBB0_7:    ;   in Loop: Header=BB0_3 Depth=2"]
+    mfma, reload = ["\tv_mfma_f32_32x32x16_bf16 v[0:15], v[20:23], v[24:27], v[0:15]"], ["\tscratch_load_dword v40, off, off offset:16"]
+    for body in (reload + mfma, mfma + reload):
+        with pytest.raises(RuntimeError, match=r"tree_attn_pipe\.s:4: a reload from scratch among the products"):
+            ge._scan_ring_assembly(pipe + body, "tree_attn_pipe.s")
+    ge._scan_ring_assembly(pipe + reload + [".LBB0_8:"] + mfma, "tree_attn_pipe.s")
+    for bad, what in ((["\tv_accvgpr_read_b32 v3, a255"], "assembly owns"), (meta, "spills 16")):
+        with pytest.raises(RuntimeError, match=r"^other\.s.*" + what):
+            ge._scan_ring_assembly(pipe + bad, "other.s")
 
 
 # ------------------------------------------------------------------------------------------------ stream layout
