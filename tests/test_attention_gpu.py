@@ -642,6 +642,75 @@ def test_pipelined_kernel_gives_the_lockstep_bits(dev, lists, cut, wide, monkeyp
     assert torch.equal(got, want), float((got.float() - want.float()).abs().max())
 
 
+@pytest.mark.parametrize("wide", [1.0, 60.0])
+@pytest.mark.parametrize("layout", ["one projection", "heads first"])
+def test_pipelined_kernel_with_several_key_heads_and_strides(dev, layout, wide, monkeypatch):
+    """head dim 512: the pipelined kernel (variant 5) against the lockstep kernel, bit for bit, with the key / value head of an item (three of
+    them, two query heads each) and the strides of q, k and v not those of contiguous tensors: q, k, v as parts of one projection's rows, and
+    k, v (strides apart from each other) with the heads outside; narrow scores and ones that send items to the exact recomputation"""
+    from spinf_serve_amd import attention
+
+    rng = np.random.default_rng(29)
+    trees = [synth._tree(rng, 700, [30, 11]), synth._tree(rng, 90, [9, 40]), synth._tree(rng, 1, [3])]
+    cfg = synth.AttnConfig("pipe heads", 6, 3, 512, 512 ** -0.5, 1.0, None, trees)
+    b = synth.pack(trees)[0]
+    n = b.length - 45   # (inside a query tile and a key tile)
+    q, k, v = (t[:n].contiguous() for t in synth.qkv(cfg, b, seed=9, device=dev))
+    k[200:280, 1] *= wide   # one key / value head only: the items of the others stay with the kernel
+    if layout == "one projection":
+        rows = torch.cat([q, k, v, torch.full((n, 1, 512), float("nan"), dtype=torch.bfloat16, device=dev)], 1)
+        qs, ks, vs = rows[:, :6], rows[:, 6:9], rows[:, 9:12]
+    else:
+        qs = q.transpose(0, 1).contiguous().transpose(0, 1)
+        ks = k.transpose(0, 1).contiguous().transpose(0, 1)
+        vs = torch.nn.functional.pad(v.transpose(0, 1), (0, 8, 0, 3), value=float("nan"))[:, :n, :512].transpose(0, 1)
+        assert ks.stride() != vs.stride()
+    assert not any(t.is_contiguous() for t in (qs, ks, vs))
+    mask = sa.TreeMask.build(b.art[:n], np.minimum(b.end[:n], n), b.pos[:n], device=dev)
+    print(f"case pipelined heads n={n} {layout} wide={wide}", flush=True)
+    monkeypatch.setattr(attention, "RING", 0)
+    want = sa.tree_attn(q, k, v, mask, cfg.scale)
+    torch.cuda.synchronize()
+    monkeypatch.setattr(attention, "RING", -1)
+    before = _exact_items()
+    got = sa.tree_attn(qs, ks, vs, mask, cfg.scale, variant=5)
+    torch.cuda.synchronize()
+    assert (_exact_items() > before) == (wide > 1)
+    assert torch.equal(got, want), float((got.float() - want.float()).abs().max())
+
+
+def test_pipelined_kernel_takes_the_calls_from_its_line_on(dev, monkeypatch):
+    """head dim 512, nothing forced: from PIPE_MIN_ITEMS_PER_WG work items per workgroup on a global layer's call goes to the pipelined
+    kernel through both entry points, one query tile less and a layer with a window do not; all give the lockstep kernel's bits"""
+    from spinf_serve_amd import attention
+    from spinf_serve_amd.masks import _static_lists
+
+    hq, hkv = 8, 2
+    tiles = -(-attention.PIPE_MIN_ITEMS_PER_WG * _static_lists(dev) // hq)
+    rng = np.random.default_rng(31)
+    trees, have = [], 0
+    while have < tiles:   # contents of one to seven query tiles
+        trees.append(synth._tree(rng, int(rng.integers(20, 800)), [int(x) for x in rng.integers(1, 30, 4)]))
+        have += -(-trees[-1].n_tokens // 128)
+    cfg = synth.AttnConfig("pipe line", hq, hkv, 512, 512 ** -0.5, 1.0, None, trees)
+    b = synth.pack(trees)[0]
+    assert b.length == 128 * have
+    q, k, v = synth.qkv(cfg, b, seed=10, device=dev)
+    for cut, window, variant in ((128 * tiles, None, 5), (128 * (tiles - 1), None, 0), (128 * tiles, 300, 0)):
+        mask = sa.TreeMask.build(b.art[:cut], np.minimum(b.end[:cut], cut), b.pos[:cut], window=window, device=dev)
+        t = [x[:cut] for x in (q, k, v)]
+        print(f"case pipelined line n={cut} window={window}", flush=True)
+        monkeypatch.setattr(attention, "RING", 0)
+        want = sa.tree_attn(*t, mask, cfg.scale)
+        torch.cuda.synchronize()
+        monkeypatch.setattr(attention, "RING", -1)
+        got = sa.tree_attn(*t, mask, cfg.scale)
+        layers = sa.tree_flex_forward(None, *(x.transpose(0, 1)[None] for x in t), mask, cfg.scale)[0][0]
+        torch.cuda.synchronize()
+        assert attention._Layer.of(mask, hq, hkv, 512, 0, False, dev).variant == variant
+        assert torch.equal(got, want) and torch.equal(layers, want)
+
+
 def test_calls_on_two_streams_do_not_share_cursors(dev):
     """calls interleaved on two streams, not synchronised with each other, give the bits of the same calls one after the other"""
     cfgs = [synth.attention_config("C2", seed=s, contents=4 + 3 * s) for s in range(2)]
