@@ -32,7 +32,7 @@ STATIC = int(os.environ.get("SPINF_ATTN_STATIC", "-1"))  # -1 = auto
 
 
 RING_MAX_ITEMS_PER_WG = 8
-PIPE_MIN_ITEMS_PER_WG = 12
+PIPE_MIN_ITEMS_PER_WG = 4
 # head dim 128: the kernel with decoupled waves over 64-key tiles (the library's variant 3) where the geometry allows
 RING_128 = False
 
@@ -93,9 +93,13 @@ def _ring_lists(device, hq, hkv, d, variant, compact, mask):
 
 
 def _pipelined(hq, d, n_wg, mask) -> bool:
-    """does a call of head dim 512 that would go to the kernel with decoupled waves go to the pipelined one (variant 5; same bits)?  Measured
-    on MI355X, global layers of 16 query heads over one key / value head: 14 items per workgroup 554 us against 610 - 621, 32 items 2.06 ms
-    against 2.16 - 2.28.  Fewer items, and layers with a window, were not compared: they stay where they were."""
+    """does a call of head dim 512 that would go to the kernel with decoupled waves go to the pipelined one (variant 5; same bits)?  Only
+    workgroups with a few short items are slower with it.  Measured on MI355X, the two in turns, time of the decoupled kernel over the
+    pipelined one's (16 heads over 1 and 8 over 2; 64 streams of 1,152 to 58,624 tokens; "items" = work items per workgroup): contents of 470
+    tokens and 56 questions 0.94 - 0.96 at 0.3 - 0.6 items, 1.00 - 1.07 at 1.2 - 3, 1.07 - 1.08 at 4, 1.08 - 1.11 from 5 to 28; trunks of
+    60 - 200 tokens with 8 branches 0.92 - 0.98 below 3 items, 1.03 at 4, 1.02 - 1.06 from 5 to 29; trunks of 2,048 1.09 - 1.14 everywhere
+    (0.6 - 28).  So the line is at the fewest items with which all of them win.  Layers with a window are not the pipelined kernel's (it has
+    no window arithmetic)."""
     return d == 512 and RING < 0 and not mask.window and mask.n_qtiles * hq >= PIPE_MIN_ITEMS_PER_WG * n_wg
 
 
