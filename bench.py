@@ -39,7 +39,7 @@ WORKLOADS = {
     "XDEC_long": "extraction-decode attention step: 64 groups x (U{1024..4096}-token prefix + 8 slots with templates of U{8..16} tokens) x 6 beams, 33 generated entries (step 32), 16 / 8 heads, head_dim 256, global layer",
     "XDEC_qwen": "XDEC's step at the Qwen-hybrid attention geometry: 24 query heads / 4 KV heads, head_dim 256 (288 rows per (group, kv head): three row chunks)",
     "XDEC_512": "XDEC's step at the head geometry of the Gemma-4 full-attention layers: 16 query heads / 1 KV head, head_dim 512 (output computed 256 head dims at a time, two launches)",
-    "mfma_valu": "rounds of one v_mfma_f32_32x32x16_bf16 and nv independent vector instructions per wave, one, two and four waves per SIMD: clocks per round of a wave and of its SIMD (spinf_diag_mfma_valu)",
+    "mfma_valu": "rounds of one v_mfma_f32_32x32x16_bf16 and nv independent vector instructions per wave, one, two and four waves per SIMD: clocks per round of a wave and of its SIMD (spinf_diag_mfma_valu); the attention kernels' fragment reads from LDS, alone and behind products (spinf_diag_lds_rate)",
     "mfma_peak": "pure v_mfma_f32_32x32x16_bf16 loop, one workgroup of eight waves on every compute unit, operands in registers: the yardstick for what the matrix cores sustain on this part",
     "LM_head": "lm head of one chunk of 1,024 read rows gathered from a 65,536-row stream: h[sel] W^T (hidden 2,560, vocabulary 262,144, bf16 MFMA, fp32 logits) + soft-capping (30) + log-softmax + 8 option columns in one pass, no logits matrix",
     "LM": "lm head read-out of one chunk of 1,024 read rows: soft-capping (30) + log-softmax over 262,144 fp32 logits + 8 option columns",
@@ -282,6 +282,20 @@ def main():
                 table[f"block-shaped rounds nv={nv} waves_per_simd={wps}"] = {
                     "clocks_per_block_oldest_wave": round(float(simd0[0, 1] - simd0[0, 0]) / (iters // 8), 1),
                     "clocks_per_block_simd": round(float(simd0[:, 1].max() - simd0[:, 0].min()) / ((iters // 8) * wps), 1)}
+        pads = {0: 16, 1: 64}   # the attention kernels' pads of K and V tiles
+        for kind, kname in ((0, "K, ds_read_b128"), (1, "V, ds_read_b64_tr_b16")):
+            for d, ktile in ((128, 64), (256, 64), (256, 32), (512, 32)):
+                for pad, reads in [(pad, 0) for pad in range(0, 129, 16)] + [(pads[kind], r) for r in (1, 2, 3)]:
+                    out = torch.zeros(8, dtype=torch.int64, device=dev)
+                    _lib.check(lib.spinf_diag_lds_rate(kind, d, ktile, pad, reads, 2000, out.data_ptr(), C.c_void_p(torch.cuda.current_stream().cuda_stream)), "spinf_diag_lds_rate")
+                    torch.cuda.synchronize()
+                    t = out.cpu().view(-1, 2)   # the four waves share the LDS: clocks per read = the whole time over all their reads; per round of a wave otherwise
+                    name = f"{kname} head_dim={d} ktile={ktile} pad={pad}"
+                    clocks = float(t[:, 1].max() - t[:, 0].min()) / (2000 * 16)
+                    if reads:
+                        table[f"{name}: one MFMA and {reads} reads"] = {"clocks_per_round": round(clocks, 1)}
+                    else:
+                        table[f"{name}: reads alone"] = {"clocks_per_read": round(clocks / 4, 2)}
         line.update(metric="clocks per MFMA of a SIMD, MFMA + nv vector instructions per round", unit="clocks", value=table["v_fma_f32 nv=6 waves_per_simd=2"]["clocks_per_mfma_simd"],
                     higher_is_better=False, ms_per_step=None, dtype="bf16", config={"workload": WORKLOADS["mfma_valu"], "iters": iters}, table=table)
         print(json.dumps(line))

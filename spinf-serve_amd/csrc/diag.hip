@@ -40,15 +40,16 @@ __global__ __launch_bounds__(512) void mfma_rate_kernel(const long iters, float*
     out[(long)blockIdx.x * blockDim.x + threadIdx.x] = s;   // keeps the loop alive
 }
 
-// ---- do a wave's vector instructions run in the shadow of its own MFMAs?
-// Every wave runs iters x { one v_mfma_f32_32x32x16_bf16 (32 clocks of the matrix pipe) on a single accumulator, then NV vector
-// instructions that depend on nothing the MFMA touches: v_fma_f32 (KIND 0) or v_exp_f32 (KIND 1) }, with one, two or four waves per
-// SIMD (KIND 2: rounds shaped like a 32 x 32 attention block at head dim 128: 8 chained MFMAs, 3 NV v_fma_f32 + NV v_exp_f32, 8 MFMAs
-// on four accumulators).  Every wave of workgroup 0 records the clock before and after its loop (s_memtime ticks, which count core clocks here: the bare
-// MFMA chain reads 32.3 per MFMA).  A round is an iteration of the loop and has the loop's branch in it: one wave per SIMD takes ~44 + 4 NV clocks per
-// round here, but 32.8 with 4 and 35.5 with 6 v_fma_f32 per MFMA when 16 rounds are unrolled into an iteration.  So a wave's vector
-// instructions do run under its own MFMAs, a branch does not; with two waves per SIMD the other wave covers the branch.  Beyond ~6
-// vector instructions per MFMA the vector ALU's issue port is the bound, which is where the attention kernels are at head dim 128.
+// ---- do a wave's vector instructions run under its own MFMAs?
+// Every wave runs iters rounds of { one v_mfma_f32_32x32x16_bf16 (32 clocks of the matrix pipe), the MFMAs going round four accumulators, and NV
+// vector instructions that depend on nothing the MFMAs touch }: v_fma_f32 (KIND 0) or v_exp_f32 (KIND 1), with one, two or four waves per SIMD.
+// 16 rounds are unrolled into an iteration of the loop: a loop's branch does not run under an MFMA, and with one round to an iteration it was what
+// such a yardstick measured (~44 + 4 NV clocks per round of a wave alone).  KIND 2: rounds shaped like a 32 x 32 attention block at head
+// dim 128: 8 chained MFMAs, 3 NV v_fma_f32 + NV v_exp_f32, 8 MFMAs on four accumulators.  Every wave of workgroup 0 records the clock before and
+// after its loop (s_memtime ticks, which count core clocks here: the bare MFMA chain reads 32.0 per MFMA).
+// What comes out: they do run under them, up to 6 v_fma_f32 or 3 v_exp_f32 per MFMA; beyond that the vector ALU's issue port is the bound.
+constexpr int ROUNDS_PER_ITER = 16;
+
 template <int NV, int KIND>
 __global__ __launch_bounds__(1024) void mfma_valu_kernel(const int iters, long long* out) {
     bf16x8 a, b;
@@ -57,22 +58,26 @@ __global__ __launch_bounds__(1024) void mfma_valu_kernel(const int iters, long l
         a[i] = (__bf16)(0.001f * (float)((threadIdx.x + i) & 15));
         b[i] = (__bf16)(0.002f * (float)((threadIdx.x * 3 + i) & 7));
     }
-    f32x16 acc;
+    f32x16 acc;   // (KIND 2: the scores)
+    f32x16 o[4];
 #pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.f;
+    for (int i = 0; i < 16; i++) acc[i] = o[0][i] = o[1][i] = o[2][i] = o[3][i] = 0.f;
     float v[16];
 #pragma unroll
     for (int i = 0; i < 16; i++) v[i] = 0.5f + 0.01f * (float)i + 0.0001f * (float)(threadIdx.x & 63);
     const float c = 0.999f, d = 0.0001f;
     __syncthreads();
     const long long t0 = __builtin_readcyclecounter();
-    f32x16 o[4];   // (KIND 2)
+    auto round = [&](f32x16& to, const int x) __attribute__((always_inline)) {
+        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(to) : "v"(a), "v"(b));
 #pragma unroll
-    for (int n = 0; n < 4; n++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) o[n][i] = 0.f;
-    for (int it = 0; it < iters; it++) {
-        if (KIND == 2) {   // an attention block's phases: 8 chained MFMAs, the softmax's vector instructions, 8 MFMAs on four accumulators
+        for (int j = 0; j < NV; j++) {
+            if (KIND == 0) asm volatile("v_fma_f32 %0, %0, %1, %2" : "+v"(v[(x * NV + j) % 16]) : "v"(c), "v"(d));
+            else asm volatile("v_exp_f32 %0, %0" : "+v"(v[(x * NV + j) % 16]));
+        }
+    };
+    if (KIND == 2) {
+        for (int it = 0; it < iters; it++) {   // an attention block's phases: 8 chained MFMAs, the softmax's vector instructions, 8 MFMAs on four accumulators
 #pragma unroll
             for (int x = 0; x < 8; x++) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
 #pragma unroll
@@ -81,14 +86,13 @@ __global__ __launch_bounds__(1024) void mfma_valu_kernel(const int iters, long l
             for (int j = 0; j < NV; j++) asm volatile("v_exp_f32 %0, %0" : "+v"(v[j % 16]));
 #pragma unroll
             for (int x = 0; x < 8; x++) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(o[x & 3]) : "v"(a), "v"(b));
-            continue;
         }
-        asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(a), "v"(b));
+    } else {
+        for (int it = 0; it < iters / ROUNDS_PER_ITER; it++) {
 #pragma unroll
-        for (int j = 0; j < NV; j++) {
-            if (KIND == 0) asm volatile("v_fma_f32 %0, %0, %1, %2" : "+v"(v[j % 16]) : "v"(c), "v"(d));
-            else asm volatile("v_exp_f32 %0, %0" : "+v"(v[j % 16]));
+            for (int x = 0; x < ROUNDS_PER_ITER; x++) round(o[x & 3], x);
         }
+        for (int it = 0; it < iters % ROUNDS_PER_ITER; it++) round(o[0], 0);
     }
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // the last MFMA's result -> vector ALU reads (assembly: the compiler adds no wait states)
     const long long t1 = __builtin_readcyclecounter();
@@ -97,6 +101,65 @@ __global__ __launch_bounds__(1024) void mfma_valu_kernel(const int iters, long l
     for (int i = 0; i < 16; i++) sum += acc[i] + v[i] + o[0][i] + o[1][i] + o[2][i] + o[3][i];
     if (sum == 12345.678f) out[0] = 0;   // keeps the loop alive (never true)
     if (blockIdx.x == 0 && (threadIdx.x & 63) == 0) {
+        out[2 * (threadIdx.x >> 6)] = t0;
+        out[2 * (threadIdx.x >> 6) + 1] = t1;
+    }
+}
+
+// ---- what do the attention kernels' fragment reads from LDS cost, alone and behind products?
+// One workgroup of four waves over a tile in the attention kernels' layout (attn_tiles.h: nreg regions of 1 KiB, row r in region r % nreg, regions
+// apart by a pad).  KIND 0: the 16-byte reads of 32 K rows, KIND 1: the transposing 8-byte reads of V.  READS 0: 16 reads to an iteration and
+// nothing else; READS 1 .. 3: 16 rounds of { one v_mfma_f32_32x32x16_bf16 on one of four accumulators, READS reads }.  Every wave records the clock
+// before and after its loop.  (A register that a read is in flight to stays the same variable up to the wait behind the loop.)
+typedef __attribute__((ext_vector_type(2))) int rate_i32x2;
+typedef __attribute__((ext_vector_type(4))) int rate_i32x4;
+constexpr int LDS_RATE_PAD = 128, LDS_RATE_REGIONS = 32;
+
+template <int KIND, int READS>
+__global__ __launch_bounds__(256) void lds_rate_kernel(const int iters, const int nreg, const int rowb, const int pitch, long long* out) {
+    __shared__ __attribute__((aligned(16))) char lds[LDS_RATE_REGIONS * (1024 + LDS_RATE_PAD)];
+    for (int i = threadIdx.x; i < (int)sizeof(lds) / 4; i += 256) ((int*)lds)[i] = 0;
+    bf16x8 a, b;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        a[i] = (__bf16)(0.001f * (float)((threadIdx.x + i) & 15));
+        b[i] = (__bf16)(0.002f * (float)((threadIdx.x * 3 + i) & 7));
+    }
+    f32x16 o[4];
+#pragma unroll
+    for (int i = 0; i < 16; i++) o[0][i] = o[1][i] = o[2][i] = o[3][i] = 0.f;
+    rate_i32x4 r[8] = {};
+    rate_i32x2 s[8] = {};
+    const int lane = threadIdx.x & 63;
+    auto off = [&](const int row) { return (row % nreg) * pitch + (row / nreg) * rowb; };
+    const unsigned base = lds_addr(lds);
+    const unsigned at = base + (KIND == 0 ? off(lane & 31) + 16 * (lane >> 5) : off(4 * (lane >> 5) + ((lane >> 2) & 3)) + 32 * ((lane >> 4) & 1) + 8 * (lane & 3));
+    const unsigned at8 = at + off(8);   // (KIND 1: rows 8 .. 15; nreg >= 16)
+    __syncthreads();
+    const long long t0 = __builtin_readcyclecounter();
+    for (int it = 0; it < iters; it++) {
+#pragma unroll
+        for (int x = 0; x < ROUNDS_PER_ITER; x++) {
+            if (READS > 0) asm volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(o[x & 3]) : "v"(a), "v"(b));
+#pragma unroll
+            for (int j = 0; j < (READS > 0 ? READS : 1); j++) {
+                const int y = (READS > 0 ? READS * x + j : x) & 7;
+                if (KIND == 0) asm volatile("ds_read_b128 %0, %1 offset:%2" : "+v"(r[y]) : "v"(at), "n"(32 * y));
+                else asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "+v"(s[y]) : "v"((y & 1) ? at8 : at), "n"(64 * (y >> 1)));
+            }
+        }
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int x = 0; x < 8; x++) asm volatile("" : "+v"(r[x]), "+v"(s[x]));
+    const long long t1 = __builtin_readcyclecounter();
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; i++) sum += o[0][i] + o[1][i] + o[2][i] + o[3][i];
+#pragma unroll
+    for (int x = 0; x < 8; x++) sum += (float)(r[x][0] + s[x][0]);
+    if (sum == 12345.678f) out[0] = 0;   // keeps the loop alive (never true)
+    if ((threadIdx.x & 63) == 0) {
         out[2 * (threadIdx.x >> 6)] = t0;
         out[2 * (threadIdx.x >> 6) + 1] = t1;
     }
@@ -567,5 +630,28 @@ extern "C" int spinf_diag_mfma_rate(int64_t iters, float* out, int64_t out_float
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "diag_mfma_rate: launch: %s", hipGetErrorString(e));
     *flops = (double)wgs * 8 * (double)iters * MFMA_PER_ITER * 2.0 * 32 * 32 * 16;
+    return SPINF_OK;
+}
+
+template <int KIND>
+static void launch_lds_rate(int reads, int iters, int nreg, int rowb, int pitch, long long* out, hipStream_t stream) {
+    switch (reads) {
+        case 0: hipLaunchKernelGGL((lds_rate_kernel<KIND, 0>), dim3(1), dim3(256), 0, stream, iters, nreg, rowb, pitch, out); break;
+        case 1: hipLaunchKernelGGL((lds_rate_kernel<KIND, 1>), dim3(1), dim3(256), 0, stream, iters, nreg, rowb, pitch, out); break;
+        case 2: hipLaunchKernelGGL((lds_rate_kernel<KIND, 2>), dim3(1), dim3(256), 0, stream, iters, nreg, rowb, pitch, out); break;
+        default: hipLaunchKernelGGL((lds_rate_kernel<KIND, 3>), dim3(1), dim3(256), 0, stream, iters, nreg, rowb, pitch, out); break;
+    }
+}
+
+extern "C" int spinf_diag_lds_rate(int32_t kind, int32_t d, int32_t ktile, int32_t pad, int32_t reads, int32_t iters, int64_t* out, void* stream) {
+    if ((d != 128 && d != 256 && d != 512) || (ktile != 32 && ktile != 64) || ktile * d * 2 / 1024 < 16 || ktile * d * 2 / 1024 > LDS_RATE_REGIONS)
+        return spinf_fail(SPINF_E_ARG, "diag_lds_rate: head dim %d with tiles of %d keys: 128 with 64, 256 with 32 or 64, 512 with 32", d, ktile);
+    if (kind < 0 || kind > 1 || pad < 0 || pad > LDS_RATE_PAD || pad % 16 || reads < 0 || reads > 3 || iters <= 0 || iters > (1 << 18) || !out)
+        return spinf_fail(SPINF_E_ARG, "diag_lds_rate: kind in {0, 1}, pad in {0, 16, .. %d}, reads in 0 .. 3, iters in 1 .. 2^18, out not null", LDS_RATE_PAD);
+    const int nreg = ktile * d * 2 / 1024;
+    if (kind == 0) launch_lds_rate<0>(reads, iters, nreg, d * 2, 1024 + pad, (long long*)out, (hipStream_t)stream);
+    else launch_lds_rate<1>(reads, iters, nreg, d * 2, 1024 + pad, (long long*)out, (hipStream_t)stream);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "diag_lds_rate: launch: %s", hipGetErrorString(e));
     return SPINF_OK;
 }

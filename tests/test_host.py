@@ -57,6 +57,10 @@ def test_c_abi_rejects_bad_arguments(lib):
     assert lib.spinf_diag_mfma_valu(4, 3, 2, 100, buf, None) == -1 and b"kind 3" in lib.spinf_last_error()
     assert lib.spinf_diag_mfma_valu(4, 0, 3, 100, buf, None) == -1 and b"waves per SIMD" in lib.spinf_last_error()
     assert lib.spinf_diag_mfma_valu(4, 0, 2, 100, None, None) == -1
+    for bad, what in (((0, 128, 32, 16, 0, 100), b"head dim 128"), ((0, 512, 64, 16, 0, 100), b"head dim 512"), ((2, 256, 64, 16, 0, 100), b"kind"),
+                      ((0, 256, 64, 144, 0, 100), b"pad"), ((0, 256, 64, 8, 0, 100), b"pad"), ((1, 256, 64, 64, 4, 100), b"reads"), ((1, 256, 64, 64, 0, 0), b"iters")):
+        assert lib.spinf_diag_lds_rate(*bad, buf, None) == -1 and what in lib.spinf_last_error()
+    assert lib.spinf_diag_lds_rate(0, 256, 64, 16, 0, 100, None, None) == -1
 
 
 def test_heads_per_item_follows_the_kernel_choice(lib):
