@@ -24,7 +24,7 @@
 // One branch is left, around the row's reference in B: its 16 maxima and lane exchange are wanted once per row, not once per tile.
 //
 // Measured, the ring kernel in turns with it: 24 contents of 470 tokens with 56 questions (28,672 tokens, 16 / 1 heads, 14 items a workgroup)
-// 552 us against 603; 46 contents with trunks around 800 (64,896 tokens, 32 items a workgroup) 2.02 ms against 2.19.  A tile takes 5.0 k clocks
+// 556 - 561 us against 609 - 611; 46 contents with trunks around 800 (64,896 tokens, 32 items a workgroup) 2.02 ms against 2.19.  A tile takes 5.0 k clocks
 // of 2.05 k products: A 1.5, B 2.8, waits for the other waves 0.7 (a build with clock stamps).  What bounds it now: the issue of everything that
 // stands behind the products of one wave; the matrix cores are busy 29 % of the time, 28,672 tokens move 1.33 GB.  Timing-only builds
 // on the longer stream: without exponentials 1.98 ms; an earlier form of this kernel 2.03 - 2.14, without requests 1.72, without V's
