@@ -9,8 +9,8 @@
 // while it does its softmax, asks for a whole tile (67 requests in a row) or polls a flag, the matrix core stands.
 // But a wave's own vector instructions do run under its own products: one product of 32 x 32 x 16 takes 32 clocks of the matrix core,
 // and 4 - 6 fused multiply-adds, 2 exponentials or 2 sixteen-byte LDS reads issued behind it cost next to nothing (32.8 - 35.6, 32.8 and 32.6
-// clocks per product measured, 8 multiply-adds 44: mfma_valu_kernel and lds_rate_kernel in diag.hip).  So the work of a tile is laid out by hand as two phases of 32 products, each product with a
-// piece of the other work behind it (scheduling barriers keep the pieces in place).
+// clocks per product measured, 8 multiply-adds 44: mfma_valu_kernel and lds_rate_kernel in diag.hip).  So the work of a tile is laid out by
+// hand as two phases of 32 products, each product with a piece of the other work behind it (scheduling barriers keep the pieces in place).
 //   A(j)  the scores of tile j, K Q^T; V of tile j is requested, and what B(j) requests is worked out
 //   B(j)  P V of tile j - 1, with mask, softmax and packing of tile j's scores beside it; K and the keys' metadata of tile j + 2 are requested,
 //         tile j + 3 is looked up
@@ -24,11 +24,11 @@
 // One branch is left, around the row's reference in B: its 16 maxima and lane exchange are wanted once per row, not once per tile.
 //
 // Measured, the ring kernel in turns with it: 24 contents of 470 tokens with 56 questions (28,672 tokens, 16 / 1 heads, 14 items a workgroup)
-// 556 - 561 us against 609 - 611; 46 contents with trunks around 800 (64,896 tokens, 32 items a workgroup) 2.02 ms against 2.19.  A tile takes 5.0 k clocks
-// of 2.05 k products: A 1.5, B 2.8, waits for the other waves 0.7 (a build with clock stamps).  What bounds it now: the issue of everything that
-// stands behind the products of one wave; the matrix cores are busy 29 % of the time, 28,672 tokens move 1.33 GB.  Timing-only builds
-// on the longer stream: without exponentials 1.98 ms; an earlier form of this kernel 2.03 - 2.14, without requests 1.72, without V's
-// reads from LDS as well 1.70.
+// 556 - 561 us against 609 - 611; 46 contents with trunks around 800 (64,896 tokens, 32 items a workgroup) 2.02 ms against 2.19.  A tile
+// takes 5.0 k clocks of 2.05 k products: A 1.5, B 2.8, waits for the other waves 0.7 (a build with clock stamps).  What bounds it now: the
+// issue of everything that stands behind the products of one wave; the matrix cores are busy 29 % of the time, 28,672 tokens move
+// 1.33 GB.  Timing-only builds on the longer stream: without exponentials 1.98 ms; an earlier form of this kernel 2.03 - 2.14, without
+// requests 1.72, without V's reads from LDS as well 1.70.
 #include <hip/hip_runtime.h>
 
 #include "attn_acc.h"
