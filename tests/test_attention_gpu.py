@@ -681,7 +681,8 @@ def test_pipelined_kernel_with_several_key_heads_and_strides(dev, layout, wide, 
 
 def test_pipelined_kernel_takes_the_calls_from_its_line_on(dev, monkeypatch):
     """head dim 512, nothing forced: from PIPE_MIN_ITEMS_PER_WG work items per workgroup on a global layer's call goes to the pipelined
-    kernel through both entry points, one query tile less and a layer with a window do not; all give the lockstep kernel's bits"""
+    kernel through both entry points, one query tile less and a layer with a window do not; all give the lockstep kernel's bits, items with
+    too wide a score range among them, and so do the entry point that allocates nothing and the replays of a recorded call"""
     from spinf_serve_amd import attention
     from spinf_serve_amd.masks import _static_lists
 
@@ -696,6 +697,7 @@ def test_pipelined_kernel_takes_the_calls_from_its_line_on(dev, monkeypatch):
     b = synth.pack(trees)[0]
     assert b.length == 128 * have
     q, k, v = synth.qkv(cfg, b, seed=10, device=dev)
+    k[2000:2100, 1] *= 60.0
     for cut, window, variant in ((128 * tiles, None, 5), (128 * (tiles - 1), None, 0), (128 * tiles, 300, 0)):
         mask = sa.TreeMask.build(b.art[:cut], np.minimum(b.end[:cut], cut), b.pos[:cut], window=window, device=dev)
         t = [x[:cut] for x in (q, k, v)]
@@ -704,11 +706,33 @@ def test_pipelined_kernel_takes_the_calls_from_its_line_on(dev, monkeypatch):
         want = sa.tree_attn(*t, mask, cfg.scale)
         torch.cuda.synchronize()
         monkeypatch.setattr(attention, "RING", -1)
+        before = _exact_items()
         got = sa.tree_attn(*t, mask, cfg.scale)
+        torch.cuda.synchronize()
+        assert _exact_items() > before
         layers = sa.tree_flex_forward(None, *(x.transpose(0, 1)[None] for x in t), mask, cfg.scale)[0][0]
         torch.cuda.synchronize()
         assert attention._Layer.of(mask, hq, hkv, 512, 0, False, dev).variant == variant
+        if variant == 5:
+            kept = t, mask, want
         assert torch.equal(got, want) and torch.equal(layers, want)
+        out = torch.full_like(want, float("nan"))
+        sa.tree_attn_noalloc(*t, mask, out, cfg.scale)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    stream, (x, mask, want) = torch.cuda.Stream(device=dev), kept
+    with torch.cuda.stream(stream):
+        sa.tree_attn(*x, mask, cfg.scale)   # (the stream's block exists from here on)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        out = sa.tree_attn(*x, mask, cfg.scale)
+    for _ in range(3):
+        out.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        assert torch.equal(sa.tree_attn(*x, mask, cfg.scale), want)   # eager work in between
 
 
 def test_calls_on_two_streams_do_not_share_cursors(dev):
