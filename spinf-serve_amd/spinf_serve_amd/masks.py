@@ -154,7 +154,8 @@ def _join(shared) -> bool:
         if shared.made is not None:
             stream.wait_event(shared.made)
         elif shared.home is not None:
-            home = torch.cuda.ExternalStream(shared.home)
+            # (the default stream's handle is 0, and of a handle of 0 ExternalStream makes a new stream)
+            home = torch.cuda.ExternalStream(shared.home) if shared.home else torch.cuda.default_stream()
             try:
                 with torch.cuda.stream(home):
                     done = torch.cuda.is_current_stream_capturing()   # (torch waits for the device before a capture begins)

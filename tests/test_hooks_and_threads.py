@@ -3,11 +3,13 @@ recurrent-layer interfaces (spinf_serve/models/gemma4.py:98-119, spinf_serve/mod
 with transformers (gemma4.py:121-122), the plan compilers under threads, and the CPU baseline's fp32 arithmetic against the
 float64 oracle."""
 
+import contextlib
 import copy
 import gc
 import pickle
 import sys
 import threading
+import time
 import types
 
 import numpy as np
@@ -325,6 +327,28 @@ def test_a_call_on_another_stream_waits_for_what_the_first_one_uploaded(monkeypa
     assert call("d", 4, sidx)[1] == [("d", "b"), ("d", None), ("d", "b")]
 
 
+@pytest.mark.parametrize("home", [0, 0x70])
+def test_the_wait_is_for_the_stream_that_uploaded_the_default_stream_too(home, monkeypatch):
+    """the default stream's handle is 0, and torch.cuda.ExternalStream(0) is not that stream: torch takes a handle of 0 for none given and
+    makes a new one (restated here, as on the GPU: its cuda_stream is not 0), which there is nothing to wait for on"""
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream, self.waits = handle, []
+
+        def wait_stream(self, other):
+            self.waits.append(other.cuda_stream)
+
+    here = Stream(0x10)
+    monkeypatch.setattr(torch.cuda, "device", lambda device: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "stream", lambda stream: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: here)
+    monkeypatch.setattr(torch.cuda, "default_stream", lambda: Stream(0))
+    monkeypatch.setattr(torch.cuda, "ExternalStream", lambda handle: Stream(handle or 0x5000))
+    assert masks._join(types.SimpleNamespace(device=None, made=None, home=home, tensors=()))
+    assert here.waits == [home]
+
+
 def test_c1_in_fp32_on_the_cpu_against_the_oracle():
     """the CPU baseline leg (fp32 scaled_dot_product_attention under a dense tree mask per content) and torch's eager
     flex_attention under the same rule agree with the float64 oracle to 1e-5 on C1"""
@@ -512,7 +536,13 @@ def test_layers_of_one_mask_on_two_streams(dev, default):
         torch.cuda._sleep(20_000_000)
         one = sa.tree_attn(q, k, v, mask, cfg.scale)
     with torch.cuda.stream(streams[1]):
-        two = [sa.tree_attn(*few, mask, cfg.scale), sa.tree_attn(q, k, v, mask, cfg.scale)]
+        two = [sa.tree_attn(*few, mask, cfg.scale)]
+        behind = torch.cuda.Event()
+        behind.record()
+        time.sleep(2e-3)   # (longer than that call takes)
+        ran = behind.query()
+        assert not (ran and not streams[0].query()), "the call has run while the stream that uploads what it reads is still busy"
+        two.append(sa.tree_attn(q, k, v, mask, cfg.scale))
         torch.cuda._sleep(20_000_000)
         two.append(sa.tree_attn(*few, mask, cfg.scale))
     buffers = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for x in (*mask._sched.values(), mask._kv) for t in x[-1].tensors}
