@@ -613,6 +613,9 @@ int device_cus(int* cus) {
     return SPINF_OK;
 }
 
+// a new block: cursors, counts and the running totals at [NLIST + 3], [NLIST + 4] start at zero
+__global__ void attn_clear_block_kernel(int* block) { block[threadIdx.x] = 0; }
+
 // -> the stream's block with room for n_items redo entries; *slot names it for release_block
 int acquire_block(long n_items, bool capturing, unsigned long long capture, hipStream_t stream, int** ptr, int* slot, bool* dirty, long* cap) {
     int dev = 0;
@@ -644,8 +647,14 @@ int acquire_block(long n_items, bool capturing, unsigned long long capture, hipS
     b.owner = stream;
     e = hipMalloc((void**)&b.ptr, (64 + b.cap) * sizeof(int));
     if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "tree_attn: hipMalloc: %s", hipGetErrorString(e));
-    e = hipMemset(b.ptr, 0, 64 * sizeof(int));   // cursors, counts and the running totals at [NLIST + 3], [NLIST + 4] start at zero
-    if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "tree_attn: cursor block: %s", hipGetErrorString(e));
+    // Cleared on the block's own stream: hipMemset clears on the default stream and returns at once, and the calls of a stream that does not
+    // wait for that one would find whatever the memory held.
+    hipLaunchKernelGGL(attn_clear_block_kernel, dim3(1), dim3(64), 0, stream, b.ptr);
+    e = hipGetLastError();
+    if (e != hipSuccess) {
+        (void)hipFree(b.ptr);
+        return spinf_fail(SPINF_E_HIP, "tree_attn: launch (cursor block): %s", hipGetErrorString(e));
+    }
     b.taken = true;
     s.blocks.push_back(b);
     *ptr = b.ptr;
@@ -814,6 +823,8 @@ extern "C" int spinf_attn_exact_items(int64_t* total) {
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess || dev < 0 || dev >= 64) return spinf_fail(SPINF_E_HIP, "attn_exact_items: hipGetDevice: %s", hipGetErrorString(e));
     std::lock_guard<std::mutex> lock(g_mu);
+    e = hipDeviceSynchronize();   // (hipMemcpy waits for the default stream only; under the lock: no block is new then)
+    if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "attn_exact_items: hipDeviceSynchronize: %s", hipGetErrorString(e));
     std::vector<const int*> blocks{(const int*)g_scratch[dev].ptr};
     for (const CursorBlock& b : g_dev[dev].blocks) blocks.push_back(b.ptr);
     for (const int* c : blocks) {
@@ -833,6 +844,8 @@ extern "C" int spinf_attn_ring_aborts(int64_t* total) {
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess || dev < 0 || dev >= 64) return spinf_fail(SPINF_E_HIP, "attn_ring_aborts: hipGetDevice: %s", hipGetErrorString(e));
     std::lock_guard<std::mutex> lock(g_mu);
+    e = hipDeviceSynchronize();   // (hipMemcpy waits for the default stream only; under the lock: no block is new then)
+    if (e != hipSuccess) return spinf_fail(SPINF_E_HIP, "attn_ring_aborts: hipDeviceSynchronize: %s", hipGetErrorString(e));
     std::vector<const int*> blocks{(const int*)g_scratch[dev].ptr};
     for (const CursorBlock& b : g_dev[dev].blocks) blocks.push_back(b.ptr);
     for (const int* c : blocks) {

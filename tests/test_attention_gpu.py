@@ -756,6 +756,40 @@ def test_calls_on_two_streams_do_not_share_cursors(dev):
         assert all(torch.equal(o, serial[i]) for o in outs[i])
 
 
+def test_a_streams_first_call_does_not_lean_on_the_default_stream(dev, monkeypatch):
+    """the first call on a stream gets a cursor block that is cleared on that stream: it neither waits for a busy default stream nor reads
+    what a clear behind it would still have to clear (the memory it comes from held something else before)"""
+    import ctypes
+
+    monkeypatch.setattr(attention, "SPREAD", 0)
+    monkeypatch.setattr(attention, "RING", 0)   # the kernels that take their items from shared cursors
+    cfg = synth.attention_config("smoke")
+    b = cfg.batches[0]
+    q, k, v = synth.qkv(cfg, b, seed=4, device=dev)
+    mask = sa.TreeMask.build(b.art, b.end, b.pos, device=dev)
+    want = sa.tree_attn(q, k, v, mask, cfg.scale)
+    hip, handle = ctypes.CDLL("libamdhip64.so"), ctypes.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ctypes.byref(handle), 1) == 0   # one that no call has been made on, and that does not wait for the default stream
+    stream = torch.cuda.ExternalStream(handle.value)
+    held = torch.full((64 + 65536,), 1 << 20, dtype=torch.int32, device=dev)
+    torch.cuda.synchronize()
+    del held
+    torch.cuda.empty_cache()
+    with torch.cuda.stream(stream):
+        out = torch.empty_like(want)   # (the memory of the call's result)
+        del out
+        mask.schedule(cfg.hq // 2)     # the wait for what the first call uploaded is over before the default stream is busy
+    torch.cuda.synchronize()
+    torch.cuda._sleep(20_000_000)
+    with torch.cuda.stream(stream):
+        got = sa.tree_attn(q, k, v, mask, cfg.scale)
+        stream.synchronize()
+    busy = not torch.cuda.default_stream().query()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    assert busy, "the call waited for the default stream"
+
+
 def test_groups_of_the_windowed_checkpoint_are_rejected_on_a_global_layer(dev):
     import ctypes as C
 
