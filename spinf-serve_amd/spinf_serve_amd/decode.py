@@ -65,11 +65,21 @@ class XCaches:
         self._plans.clear()
         self._calls.clear()
 
-    def workspace(self, device, nbytes: int) -> torch.Tensor:
+    def __setstate__(self, state):
+        """copied and saved without the workspaces: the next step makes its own, on its stream"""
+        self.__dict__.update(state, _spaces={})
+
+    def workspace(self, device, nbytes: int, stream=None) -> torch.Tensor:
+        """for a launch on the current stream of `device` (its raw handle)"""
         kept = self._spaces.setdefault(device, [])
         if not kept or kept[-1].numel() < nbytes:   # (a smaller one stays: a step in a captured graph may still write to it)
             kept.append(torch.empty(max(nbytes, 2 * kept[-1].numel() if kept else 0), dtype=torch.uint8, device=device))
-        return kept[-1]
+            kept[-1].home = stream
+        space = kept[-1]
+        if space.home != stream and not torch.cuda.is_current_stream_capturing():
+            # (the caller cannot name a buffer it does not know: when the caches go it is not handed out while this stream still writes to it)
+            space.record_stream(torch.cuda.current_stream(device))
+        return space
 
 
 class GroupKV:
@@ -162,13 +172,13 @@ def _xdecode_args(query, kp, vp, pos_p, kt, vt, pos_t, own_t, gk, gv, qpos, step
     return a
 
 
-def _xdecode_run(a, query, workspace):
+def _xdecode_run(a, query, workspace, stream=None):
     G, H, Q, d = query.shape
     out = torch.empty((G, Q, H, d), dtype=torch.bfloat16, device=query.device)
     a.q, (a.q_g, a.q_h, a.q_q, _), a.out = query.data_ptr(), query.stride(), out.data_ptr()
     if workspace is not None:
         a.workspace, a.workspace_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
-    _lib.launch(_lib.load_library().spinf_xdecode_attn_fwd, a, query.device, "spinf_xdecode_attn_fwd")
+    _lib.launch(_lib.load_library().spinf_xdecode_attn_fwd, a, query.device, "spinf_xdecode_attn_fwd", stream)
     return out
 
 
@@ -230,7 +240,9 @@ def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None
         if got is not None and got[0] == where:
             a = _lib.XdecArgs.from_buffer_copy(got[1])   # (kept as bytes: the caches can be copied and saved)
             a.scale, a.window, a.softcap = scale, window, softcap
-            return _xdecode_run(a, query, c.workspace(query.device, got[2]) if got[2] else None)
+            device = query.device
+            stream = _lib.raw_stream(device.index)
+            return _xdecode_run(a, query, c.workspace(device, got[2], stream) if got[2] else None, stream)
     per = 0
     if nsplit is None and li in c._host_len:   # the groups' own lengths are known: split sizes that balance them
         geo = (G, H, gk.shape[1], Q, gk.shape[3], kp.shape[2], c.kt[li].shape[2], d, c.beam)
@@ -241,7 +253,7 @@ def xdecode_attn(query, caches: XCaches, layer_idx: int, scale=None, window=None
     elif nsplit is None:
         nsplit, _ = plan_splits(G, H, gk.shape[1], Q, gk.shape[3], kp.shape[2], c.kt[li].shape[2], d, c.beam)
     nbytes = G * H * Q * nsplit * (d + 2) * 4 if nsplit > 1 else 0
-    work = c.workspace(query.device, nbytes) if nbytes else None
+    work = c.workspace(query.device, nbytes, _lib.raw_stream(query.device.index)) if nbytes else None
     if eager:
         a = _xdecode_args(query, *tensors, int(nsplit), int(per), int(c.beam))
         c._calls[key] = (where, bytes(a), nbytes)

@@ -224,6 +224,28 @@ def test_a_workspace_that_grows_leaves_the_smaller_one_to_the_graphs_that_write_
     assert two is not one and two.numel() >= 200 and c.workspace(cpu, 100) is two and any(w is one for w in c._spaces[cpu])
 
 
+def test_a_workspace_is_named_to_the_allocator_on_other_streams(monkeypatch):
+    """the workspace is made behind the caller's back on the stream of the step that first needs it; a step on another stream names that
+    stream to the allocator, also where the caches were copied or saved in between"""
+    capturing, named = [False], []
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing[0])
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device: "current")
+    monkeypatch.setattr(torch.Tensor, "record_stream", lambda t, stream: named.append((t.data_ptr(), stream)))
+    c, cpu = decode.XCaches(), torch.device("cpu")
+    one = c.workspace(cpu, 100, 1)
+    assert c.workspace(cpu, 100, 1) is one and not named
+    assert c.workspace(cpu, 100, 2) is one and named == [(one.data_ptr(), "current")]
+    two = c.workspace(cpu, 1000, 2)
+    assert c.workspace(cpu, 1000, 2) is two and len(named) == 1
+    capturing[0] = True
+    assert c.workspace(cpu, 1000, 1) is two and len(named) == 1
+    capturing[0] = False
+    for how in (copy.copy, copy.deepcopy, lambda x: pickle.loads(pickle.dumps(x))):
+        other = how(c).workspace(cpu, 10, 1)
+        assert other is not two and other.numel() == 10 and len(named) == 1
+    assert c.workspace(cpu, 1000, 1) is two and named[-1] == (two.data_ptr(), "current")
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("how", [copy.deepcopy, lambda c: pickle.loads(pickle.dumps(c))])
 def test_caches_are_copied_and_saved_after_a_step(dev, how):
