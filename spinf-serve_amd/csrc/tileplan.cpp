@@ -198,14 +198,15 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
             }
             if (B.job == -3) B.job = -2;
         }
-        // image groups: the distinct groups of every block (sorted), the last position of every group
+        // image groups: the distinct groups of every block (sorted), the first and last position of every group
         std::vector<std::vector<int32_t>> bgrp(grp ? nb : 0);
-        std::unordered_map<int32_t, int64_t> glast;
+        std::unordered_map<int32_t, int64_t> gfirst, glast;
         if (grp) {
             for (int64_t i = 0; i < n; i++) {
                 if (grp[i] < 0) continue;
                 std::vector<int32_t>& g = bgrp[i / SPINF_SUB];
                 if (std::find(g.begin(), g.end(), grp[i]) == g.end()) g.push_back(grp[i]);
+                gfirst.emplace(grp[i], i);
                 glast[grp[i]] = i;
             }
             for (auto& g : bgrp) std::sort(g.begin(), g.end());
@@ -224,13 +225,16 @@ extern "C" int spinf_tileplan_build_ktile(const int32_t* art, const int32_t* end
         p->kv_bits.reserve((size_t)nqt * 8);
         for (int64_t t = 0; t < nqt; t++) {
             const int64_t q0 = t * SPINF_QTILE, q1 = std::min<int64_t>(n, q0 + SPINF_QTILE);
-            int64_t lo_key = q0, hi_key = q1;   // keys [lo_key, hi_key) can matter: the rows' jobs so far, and their groups to the end
+            int64_t lo_key = q0, hi_key = q1;   // keys [lo_key, hi_key) can matter: the rows' jobs so far, and their groups (a group may lie in several jobs)
             for (int64_t rb = q0 / SPINF_SUB; rb < nb && blk[rb].lo < q1; rb++) {
                 lo_key = std::min<int64_t>(lo_key, blk[rb].first);
                 if (group[t] < 0) group[t] = blk[rb].lead;
             }
-            for (int64_t q = q0; grp && q < q1; q++)
-                if (grp[q] >= 0) hi_key = std::max(hi_key, glast[grp[q]] + 1);
+            for (int64_t q = q0; grp && q < q1; q++) {
+                if (grp[q] < 0) continue;
+                lo_key = std::min(lo_key, gfirst[grp[q]]);
+                hi_key = std::max(hi_key, glast[grp[q]] + 1);
+            }
             // Most tile pairs are one thing throughout, and settled as a whole: nothing seen (every key's subtree has ended, or lies behind the
             // window, and the tile before the rows), or everything (rows and keys of one job, the keys before the rows and their
             // subtrees to the tile's end, all within the window).  Block by block the tests below say the same.  (One host core, a

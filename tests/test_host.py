@@ -393,6 +393,18 @@ def test_tileplan_with_image_groups_is_exact():
     assert plain.kv_idx[plain.qt_ptr[0] : plain.qt_ptr[1]].tolist() == [0, 1]
 
 
+@pytest.mark.parametrize("window,windowed", [(None, False), (40, False), (40, True)])
+def test_tileplan_with_groups_that_lie_in_several_jobs(window, windowed):
+    """the predicate looks at group numbers alone: a number used in two jobs, or a span over a job's end and its pads, is seen both ways"""
+    s = pack_stream([Job([1] * 300, [[2] * 20]), Job([3] * 100, []), Job([4] * 200, [[5] * 30])], align=True)
+    for spans in ([(250, 420)], [(10, 30), (500, 520)], [(310, 330), (384, 400), (700, 710)]):
+        grp = np.full(len(s.art), -1, np.int32)
+        for a, e in spans:
+            grp[a:e] = 7
+        _check_plan(s.art, s.end, s.pos, window, grp, windowed)
+        _check_plan(s.art, s.end, s.pos, window, np.where(s.art < 0, -1, grp).astype(np.int32), windowed)
+
+
 def test_tileplan_is_exact_on_golden_streams(golden):
     for case in golden["cases"]:
         for b in case["batches"]:
